@@ -60,26 +60,145 @@ __global__ void k_outcnt_from_V(const int32_t* __restrict__ V, int32_t n, double
     out_w[u] = (double)c;
 }
 
-// One thread per row, sequential in CSR order: the summation order of
-// pagerank.cu:308-315.
-__global__ void k_row_out(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
-                          const double* __restrict__ W, int32_t n, double* __restrict__ out_w,
-                          int32_t* __restrict__ outcnt) {
-    const int32_t u = blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= n) return;
+// The weight of arc p as the build counts it (pagerank.cu:308-315): 0 when
+// its endpoint is outside [0, n) or the weight is not finite or negative.
+template <bool HasW>
+__device__ __forceinline__ double arc_weight(const int32_t* __restrict__ E, const double* __restrict__ W, int64_t p,
+                                             int32_t n, int32_t& cnt) {
+    const int32_t v = E[p];
+    if (v < 0 || v >= n) return 0.0;
+    ++cnt;
+    if (!HasW) return 1.0;
+    const double w = W[p];
+    return (!isfinite(w) || w < 0.0) ? 0.0 : w;
+}
+
+// Out-weight and valid out-arc count of every row.  The sum is the one of
+// adding the row's weights one after the other in CSR order (pagerank.cu:308-315),
+// bit for bit.  kOutLanes lanes share a row: they load that many arcs
+// together and each adds them in order (shuffles inside the group), so the
+// only serial part is the chain of additions; one thread walking a row by
+// itself paid a memory latency per arc (95 ns: 7.6 ms for the longest row of
+// an 11M-arc R-MAT graph, 4.3 ms at 8M arcs, whatever the other rows did).
+// Rows longer than kOutLong go to k_row_out_long.
+constexpr int kOutLanes = 8;
+constexpr int32_t kOutLong = 1024;
+template <bool HasW>
+__global__ __launch_bounds__(256) void k_row_out(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
+                                                 const double* __restrict__ W, int32_t n,
+                                                 double* __restrict__ out_w, int32_t* __restrict__ outcnt,
+                                                 int32_t* __restrict__ long_rows, uint32_t* __restrict__ n_long) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (int64_t)n * kOutLanes) return;  // whole groups: 64 is a multiple of kOutLanes
+    const int32_t u = (int32_t)(t / kOutLanes);
+    const int sub = (int)(t % kOutLanes);
+    const int32_t beg = V[u], end = V[u + 1];
+    if (end - beg > kOutLong) {
+        if (sub == 0) long_rows[atomicAdd(n_long, 1u)] = u;
+        return;
+    }
     double s = 0.0;
     int32_t c = 0;
-    const int32_t end = V[u + 1];
-    for (int32_t p = V[u]; p < end; ++p) {
-        const int32_t v = E[p];
-        if (v < 0 || v >= n) continue;
-        double w = W ? W[p] : 1.0;
-        if (!isfinite(w) || w < 0.0) w = 0.0;
-        s += w;
-        ++c;
+    double w = (int64_t)beg + sub < end ? arc_weight<HasW>(E, W, (int64_t)beg + sub, n, c) : 0.0;
+    for (int64_t p = beg; p < end; p += kOutLanes) {
+        const int64_t nx = p + kOutLanes + sub;  // the next arcs are loaded before these are added
+        const double wn = nx < end ? arc_weight<HasW>(E, W, nx, n, c) : 0.0;
+        if (HasW) {
+#pragma unroll
+            for (int j = 0; j < kOutLanes; ++j) s += __shfl(w, j, kOutLanes);
+        }
+        w = wn;
     }
-    out_w[u] = s;
-    outcnt[u] = c;
+#pragma unroll
+    for (int off = kOutLanes / 2; off > 0; off >>= 1) c += __shfl_xor(c, off, kOutLanes);
+    if (sub == 0) {
+        out_w[u] = HasW ? s : (double)c;
+        outcnt[u] = c;
+    }
+}
+
+// Exponent of the lowest set bit of w > 0 (finite).
+__device__ __forceinline__ int32_t lowest_bit(double w) {
+    const uint64_t b = (uint64_t)__double_as_longlong(w);
+    const int32_t e = (int32_t)((b >> 52) & 0x7ffu);
+    const uint64_t f = b & 0xfffffffffffffull;
+    return e == 0 ? -1074 + (__ffsll((unsigned long long)f) - 1)
+                  : e - 1075 + (__ffsll((unsigned long long)(f | 0x10000000000000ull)) - 1);
+}
+
+// Rows above kOutLong arcs, one workgroup each.  When every partial sum is
+// exact the order does not matter: all weights are multiples of 2^low, so
+// with a total below 2^(low + 53) nothing was rounded (a rounded partial
+// sum is at least that, and sums of non-negative terms never shrink), and
+// the parallel sum is the sequential one.  That holds for unit weights and
+// for weights that came from 32-bit floats.  Other rows are staged through
+// LDS and added in CSR order by one wavefront.
+constexpr int kLongStage = 1024;
+constexpr int kLongBlocks = 1024;
+template <bool HasW>
+__global__ __launch_bounds__(256) void k_row_out_long(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
+                                                      const double* __restrict__ W, int32_t n,
+                                                      double* __restrict__ out_w, int32_t* __restrict__ outcnt,
+                                                      const int32_t* __restrict__ long_rows,
+                                                      const uint32_t* __restrict__ n_long) {
+    __shared__ double stage[2][kLongStage];
+    __shared__ double sh_s[4];
+    __shared__ int32_t sh_c[4], sh_low[4];
+    const int t = threadIdx.x;
+    const uint32_t rows = *n_long;
+    for (uint32_t i = blockIdx.x; i < rows; i += gridDim.x) {
+        const int32_t u = long_rows[i];
+        const int32_t beg = V[u], end = V[u + 1];
+        double s = 0.0;
+        int32_t c = 0, low = 4096;
+        for (int64_t p = (int64_t)beg + t; p < end; p += 256) {
+            const double w = arc_weight<HasW>(E, W, p, n, c);
+            s += w;
+            if (HasW && w > 0.0) low = min(low, lowest_bit(w));
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            s += __shfl_xor(s, off, kWave);
+            c += __shfl_xor(c, off, kWave);
+            low = min(low, __shfl_xor(low, off, kWave));
+        }
+        if (lane_id() == 0) {
+            sh_s[wave_id()] = s;
+            sh_c[wave_id()] = c;
+            sh_low[wave_id()] = low;
+        }
+        __syncthreads();
+        s = (sh_s[0] + sh_s[1]) + (sh_s[2] + sh_s[3]);
+        c = sh_c[0] + sh_c[1] + sh_c[2] + sh_c[3];
+        low = min(min(sh_low[0], sh_low[1]), min(sh_low[2], sh_low[3]));
+        const bool exact = !HasW || low == 4096 || s < ldexp(1.0, low + 53);  // uniform over the workgroup
+        if (!exact) {
+            int32_t dummy = 0;
+            double run = 0.0;
+            for (int32_t q = t; q < kLongStage; q += 256)
+                stage[0][q] = (int64_t)beg + q < end ? arc_weight<HasW>(E, W, (int64_t)beg + q, n, dummy) : 0.0;
+            __syncthreads();
+            int cur = 0;
+            for (int64_t p = beg; p < end; p += kLongStage, cur ^= 1) {
+                if (wave_id() == 0) {  // every lane reads the same entries
+                    const double* st = stage[cur];
+#pragma unroll 16
+                    for (int q = 0; q < kLongStage; ++q) run += st[q];
+                } else {
+                    const int64_t nb = p + kLongStage;
+                    for (int32_t q = t - kWave; q < kLongStage; q += 256 - kWave)
+                        stage[cur ^ 1][q] = nb + q < end ? arc_weight<HasW>(E, W, nb + q, n, dummy) : 0.0;
+                }
+                __syncthreads();
+            }
+            s = run;
+        }
+        if (t == 0) {
+            out_w[u] = s;
+            outcnt[u] = c;
+        }
+        __syncthreads();  // sh_* are reused by the next row
+    }
 }
 
 // deg (0 == dangling), dangling count, max out-degree.
@@ -841,9 +960,11 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
     g.alpha_orig = alpha;
     const auto t_start = std::chrono::steady_clock::now();
 
-    DevBuf ctr;
-    EGX_TRY(ctr.alloc(4 * sizeof(uint32_t)));
-    EGX_HIP_TRY(hipMemsetAsync(ctr.p, 0, 4 * sizeof(uint32_t), s), EGX_DEVICE_ERR);
+    // [0] invalid endpoints, [1] dangling nodes, [2] largest out-degree,
+    // [3] largest in-degree, [4] rows longer than kOutLong
+    DevBuf ctr, long_rows;
+    EGX_TRY(ctr.alloc(5 * sizeof(uint32_t)));
+    EGX_HIP_TRY(hipMemsetAsync(ctr.p, 0, 5 * sizeof(uint32_t), s), EGX_DEVICE_ERR);
 
     EGX_TRY(g.out_w.alloc((size_t)std::max(n, 1) * 8));
     EGX_TRY(g.deg.alloc((size_t)std::max(n, 1) * 4));
@@ -868,11 +989,27 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
     EGX_HIP_TRY(hipMemcpyAsync(&invalid, ctr.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     if (n > 0) {
-        if (!g.weighted && invalid == 0)
+        if (!dW && invalid == 0) {
             k_outcnt_from_V<<<nblocks(n, 256), 256, 0, s>>>(dV, n, g.out_w.as<double>(), outcnt_p);
-        else
-            k_row_out<<<nblocks(n, 64), 64, 0, s>>>(dV, dE, dW, n, g.out_w.as<double>(), outcnt_p);
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        } else {
+            // at most m / kOutLong rows are longer than kOutLong
+            const int64_t max_long = m / kOutLong;
+            EGX_TRY(long_rows.alloc((size_t)std::max<int64_t>(max_long, 1) * 4));
+            int32_t* lr = long_rows.as<int32_t>();
+            uint32_t* nl = ctr.as<uint32_t>() + 4;
+            const unsigned lb = (unsigned)std::min<int64_t>(max_long, kLongBlocks);
+            const unsigned sb = nblocks((int64_t)n * kOutLanes, 256);
+            if (dW) k_row_out<true><<<sb, 256, 0, s>>>(dV, dE, dW, n, g.out_w.as<double>(), outcnt_p, lr, nl);
+            else k_row_out<false><<<sb, 256, 0, s>>>(dV, dE, nullptr, n, g.out_w.as<double>(), outcnt_p, lr, nl);
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+            if (lb > 0) {
+                if (dW) k_row_out_long<true><<<lb, 256, 0, s>>>(dV, dE, dW, n, g.out_w.as<double>(), outcnt_p, lr, nl);
+                else k_row_out_long<false><<<lb, 256, 0, s>>>(dV, dE, nullptr, n, g.out_w.as<double>(), outcnt_p, lr,
+                                                              nl);
+                EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+            }
+        }
         if (g.adjacency) {
             k_unit_out_w<<<nblocks(n, 256), 256, 0, s>>>(g.out_w.as<double>(), n);
             EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);

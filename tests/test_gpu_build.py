@@ -1,0 +1,47 @@
+"""Device build at the edges of its kernels' row and tile sizes, bit for bit against the oracle."""
+import numpy as np
+import pytest
+
+from eggpu_amd import native
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# out-degrees around the lanes per row (8), the long-row limit (1024) and the long rows' staging chunk (1024)
+OUT_LENGTHS = [0, 1, 7, 8, 9, 15, 16, 17, 1023, 1024, 1025, 2047, 2048, 2049, 5000]
+
+
+def _weights(rng, kind, m):
+    if kind == "float32":  # every partial sum exact
+        return rng.uniform(0.1, 1.0, m).astype(np.float32).astype(np.float64)
+    if kind == "wide":  # exponents too far apart for exact sums
+        return np.ldexp(rng.uniform(0.5, 1.0, m), rng.integers(-60, 60, m))
+    if kind == "subnormal":
+        return rng.integers(1, 1 << 20, m) * 5e-324
+    w = rng.uniform(0.1, 2.0, m)
+    if kind == "bad":
+        idx = rng.choice(m, m // 5, replace=False)
+        w[idx] = rng.choice([-1.0, np.nan, np.inf, -np.inf, 0.0, -0.0], len(idx))
+    return w
+
+
+@pytest.mark.parametrize("kind", ["float32", "double", "wide", "subnormal", "bad"])
+@pytest.mark.parametrize("invalid", [False, True])
+def test_out_weight_sums_bit_exact(gpu_ready, kind, invalid):
+    print(f"out weights {kind} invalid={invalid}", flush=True)
+    rng = np.random.default_rng(5)
+    lengths = np.array(OUT_LENGTHS * 3)
+    n = len(lengths)
+    V = np.zeros(n + 1, np.int32)
+    V[1:] = np.cumsum(lengths)
+    m = int(V[-1])
+    E = rng.integers(0, n, m).astype(np.int32)
+    if invalid:
+        E[rng.choice(m, m // 7, replace=False)] = n + 3
+    W = _weights(rng, kind, m)
+    with native.DeviceGraph.from_csr(V, E, W, alpha=0.85) as g:
+        got = g.download_csc()
+    want = O.build_inbound(V, E, W, 0.85)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    assert np.array_equal(got[2].view(np.uint32), want[2].view(np.uint32))
+    assert np.array_equal(got[3], want[3])
