@@ -1,5 +1,6 @@
 // egx_api.hip -- the C ABI declared in include/egx.h.
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cmath>
 #include <cctype>
@@ -80,6 +81,7 @@ hipError_t take_stream(int dev, hipStream_t* s) {
 void give_stream(int dev, hipStream_t s) {
     if (!s) return;
     (void)hipStreamSynchronize(s);
+    pool_stream_idle(s);
     StreamPool& p = stream_pool();
     {
         std::lock_guard<std::mutex> lk(p.mu);
@@ -182,14 +184,15 @@ int graph_from_host_csr(const int32_t* V, const int32_t* E, const double* W, int
     std::unique_ptr<egx_graph> h;
     EGX_TRY(new_graph(h));
     Graph& g = h->g;
+    StreamScope scope(g.stream);
     DevBuf dV, dE, dW;
     EGX_TRY(dV.alloc(((size_t)n + 1) * 4));
     EGX_TRY(dE.alloc((size_t)std::max(m, 1) * 4));
     // pageable copies: a pinned staging arena measured 0.3 ms faster per
     // build at R-MAT 14 but its first allocation (1 MB) took 7-8 ms
-    if (n > 0) EGX_HIP_TRY(hipMemcpy(dV.p, V, ((size_t)n + 1) * 4, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
-    else EGX_HIP_TRY(hipMemset(dV.p, 0, 4), EGX_DEVICE_ERR);
-    if (m > 0) EGX_HIP_TRY(hipMemcpy(dE.p, E, (size_t)m * 4, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
+    if (n > 0) EGX_HIP_TRY(hipMemcpyWithStream(dV.p, V, ((size_t)n + 1) * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
+    else EGX_HIP_TRY(hipMemsetAsync(dV.p, 0, 4, g.stream), EGX_DEVICE_ERR);
+    if (m > 0) EGX_HIP_TRY(hipMemcpyWithStream(dE.p, E, (size_t)m * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
     // weights that are all exactly 1 (the reference's unweighted_W, gen_CSR
     // graph.cpp:881) give the unweighted graph: the same pull CSC bit for bit
     // (in_val = fl32(alpha * (1/outdeg)) either way), iterated by the
@@ -199,7 +202,7 @@ int graph_from_host_csr(const int32_t* V, const int32_t* E, const double* W, int
     const bool upload_w = W && (!unit || keep_csr);
     if (upload_w) {
         EGX_TRY(dW.alloc((size_t)std::max(m, 1) * 8));
-        if (m > 0) EGX_HIP_TRY(hipMemcpy(dW.p, W, (size_t)m * 8, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
+        if (m > 0) EGX_HIP_TRY(hipMemcpyWithStream(dW.p, W, (size_t)m * 8, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
     }
     EGX_TRY(build_from_device_csr(g, dV.as<int32_t>(), dE.as<int32_t>(), (W && !unit) ? dW.as<double>() : nullptr,
                                   n, m, alpha));
@@ -210,6 +213,8 @@ int graph_from_host_csr(const int32_t* V, const int32_t* E, const double* W, int
         g.csr_m = m;
         g.have_csr = true;
     }
+    // the build has waited for its stream
+    for (DevBuf* d : {&dV, &dE, &dW}) d->release_idle();
     out = std::move(h);
     return EGX_SUCC;
 }
@@ -299,6 +304,8 @@ size_t budget_bytes(const ThreadRegistry& r) {
     }
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || total_b == 0) return (size_t)2 << 30;
+    int dev = -1;
+    if (hipGetDevice(&dev) == hipSuccess) free_b += pool_idle_bytes(dev);
     return std::max<size_t>((free_b + resident(r)) / 4, (size_t)256 << 20);
 }
 
@@ -344,6 +351,7 @@ int make_graph(std::unique_ptr<egx_graph>& out) { return new_graph(out); }
 Graph::~Graph() {
     if (device >= 0) (void)hipSetDevice(device);
     if (stream) (void)hipStreamSynchronize(stream);
+    for (DevBuf* b : buffers()) b->release_idle();
     give_state_slot(host_state);
     if (host_result) (void)hipHostFree(host_result);
     if (ev0) (void)hipEventDestroy(ev0);
@@ -351,16 +359,19 @@ Graph::~Graph() {
     give_stream(device, stream);
 }
 
+std::array<DevBuf*, Graph::kBuffers> Graph::buffers() {
+    return {&in_row, &in_col, &in_val, &w_csc,  &out_w,  &out_cnt, &deg,    &csr_V,
+            &csr_E,  &csr_W,  &perm,   &rank,   &p_row,  &p_col,   &p_val,  &p_w,
+            &p_outw, &p_deg,  &p_nval, &tiles,  &t_col,  &t_pos,  &t_val,  &hsegs,
+            &hrows,  &hub_part, &x[0],  &x[1],
+            &s[0],   &s[1],   &state,  &partials, &red_part, &out,    &tele,
+            &pb_src, &pb_dst, &pb_vals, &pb_vgrp, &pb_mask, &pb_scatter, &pb_sum, &pb_hrows,
+            &pb_hub_part, &pb_w, &pb_arc};
+}
+
 size_t Graph::device_bytes() const {
-    const DevBuf* bufs[] = {&in_row, &in_col, &in_val, &w_csc,  &out_w,  &out_cnt, &deg,    &csr_V,
-                            &csr_E,  &csr_W,  &perm,   &rank,   &p_row,  &p_col,   &p_val,  &p_w,
-                            &p_outw, &p_deg,  &p_nval, &tiles,  &t_col,  &t_pos,  &t_val,  &hsegs,
-                            &hrows,  &hub_part, &x[0],  &x[1],
-                            &s[0],   &s[1],   &state,  &partials, &red_part, &out,    &tele,
-                            &pb_src, &pb_dst, &pb_vals, &pb_vgrp, &pb_mask, &pb_scatter, &pb_sum, &pb_hrows,
-                            &pb_hub_part, &pb_w, &pb_arc};
     size_t total = 0;
-    for (const DevBuf* b : bufs) total += b->bytes;
+    for (const DevBuf* b : const_cast<Graph*>(this)->buffers()) total += b->bytes;
     return total;
 }
 
@@ -423,6 +434,7 @@ int egx_graph_rmat_n(int32_t n, int64_t nedges, double a, double b, double c, ui
     *out = nullptr;
     std::unique_ptr<egx_graph> h;
     EGX_TRY(egx::new_graph(h));
+    egx::StreamScope scope(h->g.stream);
     egx::DevBuf V, E;
     int64_t m = 0;
     EGX_TRY(egx::gen_rmat_csr(n, nedges, seed, egx::threshold32(a), egx::threshold32(a + b),
@@ -438,6 +450,7 @@ int egx_graph_er(int32_t n, int64_t nedges, uint64_t seed, int32_t weighted, dou
     *out = nullptr;
     std::unique_ptr<egx_graph> h;
     EGX_TRY(egx::new_graph(h));
+    egx::StreamScope scope(h->g.stream);
     egx::DevBuf V, E;
     int64_t m = 0;
     EGX_TRY(egx::gen_er_csr(n, nedges, seed, V, E, m, h->g.stream));
@@ -483,6 +496,7 @@ int egx_graph_set_bins(egx_graph* gh, const egx_bin_opts* opts) {
     std::lock_guard<std::mutex> lk(g.mu);
     egx::DeviceGuard dg(g.device);
     if (!dg.ok) return EGX_DEVICE_ERR;
+    egx::StreamScope scope(g.stream);
     egx::BinCfg cfg = g.bins;
     if (opts->thread_row_max > 0) cfg.thread_row_max = opts->thread_row_max;
     if (opts->wave_row_max > 0) cfg.wave_row_max = opts->wave_row_max;
@@ -507,6 +521,7 @@ int egx_graph_download_csc(const egx_graph* gh, int32_t* in_row, int32_t* in_col
     std::lock_guard<std::mutex> lk(g.mu);
     egx::DeviceGuard dg(g.device);
     if (!dg.ok) return EGX_DEVICE_ERR;
+    egx::StreamScope scope(g.stream);
     return egx::download_csc(g, in_row, in_col, in_val, dangling01);
 }
 
@@ -574,6 +589,7 @@ int egx_graph_pagerank_ex(egx_graph* gh, const egx_solve_opts* opts, double* PR,
     std::lock_guard<std::mutex> lk(g.mu);
     egx::DeviceGuard dg(g.device);
     if (!dg.ok) return EGX_DEVICE_ERR;
+    egx::StreamScope scope(g.stream);
     egx::SolveStats st;
     int rc = after_launches(egx::solve_pagerank(g, solve_params(opts, flags), PR, &st));
     copy_stats(st, stats);
@@ -590,6 +606,7 @@ int egx_graph_ppr_single(egx_graph* gh, const int32_t* seeds, int32_t nseeds, co
     std::lock_guard<std::mutex> lk(g.mu);
     egx::DeviceGuard dg(g.device);
     if (!dg.ok) return EGX_DEVICE_ERR;
+    egx::StreamScope scope(g.stream);
     std::vector<int32_t> uniq(seeds, seeds + nseeds);
     for (int32_t v : uniq)
         if (v < 0 || v >= g.n) {
@@ -649,6 +666,7 @@ int egx_multi_pagerank(egx_graph* const* graphs, int32_t count, const egx_solve_
         rc = EGX_DEVICE_ERR;
     }
     egx::SolveStats st;
+    egx::StreamScope scope(s);
     if (rc == EGX_SUCC)
         rc = after_launches(egx::solve_pagerank_multi(gs, solve_params(opts, flags), PR, iterations, &st, s, ev0, ev1));
     if (s) (void)hipStreamSynchronize(s);
@@ -756,6 +774,7 @@ int egx_pagerank(const int32_t* V, const int32_t* E, const double* W, int32_t le
 void egx_pagerank_cache_reset(void) {
     egx::ThreadRegistry& r = egx::t_reg;
     r.entries.clear();
+    egx::pool_trim();
     r.owner_device = -1;
     r.clock = 0;
     egx::g_hits = egx::g_misses = egx::g_builds = egx::g_refreshes = egx::g_evictions = 0;

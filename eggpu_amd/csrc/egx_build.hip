@@ -404,7 +404,7 @@ int build_tile_sort(Graph& g, const BinCfg& cfg) {
     if (!cfg.tile_sort || g.n_tiles == 0) return EGX_SUCC;
     hipStream_t s = g.stream;
     int32_t base32 = 0;
-    EGX_HIP_TRY(hipMemcpy(&base32, g.it_row + g.n_hub, 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(&base32, g.it_row + g.n_hub, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     const int64_t base = base32;
     const int64_t mt = g.m - base;
     if (mt <= 0) return EGX_SUCC;
@@ -701,7 +701,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     EGX_TRY(exclusive_scan_u32(soff.as<uint32_t>(), soff.as<uint32_t>(), runs + 1, s));
     std::vector<uint32_t> soff_h((size_t)runs + 1);
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpy(soff_h.data(), soff.p, soff_h.size() * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(soff_h.data(), soff.p, soff_h.size() * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     const int64_t slots = soff_h[(size_t)runs];
     if (slots > INT32_MAX) {
         set_last_error("propagation-blocked layout: too many slots");
@@ -757,7 +757,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     EGX_TRY(exclusive_scan_u32(voff.as<uint32_t>(), voff.as<uint32_t>(), runs + 1, s));
     std::vector<uint32_t> voff_h((size_t)runs + 1);  // bin-major: sub-bin b, chunk c at b*S + c
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpy(voff_h.data(), voff.p, voff_h.size() * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(voff_h.data(), voff.p, voff_h.size() * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     const int64_t nvals = voff_h[(size_t)runs];
     if (nvals > INT32_MAX) {
         set_last_error("propagation-blocked layout: too many value slots");
@@ -776,7 +776,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     int32_t bad_h = 0;
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpy(&bad_h, bad.p, 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(&bad_h, bad.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
 
     // scatter work: contiguous group ranges of at most scat_slots slots per chunk
     // (a graph laid out for shared launches takes the largest items: the set fills the device)
@@ -847,12 +847,12 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     EGX_TRY(g.pb_hrows.alloc(std::max<size_t>(hrows.size(), 1) * sizeof(HubRow)));
     EGX_TRY(g.pb_hub_part.alloc((size_t)std::max<int64_t>(parts, 1) * 8));
     if (!scat.empty())
-        EGX_HIP_TRY(hipMemcpy(g.pb_scatter.p, scat.data(), scat.size() * sizeof(PbScatter), hipMemcpyHostToDevice),
+        EGX_HIP_TRY(hipMemcpyWithStream(g.pb_scatter.p, scat.data(), scat.size() * sizeof(PbScatter), hipMemcpyHostToDevice, s),
                     EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpy(g.pb_sum.p, sums.data(), sums.size() * sizeof(PbSum), hipMemcpyHostToDevice),
+    EGX_HIP_TRY(hipMemcpyWithStream(g.pb_sum.p, sums.data(), sums.size() * sizeof(PbSum), hipMemcpyHostToDevice, s),
                 EGX_DEVICE_ERR);
     if (!hrows.empty())
-        EGX_HIP_TRY(hipMemcpy(g.pb_hrows.p, hrows.data(), hrows.size() * sizeof(HubRow), hipMemcpyHostToDevice),
+        EGX_HIP_TRY(hipMemcpyWithStream(g.pb_hrows.p, hrows.data(), hrows.size() * sizeof(HubRow), hipMemcpyHostToDevice, s),
                     EGX_DEVICE_ERR);
     g.n_pb_scatter = (int64_t)scat.size();
     g.n_pb_sum = (int64_t)sums.size();
@@ -889,7 +889,7 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in) {
     if (n <= 0) return EGX_SUCC;
     std::vector<int32_t> row((size_t)n + 1);
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpy(row.data(), g.it_row, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(row.data(), g.it_row, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
 
     // hub rows [0, n_hub): fixed-size segments
     std::vector<HubSeg> segs;
@@ -914,11 +914,11 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in) {
     g.n_hseg = (int64_t)segs.size();
     EGX_TRY(g.hsegs.alloc(std::max<size_t>(segs.size(), 1) * sizeof(HubSeg)));
     if (!segs.empty())
-        EGX_HIP_TRY(hipMemcpy(g.hsegs.p, segs.data(), segs.size() * sizeof(HubSeg), hipMemcpyHostToDevice),
+        EGX_HIP_TRY(hipMemcpyWithStream(g.hsegs.p, segs.data(), segs.size() * sizeof(HubSeg), hipMemcpyHostToDevice, s),
                     EGX_DEVICE_ERR);
     EGX_TRY(g.hrows.alloc(std::max<size_t>(hub_rows.size(), 1) * sizeof(HubRow)));
     if (!hub_rows.empty())
-        EGX_HIP_TRY(hipMemcpy(g.hrows.p, hub_rows.data(), hub_rows.size() * sizeof(HubRow), hipMemcpyHostToDevice),
+        EGX_HIP_TRY(hipMemcpyWithStream(g.hrows.p, hub_rows.data(), hub_rows.size() * sizeof(HubRow), hipMemcpyHostToDevice, s),
                     EGX_DEVICE_ERR);
     EGX_TRY(g.hub_part.alloc(std::max<size_t>(segs.size(), 1) * 8));
 
@@ -931,7 +931,7 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in) {
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     std::vector<int32_t> ts((size_t)g.n_tiles + 1);
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpy(ts.data(), g.tiles.p, ts.size() * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(ts.data(), g.tiles.p, ts.size() * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     for (int64_t k = 0; k < g.n_tiles; ++k) {
         const int64_t r = ts[(size_t)k + 1] - ts[(size_t)k];
         const int64_t arcs = (int64_t)row[(size_t)ts[(size_t)k + 1]] - row[(size_t)ts[(size_t)k]];
@@ -1077,6 +1077,7 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
         }
     }
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
+    pool_stream_idle(s);
     g.build_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
     return EGX_SUCC;
 }
@@ -1129,7 +1130,7 @@ int build_layout(Graph& g, const BinCfg& cfg) {
     EGX_TRY(radix_sort_u32(keys.as<uint32_t>(), keys_alt.as<uint32_t>(), g.perm.as<uint32_t>(),
                            vals_alt.as<uint32_t>(), n, bits + 1, s));
     uint32_t nh = 0;
-    EGX_HIP_TRY(hipMemcpy(&nh, hubs.p, 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(&nh, hubs.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     keys.release();
     keys_alt.release();
     vals_alt.release();
@@ -1213,13 +1214,13 @@ int download_csc(Graph& g, int32_t* in_row, int32_t* in_col, float* in_val, int3
     hipStream_t s = g.stream;
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     if (in_row)
-        EGX_HIP_TRY(hipMemcpy(in_row, g.in_row.p, ((size_t)g.n + 1) * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyWithStream(in_row, g.in_row.p, ((size_t)g.n + 1) * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     if (in_col && g.m > 0)
-        EGX_HIP_TRY(hipMemcpy(in_col, g.in_col.p, (size_t)g.m * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyWithStream(in_col, g.in_col.p, (size_t)g.m * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     if (in_val && g.m > 0) {
         // values for the alpha of the last build or solve
         if (g.weighted && g.alpha_orig == g.alpha_vals) {
-            EGX_HIP_TRY(hipMemcpy(in_val, g.in_val.p, (size_t)g.m * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+            EGX_HIP_TRY(hipMemcpyWithStream(in_val, g.in_val.p, (size_t)g.m * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
         } else {
             DevBuf tmp;
             EGX_TRY(tmp.alloc((size_t)g.m * 4));
@@ -1232,12 +1233,12 @@ int download_csc(Graph& g, int32_t* in_row, int32_t* in_col, float* in_val, int3
                                                                g.alpha_vals, tmp.as<float>());
             EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
             EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-            EGX_HIP_TRY(hipMemcpy(in_val, tmp.p, (size_t)g.m * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+            EGX_HIP_TRY(hipMemcpyWithStream(in_val, tmp.p, (size_t)g.m * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
         }
     }
     if (dangling01 && g.n > 0) {
         std::vector<float> d((size_t)g.n);
-        EGX_HIP_TRY(hipMemcpy(d.data(), g.deg.p, (size_t)g.n * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyWithStream(d.data(), g.deg.p, (size_t)g.n * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
         for (int32_t i = 0; i < g.n; ++i) dangling01[i] = (d[(size_t)i] == 0.0f) ? 1 : 0;
     }
     return EGX_SUCC;

@@ -44,24 +44,57 @@ void set_last_error(const std::string& msg);
         if (egx_rc_ != EGX_SUCC) return egx_rc_; \
     } while (0)
 
-// A device allocation that frees itself.  Build-time temporaries only; the
+// A device allocation that frees itself.  Inside a StreamScope (or with the
+// stream named) it is taken from, and returned to, the process's block pool
+// (DevPool, egx_prim.hip); otherwise it is hipMalloc'ed and hipFree'd.  The
 // iteration path allocates nothing.
 struct DevBuf {
     void* p = nullptr;
-    size_t bytes = 0;
+    size_t bytes = 0;              // as asked for
+    size_t cap = 0;                // of the pooled block (0: not pooled)
+    int dev = -1;                  // its device
+    hipStream_t stream = nullptr;  // the stream whose order its uses follow
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes) { o.p = nullptr; o.bytes = 0; }
+    DevBuf(DevBuf&& o) noexcept { take(o); }
     DevBuf& operator=(DevBuf&& o) noexcept {
-        if (this != &o) { release(); p = o.p; bytes = o.bytes; o.p = nullptr; o.bytes = 0; }
+        if (this != &o) { release(); take(o); }
         return *this;
     }
     ~DevBuf() { release(); }
-    int alloc(size_t nbytes);
+    int alloc(size_t nbytes);  // on the calling thread's StreamScope stream, if any
+    int alloc(size_t nbytes, hipStream_t s);
     void release();
+    // release() when nothing that uses the buffer is queued or running
+    void release_idle() { stream = nullptr; release(); }
     template <typename T> T* as() const { return static_cast<T*>(p); }
+
+   private:
+    void take(DevBuf& o) {
+        p = o.p; bytes = o.bytes; cap = o.cap; dev = o.dev; stream = o.stream;
+        o.p = nullptr; o.bytes = 0; o.cap = 0; o.dev = -1; o.stream = nullptr;
+    }
 };
+
+// Allocations of the calling thread inside the scope belong to stream s.
+struct StreamScope {
+    explicit StreamScope(hipStream_t s);
+    ~StreamScope();
+    StreamScope(const StreamScope&) = delete;
+    StreamScope& operator=(const StreamScope&) = delete;
+
+   private:
+    hipStream_t prev;
+};
+
+// Everything queued on stream s has finished: its pooled blocks may be used
+// on any stream.  Called before a stream is destroyed or handed on.
+void pool_stream_idle(hipStream_t s);
+// Bytes idle in the pool on device dev.
+size_t pool_idle_bytes(int dev);
+// Give every idle block back to the device.
+void pool_trim();
 
 // ---------------------------------------------------------------------------
 // wave64 reductions

@@ -146,21 +146,22 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
     EGX_TRY(make_graph(h));
     Graph& g = h->g;
     g.adjacency = true;
+    StreamScope scope(g.stream);
     DevBuf dV, dE, dW, dx;
     EGX_TRY(dV.alloc(((size_t)n + 1) * 4));
     EGX_TRY(dE.alloc((size_t)m * 4));
-    EGX_HIP_TRY(hipMemcpy(dV.p, V, ((size_t)n + 1) * 4, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpy(dE.p, E, (size_t)m * 4, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(dV.p, V, ((size_t)n + 1) * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(dE.p, E, (size_t)m * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
     if (W) {
         EGX_TRY(dW.alloc((size_t)m * 8));
-        EGX_HIP_TRY(hipMemcpy(dW.p, W, (size_t)m * 8, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyWithStream(dW.p, W, (size_t)m * 8, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
     }
     EGX_TRY(build_from_device_csr(g, dV.as<int32_t>(), dE.as<int32_t>(), W ? dW.as<double>() : nullptr, n, m, 1.0));
     dV.release();
     dE.release();
     dW.release();
     EGX_TRY(dx.alloc((size_t)n * 8));
-    EGX_HIP_TRY(hipMemcpy(dx.p, x.data(), (size_t)n * 8, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(dx.p, x.data(), (size_t)n * 8, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
 
     SolveParams p;
     p.alpha = 1.0;

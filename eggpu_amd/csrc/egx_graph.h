@@ -34,6 +34,7 @@
 // double buffered, sized for FP64; partials (3 x grid, SoA), hub_part, out.
 #pragma once
 
+#include <array>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -223,6 +224,8 @@ struct Graph {
     char* host_result = nullptr;
 
     ~Graph();
+    static constexpr size_t kBuffers = 46;  // every DevBuf above
+    std::array<DevBuf*, kBuffers> buffers();
     size_t device_bytes() const;
 };
 

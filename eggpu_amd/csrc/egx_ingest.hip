@@ -154,6 +154,7 @@ extern "C" int egx_graph_from_csr_files(const char* offsets_path, const char* in
     EGX_TRY(make_graph(h));
     Graph& g = h->g;
     hipStream_t s = g.stream;
+    StreamScope scope(s);
     DevBuf dV, dE, dW, flags;
     EGX_TRY(dV.alloc(((size_t)n + 1) * 4));
     EGX_TRY(dE.alloc((size_t)std::max(m, 1) * 4));
@@ -176,8 +177,8 @@ extern "C" int egx_graph_from_csr_files(const char* offsets_path, const char* in
 
     // offsets first: the row checks and the build walk them
     int32_t ends[2] = {0, 0};
-    EGX_HIP_TRY(hipMemcpy(&ends[0], dV.p, 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpy(&ends[1], dV.as<int32_t>() + n, 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(&ends[0], dV.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(&ends[1], dV.as<int32_t>() + n, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     if (ends[0] != 0 || ends[1] != m) {
         set_last_error("invalid CSR offsets: first offset must be zero and final offset must equal num_entries");
         return EGX_UNSUPPORTED_GRAPH;

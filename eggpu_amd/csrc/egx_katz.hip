@@ -98,18 +98,19 @@ extern "C" int egx_katz_csr(const int32_t* V, const int32_t* E, int32_t n, int32
         EGX_TRY(make_graph(h));
         Graph& g = h->g;
         g.adjacency = true;
+        StreamScope scope(g.stream);
         DevBuf dV, dE, dB, bias;
         EGX_TRY(dV.alloc(((size_t)n + 1) * 4));
         EGX_TRY(dE.alloc((size_t)m * 4));
-        EGX_HIP_TRY(hipMemcpy(dV.p, Vt.data(), ((size_t)n + 1) * 4, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
-        EGX_HIP_TRY(hipMemcpy(dE.p, Et.data(), (size_t)m * 4, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyWithStream(dV.p, Vt.data(), ((size_t)n + 1) * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyWithStream(dE.p, Et.data(), (size_t)m * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
         EGX_TRY(build_from_device_csr(g, dV.as<int32_t>(), dE.as<int32_t>(), nullptr, n, m, alpha));
         dV.release();
         dE.release();
         EGX_TRY(bias.alloc((size_t)n * 8));
         if (beta) {
             EGX_TRY(dB.alloc((size_t)n * 8));
-            EGX_HIP_TRY(hipMemcpy(dB.p, beta, (size_t)n * 8, hipMemcpyHostToDevice), EGX_DEVICE_ERR);
+            EGX_HIP_TRY(hipMemcpyWithStream(dB.p, beta, (size_t)n * 8, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
         }
         k_katz_bias<<<nblk(n, 256), 256, 0, g.stream>>>(beta ? dB.as<double>() : nullptr, beta_scalar,
                                                          g.reordered ? g.perm.as<int32_t>() : nullptr, n,

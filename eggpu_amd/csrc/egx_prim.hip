@@ -3,16 +3,174 @@
 //
 // Written for gfx950 wave64: the radix rank uses 64-lane ballots to find the
 // lanes that share a digit, so one tile needs no per-thread digit counters.
+#include <algorithm>
+#include <mutex>
+#include <new>
+#include <vector>
+
 #include "egx_common.h"
 
 namespace egx {
 
-int DevBuf::alloc(size_t nbytes) {
+namespace {
+
+// Device blocks of released buffers, kept for the next ones of their size.
+// A graph build allocates and frees some 70 buffers; hipMalloc and hipFree
+// took 13 ms of a 21 ms build and solve of an 11M-arc weighted graph (hipFree
+// waits for the device, 120 us at a time) and 6 ms at 5M arcs.
+//
+// A block that its stream may still be working on (tagged with that
+// stream) goes to a buffer of the same stream only, whose work is queued
+// behind it; once the stream is known to be idle the tag is dropped and any
+// stream may have it.  The allocator itself never waits.  At most kPoolBytes
+// (and kPoolBlocks blocks) stay idle per process (the oldest blocks are freed first, a larger block
+// at once); a failed hipMalloc gives all of them back and tries again, and so
+// does egx_pagerank_cache_reset.
+constexpr size_t kPoolBytes = (size_t)4 << 30;
+constexpr size_t kPoolBlocks = 4096;
+
+struct PoolBlock {
+    void* p;
+    size_t cap;
+    int dev;
+    hipStream_t stream;  // null: idle
+};
+
+struct DevPool {
+    std::mutex mu;
+    std::vector<PoolBlock> idle;  // oldest first
+    size_t bytes = 0;
+};
+
+DevPool& dev_pool() {
+    static DevPool* p = new DevPool();  // never destroyed: buffers may outlive static objects
+    return *p;
+}
+
+thread_local hipStream_t t_alloc_stream = nullptr;
+
+// Block sizes: eight steps per power of two, at least 512 bytes, so that
+// builds of nearly equal graphs share blocks.
+size_t block_size(size_t n) {
+    if (n <= 512) return 512;
+    size_t top = 512;
+    while (top <= n / 2) top *= 2;
+    const size_t step = top / 8;
+    return (n + step - 1) / step * step;
+}
+
+// The smallest fitting block that stream s may use, at most a quarter larger.
+bool pool_take(size_t need, int dev, hipStream_t s, PoolBlock* out) {
+    DevPool& pool = dev_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    size_t best = pool.idle.size();
+    for (size_t i = pool.idle.size(); i-- > 0;) {
+        const PoolBlock& b = pool.idle[i];
+        if (b.dev != dev || b.cap < need || b.cap - need > need / 4 || (b.stream && b.stream != s)) continue;
+        if (best == pool.idle.size() || b.cap < pool.idle[best].cap) best = i;
+        if (b.cap == need) break;
+    }
+    if (best == pool.idle.size()) return false;
+    *out = pool.idle[best];
+    pool.bytes -= out->cap;
+    pool.idle.erase(pool.idle.begin() + (std::ptrdiff_t)best);
+    return true;
+}
+
+void pool_give(const PoolBlock& b) {
+    DevPool& pool = dev_pool();
+    if (b.cap > kPoolBytes / 4) {
+        (void)hipFree(b.p);
+        return;
+    }
+    PoolBlock add = b;
+    for (;;) {
+        PoolBlock drop;  // freed outside the lock: hipFree waits for the device
+        {
+            std::lock_guard<std::mutex> lk(pool.mu);
+            if (add.p && pool.bytes + add.cap <= kPoolBytes && pool.idle.size() < kPoolBlocks) {
+                try {
+                    pool.idle.push_back(add);
+                    pool.bytes += add.cap;
+                    return;
+                } catch (const std::bad_alloc&) {
+                    drop = add;
+                    add.p = nullptr;
+                }
+            } else {
+                // the new block fits once older ones have gone
+                drop = pool.idle.front();
+                pool.bytes -= drop.cap;
+                pool.idle.erase(pool.idle.begin());
+            }
+        }
+        (void)hipFree(drop.p);
+        if (!add.p) return;
+    }
+}
+
+}  // namespace
+
+StreamScope::StreamScope(hipStream_t s) : prev(t_alloc_stream) { t_alloc_stream = s; }
+StreamScope::~StreamScope() { t_alloc_stream = prev; }
+
+void pool_stream_idle(hipStream_t s) {
+    if (!s) return;
+    DevPool& pool = dev_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    for (PoolBlock& b : pool.idle)
+        if (b.stream == s) b.stream = nullptr;
+}
+
+size_t pool_idle_bytes(int dev) {
+    DevPool& pool = dev_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    size_t n = 0;
+    for (const PoolBlock& b : pool.idle) n += b.dev == dev ? b.cap : 0;
+    return n;
+}
+
+void pool_trim() {
+    std::vector<PoolBlock> out;
+    {
+        DevPool& pool = dev_pool();
+        std::lock_guard<std::mutex> lk(pool.mu);
+        out.swap(pool.idle);
+        pool.bytes = 0;
+    }
+    for (const PoolBlock& b : out) (void)hipFree(b.p);
+}
+
+int DevBuf::alloc(size_t nbytes) { return alloc(nbytes, t_alloc_stream); }
+
+int DevBuf::alloc(size_t nbytes, hipStream_t s) {
     release();
     if (nbytes == 0) nbytes = 16;
-    hipError_t e = hipMalloc(&p, nbytes);
+    size_t need = nbytes;
+    if (s) {
+        int d = -1;
+        EGX_HIP_TRY(hipGetDevice(&d), EGX_DEVICE_ERR);
+        need = block_size(nbytes);
+        PoolBlock b;
+        if (pool_take(need, d, s, &b)) {
+            p = b.p;
+            bytes = nbytes;
+            cap = b.cap;
+            dev = d;
+            stream = s;
+            return EGX_SUCC;
+        }
+        dev = d;
+    }
+    hipError_t e = hipMalloc(&p, need);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        pool_trim();  // idle blocks may be what is missing
+        e = hipMalloc(&p, need);
+    }
     if (e != hipSuccess) {
         p = nullptr;
+        dev = -1;
         set_last_error(std::string("hipMalloc(") + std::to_string(nbytes) + "): " + hipGetErrorString(e));
         // the failure is reported here; clear HIP's sticky last error so the
         // next launch check does not report it again (a caller that falls
@@ -21,13 +179,21 @@ int DevBuf::alloc(size_t nbytes) {
         return EGX_FAILED_TO_ALLOCATE_DEVICE_MEM;
     }
     bytes = nbytes;
+    cap = s ? need : 0;
+    stream = s;
     return EGX_SUCC;
 }
 
 void DevBuf::release() {
-    if (p) (void)hipFree(p);
+    if (p) {
+        if (cap) pool_give(PoolBlock{p, cap, dev, stream});
+        else (void)hipFree(p);
+    }
     p = nullptr;
     bytes = 0;
+    cap = 0;
+    dev = -1;
+    stream = nullptr;
 }
 
 namespace {
@@ -126,14 +292,12 @@ int scan_impl(const T* in, T* out, int64_t n, hipStream_t s) {
         return EGX_SUCC;
     }
     DevBuf part;
-    EGX_TRY(part.alloc((size_t)nb * sizeof(T)));
+    EGX_TRY(part.alloc((size_t)nb * sizeof(T), s));  // released in s's order: no wait
     k_scan_reduce<T><<<(unsigned)nb, kScanThreads, 0, s>>>(in, n, part.as<T>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     EGX_TRY(scan_impl<T>(part.as<T>(), part.as<T>(), nb, s));
     k_scan_tile<T><<<(unsigned)nb, kScanThreads, 0, s>>>(in, out, n, part.as<T>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    // part is freed when this returns; the stream must finish using it first.
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     return EGX_SUCC;
 }
 
@@ -233,7 +397,7 @@ int radix_sort_impl(K* keys, K* keys_alt, uint32_t* vals, uint32_t* vals_alt, in
     const int64_t nb64 = (n + kSortTile - 1) / kSortTile;
     const uint32_t nb = (uint32_t)nb64;
     DevBuf counts;
-    EGX_TRY(counts.alloc((size_t)256 * nb * sizeof(uint32_t)));
+    EGX_TRY(counts.alloc((size_t)256 * nb * sizeof(uint32_t), s));
     const bool has_val = vals != nullptr;
     K* kin = keys;
     K* kout = keys_alt;
@@ -260,7 +424,6 @@ int radix_sort_impl(K* keys, K* keys_alt, uint32_t* vals, uint32_t* vals_alt, in
             EGX_HIP_TRY(hipMemcpyAsync(vals, vin, (size_t)n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s),
                         EGX_DEVICE_ERR);
     }
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     return EGX_SUCC;
 }
 

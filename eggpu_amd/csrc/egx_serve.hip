@@ -570,7 +570,7 @@ int egx_server_open(egx_graph* const* pool, int32_t count, const egx_server_opts
             egx::set_last_error(hipGetErrorString(e));
             return EGX_DEVICE_ERR;
         }
-        sv->opts.hbm_budget_bytes = (int64_t)(0.8 * (double)free_b);
+        sv->opts.hbm_budget_bytes = (int64_t)(0.8 * (double)(free_b + egx::pool_idle_bytes(sv->device)));
     }
     sv->stats.budget_bytes = sv->opts.hbm_budget_bytes;
     for (const egx_graph_info& inf : sv->info)

@@ -1003,6 +1003,10 @@ struct Batch {
     ~Batch() {
         if (device >= 0) (void)hipSetDevice(device);
         if (stream) (void)hipStreamSynchronize(stream);
+        for (DevBuf* d : {&X[0], &X[1], &nval, &tslot, &ptab, &cols, &ctl, &partials, &red_part, &hub_part, &hsegs,
+                          &hrows, &wave_rows, &out, &upd})
+            d->release_idle();
+        pool_stream_idle(stream);
         drop_step_graphs();
         if (pinned) (void)hipHostFree(pinned);
         if (arena) (void)hipHostFree(arena);
@@ -1021,7 +1025,7 @@ struct Batch {
 int ensure_nval(Graph& g) {
     const size_t bytes = ((size_t)std::max<int64_t>(g.m, 1) + kArcPad) * 4;
     if (g.p_nval.p && g.p_nval.bytes >= bytes) return EGX_SUCC;
-    EGX_TRY(g.p_nval.alloc(bytes));
+    EGX_TRY(g.p_nval.alloc(bytes, g.stream));  // it outlives the batch that asks for it
     EGX_HIP_TRY(hipMemsetAsync(g.p_nval.as<float>() + g.m, 0, kArcPad * 4, g.stream), EGX_DEVICE_ERR);
     if (g.m > 0) {
         k_nval<<<nblk(g.m, 256), 256, 0, g.stream>>>(g.it_col, g.it_w, g.it_outw, g.m, g.weighted ? 1 : 0,
@@ -1041,6 +1045,7 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
     EGX_HIP_TRY(hipStreamCreate(&b->stream), EGX_DEVICE_ERR);
     EGX_HIP_TRY(hipEventCreate(&b->ev0), EGX_DEVICE_ERR);
     EGX_HIP_TRY(hipEventCreate(&b->ev1), EGX_DEVICE_ERR);
+    StreamScope scope(b->stream);
     const int32_t n = g.n;
     if (n <= 0 || g.m <= 0) {
         set_last_error("batched PageRank needs a graph with nodes and arcs");
@@ -1072,12 +1077,12 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
     if (const char* e = std::getenv("EGGPU_AMD_BATCH_GRAPHS")) b->use_graph = std::strcmp(e, "0") != 0;
     if (g.reordered) {
         b->rank_h.resize((size_t)n);
-        EGX_HIP_TRY(hipMemcpy(b->rank_h.data(), g.rank.p, (size_t)n * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyWithStream(b->rank_h.data(), g.rank.p, (size_t)n * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     }
 
     // hub segments of the SpMM (hub rows are the iteration-layout prefix)
     std::vector<int32_t> row((size_t)g.n_hub + 1);
-    EGX_HIP_TRY(hipMemcpy(row.data(), g.it_row, row.size() * 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(row.data(), g.it_row, row.size() * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     std::vector<HubSeg> segs;
     std::vector<HubRow> hrows;
     for (int32_t v = 0; v < g.n_hub; ++v) {
@@ -1101,17 +1106,17 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
     EGX_TRY(b->hsegs.alloc(std::max<size_t>(segs.size(), 1) * sizeof(HubSeg)));
     EGX_TRY(b->hrows.alloc(std::max<size_t>(hrows.size(), 1) * sizeof(HubRow)));
     if (!segs.empty())
-        EGX_HIP_TRY(hipMemcpy(b->hsegs.p, segs.data(), segs.size() * sizeof(HubSeg), hipMemcpyHostToDevice),
+        EGX_HIP_TRY(hipMemcpyWithStream(b->hsegs.p, segs.data(), segs.size() * sizeof(HubSeg), hipMemcpyHostToDevice, s),
                     EGX_DEVICE_ERR);
     if (!hrows.empty())
-        EGX_HIP_TRY(hipMemcpy(b->hrows.p, hrows.data(), hrows.size() * sizeof(HubRow), hipMemcpyHostToDevice),
+        EGX_HIP_TRY(hipMemcpyWithStream(b->hrows.p, hrows.data(), hrows.size() * sizeof(HubRow), hipMemcpyHostToDevice, s),
                     EGX_DEVICE_ERR);
     EGX_TRY(b->hub_part.alloc(std::max<size_t>(segs.size(), 1) * kCols * 8));
 
     // merge-path split of the other rows: about 8 wavefronts per CU-slot
     int32_t row_end_hub = 0, row_end = 0;
-    EGX_HIP_TRY(hipMemcpy(&row_end_hub, g.it_row + g.n_hub, 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpy(&row_end, g.it_row + n, 4, hipMemcpyDeviceToHost), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(&row_end_hub, g.it_row + g.n_hub, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipMemcpyWithStream(&row_end, g.it_row + n, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     // wavefront k holds the rows whose merge-path diagonal starts in its share
     const int64_t work = (int64_t)(row_end - row_end_hub) + kRowItems * (int64_t)(n - g.n_hub);
     int64_t waves = std::min<int64_t>(16384, std::max<int64_t>(1, (work + 511) / 512));
@@ -1233,6 +1238,7 @@ int batch_set_width(Batch& b, int32_t want) {
     const int64_t total = (int64_t)b.n * want;
     int next;
     if (want > b.cap_cols) {
+        StreamScope scope(s);
         DevBuf nx[2];
         EGX_TRY(nx[0].alloc((size_t)total * 4));
         EGX_TRY(nx[1].alloc((size_t)total * 4));
