@@ -386,6 +386,20 @@ __global__ void k_layout_slots(const int32_t* __restrict__ p_row, const int32_t*
     }
 }
 
+__global__ void k_check_arcs(const int32_t* __restrict__ E, const double* __restrict__ W, int32_t n, int64_t m,
+                             uint32_t* __restrict__ flags) {
+    uint32_t f = 0;
+    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < m; p += (int64_t)gridDim.x * blockDim.x) {
+        const int32_t v = E[p];
+        if (v < 0 || v >= n) f |= kArcBadEndpoint;
+        if (W) {
+            const double w = W[p];
+            if (!isfinite(w) || w < 0.0) f |= kArcBadWeight;
+        }
+    }
+    if (f) atomicOr(flags, f);
+}
+
 __global__ void k_set_last(int32_t* __restrict__ arr, int64_t idx, int32_t value) {
     if (blockIdx.x == 0 && threadIdx.x == 0) arr[idx] = value;
 }
@@ -942,6 +956,35 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in) {
     const int rc = build_blocked(g, cfg, layout_changed);
     if (rc != EGX_SUCC) g.bins.blocked = 0;  // the pull layout stays usable
     return rc;
+}
+
+int check_arcs(const int32_t* dE, const double* dW, int32_t n, int64_t m, uint32_t* flags, hipStream_t s) {
+    EGX_HIP_TRY(hipMemsetAsync(flags, 0, sizeof(uint32_t), s), EGX_DEVICE_ERR);
+    if (m <= 0) return EGX_SUCC;
+    const unsigned blocks = (unsigned)std::min<int64_t>((m + 255) / 256, 4096);
+    k_check_arcs<<<blocks, 256, 0, s>>>(dE, dW, n, m, flags);
+    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    return EGX_SUCC;
+}
+
+int transpose_csr(const int32_t* dV, const int32_t* dE, int32_t n, int64_t m, DevBuf& Vt, DevBuf& Et,
+                  hipStream_t s) {
+    // a stable sort of (head, source) pairs in arc order
+    const size_t mm = (size_t)std::max<int64_t>(m, 1);
+    DevBuf keys, keys_alt, vals_alt;
+    EGX_TRY(keys.alloc(mm * 4, s));
+    EGX_TRY(keys_alt.alloc(mm * 4, s));
+    EGX_TRY(vals_alt.alloc(mm * 4, s));
+    EGX_TRY(Et.alloc(mm * 4, s));
+    EGX_TRY(Vt.alloc(((size_t)n + 1) * 4, s));
+    if (m > 0) {
+        EGX_HIP_TRY(hipMemcpyAsync(keys.p, dE, (size_t)m * 4, hipMemcpyDeviceToDevice, s), EGX_DEVICE_ERR);
+        k_expand_src<<<nblocks(m, 256), 256, 0, s>>>(dV, n, m, Et.as<int32_t>());
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    }
+    EGX_TRY(radix_sort_u32(keys.as<uint32_t>(), keys_alt.as<uint32_t>(), Et.as<uint32_t>(), vals_alt.as<uint32_t>(),
+                           m, bits_for((uint64_t)std::max(n - 1, 0)), s));
+    return lower_bound_iota_u32(keys.as<uint32_t>(), m, Vt.as<int32_t>(), (int64_t)n + 1, s);
 }
 
 // out_w[u] = 1: adjacency values keep alpha * w undivided.

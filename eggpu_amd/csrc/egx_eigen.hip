@@ -55,17 +55,29 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
             set_last_error("invalid CSR offsets: offsets must be monotonic");
             return EGX_UNSUPPORTED_GRAPH;
         }
-    for (int32_t p = 0; p < m; ++p)
-        if (E[p] < 0 || E[p] >= n) {
-            set_last_error("invalid CSR index: endpoint is outside [0, num_nodes)");
-            return EGX_UNSUPPORTED_GRAPH;
-        }
-    if (W)
+    auto bad_endpoint = [] {
+        set_last_error("invalid CSR index: endpoint is outside [0, num_nodes)");
+        return EGX_UNSUPPORTED_GRAPH;
+    };
+    auto bad_weight = [] {
+        set_last_error("eigenvector centrality takes finite, non-negative weights");
+        return EGX_UNSUPPORTED_GRAPH;
+    };
+    // The arcs are checked on the device, once they are there; calls that
+    // end before that check them here.
+    auto host_check = [&]() -> int {
         for (int32_t p = 0; p < m; ++p)
-            if (!std::isfinite(W[p]) || W[p] < 0.0) {
-                set_last_error("eigenvector centrality takes finite, non-negative weights");
-                return EGX_UNSUPPORTED_GRAPH;
-            }
+            if (E[p] < 0 || E[p] >= n) return bad_endpoint();
+        if (W)
+            for (int32_t p = 0; p < m; ++p)
+                if (!std::isfinite(W[p]) || W[p] < 0.0) return bad_weight();
+        return EGX_SUCC;
+    };
+    auto bad_start = [&](const char* what) {
+        EGX_TRY(host_check());
+        set_last_error(what);
+        return (int)EGX_UNSUPPORTED_GRAPH;
+    };
 
     // the normalised start, caller order
     std::vector<double> x((size_t)n);
@@ -73,8 +85,7 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
         double s1 = 0.0;
         for (int32_t v = 0; v < n; ++v) s1 += std::fabs(x0[v]);
         if (!(s1 > 0.0) || !std::isfinite(s1)) {
-            set_last_error("eigenvector centrality: the start vector's absolute sum must be finite and positive");
-            return EGX_UNSUPPORTED_GRAPH;
+            return bad_start("eigenvector centrality: the start vector's absolute sum must be finite and positive");
         }
         for (int32_t v = 0; v < n; ++v) x[(size_t)v] = x0[v] / s1;
     } else {
@@ -82,8 +93,7 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
         for (int32_t v = 0; v < n; ++v) ss += x0[v] * x0[v];
         const double nrm = std::sqrt(ss);
         if (!std::isfinite(nrm)) {
-            set_last_error("eigenvector centrality: the start vector must be finite");
-            return EGX_UNSUPPORTED_GRAPH;
+            return bad_start("eigenvector centrality: the start vector must be finite");
         }
         if (nrm < 1e-12) {
             for (int32_t v = 0; v < n; ++v) x[(size_t)v] = 1.0 / std::sqrt((double)n);
@@ -94,11 +104,11 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
     }
     for (int32_t v = 0; v < n; ++v)
         if (!std::isfinite(x[(size_t)v])) {
-            set_last_error("eigenvector centrality: the start vector must be finite");
-            return EGX_UNSUPPORTED_GRAPH;
+            return bad_start("eigenvector centrality: the start vector must be finite");
         }
 
     if (o.max_iter == 0) {
+        EGX_TRY(host_check());
         std::memcpy(out, x.data(), (size_t)n * 8);
         if (stop) *stop = 2;
         return EGX_SUCC;
@@ -143,11 +153,15 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
     }
 
     std::unique_ptr<egx_graph> h;
-    EGX_TRY(make_graph(h));
+    const int made = make_graph(h);
+    if (made != EGX_SUCC) {
+        EGX_TRY(host_check());
+        return made;
+    }
     Graph& g = h->g;
     g.adjacency = true;
     StreamScope scope(g.stream);
-    DevBuf dV, dE, dW, dx;
+    DevBuf dV, dE, dW, dx, flags;
     EGX_TRY(dV.alloc(((size_t)n + 1) * 4));
     EGX_TRY(dE.alloc((size_t)m * 4));
     EGX_HIP_TRY(hipMemcpyWithStream(dV.p, V, ((size_t)n + 1) * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
@@ -156,6 +170,12 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
         EGX_TRY(dW.alloc((size_t)m * 8));
         EGX_HIP_TRY(hipMemcpyWithStream(dW.p, W, (size_t)m * 8, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
     }
+    uint32_t bad = 0;
+    EGX_TRY(flags.alloc(4));
+    EGX_TRY(check_arcs(dE.as<int32_t>(), W ? dW.as<double>() : nullptr, n, m, flags.as<uint32_t>(), g.stream));
+    EGX_HIP_TRY(hipMemcpyWithStream(&bad, flags.p, 4, hipMemcpyDeviceToHost, g.stream), EGX_DEVICE_ERR);
+    if (bad & kArcBadEndpoint) return bad_endpoint();
+    if (bad & kArcBadWeight) return bad_weight();
     EGX_TRY(build_from_device_csr(g, dV.as<int32_t>(), dE.as<int32_t>(), W ? dW.as<double>() : nullptr, n, m, 1.0));
     dV.release();
     dE.release();

@@ -233,6 +233,15 @@ struct Graph {
 int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const double* dW, int32_t n,
                           int64_t m, double alpha);
 int build_layout(Graph& g, const BinCfg& cfg);
+// Queue the device check of a host CSR's arcs on s: *flags (device, zeroed
+// here) gets kArcBadEndpoint / kArcBadWeight (not finite or negative; dW may
+// be null).
+constexpr uint32_t kArcBadEndpoint = 1u, kArcBadWeight = 2u;
+int check_arcs(const int32_t* dE, const double* dW, int32_t n, int64_t m, uint32_t* flags, hipStream_t s);
+// Queue the transposed arcs of (dV, dE) on s, stable in source order: row v
+// of (Vt, Et) lists the u with u->v.  Endpoints outside [0, n) leave Vt and Et unspecified.
+int transpose_csr(const int32_t* dV, const int32_t* dE, int32_t n, int64_t m, DevBuf& Vt, DevBuf& Et,
+                  hipStream_t s);
 int rebuild_bins(Graph& g, const BinCfg& cfg);
 int refresh_alpha(Graph& g, double alpha);
 int download_csc(Graph& g, int32_t* in_row, int32_t* in_col, float* in_val, int32_t* dangling01);

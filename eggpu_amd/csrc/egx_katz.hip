@@ -10,8 +10,9 @@
 //   no stop within max_iter: RuntimeError;  normalized: x / ||x||_2
 //
 // Row u of A x sums x over u's out-neighbours, so the pull layout is built
-// from the transposed arcs: the device build transposes its input once more,
-// which turns the host transpose back into "row u reads E[V[u]..V[u+1])".
+// from the transposed arcs (one stable radix sort on the device; the host
+// loop that did it took 25 ms of the 31 ms call at 8M draws): the device build transposes its
+// input once more, which turns that back into "row u reads E[V[u]..V[u+1])".
 // The graph is built in adjacency mode (unit weights, out-weight 1 for every
 // node), so the unweighted kernels compute x'[u] = alpha * (sum of x over the
 // row) + b[u] with alpha applied in FP64, as alpha * A @ x + b does; iterates
@@ -38,6 +39,31 @@ __global__ void k_katz_bias(const double* __restrict__ beta, double beta_scalar,
     const int32_t v = perm ? perm[r] : r;
     bias[r] = beta ? beta[v] : beta_scalar;
 }
+
+// ||x||_2 in a fixed order: per-block sums, added again by every block of
+// the scaling launch.
+constexpr int kNormBlocks = 256;
+__global__ __launch_bounds__(256) void k_katz_squares(const double* __restrict__ x, int32_t n,
+                                                      double* __restrict__ part) {
+    __shared__ double sh[12];
+    double s = 0.0, z0 = 0.0, z1 = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)kNormBlocks * 256) s += x[i] * x[i];
+    block_sum3(s, z0, z1, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+__global__ __launch_bounds__(256) void k_katz_scale(const double* __restrict__ part, int32_t n,
+                                                    double* __restrict__ x) {
+    __shared__ double sh[12];
+    __shared__ double norm;
+    double s = part[threadIdx.x], z0 = 0.0, z1 = 0.0;
+    block_sum3(s, z0, z1, sh);
+    if (threadIdx.x == 0) norm = sqrt(s);
+    __syncthreads();
+    if (!(norm > 0.0)) return;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) x[i] /= norm;
+}
+static_assert(kNormBlocks == 256, "k_katz_scale reads one partial sum per thread");
 
 inline unsigned nblk(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
@@ -71,11 +97,10 @@ extern "C" int egx_katz_csr(const int32_t* V, const int32_t* E, int32_t n, int32
             set_last_error("invalid CSR offsets: offsets must be monotonic");
             return EGX_UNSUPPORTED_GRAPH;
         }
-    for (int32_t p = 0; p < m; ++p)
-        if (E[p] < 0 || E[p] >= n) {
-            set_last_error("invalid CSR index: endpoint is outside [0, num_nodes)");
-            return EGX_UNSUPPORTED_GRAPH;
-        }
+    auto bad_endpoint = [] {
+        set_last_error("invalid CSR index: endpoint is outside [0, num_nodes)");
+        return EGX_UNSUPPORTED_GRAPH;
+    };
     auto b_at = [&](int32_t v) { return beta ? beta[v] : beta_scalar; };
     if (m == 0) {
         // x_1 = b; the test after update k compares x_k with x_{k-1}
@@ -86,24 +111,32 @@ extern "C" int egx_katz_csr(const int32_t* V, const int32_t* E, int32_t n, int32
         for (int32_t v = 0; v < n; ++v) out[v] = first ? 1.0 : b_at(v);
         if (iterations) *iterations = first ? 1 : 2;
     } else {
-        // transposed arcs, stable in source order: row v of (Vt, Et) lists the u with u->v
-        std::vector<int32_t> Vt((size_t)n + 1, 0), Et((size_t)m), pos;
-        for (int32_t p = 0; p < m; ++p) Vt[(size_t)E[p] + 1] += 1;
-        for (int32_t v = 0; v < n; ++v) Vt[(size_t)v + 1] += Vt[(size_t)v];
-        pos.assign(Vt.begin(), Vt.end() - 1);
-        for (int32_t u = 0; u < n; ++u)
-            for (int32_t p = V[u]; p < V[u + 1]; ++p) Et[(size_t)pos[(size_t)E[p]]++] = u;
-
         std::unique_ptr<egx_graph> h;
-        EGX_TRY(make_graph(h));
+        int rc = make_graph(h);
+        if (rc != EGX_SUCC) {
+            // without a device an invalid endpoint is still the error to report
+            for (int32_t p = 0; p < m; ++p)
+                if (E[p] < 0 || E[p] >= n) return bad_endpoint();
+            return rc;
+        }
         Graph& g = h->g;
+        hipStream_t s = g.stream;
         g.adjacency = true;
-        StreamScope scope(g.stream);
-        DevBuf dV, dE, dB, bias;
-        EGX_TRY(dV.alloc(((size_t)n + 1) * 4));
-        EGX_TRY(dE.alloc((size_t)m * 4));
-        EGX_HIP_TRY(hipMemcpyWithStream(dV.p, Vt.data(), ((size_t)n + 1) * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
-        EGX_HIP_TRY(hipMemcpyWithStream(dE.p, Et.data(), (size_t)m * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
+        StreamScope scope(s);
+        DevBuf dV, dE, dB, bias, flags, res, part;
+        {
+            DevBuf cV, cE;
+            EGX_TRY(cV.alloc(((size_t)n + 1) * 4));
+            EGX_TRY(cE.alloc((size_t)m * 4));
+            EGX_TRY(flags.alloc(4));
+            EGX_HIP_TRY(hipMemcpyWithStream(cV.p, V, ((size_t)n + 1) * 4, hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
+            EGX_HIP_TRY(hipMemcpyWithStream(cE.p, E, (size_t)m * 4, hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
+            EGX_TRY(check_arcs(cE.as<int32_t>(), nullptr, n, m, flags.as<uint32_t>(), s));
+            EGX_TRY(transpose_csr(cV.as<int32_t>(), cE.as<int32_t>(), n, m, dV, dE, s));
+        }
+        uint32_t bad = 0;
+        EGX_HIP_TRY(hipMemcpyWithStream(&bad, flags.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+        if (bad) return bad_endpoint();
         EGX_TRY(build_from_device_csr(g, dV.as<int32_t>(), dE.as<int32_t>(), nullptr, n, m, alpha));
         dV.release();
         dE.release();
@@ -122,12 +155,24 @@ extern "C" int egx_katz_csr(const int32_t* V, const int32_t* E, int32_t n, int32
         p.tol = tol;
         p.precision = EGX_PRECISION_FP64;
         p.bias = bias.as<double>();
+        EGX_TRY(res.alloc((size_t)n * 8));
+        p.out_device = res.as<double>();
         SolveStats st;
-        EGX_TRY(solve_pagerank(g, p, out, &st));
+        EGX_TRY(solve_pagerank(g, p, nullptr, &st));
         const PrState* hs = static_cast<const PrState*>(g.host_state);
         if (iterations) *iterations = hs->iter;
         if (kernel_seconds) *kernel_seconds = st.kernel_seconds;
-        if (!(hs->err < tol)) return EGX_SUCC;  // stopped by max_iter
+        const bool stopped = hs->err < tol;  // else by max_iter
+        if (stopped && normalized) {
+            EGX_TRY(part.alloc(kNormBlocks * 8));
+            k_katz_squares<<<kNormBlocks, 256, 0, s>>>(res.as<double>(), n, part.as<double>());
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+            k_katz_scale<<<nblk(n, 1024), 256, 0, s>>>(part.as<double>(), n, res.as<double>());
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        }
+        EGX_HIP_TRY(hipMemcpyWithStream(out, res.p, (size_t)n * 8, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+        if (converged) *converged = stopped ? 1 : 0;
+        return EGX_SUCC;
     }
     if (converged) *converged = 1;
     if (normalized) {

@@ -45,3 +45,42 @@ def test_out_weight_sums_bit_exact(gpu_ready, kind, invalid):
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     assert np.array_equal(got[2].view(np.uint32), want[2].view(np.uint32))
     assert np.array_equal(got[3], want[3])
+
+
+@pytest.mark.parametrize("n,m", [(1, 3), (2, 2), (255, 1000), (257, 4096), (65537, 200001)])
+def test_katz_transposes_and_normalises_on_the_device(gpu_ready, n, m):
+    """Unsorted rows with duplicates; sums differ from the oracle's in FP64 order only."""
+    print(f"katz n={n} m={m}", flush=True)
+    rng = np.random.default_rng(n)
+    src = np.sort(rng.integers(0, n, m))
+    E = rng.integers(0, n, m).astype(np.int32)
+    V = np.zeros(n + 1, np.int32)
+    V[1:] = np.cumsum(np.bincount(src, minlength=n))
+    beta = rng.uniform(0.5, 1.5, n)
+    alpha = 0.5 / np.diff(V).max()
+    for normalized in (True, False):
+        got, it, converged, _ = native.katz_csr(V, E, alpha=alpha, beta=beta, normalized=normalized)
+        want, it_ref = O.katz_rows(n, src, E, alpha=alpha, beta=beta, normalized=normalized)
+        assert converged and it == it_ref
+        assert np.abs(got - want).max() <= 1e-12 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("bad", [-1, 300])
+@pytest.mark.parametrize("at", [0, 4999])
+def test_bad_arcs_are_refused(gpu_ready, bad, at):
+    print(f"bad arcs {bad} at {at}", flush=True)
+    rng = np.random.default_rng(3)
+    V = np.linspace(0, 5000, 301).astype(np.int32)
+    E = rng.integers(0, 300, 5000).astype(np.int32)
+    W = rng.uniform(0.1, 1.0, 5000)
+    broken = E.copy()
+    broken[at] = bad
+    for call in (lambda: native.katz_csr(V, broken), lambda: native.eigenvector_csr(V, broken, W),
+                 lambda: native.eigenvector_csr(V, broken, None, max_iter=0)):
+        with pytest.raises(native.EgxError, match="outside"):
+            call()
+    for w in (-1.0, np.nan, np.inf):
+        bad_w = W.copy()
+        bad_w[at] = w
+        with pytest.raises(native.EgxError, match="non-negative weights"):
+            native.eigenvector_csr(V, E, bad_w)
