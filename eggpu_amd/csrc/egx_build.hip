@@ -82,7 +82,7 @@ __device__ __forceinline__ double arc_weight(const int32_t* __restrict__ E, cons
 // an 11M-arc R-MAT graph, 4.3 ms at 8M arcs, whatever the other rows did).
 // Rows longer than kOutLong go to k_row_out_long.
 constexpr int kOutLanes = 8;
-constexpr int32_t kOutLong = 1024;
+constexpr int32_t kOutLong = 256;
 template <bool HasW>
 __global__ __launch_bounds__(256) void k_row_out(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
                                                  const double* __restrict__ W, int32_t n,
@@ -436,8 +436,7 @@ int build_tile_sort(Graph& g, const BinCfg& cfg) {
         k_tile_sort_keys<<<nt, 256, 0, s>>>(g.it_row, g.it_col, g.tiles.as<int32_t>(), keys.as<uint64_t>(),
                                             vals.as<uint32_t>(), base);
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        EGX_TRY(radix_sort_u64(keys.as<uint64_t>(), keys_alt.as<uint64_t>(), vals.as<uint32_t>(),
-                               vals_alt.as<uint32_t>(), mt, 32 + bits_for((uint64_t)g.n_tiles), s));
+        EGX_TRY(radix_sort_u64(keys, keys_alt, &vals, &vals_alt, mt, 32 + bits_for((uint64_t)g.n_tiles), s));
         k_tile_sorted_arrays<<<nt, 256, 0, s>>>(g.it_row, g.tiles.as<int32_t>(), keys.as<uint64_t>(),
                                                 vals.as<uint32_t>(), g.it_val, base, g.t_col.as<int32_t>(),
                                                 g.t_pos.as<uint16_t>(), g.weighted ? g.t_val.as<float>() : nullptr);
@@ -704,8 +703,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
         k_pb_keys<<<nblocks(m, tb), tb, 0, s>>>(g.it_col, rowof.as<int32_t>(), m, B, keys.as<uint32_t>(),
                                                 vals.as<uint32_t>());
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        EGX_TRY(radix_sort_u32(keys.as<uint32_t>(), keys_alt.as<uint32_t>(), vals.as<uint32_t>(),
-                               vals_alt.as<uint32_t>(), m, bits_for((uint64_t)(runs - 1)), s));
+        EGX_TRY(radix_sort_u32(keys, keys_alt, &vals, &vals_alt, m, bits_for((uint64_t)(runs - 1)), s));
     }
     EGX_TRY(lb.alloc((size_t)(runs + 1) * 4));
     EGX_TRY(lower_bound_iota_u32(keys.as<uint32_t>(), m, lb.as<int32_t>(), runs + 1, s));
@@ -982,8 +980,7 @@ int transpose_csr(const int32_t* dV, const int32_t* dE, int32_t n, int64_t m, De
         k_expand_src<<<nblocks(m, 256), 256, 0, s>>>(dV, n, m, Et.as<int32_t>());
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     }
-    EGX_TRY(radix_sort_u32(keys.as<uint32_t>(), keys_alt.as<uint32_t>(), Et.as<uint32_t>(), vals_alt.as<uint32_t>(),
-                           m, bits_for((uint64_t)std::max(n - 1, 0)), s));
+    EGX_TRY(radix_sort_u32(keys, keys_alt, &Et, &vals_alt, m, bits_for((uint64_t)std::max(n - 1, 0)), s));
     return lower_bound_iota_u32(keys.as<uint32_t>(), m, Vt.as<int32_t>(), (int64_t)n + 1, s);
 }
 
@@ -1063,8 +1060,7 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
     }
 
     // stable sort of (dst-or-sentinel, slot-or-src) on the bits that can hold n
-    EGX_TRY(radix_sort_u32(keys.as<uint32_t>(), keys_alt.as<uint32_t>(), vals.as<uint32_t>(),
-                           vals_alt.as<uint32_t>(), m, bits_for((uint64_t)n), s));
+    EGX_TRY(radix_sort_u32(keys, keys_alt, &vals, &vals_alt, m, bits_for((uint64_t)n), s));
     keys_alt.release();
     vals_alt.release();
 
@@ -1170,8 +1166,7 @@ int build_layout(Graph& g, const BinCfg& cfg) {
                                                    cfg.wave_row_max, bits, maxdeg, cfg.reorder,
                                                    keys.as<uint32_t>(), g.perm.as<uint32_t>(), hubs.as<uint32_t>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    EGX_TRY(radix_sort_u32(keys.as<uint32_t>(), keys_alt.as<uint32_t>(), g.perm.as<uint32_t>(),
-                           vals_alt.as<uint32_t>(), n, bits + 1, s));
+    EGX_TRY(radix_sort_u32(keys, keys_alt, &g.perm, &vals_alt, n, bits + 1, s));
     uint32_t nh = 0;
     EGX_HIP_TRY(hipMemcpyWithStream(&nh, hubs.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     keys.release();

@@ -146,13 +146,14 @@ __device__ __forceinline__ void block_sum3(double& a, double& b, double& c, doub
 int exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s);
 int exclusive_scan_i64(const int64_t* in, int64_t* out, int64_t n, hipStream_t s);
 
-// Stable LSD radix sort on bits [0, nbits) of the keys.  Values optional
-// (nullptr).  The sorted result is left in keys/vals; alt buffers are
-// scratch of the same size.
-int radix_sort_u32(uint32_t* keys, uint32_t* keys_alt, uint32_t* vals, uint32_t* vals_alt,
-                   int64_t n, int nbits, hipStream_t s);
-int radix_sort_u64(uint64_t* keys, uint64_t* keys_alt, uint32_t* vals, uint32_t* vals_alt,
-                   int64_t n, int nbits, hipStream_t s);
+// Stable LSD radix sort of n keys on bits [0, nbits), queued on s.  Values
+// (uint32) optional (nullptr).  The sorted arrays are in keys / vals
+// afterwards, which may have changed places with the alt buffers (scratch of
+// the same size).
+int radix_sort_u32(DevBuf& keys, DevBuf& keys_alt, DevBuf* vals, DevBuf* vals_alt, int64_t n, int nbits,
+                   hipStream_t s);
+int radix_sort_u64(DevBuf& keys, DevBuf& keys_alt, DevBuf* vals, DevBuf* vals_alt, int64_t n, int nbits,
+                   hipStream_t s);
 
 // out[i] = number of keys < probe(i) in the sorted array, for i in [0, nprobe):
 // probe(i) = i (u32 keys) or i << shift (u64 keys).

@@ -109,7 +109,7 @@ int keys_to_csr(DevBuf& keys, int64_t nedges, int32_t n, int32_t bits, DevBuf& V
     {
         DevBuf alt;
         EGX_TRY(alt.alloc((size_t)std::max<int64_t>(nedges, 1) * 8));
-        EGX_TRY(radix_sort_u64(keys.as<uint64_t>(), alt.as<uint64_t>(), nullptr, nullptr, nedges, 2 * bits, s));
+        EGX_TRY(radix_sort_u64(keys, alt, nullptr, nullptr, nedges, 2 * bits, s));
     }
     DevBuf flags, pos, ukeys;
     EGX_TRY(flags.alloc((size_t)std::max<int64_t>(nedges, 1) * 4));

@@ -1,11 +1,12 @@
-// egx_prim.hip -- device primitives for the graph build: exclusive scan,
-// stable LSD radix sort (8-bit digits) and lower-bound probes.
+// egx_prim.hip -- device blocks, and device primitives for the graph build:
+// exclusive scan, stable LSD radix sort and lower-bound probes.
 //
 // Written for gfx950 wave64: the radix rank uses 64-lane ballots to find the
 // lanes that share a digit, so one tile needs no per-thread digit counters.
 #include <algorithm>
 #include <mutex>
 #include <new>
+#include <utility>
 #include <vector>
 
 #include "egx_common.h"
@@ -304,127 +305,229 @@ int scan_impl(const T* in, T* out, int64_t n, hipStream_t s) {
 // ---------------------------------------------------------------------------
 // radix sort
 // ---------------------------------------------------------------------------
-constexpr int kSortThreads = 256;
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kSortThreads * kSortItems;
+// Stable LSD, up to kDigitBits bits per pass (the passes share the key bits
+// evenly, so 17 or 18 bits take two passes and 25 bits three).  One
+// workgroup takes a tile of kSortThreads * ITEMS keys; counts holds the
+// tiles' digit counts.
+constexpr int kSortThreads = 512;
 constexpr int kSortWaves = kSortThreads / kWave;
+constexpr int kDigitBits = 9;
+constexpr int kBins = 1 << kDigitBits;
+static_assert(kBins == kSortThreads, "thread t owns digit t");
+constexpr int kItemsSmall = 4;   // tiles of 2048 keys: R-MAT 14's 228K arcs fill 112 workgroups
+constexpr int kItemsLarge = 16;  // tiles of 8192 keys (4096 of 64 bits): runs of 64 bytes and more per digit
+// Up to this many tiles, counts stay tile-major and each tile adds up the
+// ones before it itself (one launch less than three scan launches: 57K
+// counters took 10 us to scan); above, a digit-major scan.
+constexpr uint32_t kSelfScanTiles = 128;
 
-template <typename K>
-__global__ __launch_bounds__(kSortThreads) void k_radix_upsweep(const K* __restrict__ keys, int64_t n,
-                                                                int shift, uint32_t* __restrict__ counts,
-                                                                uint32_t nblocks) {
-    __shared__ uint32_t hist[256];
-    hist[threadIdx.x] = 0;
+template <typename K, int ITEMS>
+__global__ __launch_bounds__(kSortThreads) void k_radix_upsweep(const K* __restrict__ keys, int64_t n, int shift,
+                                                                uint32_t mask, uint32_t* __restrict__ counts,
+                                                                uint32_t nblocks, int tile_major) {
+    // two copies, by wavefront parity: fewer lanes meet on one hot digit
+    __shared__ uint32_t hist[2][kBins];
+    hist[0][threadIdx.x] = 0;
+    hist[1][threadIdx.x] = 0;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * kSortTile;
-#pragma unroll 4
-    for (int i = 0; i < kSortItems; ++i) {
-        int64_t idx = base + (int64_t)i * kSortThreads + threadIdx.x;
-        if (idx < n) {
-            uint32_t d = (uint32_t)(keys[idx] >> shift) & 255u;
-            atomicAdd(&hist[d], 1u);
-        }
+    const int64_t base = (int64_t)blockIdx.x * (kSortThreads * ITEMS);
+    uint32_t* h = hist[wave_id() & 1];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const int64_t idx = base + (int64_t)i * kSortThreads + threadIdx.x;
+        if (idx < n) atomicAdd(&h[(uint32_t)(keys[idx] >> shift) & mask], 1u);
     }
     __syncthreads();
-    counts[(size_t)threadIdx.x * nblocks + blockIdx.x] = hist[threadIdx.x];
+    if (threadIdx.x <= mask) {
+        const uint32_t c = hist[0][threadIdx.x] + hist[1][threadIdx.x];
+        if (tile_major) counts[(size_t)blockIdx.x * kBins + threadIdx.x] = c;
+        else counts[(size_t)threadIdx.x * nblocks + blockIdx.x] = c;
+    }
 }
 
-// Stable scatter: within the tile, key i*256+t precedes key (i+1)*256+t' and
-// key i*256+t precedes i*256+t+1, which is the tile's input order.
-template <typename K, bool HAS_VAL>
+// Exclusive sum over the workgroup of one value per thread.
+__device__ __forceinline__ uint32_t sort_block_scan(uint32_t v, uint32_t* sh_w) {
+    uint32_t inc = v;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const uint32_t o = __shfl_up(inc, off, kWave);
+        if (lane_id() >= off) inc += o;
+    }
+    if (lane_id() == kWave - 1) sh_w[wave_id()] = inc;
+    __syncthreads();
+    uint32_t base = 0;
+    for (int w = 0; w < wave_id(); ++w) base += sh_w[w];
+    __syncthreads();
+    return base + inc - v;
+}
+
+// Stable scatter of one tile.  Wavefront w holds the tile's keys [w * 64 *
+// ITEMS, ...), 64 consecutive ones per step, and ranks them by itself: the
+// lanes that share a digit find each other by ballots, and a counter per
+// (wavefront, digit) in LDS carries the count over the steps, so the ranking
+// needs no barrier.  The tile is then put in digit order in LDS and written
+// out by consecutive threads, so that each digit's run is stored in
+// consecutive addresses.  The form with four barriers per 256 keys and
+// stores in key order took 2.05 ms per pass over 263M pairs and 15 us over
+// 228K.
+template <typename K, bool HAS_VAL, int ITEMS>
 __global__ __launch_bounds__(kSortThreads) void k_radix_downsweep(
     const K* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, K* __restrict__ keys_out,
-    uint32_t* __restrict__ vals_out, int64_t n, int shift, const uint32_t* __restrict__ offsets,
-    uint32_t nblocks) {
-    __shared__ uint32_t gbase[256];
-    __shared__ uint32_t run[256];
-    __shared__ uint32_t wcnt[kSortWaves][256];
+    uint32_t* __restrict__ vals_out, int64_t n, int shift, uint32_t mask, int bits,
+    const uint32_t* __restrict__ offsets, uint32_t nblocks, int tile_major) {
+    constexpr int kTile = kSortThreads * ITEMS;
+    __shared__ K stage[kTile];
+    __shared__ uint32_t wcnt[kSortWaves][kBins];
+    __shared__ uint32_t start[kBins];   // first position of the digit in the tile
+    __shared__ uint32_t gbase[kBins];   // its first position in the output
+    __shared__ uint32_t sh_w[kSortWaves];
     const int t = threadIdx.x;
     const int lane = lane_id();
     const int w = wave_id();
-    gbase[t] = offsets[(size_t)t * nblocks + blockIdx.x];
-    run[t] = 0;
-    const uint64_t lt_mask = (lane == 0) ? 0ull : ((1ull << lane) - 1ull);
-    const int64_t base = (int64_t)blockIdx.x * kSortTile;
-    for (int r = 0; r < kSortItems; ++r) {
-        const int64_t idx = base + (int64_t)r * kSortThreads + t;
-        const bool valid = idx < n;
-        K key = valid ? keys_in[idx] : (K)0;
-        uint32_t val = 0;
-        if (HAS_VAL && valid) val = vals_in[idx];
-        const uint32_t d = (uint32_t)(key >> shift) & 255u;
+    const int64_t base = (int64_t)blockIdx.x * kTile;
+    const int32_t count = (int32_t)min((int64_t)kTile, n - base);  // keys of this tile
+    const int32_t wbase = w * (kWave * ITEMS) + lane;
+    K key[ITEMS];
+    uint32_t val[HAS_VAL ? ITEMS : 1];
 #pragma unroll
-        for (int ww = 0; ww < kSortWaves; ++ww) wcnt[ww][t] = 0;
-        __syncthreads();
-        uint64_t peers = __ballot(valid);
+    for (int r = 0; r < ITEMS; ++r) {
+        const int32_t i = wbase + r * kWave;
+        const int64_t at = base + (i < count ? i : 0);
+        key[r] = keys_in[at];
+        if (HAS_VAL) val[r] = vals_in[at];
+    }
 #pragma unroll
-        for (int bit = 0; bit < 8; ++bit) {
-            const bool set = (d >> bit) & 1u;
-            const uint64_t b = __ballot(set);
-            peers &= set ? b : ~b;
-        }
-        const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
-        if (valid && rank == 0) wcnt[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        {
-            uint32_t acc = run[t];
-#pragma unroll
-            for (int ww = 0; ww < kSortWaves; ++ww) {
-                uint32_t c = wcnt[ww][t];
-                wcnt[ww][t] = acc;
-                acc += c;
+    for (int ww = 0; ww < kSortWaves; ++ww) wcnt[ww][t] = 0;
+    // this tile's first output position of every digit
+    uint32_t tot = 0, before = 0;
+    if (tile_major) {
+        if ((uint32_t)t <= mask) {
+#pragma unroll 8
+            for (uint32_t b = 0; b < nblocks; ++b) {
+                const uint32_t c = offsets[(size_t)b * kBins + t];
+                tot += c;
+                before += b < blockIdx.x ? c : 0u;
             }
-            run[t] = acc;
         }
-        __syncthreads();
-        if (valid) {
-            const uint32_t dest = gbase[d] + wcnt[w][d] + rank;
-            keys_out[dest] = key;
-            if (HAS_VAL) vals_out[dest] = val;
+    } else if ((uint32_t)t <= mask) {
+        before = offsets[(size_t)t * nblocks + blockIdx.x];
+    }
+    __syncthreads();
+    if (tile_major) before += sort_block_scan(tot, sh_w);
+    gbase[t] = before;
+    const uint64_t lt_mask = (1ull << lane) - 1ull;
+    uint32_t rank[ITEMS];
+    volatile uint32_t* cnt = wcnt[w];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const bool valid = wbase + r * kWave < count;
+        // keys past the end take the last digit: they rank behind its keys
+        const uint32_t d = valid ? (uint32_t)(key[r] >> shift) & mask : mask;
+        uint64_t peers = ~0ull;
+#pragma unroll
+        for (int bit = 0; bit < kDigitBits; ++bit) {
+            if (bit < bits) {
+                const bool set = (d >> bit) & 1u;
+                const uint64_t b = __ballot(set);
+                peers &= set ? b : ~b;
+            }
         }
+        const uint32_t pre = cnt[d];
+        const uint32_t mine = (uint32_t)__popcll(peers & lt_mask);
+        __builtin_amdgcn_wave_barrier();
+        if (mine == 0) cnt[d] = pre + (uint32_t)__popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+        rank[r] = pre + mine;
+    }
+    __syncthreads();
+    {
+        uint32_t acc = 0;
+#pragma unroll
+        for (int ww = 0; ww < kSortWaves; ++ww) {
+            const uint32_t c = wcnt[ww][t];
+            wcnt[ww][t] = acc;
+            acc += c;
+        }
+        start[t] = sort_block_scan(acc, sh_w);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const bool valid = wbase + r * kWave < count;
+        const uint32_t d = valid ? (uint32_t)(key[r] >> shift) & mask : mask;
+        rank[r] += start[d] + wcnt[w][d];
+        stage[rank[r]] = key[r];
+    }
+    __syncthreads();
+    uint32_t dest[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const int32_t i = r * kSortThreads + t;
+        if (i < count) {
+            const K k = stage[i];
+            const uint32_t d = (uint32_t)(k >> shift) & mask;
+            dest[r] = gbase[d] + ((uint32_t)i - start[d]);
+            keys_out[dest[r]] = k;
+        }
+    }
+    if (HAS_VAL) {
         __syncthreads();
+        uint32_t* vstage = reinterpret_cast<uint32_t*>(stage);
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) vstage[rank[r]] = val[HAS_VAL ? r : 0];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const int32_t i = r * kSortThreads + t;
+            if (i < count) vals_out[dest[r]] = vstage[i];
+        }
     }
 }
 
+template <typename K, int ITEMS>
+int radix_passes(DevBuf& keys, DevBuf& keys_alt, DevBuf* vals, DevBuf* vals_alt, int64_t n, int nbits,
+                 hipStream_t s) {
+    const uint32_t nb = (uint32_t)((n + kSortThreads * ITEMS - 1) / (kSortThreads * ITEMS));
+    const int passes = (nbits + kDigitBits - 1) / kDigitBits;
+    const int tile_major = nb <= kSelfScanTiles ? 1 : 0;
+    DevBuf counts;
+    EGX_TRY(counts.alloc((size_t)kBins * nb * sizeof(uint32_t), s));
+    for (int q = 0, shift = 0; q < passes; ++q) {
+        const int bits = (nbits - shift + passes - q - 1) / (passes - q);
+        const uint32_t mask = (1u << bits) - 1u;
+        k_radix_upsweep<K, ITEMS><<<nb, kSortThreads, 0, s>>>(keys.as<K>(), n, shift, mask, counts.as<uint32_t>(), nb,
+                                                              tile_major);
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        if (!tile_major)
+            EGX_TRY(scan_impl<uint32_t>(counts.as<uint32_t>(), counts.as<uint32_t>(), (int64_t)(mask + 1) * nb, s));
+        if (vals)
+            k_radix_downsweep<K, true, ITEMS><<<nb, kSortThreads, 0, s>>>(
+                keys.as<K>(), vals->as<uint32_t>(), keys_alt.as<K>(), vals_alt->as<uint32_t>(), n, shift, mask, bits,
+                counts.as<uint32_t>(), nb, tile_major);
+        else
+            k_radix_downsweep<K, false, ITEMS><<<nb, kSortThreads, 0, s>>>(keys.as<K>(), nullptr, keys_alt.as<K>(),
+                                                                           nullptr, n, shift, mask, bits,
+                                                                           counts.as<uint32_t>(), nb, tile_major);
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        std::swap(keys, keys_alt);
+        if (vals) std::swap(*vals, *vals_alt);
+        shift += bits;
+    }
+    return EGX_SUCC;
+}
+
 template <typename K>
-int radix_sort_impl(K* keys, K* keys_alt, uint32_t* vals, uint32_t* vals_alt, int64_t n, int nbits,
+int radix_sort_impl(DevBuf& keys, DevBuf& keys_alt, DevBuf* vals, DevBuf* vals_alt, int64_t n, int nbits,
                     hipStream_t s) {
     if (n <= 1 || nbits <= 0) return EGX_SUCC;
     if (n > (int64_t)0xFFFFFFFFll) {
         set_last_error("radix sort: more than 2^32-1 keys");
         return EGX_UNSUPPORTED_GRAPH;
     }
-    const int64_t nb64 = (n + kSortTile - 1) / kSortTile;
-    const uint32_t nb = (uint32_t)nb64;
-    DevBuf counts;
-    EGX_TRY(counts.alloc((size_t)256 * nb * sizeof(uint32_t), s));
-    const bool has_val = vals != nullptr;
-    K* kin = keys;
-    K* kout = keys_alt;
-    uint32_t* vin = vals;
-    uint32_t* vout = vals_alt;
-    int passes = 0;
-    for (int shift = 0; shift < nbits; shift += 8, ++passes) {
-        k_radix_upsweep<K><<<nb, kSortThreads, 0, s>>>(kin, n, shift, counts.as<uint32_t>(), nb);
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        EGX_TRY(scan_impl<uint32_t>(counts.as<uint32_t>(), counts.as<uint32_t>(), (int64_t)256 * nb, s));
-        if (has_val)
-            k_radix_downsweep<K, true><<<nb, kSortThreads, 0, s>>>(kin, vin, kout, vout, n, shift,
-                                                                   counts.as<uint32_t>(), nb);
-        else
-            k_radix_downsweep<K, false><<<nb, kSortThreads, 0, s>>>(kin, nullptr, kout, nullptr, n,
-                                                                    shift, counts.as<uint32_t>(), nb);
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        K* tk = kin; kin = kout; kout = tk;
-        uint32_t* tv = vin; vin = vout; vout = tv;
-    }
-    if (passes & 1) {
-        EGX_HIP_TRY(hipMemcpyAsync(keys, kin, (size_t)n * sizeof(K), hipMemcpyDeviceToDevice, s), EGX_DEVICE_ERR);
-        if (has_val)
-            EGX_HIP_TRY(hipMemcpyAsync(vals, vin, (size_t)n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s),
-                        EGX_DEVICE_ERR);
-    }
-    return EGX_SUCC;
+    if (n <= (int64_t)kSelfScanTiles * kSortThreads * kItemsSmall)
+        return radix_passes<K, kItemsSmall>(keys, keys_alt, vals, vals_alt, n, nbits, s);
+    constexpr int kItems = sizeof(K) == 8 ? kItemsLarge / 2 : kItemsLarge;
+    return radix_passes<K, kItems>(keys, keys_alt, vals, vals_alt, n, nbits, s);
 }
 
 template <typename K>
@@ -451,12 +554,12 @@ int exclusive_scan_i64(const int64_t* in, int64_t* out, int64_t n, hipStream_t s
     return scan_impl<int64_t>(in, out, n, s);
 }
 
-int radix_sort_u32(uint32_t* keys, uint32_t* keys_alt, uint32_t* vals, uint32_t* vals_alt, int64_t n,
-                   int nbits, hipStream_t s) {
+int radix_sort_u32(DevBuf& keys, DevBuf& keys_alt, DevBuf* vals, DevBuf* vals_alt, int64_t n, int nbits,
+                   hipStream_t s) {
     return radix_sort_impl<uint32_t>(keys, keys_alt, vals, vals_alt, n, nbits, s);
 }
-int radix_sort_u64(uint64_t* keys, uint64_t* keys_alt, uint32_t* vals, uint32_t* vals_alt, int64_t n,
-                   int nbits, hipStream_t s) {
+int radix_sort_u64(DevBuf& keys, DevBuf& keys_alt, DevBuf* vals, DevBuf* vals_alt, int64_t n, int nbits,
+                   hipStream_t s) {
     return radix_sort_impl<uint64_t>(keys, keys_alt, vals, vals_alt, n, nbits, s);
 }
 

@@ -84,3 +84,19 @@ def test_bad_arcs_are_refused(gpu_ready, bad, at):
         bad_w[at] = w
         with pytest.raises(native.EgxError, match="non-negative weights"):
             native.eigenvector_csr(V, E, bad_w)
+
+
+# arcs around the sort's tiles (2048 keys up to 128 tiles, 8192 above) and key widths of one to three passes
+@pytest.mark.parametrize("n,m", [(1, 1), (2, 2047), (3, 2048), (511, 2049), (512, 4097), (513, 8191), (70000, 262144),
+                                 (131072, 262145), (262143, 270337), (300001, 999999)])
+def test_sorted_build_bit_exact(gpu_ready, n, m):
+    print(f"sort n={n} m={m}", flush=True)
+    rng = np.random.default_rng(m)
+    src = np.sort(rng.integers(0, n, m))
+    E = np.minimum(rng.integers(0, n, m), rng.integers(0, n, m)).astype(np.int32)  # skewed heads
+    V = np.zeros(n + 1, np.int32)
+    V[1:] = np.cumsum(np.bincount(src, minlength=n))
+    with native.DeviceGraph.from_csr(V, E) as g:
+        got = g.download_csc()
+    want = O.build_inbound(V, E, None, 0.85)
+    assert all(np.array_equal(a, b) for a, b in zip(got, want[:4]))
