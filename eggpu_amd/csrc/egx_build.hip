@@ -26,30 +26,137 @@ namespace egx {
 
 namespace {
 
-__global__ void k_expand_src(const int32_t* __restrict__ V, int32_t n, int64_t m, int32_t* __restrict__ src) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= m) return;
-    // last u with V[u] <= p (V is monotonic, V[n] = m > p)
-    int32_t lo = 0, hi = n + 1;
-    while (lo < hi) {
-        int32_t mid = (lo + hi) >> 1;
-        if ((int64_t)V[mid] <= p) lo = mid + 1;
-        else hi = mid;
+// Row of every arc of a run.  One binary search per arc over the whole
+// offset array was 80-100 us of every pass over 7-9M arcs (20 dependent
+// loads each).  A workgroup now finds the rows of its first and last arc by
+// a 64-way search (four loads deep at a million rows), marks the first arc
+// of each row in between and spreads the marks by a running maximum.
+constexpr int kRunThreads = 512;
+constexpr int kRunItems = 8;
+constexpr int kRunArcs = kRunThreads * kRunItems;  // arcs per workgroup
+struct RunRows {
+    int4 mark[kRunArcs / 4];
+    int32_t wave_max[kRunThreads / kWave];
+    int32_t ends[2];
+};
+
+// The last u in [0, n] with V[u] <= p, for V[0] <= p < V[n]; all 64 lanes take part.
+__device__ __forceinline__ int32_t wave_row_of(const int32_t* __restrict__ V, int32_t n, int64_t p) {
+    int32_t lo = 0;
+    int64_t hi = (int64_t)n + 1;
+    while (hi - lo > 1) {
+        const int64_t w = (hi - lo + kWave - 1) / kWave;
+        const int64_t at = lo + (lane_id() + 1) * w;
+        const bool below = at < hi && (int64_t)V[at] <= p;
+        const int32_t c = __popcll(__ballot(below));
+        lo = (int32_t)(lo + c * w);
+        hi = min(hi, lo + w);
     }
-    src[p] = lo - 1;
+    return lo;
 }
 
-__global__ void k_make_sort_keys(const int32_t* __restrict__ E, const int32_t* __restrict__ src, int32_t n,
-                                 int64_t m, int weighted, uint32_t* __restrict__ keys,
-                                 uint32_t* __restrict__ vals, uint32_t* __restrict__ invalid_count) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= m) return;
-    const int32_t v = E[p];
-    const bool valid = (0 <= v) && (v < n);
-    keys[p] = valid ? (uint32_t)v : (uint32_t)n;
-    vals[p] = weighted ? (uint32_t)p : (uint32_t)src[p];
-    if (!valid) atomicAdd(invalid_count, 1u);
+// rows: rows[i] = row of arc q0 + i, i in [0, cnt), cnt <= kRunArcs, q0 + cnt <= V[n].
+// Every thread of a kRunThreads workgroup takes part; the result is valid
+// after the call.
+__device__ __forceinline__ const int32_t* run_rows(const int32_t* __restrict__ V, int32_t n, int64_t q0, int32_t cnt,
+                                                   RunRows& sh) {
+    const int t = threadIdx.x;
+    int32_t* mark = reinterpret_cast<int32_t*>(sh.mark);
+    if (wave_id() < 2) {
+        const int32_t r = wave_row_of(V, n, wave_id() == 0 ? q0 : q0 + cnt - 1);
+        if (lane_id() == 0) sh.ends[wave_id()] = r;
+    }
+    for (int i = t; i < kRunArcs / 4; i += kRunThreads) sh.mark[i] = int4{0, 0, 0, 0};
+    __syncthreads();
+    const int32_t first = sh.ends[0], last = sh.ends[1];
+    // a row's first arc gets the row; of the rows that share it (all but the last have no arcs) the last wins
+    for (int32_t r = first + 1 + t; r <= last; r += kRunThreads) atomicMax(&mark[V[r] - q0], r);
+    if (t == 0) atomicMax(&mark[0], first);
+    __syncthreads();
+    int4 a = sh.mark[2 * t], b = sh.mark[2 * t + 1];
+    a.y = max(a.y, a.x); a.z = max(a.z, a.y); a.w = max(a.w, a.z);
+    b.x = max(b.x, a.w); b.y = max(b.y, b.x); b.z = max(b.z, b.y); b.w = max(b.w, b.z);
+    int32_t inc = b.w;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int32_t o = __shfl_up(inc, off, kWave);
+        if (lane_id() >= off) inc = max(inc, o);
+    }
+    int32_t prev = __shfl_up(inc, 1, kWave);
+    if (lane_id() == 0) prev = 0;
+    if (lane_id() == kWave - 1) sh.wave_max[wave_id()] = inc;
+    __syncthreads();
+    for (int w = 0; w < wave_id(); ++w) prev = max(prev, sh.wave_max[w]);
+    sh.mark[2 * t] = int4{max(a.x, prev), max(a.y, prev), max(a.z, prev), max(a.w, prev)};
+    sh.mark[2 * t + 1] = int4{max(b.x, prev), max(b.y, prev), max(b.z, prev), max(b.w, prev)};
+    __syncthreads();
+    return mark;
 }
+static_assert(kRunItems == 8, "a thread spreads two int4 of marks");
+
+__global__ __launch_bounds__(kRunThreads) void k_expand_src(const int32_t* __restrict__ V, int32_t n, int64_t m,
+                                                            int32_t* __restrict__ src) {
+    __shared__ RunRows sh;
+    const int64_t q0 = (int64_t)blockIdx.x * kRunArcs;
+    const int32_t cnt = (int32_t)min((int64_t)kRunArcs, m - q0);
+    const int32_t* rows = run_rows(V, n, q0, cnt, sh);
+    for (int32_t i = threadIdx.x; i < cnt; i += kRunThreads) src[q0 + i] = rows[i];
+}
+
+// What a weighted arc carries to its place in the pull CSC: gathered as one
+// 16-byte record instead of its weight, source and the source's out-weight
+// one by one (k_fill_csc over 9.3M arcs: 310 us).
+struct __align__(16) ArcRec {
+    double w;     // sanitised weight
+    int32_t src;
+    float val;    // fl32(alpha * (w / outW[src])), pagerank.cu:344
+};
+
+// Sort keys (head, or n past the valid ones) and payloads of every arc: the
+// source, or for weighted arcs the arc's slot, with its record.
+template <bool HasW>
+__global__ __launch_bounds__(kRunThreads) void k_arc_keys(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
+                                                          const double* __restrict__ W,
+                                                          const double* __restrict__ out_w, int32_t n, int64_t m,
+                                                          double alpha, uint32_t* __restrict__ keys,
+                                                          uint32_t* __restrict__ vals, ArcRec* __restrict__ rec,
+                                                          uint32_t* __restrict__ invalid_count) {
+    __shared__ RunRows sh;
+    __shared__ uint32_t bad;
+    if (threadIdx.x == 0) bad = 0;  // run_rows has barriers before it is used
+    const int64_t q0 = (int64_t)blockIdx.x * kRunArcs;
+    const int32_t cnt = (int32_t)min((int64_t)kRunArcs, m - q0);
+    const int32_t* rows = run_rows(V, n, q0, cnt, sh);
+    for (int32_t i = threadIdx.x; i < cnt; i += kRunThreads) {
+        const int64_t p = q0 + i;
+        const int32_t v = E[p];
+        const int32_t u = rows[i];
+        const bool valid = (0 <= v) && (v < n);
+        keys[p] = valid ? (uint32_t)v : (uint32_t)n;
+        vals[p] = HasW ? (uint32_t)p : (uint32_t)u;
+        if (!valid) atomicAdd(&bad, 1u);
+        if (HasW) {
+            double w = W[p];
+            if (!isfinite(w) || w < 0.0) w = 0.0;
+            const double denom = out_w[u];
+            rec[p] = ArcRec{w, u, (denom > 0.0) ? (float)(alpha * (w / denom)) : 0.0f};
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && bad) atomicAdd(invalid_count, bad);
+}
+
+// Counters of a build.
+enum : int {
+    kCtrInvalid,   // arcs with an endpoint outside [0, n)
+    kCtrDangling,  // nodes without out-weight
+    kCtrMaxOut,    // largest out-degree
+    kCtrMaxIn,     // largest in-degree
+    kCtrLong,      // rows longer than kOutLong
+    kCtrHubs,      // rows above the hub threshold
+    kCtrWaveRows,  // rows of tiles reduced a wavefront per row
+    kCtrWords
+};
 
 __global__ void k_outcnt_from_V(const int32_t* __restrict__ V, int32_t n, double* __restrict__ out_w,
                                 int32_t* __restrict__ outcnt) {
@@ -201,44 +308,57 @@ __global__ __launch_bounds__(256) void k_row_out_long(const int32_t* __restrict_
     }
 }
 
-// deg (0 == dangling), dangling count, max out-degree.
-__global__ void k_node_arrays(const double* __restrict__ out_w, const int32_t* __restrict__ outcnt, int32_t n,
-                              int weighted, float* __restrict__ deg, uint32_t* __restrict__ ctr) {
-    __shared__ uint32_t sh_d, sh_max;
-    if (threadIdx.x == 0) { sh_d = 0; sh_max = 0; }
+// Sum / maximum over a 256-thread workgroup, valid in thread 0.
+__device__ __forceinline__ uint32_t block_sum_u32(uint32_t v, uint32_t* sh) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
     __syncthreads();
-    const int32_t u = blockIdx.x * blockDim.x + threadIdx.x;
-    if (u < n) {
+    if (lane_id() == 0) sh[wave_id()] = v;
+    __syncthreads();
+    return sh[0] + sh[1] + sh[2] + sh[3];
+}
+__device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t* sh) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, kWave));
+    __syncthreads();
+    if (lane_id() == 0) sh[wave_id()] = v;
+    __syncthreads();
+    return max(max(sh[0], sh[1]), max(sh[2], sh[3]));
+}
+
+// Node passes with counters run at most this many workgroups: each adds to a
+// counter once, and device-wide atomics on one address cost some 25 ns each
+// (one per 256 nodes took 67 us at 700K nodes).
+constexpr int kNodeBlocks = 512;
+
+// deg (0 == dangling), dangling count, max out-degree.
+__global__ __launch_bounds__(256) void k_node_arrays(const double* __restrict__ out_w,
+                                                     const int32_t* __restrict__ outcnt, int32_t n, int weighted,
+                                                     float* __restrict__ deg, uint32_t* __restrict__ ctr) {
+    __shared__ uint32_t sh[4];
+    uint32_t nd = 0, most = 0;
+    for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < n; u += (int64_t)gridDim.x * 256) {
         const bool dang = !(out_w[u] > 0.0);  // pagerank.cu:323-326: outW <= 0
         deg[u] = weighted ? (dang ? 0.0f : 1.0f) : (dang ? 0.0f : (float)outcnt[u]);
-        if (dang) atomicAdd(&sh_d, 1u);
-        atomicMax(&sh_max, (uint32_t)outcnt[u]);
+        nd += dang ? 1u : 0u;
+        most = max(most, (uint32_t)outcnt[u]);
     }
-    __syncthreads();
+    nd = block_sum_u32(nd, sh);
+    most = block_max_u32(most, sh);
     if (threadIdx.x == 0) {
-        if (sh_d) atomicAdd(&ctr[1], sh_d);
-        atomicMax(&ctr[2], sh_max);
+        if (nd) atomicAdd(&ctr[kCtrDangling], nd);
+        if (most) atomicMax(&ctr[kCtrMaxOut], most);
     }
 }
 
-__global__ void k_fill_csc(const uint32_t* __restrict__ vals, const int32_t* __restrict__ src,
-                           const double* __restrict__ W, const double* __restrict__ out_w, int64_t m_valid,
-                           int weighted, double alpha, int32_t* __restrict__ in_col, float* __restrict__ in_val,
-                           double* __restrict__ w_csc) {
+__global__ void k_fill_csc(const uint32_t* __restrict__ vals, const ArcRec* __restrict__ rec, int64_t m_valid,
+                           int32_t* __restrict__ in_col, float* __restrict__ in_val, double* __restrict__ w_csc) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= m_valid) return;
-    const uint32_t val = vals[q];
-    if (weighted) {
-        const int32_t u = src[val];
-        double w = W ? W[val] : 1.0;
-        if (!isfinite(w) || w < 0.0) w = 0.0;
-        const double denom = out_w[u];
-        in_col[q] = u;
-        w_csc[q] = w;
-        in_val[q] = (denom > 0.0) ? (float)(alpha * (w / denom)) : 0.0f;
-    } else {
-        in_col[q] = (int32_t)val;
-    }
+    const ArcRec r = rec[vals[q]];
+    in_col[q] = r.src;
+    w_csc[q] = r.w;
+    in_val[q] = r.val;
 }
 
 __global__ void k_refresh_vals(const int32_t* __restrict__ in_col, const double* __restrict__ w_csc,
@@ -259,14 +379,22 @@ __global__ void k_unit_vals(const int32_t* __restrict__ in_col, const double* __
     in_val[q] = (denom > 0.0) ? (float)(alpha * (1.0 / denom)) : 0.0f;
 }
 
-__global__ void k_max_in_degree(const int32_t* __restrict__ in_row, int32_t n, uint32_t* __restrict__ out) {
-    __shared__ uint32_t sh;
-    if (threadIdx.x == 0) sh = 0;
-    __syncthreads();
-    const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < n) atomicMax(&sh, (uint32_t)(in_row[v + 1] - in_row[v]));
-    __syncthreads();
-    if (threadIdx.x == 0) atomicMax(out, sh);
+// Largest in-degree, and the rows above the hub threshold.
+__global__ __launch_bounds__(256) void k_in_degrees(const int32_t* __restrict__ in_row, int32_t n, int32_t hub,
+                                                    uint32_t* __restrict__ ctr) {
+    __shared__ uint32_t sh[4];
+    uint32_t most = 0, hubs = 0;
+    for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (int64_t)gridDim.x * 256) {
+        const int32_t d = in_row[v + 1] - in_row[v];
+        most = max(most, (uint32_t)d);
+        hubs += d > hub ? 1u : 0u;
+    }
+    most = block_max_u32(most, sh);
+    hubs = block_sum_u32(hubs, sh);
+    if (threadIdx.x == 0) {
+        if (most) atomicMax(&ctr[kCtrMaxIn], most);
+        if (hubs) atomicAdd(&ctr[kCtrHubs], hubs);
+    }
 }
 
 // Relabelling key: hub rows (in-degree > hub) first, then descending
@@ -274,20 +402,13 @@ __global__ void k_max_in_degree(const int32_t* __restrict__ in_row, int32_t n, u
 // equal keys.  perm[r] = original id of row r, rank = its inverse.
 __global__ void k_layout_keys(const int32_t* __restrict__ in_row, const int32_t* __restrict__ out_cnt, int32_t n,
                               int32_t hub, int32_t bits, uint32_t maxdeg, int reorder, uint32_t* __restrict__ keys,
-                              uint32_t* __restrict__ vals, uint32_t* __restrict__ n_hub) {
-    __shared__ uint32_t sh;
-    if (threadIdx.x == 0) sh = 0;
-    __syncthreads();
+                              uint32_t* __restrict__ vals) {
     const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < n) {
-        const bool is_hub = (in_row[v + 1] - in_row[v]) > hub;
-        const uint32_t sec = reorder ? (maxdeg - (uint32_t)out_cnt[v]) : 0u;
-        keys[v] = ((is_hub ? 0u : 1u) << bits) | sec;
-        vals[v] = (uint32_t)v;
-        if (is_hub) atomicAdd(&sh, 1u);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && sh) atomicAdd(n_hub, sh);
+    if (v >= n) return;
+    const bool is_hub = (in_row[v + 1] - in_row[v]) > hub;
+    const uint32_t sec = reorder ? (maxdeg - (uint32_t)out_cnt[v]) : 0u;
+    keys[v] = ((is_hub ? 0u : 1u) << bits) | sec;
+    vals[v] = (uint32_t)v;
 }
 
 // tiles[k] = first row v in [n_hub, n] whose merge-path diagonal
@@ -361,29 +482,41 @@ __global__ void k_layout_nodes(const uint32_t* __restrict__ perm, const int32_t*
     p_outw[r] = out_w[v];
 }
 
-// One thread per relabelled CSC slot: find its row, copy the arc with its
-// source relabelled.
-__global__ void k_layout_slots(const int32_t* __restrict__ p_row, const int32_t* __restrict__ perm,
-                               const int32_t* __restrict__ rank, const int32_t* __restrict__ in_row,
-                               const int32_t* __restrict__ in_col, const float* __restrict__ in_val,
-                               const double* __restrict__ w_csc, int32_t n, int64_t m, int weighted,
-                               int32_t* __restrict__ p_col, float* __restrict__ p_val, double* __restrict__ p_w) {
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= m) return;
-    int32_t lo = 0, hi = n + 1;  // last r with p_row[r] <= q
-    while (lo < hi) {
-        const int32_t mid = (lo + hi) >> 1;
-        if ((int64_t)p_row[mid] <= q) lo = mid + 1;
-        else hi = mid;
+// Every relabelled CSC slot: its row, and the arc with its source relabelled.
+__global__ __launch_bounds__(kRunThreads) void k_layout_slots(
+    const int32_t* __restrict__ p_row, const int32_t* __restrict__ perm, const int32_t* __restrict__ rank,
+    const int32_t* __restrict__ in_row, const int32_t* __restrict__ in_col, const float* __restrict__ in_val,
+    const double* __restrict__ w_csc, int32_t n, int64_t m, int weighted, int32_t* __restrict__ p_col,
+    float* __restrict__ p_val, double* __restrict__ p_w) {
+    __shared__ RunRows sh;
+    const int64_t q0 = (int64_t)blockIdx.x * kRunArcs;
+    const int32_t cnt = (int32_t)min((int64_t)kRunArcs, m - q0);
+    const int32_t* rows = run_rows(p_row, n, q0, cnt, sh);
+#pragma unroll 4
+    for (int32_t i = threadIdx.x; i < cnt; i += kRunThreads) {
+        const int64_t q = q0 + i;
+        const int32_t r = rows[i];
+        const int64_t src_slot = (int64_t)in_row[perm[r]] + (q - p_row[r]);
+        p_col[q] = rank[in_col[src_slot]];
+        if (weighted) {
+            p_val[q] = in_val[src_slot];
+            p_w[q] = w_csc[src_slot];
+        }
     }
-    const int32_t r = lo - 1;
-    const int32_t v = perm[r];
-    const int64_t src_slot = (int64_t)in_row[v] + (q - p_row[r]);
-    p_col[q] = rank[in_col[src_slot]];
-    if (weighted) {
-        p_val[q] = in_val[src_slot];
-        p_w[q] = w_csc[src_slot];
+}
+
+// Rows of tiles whose mean row length is above thread_row_max (egx_graph_info).
+__global__ __launch_bounds__(256) void k_tile_stats(const int32_t* __restrict__ row, const int32_t* __restrict__ tiles,
+                                                    int64_t n_tiles, int32_t thread_row_max,
+                                                    uint32_t* __restrict__ ctr) {
+    __shared__ uint32_t sh[4];
+    uint32_t rows = 0;
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n_tiles; k += (int64_t)gridDim.x * 256) {
+        const int32_t r0 = tiles[k], r1 = tiles[k + 1];
+        if ((int64_t)(row[r1] - row[r0]) > (int64_t)thread_row_max * (r1 - r0)) rows += (uint32_t)(r1 - r0);
     }
+    rows = block_sum_u32(rows, sh);
+    if (threadIdx.x == 0 && rows) atomicAdd(&ctr[kCtrWaveRows], rows);
 }
 
 __global__ void k_check_arcs(const int32_t* __restrict__ E, const double* __restrict__ W, int32_t n, int64_t m,
@@ -403,6 +536,9 @@ __global__ void k_check_arcs(const int32_t* __restrict__ E, const double* __rest
 __global__ void k_set_last(int32_t* __restrict__ arr, int64_t idx, int32_t value) {
     if (blockIdx.x == 0 && threadIdx.x == 0) arr[idx] = value;
 }
+
+// The in-degree above which a row is a hub row.
+inline int32_t hub_threshold(const BinCfg& cfg) { return std::min(std::max(cfg.wave_row_max, 1), kTileLds - 256); }
 
 inline unsigned nblocks(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
@@ -425,7 +561,7 @@ int build_tile_sort(Graph& g, const BinCfg& cfg) {
     const size_t mm = (size_t)std::max<int64_t>(g.m, 1);
     EGX_TRY(g.t_col.alloc(mm * 4));
     EGX_TRY(g.t_pos.alloc(mm * 2));
-    if (g.weighted) EGX_TRY(g.t_val.alloc(mm * 4));
+    if (g.has_values()) EGX_TRY(g.t_val.alloc(mm * 4));
     {
         DevBuf keys, keys_alt, vals, vals_alt;
         EGX_TRY(keys.alloc((size_t)mt * 8));
@@ -439,7 +575,7 @@ int build_tile_sort(Graph& g, const BinCfg& cfg) {
         EGX_TRY(radix_sort_u64(keys, keys_alt, &vals, &vals_alt, mt, 32 + bits_for((uint64_t)g.n_tiles), s));
         k_tile_sorted_arrays<<<nt, 256, 0, s>>>(g.it_row, g.tiles.as<int32_t>(), keys.as<uint64_t>(),
                                                 vals.as<uint32_t>(), g.it_val, base, g.t_col.as<int32_t>(),
-                                                g.t_pos.as<uint16_t>(), g.weighted ? g.t_val.as<float>() : nullptr);
+                                                g.t_pos.as<uint16_t>(), g.has_values() ? g.t_val.as<float>() : nullptr);
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     }
@@ -452,12 +588,21 @@ namespace {
 // Run key of every arc, (chunk of its source) * B + (sub-bin of its row),
 // with the arc's CSC position as the value: a stable sort by key keeps CSC
 // order (row, then position) inside every run.
-__global__ void k_pb_keys(const int32_t* __restrict__ col, const int32_t* __restrict__ rowof, int64_t m,
-                          int64_t B, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= m) return;
-    keys[e] = (uint32_t)((int64_t)(col[e] / kPbChunk) * B + rowof[e] / kPbRows);
-    vals[e] = (uint32_t)e;
+__global__ __launch_bounds__(kRunThreads) void k_pb_keys(const int32_t* __restrict__ row,
+                                                         const int32_t* __restrict__ col, int32_t n, int64_t m,
+                                                         int64_t B, uint32_t* __restrict__ keys,
+                                                         uint32_t* __restrict__ vals, int32_t* __restrict__ rowof) {
+    __shared__ RunRows sh;
+    const int64_t q0 = (int64_t)blockIdx.x * kRunArcs;
+    const int32_t cnt = (int32_t)min((int64_t)kRunArcs, m - q0);
+    const int32_t* rows = run_rows(row, n, q0, cnt, sh);
+    for (int32_t i = threadIdx.x; i < cnt; i += kRunThreads) {
+        const int64_t e = q0 + i;
+        const int32_t r = rows[i];
+        keys[e] = (uint32_t)((int64_t)(col[e] / kPbChunk) * B + r / kPbRows);
+        vals[e] = (uint32_t)e;
+        rowof[e] = r;
+    }
 }
 
 // Source slots of every run (its arcs rounded up to kPbVec) from the lower
@@ -698,10 +843,8 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
         EGX_TRY(vals.alloc((size_t)m * 4));
         EGX_TRY(keys_alt.alloc((size_t)m * 4));
         EGX_TRY(vals_alt.alloc((size_t)m * 4));
-        k_expand_src<<<nblocks(m, tb), tb, 0, s>>>(g.it_row, n, m, rowof.as<int32_t>());
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        k_pb_keys<<<nblocks(m, tb), tb, 0, s>>>(g.it_col, rowof.as<int32_t>(), m, B, keys.as<uint32_t>(),
-                                                vals.as<uint32_t>());
+        k_pb_keys<<<nblocks(m, kRunArcs), kRunThreads, 0, s>>>(g.it_row, g.it_col, n, m, B, keys.as<uint32_t>(),
+                                                               vals.as<uint32_t>(), rowof.as<int32_t>());
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         EGX_TRY(radix_sort_u32(keys, keys_alt, &vals, &vals_alt, m, bits_for((uint64_t)(runs - 1)), s));
     }
@@ -729,7 +872,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     EGX_TRY(srow.alloc((size_t)slots * 4));
     EGX_HIP_TRY(hipMemsetAsync(bad.p, 0, 4, s), EGX_DEVICE_ERR);
     EGX_HIP_TRY(hipMemsetAsync(srow.p, 0xFF, (size_t)slots * 4, s), EGX_DEVICE_ERR);
-    if (g.weighted) {
+    if (g.has_values()) {
         EGX_TRY(g.pb_arc.alloc((size_t)slots * 4));
         EGX_HIP_TRY(hipMemsetAsync(g.pb_arc.p, 0xFF, (size_t)slots * 4, s), EGX_DEVICE_ERR);
     }
@@ -738,9 +881,9 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     k_pb_place<<<nblocks(m, tb), tb, 0, s>>>(keys.as<uint32_t>(), vals.as<uint32_t>(), lb.as<int32_t>(),
                                              soff.as<uint32_t>(), g.it_col, rowof.as<int32_t>(), m, runs, B,
                                              g.pb_src.as<uint16_t>(), srow.as<int32_t>(),
-                                             g.weighted ? g.pb_arc.as<int32_t>() : nullptr, bad.as<int32_t>());
+                                             g.has_values() ? g.pb_arc.as<int32_t>() : nullptr, bad.as<int32_t>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    if (g.weighted) {
+    if (g.has_values()) {
         EGX_TRY(g.pb_w.alloc((size_t)slots * 4));
         k_pb_gather_w<<<nblocks(slots, tb), tb, 0, s>>>(g.pb_arc.as<int32_t>(), g.it_val, slots, m,
                                                         g.pb_w.as<float>());
@@ -757,7 +900,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     EGX_TRY(g.pb_mask.alloc((size_t)groups));
     EGX_TRY(gs.alloc((size_t)(groups + 1) * 4));
     // merged stretches for the weighted kernels (the solve's weight choice)
-    const bool merge = g.weighted && (!g.adjacency || g.adjacency_weights);
+    const bool merge = g.has_values();
     k_pb_masks<<<nblocks(groups + 1, tb), tb, 0, s>>>(srow.as<int32_t>(), groups, soff.as<uint32_t>(), S, B, merge,
                                                       g.pb_mask.as<uint8_t>(), gs.as<uint32_t>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
@@ -879,11 +1022,10 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     return EGX_SUCC;
 }
 
-int rebuild_bins(Graph& g, const BinCfg& cfg_in) {
+int rebuild_bins(Graph& g, const BinCfg& cfg_in, int32_t known_hubs) {
     BinCfg cfg = cfg_in;
     if (cfg.thread_row_max < 0) cfg.thread_row_max = 0;
-    if (cfg.wave_row_max < 1) cfg.wave_row_max = 1;
-    if (cfg.wave_row_max > kTileLds - 256) cfg.wave_row_max = kTileLds - 256;
+    cfg.wave_row_max = hub_threshold(cfg);
     if (cfg.tile_items < 256) cfg.tile_items = 256;
     if (cfg.tile_items > kTileLds - cfg.wave_row_max) cfg.tile_items = kTileLds - cfg.wave_row_max;
     if (cfg.hub_segment < 256) cfg.hub_segment = 256;
@@ -892,18 +1034,19 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in) {
     if (cfg.blocked != 0) cfg.blocked = 1;
     const bool layout_changed =
         !g.layout_built || g.layout_hub != cfg.wave_row_max || g.layout_reorder != cfg.reorder;
-    if (layout_changed) EGX_TRY(build_layout(g, cfg));
+    if (layout_changed) EGX_TRY(build_layout(g, cfg, known_hubs));
     g.bins = cfg;
     hipStream_t s = g.stream;
     const int32_t n = g.n;
     g.n_hseg = g.n_hrows = g.n_tiles = 0;
     g.rows_thread = g.rows_wave = 0;
     if (n <= 0) return EGX_SUCC;
-    std::vector<int32_t> row((size_t)n + 1);
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpyWithStream(row.data(), g.it_row, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
 
     // hub rows [0, n_hub): fixed-size segments
+    std::vector<int32_t> row((size_t)g.n_hub + 1, 0);
+    if (g.n_hub > 0)
+        EGX_HIP_TRY(hipMemcpyWithStream(row.data(), g.it_row, row.size() * 4, hipMemcpyDeviceToHost, s),
+                    EGX_DEVICE_ERR);
     std::vector<HubSeg> segs;
     std::vector<HubRow> hub_rows;
     for (int32_t v = 0; v < g.n_hub; ++v) {
@@ -926,29 +1069,40 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in) {
     g.n_hseg = (int64_t)segs.size();
     EGX_TRY(g.hsegs.alloc(std::max<size_t>(segs.size(), 1) * sizeof(HubSeg)));
     if (!segs.empty())
-        EGX_HIP_TRY(hipMemcpyWithStream(g.hsegs.p, segs.data(), segs.size() * sizeof(HubSeg), hipMemcpyHostToDevice, s),
+        EGX_HIP_TRY(hipMemcpyAsync(g.hsegs.p, segs.data(), segs.size() * sizeof(HubSeg), hipMemcpyHostToDevice, s),
                     EGX_DEVICE_ERR);
     EGX_TRY(g.hrows.alloc(std::max<size_t>(hub_rows.size(), 1) * sizeof(HubRow)));
     if (!hub_rows.empty())
-        EGX_HIP_TRY(hipMemcpyWithStream(g.hrows.p, hub_rows.data(), hub_rows.size() * sizeof(HubRow), hipMemcpyHostToDevice, s),
+        EGX_HIP_TRY(hipMemcpyAsync(g.hrows.p, hub_rows.data(), hub_rows.size() * sizeof(HubRow),
+                                   hipMemcpyHostToDevice, s),
                     EGX_DEVICE_ERR);
     EGX_TRY(g.hub_part.alloc(std::max<size_t>(segs.size(), 1) * 8));
 
     // merge-path tiles over rows [n_hub, n)
-    const int64_t items = ((int64_t)row[(size_t)n] - row[(size_t)g.n_hub]) + (int64_t)(n - g.n_hub);
+    const int64_t items = (g.m - row[(size_t)g.n_hub]) + (int64_t)(n - g.n_hub);
     g.n_tiles = (items + cfg.tile_items - 1) / cfg.tile_items;
+    DevBuf ctr;
+    EGX_TRY(ctr.alloc(kCtrWords * sizeof(uint32_t)));
+    EGX_HIP_TRY(hipMemsetAsync(ctr.p, 0, kCtrWords * sizeof(uint32_t), s), EGX_DEVICE_ERR);
     EGX_TRY(g.tiles.alloc(((size_t)g.n_tiles + 1) * 4));
     k_tile_starts<<<nblocks(g.n_tiles + 1, 256), 256, 0, s>>>(g.it_row, g.n_hub, n, cfg.tile_items, g.n_tiles,
                                                                g.tiles.as<int32_t>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    std::vector<int32_t> ts((size_t)g.n_tiles + 1);
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpyWithStream(ts.data(), g.tiles.p, ts.size() * 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-    for (int64_t k = 0; k < g.n_tiles; ++k) {
-        const int64_t r = ts[(size_t)k + 1] - ts[(size_t)k];
-        const int64_t arcs = (int64_t)row[(size_t)ts[(size_t)k + 1]] - row[(size_t)ts[(size_t)k]];
-        if (arcs > (int64_t)cfg.thread_row_max * r) g.rows_wave += r;
-        else g.rows_thread += r;
+    if (g.n_tiles > 0) {
+        k_tile_stats<<<std::min<unsigned>(nblocks(g.n_tiles, 256), kNodeBlocks), 256, 0, s>>>(
+            g.it_row, g.tiles.as<int32_t>(), g.n_tiles, cfg.thread_row_max, ctr.as<uint32_t>());
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    }
+    // (also waits for the copies out of segs and hub_rows)
+    uint32_t wave_rows = 0;
+    EGX_HIP_TRY(hipMemcpyWithStream(&wave_rows, ctr.as<uint32_t>() + kCtrWaveRows, 4, hipMemcpyDeviceToHost, s),
+                EGX_DEVICE_ERR);
+    g.rows_wave = wave_rows;
+    g.rows_thread = (int64_t)(n - g.n_hub) - g.rows_wave;
+    if (layout_changed) {
+        float ms = 0.0f;
+        EGX_HIP_TRY(hipEventElapsedTime(&ms, g.ev0, g.ev1), EGX_DEVICE_ERR);
+        g.layout_seconds = (double)ms * 1e-3;
     }
     EGX_TRY(build_tile_sort(g, cfg));
     const int rc = build_blocked(g, cfg, layout_changed);
@@ -977,7 +1131,7 @@ int transpose_csr(const int32_t* dV, const int32_t* dE, int32_t n, int64_t m, De
     EGX_TRY(Vt.alloc(((size_t)n + 1) * 4, s));
     if (m > 0) {
         EGX_HIP_TRY(hipMemcpyAsync(keys.p, dE, (size_t)m * 4, hipMemcpyDeviceToDevice, s), EGX_DEVICE_ERR);
-        k_expand_src<<<nblocks(m, 256), 256, 0, s>>>(dV, n, m, Et.as<int32_t>());
+        k_expand_src<<<nblocks(m, kRunArcs), kRunThreads, 0, s>>>(dV, n, m, Et.as<int32_t>());
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     }
     EGX_TRY(radix_sort_u32(keys, keys_alt, &Et, &vals_alt, m, bits_for((uint64_t)std::max(n - 1, 0)), s));
@@ -999,110 +1153,130 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
     g.alpha_vals = alpha;
     g.alpha_orig = alpha;
     const auto t_start = std::chrono::steady_clock::now();
-
-    // [0] invalid endpoints, [1] dangling nodes, [2] largest out-degree,
-    // [3] largest in-degree, [4] rows longer than kOutLong
-    DevBuf ctr, long_rows;
-    EGX_TRY(ctr.alloc(5 * sizeof(uint32_t)));
-    EGX_HIP_TRY(hipMemsetAsync(ctr.p, 0, 5 * sizeof(uint32_t), s), EGX_DEVICE_ERR);
-
-    EGX_TRY(g.out_w.alloc((size_t)std::max(n, 1) * 8));
-    EGX_TRY(g.deg.alloc((size_t)std::max(n, 1) * 4));
-    EGX_TRY(g.out_cnt.alloc((size_t)std::max(n, 1) * 4));
-    int32_t* outcnt_p = g.out_cnt.as<int32_t>();
-
-    DevBuf src, keys, keys_alt, vals, vals_alt;
+    const bool values = g.has_values();
     const size_t mm = (size_t)std::max<int64_t>(m, 1);
-    EGX_TRY(src.alloc(mm * 4));
+    const size_t nn = (size_t)std::max(n, 1);
+
+    // The sizes that the host needs (valid arcs, hub rows, the largest
+    // out-degree) come back in one copy, after everything that does not
+    // depend on them has been queued.
+    DevBuf ctr_buf, long_rows, keys, keys_alt, vals, vals_alt, rec;
+    EGX_TRY(ctr_buf.alloc(kCtrWords * sizeof(uint32_t)));
+    uint32_t* ctr = ctr_buf.as<uint32_t>();
+    EGX_HIP_TRY(hipMemsetAsync(ctr, 0, kCtrWords * sizeof(uint32_t), s), EGX_DEVICE_ERR);
+    EGX_TRY(g.out_w.alloc(nn * 8));
+    EGX_TRY(g.deg.alloc(nn * 4));
+    EGX_TRY(g.out_cnt.alloc(nn * 4));
+    EGX_TRY(g.in_row.alloc(((size_t)n + 1) * 4));
+    int32_t* outcnt_p = g.out_cnt.as<int32_t>();
+    double* out_w = g.out_w.as<double>();
     EGX_TRY(keys.alloc(mm * 4));
     EGX_TRY(keys_alt.alloc(mm * 4));
-    EGX_TRY(vals.alloc(mm * 4));
-    EGX_TRY(vals_alt.alloc(mm * 4));
-    if (m > 0) {
-        k_expand_src<<<nblocks(m, 256), 256, 0, s>>>(dV, n, m, src.as<int32_t>());
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        k_make_sort_keys<<<nblocks(m, 256), 256, 0, s>>>(dE, src.as<int32_t>(), n, m, g.weighted ? 1 : 0,
-                                                          keys.as<uint32_t>(), vals.as<uint32_t>(), ctr.as<uint32_t>());
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    }
-    uint32_t invalid = 0;
-    EGX_HIP_TRY(hipMemcpyAsync(&invalid, ctr.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    if (n > 0) {
-        if (!dW && invalid == 0) {
-            k_outcnt_from_V<<<nblocks(n, 256), 256, 0, s>>>(dV, n, g.out_w.as<double>(), outcnt_p);
-            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        } else {
-            // at most m / kOutLong rows are longer than kOutLong
-            const int64_t max_long = m / kOutLong;
-            EGX_TRY(long_rows.alloc((size_t)std::max<int64_t>(max_long, 1) * 4));
-            int32_t* lr = long_rows.as<int32_t>();
-            uint32_t* nl = ctr.as<uint32_t>() + 4;
-            const unsigned lb = (unsigned)std::min<int64_t>(max_long, kLongBlocks);
-            const unsigned sb = nblocks((int64_t)n * kOutLanes, 256);
-            if (dW) k_row_out<true><<<sb, 256, 0, s>>>(dV, dE, dW, n, g.out_w.as<double>(), outcnt_p, lr, nl);
-            else k_row_out<false><<<sb, 256, 0, s>>>(dV, dE, nullptr, n, g.out_w.as<double>(), outcnt_p, lr, nl);
-            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-            if (lb > 0) {
-                if (dW) k_row_out_long<true><<<lb, 256, 0, s>>>(dV, dE, dW, n, g.out_w.as<double>(), outcnt_p, lr, nl);
-                else k_row_out_long<false><<<lb, 256, 0, s>>>(dV, dE, nullptr, n, g.out_w.as<double>(), outcnt_p, lr,
-                                                              nl);
-                EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-            }
-        }
-        if (g.adjacency) {
-            k_unit_out_w<<<nblocks(n, 256), 256, 0, s>>>(g.out_w.as<double>(), n);
-            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        }
-        k_node_arrays<<<nblocks(n, 256), 256, 0, s>>>(g.out_w.as<double>(), outcnt_p, n,
-                                                       g.weighted ? 1 : 0, g.deg.as<float>(), ctr.as<uint32_t>());
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    }
+    EGX_TRY(vals.alloc((mm + kArcPad) * 4));
+    EGX_TRY(vals_alt.alloc((mm + kArcPad) * 4));
+    if (values) EGX_TRY(rec.alloc(mm * sizeof(ArcRec)));
 
+    // out-weights and counts by the arcs themselves (weights, or endpoints to skip), or by the offsets
+    auto out_by_arcs = [&]() -> int {
+        // at most m / kOutLong rows are longer than kOutLong
+        const int64_t max_long = m / kOutLong;
+        EGX_TRY(long_rows.alloc((size_t)std::max<int64_t>(max_long, 1) * 4));
+        int32_t* lr = long_rows.as<int32_t>();
+        uint32_t* nl = ctr + kCtrLong;
+        const unsigned lb = (unsigned)std::min<int64_t>(max_long, kLongBlocks);
+        const unsigned sb = nblocks((int64_t)n * kOutLanes, 256);
+        if (dW) k_row_out<true><<<sb, 256, 0, s>>>(dV, dE, dW, n, out_w, outcnt_p, lr, nl);
+        else k_row_out<false><<<sb, 256, 0, s>>>(dV, dE, nullptr, n, out_w, outcnt_p, lr, nl);
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        if (lb > 0) {
+            if (dW) k_row_out_long<true><<<lb, 256, 0, s>>>(dV, dE, dW, n, out_w, outcnt_p, lr, nl);
+            else k_row_out_long<false><<<lb, 256, 0, s>>>(dV, dE, nullptr, n, out_w, outcnt_p, lr, nl);
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        }
+        return EGX_SUCC;
+    };
+    auto unit_out = [&]() -> int {
+        if (!g.adjacency) return EGX_SUCC;
+        k_unit_out_w<<<nblocks(n, 256), 256, 0, s>>>(out_w, n);
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        return EGX_SUCC;
+    };
+    const unsigned node_blocks = std::min<unsigned>(nblocks(n, 256), kNodeBlocks);
+    auto node_arrays = [&]() -> int {
+        k_node_arrays<<<node_blocks, 256, 0, s>>>(out_w, outcnt_p, n, g.weighted ? 1 : 0, g.deg.as<float>(), ctr);
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        return EGX_SUCC;
+    };
+    if (n > 0) {
+        if (dW) {
+            EGX_TRY(out_by_arcs());
+        } else {
+            k_outcnt_from_V<<<nblocks(n, 256), 256, 0, s>>>(dV, n, out_w, outcnt_p);
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        }
+        EGX_TRY(unit_out());
+        EGX_TRY(node_arrays());
+    }
+    if (m > 0) {
+        const unsigned rb = nblocks(m, kRunArcs);
+        if (values)
+            k_arc_keys<true><<<rb, kRunThreads, 0, s>>>(dV, dE, dW, out_w, n, m, alpha, keys.as<uint32_t>(),
+                                                        vals.as<uint32_t>(), rec.as<ArcRec>(), ctr + kCtrInvalid);
+        else
+            k_arc_keys<false><<<rb, kRunThreads, 0, s>>>(dV, dE, nullptr, nullptr, n, m, alpha, keys.as<uint32_t>(),
+                                                         vals.as<uint32_t>(), nullptr, ctr + kCtrInvalid);
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    }
     // stable sort of (dst-or-sentinel, slot-or-src) on the bits that can hold n
     EGX_TRY(radix_sort_u32(keys, keys_alt, &vals, &vals_alt, m, bits_for((uint64_t)n), s));
+    EGX_TRY(lower_bound_iota_u32(keys.as<uint32_t>(), m, g.in_row.as<int32_t>(), (int64_t)n + 1, s));
+    if (n > 0) {
+        k_in_degrees<<<node_blocks, 256, 0, s>>>(g.in_row.as<int32_t>(), n, hub_threshold(g.bins), ctr);
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    }
+    uint32_t hctr[kCtrWords];
+    EGX_HIP_TRY(hipMemcpyWithStream(hctr, ctr, sizeof(hctr), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+    if (hctr[kCtrInvalid] > 0 && !dW && n > 0) {
+        // skipped endpoints: the offsets counted them
+        EGX_HIP_TRY(hipMemsetAsync(ctr, 0, kCtrWords * sizeof(uint32_t), s), EGX_DEVICE_ERR);
+        EGX_TRY(out_by_arcs());
+        EGX_TRY(unit_out());
+        EGX_TRY(node_arrays());
+        uint32_t again[kCtrWords];
+        EGX_HIP_TRY(hipMemcpyWithStream(again, ctr, sizeof(again), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+        hctr[kCtrDangling] = again[kCtrDangling];
+        hctr[kCtrMaxOut] = again[kCtrMaxOut];
+    }
+    const int64_t m_valid = m - (int64_t)hctr[kCtrInvalid];
+    g.m = m_valid;
+    g.n_dangling = hctr[kCtrDangling];
+    g.max_out_degree = (int32_t)hctr[kCtrMaxOut];
+    g.max_in_degree = (int32_t)hctr[kCtrMaxIn];
+    keys.release();
     keys_alt.release();
     vals_alt.release();
 
-    EGX_TRY(g.in_row.alloc(((size_t)n + 1) * 4));
-    EGX_TRY(lower_bound_iota_u32(keys.as<uint32_t>(), m, g.in_row.as<int32_t>(), (int64_t)n + 1, s));
-    int32_t m_valid = 0;
-    EGX_HIP_TRY(hipMemcpyAsync(&m_valid, g.in_row.as<int32_t>() + n, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    g.m = m_valid;
-
-    EGX_TRY(g.in_col.alloc(((size_t)std::max(m_valid, 1) + kArcPad) * 4));
-    EGX_HIP_TRY(hipMemsetAsync(g.in_col.as<int32_t>() + m_valid, 0, kArcPad * 4, s), EGX_DEVICE_ERR);
-    if (g.weighted) {
-        EGX_TRY(g.in_val.alloc((size_t)std::max(m_valid, 1) * 4));
-        EGX_TRY(g.w_csc.alloc((size_t)std::max(m_valid, 1) * 8));
+    if (values) {
+        const size_t mv = (size_t)std::max<int64_t>(m_valid, 1);
+        EGX_TRY(g.in_col.alloc((mv + kArcPad) * 4));
+        EGX_TRY(g.in_val.alloc(mv * 4));
+        EGX_TRY(g.w_csc.alloc(mv * 8));
+        if (m_valid > 0) {
+            k_fill_csc<<<nblocks(m_valid, 256), 256, 0, s>>>(vals.as<uint32_t>(), rec.as<ArcRec>(), m_valid,
+                                                              g.in_col.as<int32_t>(), g.in_val.as<float>(),
+                                                              g.w_csc.as<double>());
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        }
+        vals.release();
+        rec.release();
     } else {
+        g.in_col = std::move(vals);  // the sorted sources
         g.in_val.release();
         g.w_csc.release();
     }
-    if (m_valid > 0) {
-        k_fill_csc<<<nblocks(m_valid, 256), 256, 0, s>>>(vals.as<uint32_t>(), src.as<int32_t>(), dW,
-                                                          g.out_w.as<double>(), m_valid, g.weighted ? 1 : 0, alpha,
-                                                          g.in_col.as<int32_t>(), g.in_val.as<float>(),
-                                                          g.w_csc.as<double>());
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    }
-    if (n > 0) {
-        k_max_in_degree<<<nblocks(n, 256), 256, 0, s>>>(g.in_row.as<int32_t>(), n, ctr.as<uint32_t>() + 3);
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    }
-    uint32_t hctr[4];
-    EGX_HIP_TRY(hipMemcpyAsync(hctr, ctr.p, sizeof(hctr), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    g.n_dangling = hctr[1];
-    g.max_out_degree = (int32_t)hctr[2];
-    g.max_in_degree = (int32_t)hctr[3];
-
-    src.release();
-    keys.release();
-    vals.release();
+    EGX_HIP_TRY(hipMemsetAsync(g.in_col.as<int32_t>() + m_valid, 0, kArcPad * 4, s), EGX_DEVICE_ERR);
     g.layout_built = false;
-    EGX_TRY(rebuild_bins(g, g.bins));
+    EGX_TRY(rebuild_bins(g, g.bins, (int32_t)hctr[kCtrHubs]));
     // large PageRank graphs iterate propagation-blocked; one the layout
     // cannot hold keeps the pull layout alone
     if (!g.adjacency && m >= kPbDefaultArcs && !g.bins.blocked) {
@@ -1121,7 +1295,7 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
     return EGX_SUCC;
 }
 
-int build_layout(Graph& g, const BinCfg& cfg) {
+int build_layout(Graph& g, const BinCfg& cfg, int32_t known_hubs) {
     hipStream_t s = g.stream;
     const int32_t n = g.n;
     const int64_t m = g.m;
@@ -1155,20 +1329,29 @@ int build_layout(Graph& g, const BinCfg& cfg) {
     EGX_HIP_TRY(hipEventRecord(g.ev0, s), EGX_DEVICE_ERR);
     const uint32_t maxdeg = (uint32_t)g.max_out_degree;
     const int bits = cfg.reorder ? bits_for(maxdeg) : 0;
-    DevBuf keys, keys_alt, vals_alt, cnt, hubs;
+    DevBuf keys, keys_alt, vals_alt, cnt;
+    int32_t nh = known_hubs;
+    if (nh < 0) {
+        DevBuf ctr;
+        uint32_t hubs = 0;
+        EGX_TRY(ctr.alloc(kCtrWords * sizeof(uint32_t)));
+        EGX_HIP_TRY(hipMemsetAsync(ctr.p, 0, kCtrWords * sizeof(uint32_t), s), EGX_DEVICE_ERR);
+        k_in_degrees<<<std::min<unsigned>(nblocks(n, 256), kNodeBlocks), 256, 0, s>>>(
+            g.in_row.as<int32_t>(), n, cfg.wave_row_max, ctr.as<uint32_t>());
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyWithStream(&hubs, ctr.as<uint32_t>() + kCtrHubs, 4, hipMemcpyDeviceToHost, s),
+                    EGX_DEVICE_ERR);
+        nh = (int32_t)hubs;
+    }
     EGX_TRY(keys.alloc((size_t)n * 4));
     EGX_TRY(keys_alt.alloc((size_t)n * 4));
     EGX_TRY(g.perm.alloc((size_t)n * 4));
     EGX_TRY(vals_alt.alloc((size_t)n * 4));
-    EGX_TRY(hubs.alloc(4));
-    EGX_HIP_TRY(hipMemsetAsync(hubs.p, 0, 4, s), EGX_DEVICE_ERR);
     k_layout_keys<<<nblocks(n, 256), 256, 0, s>>>(g.in_row.as<int32_t>(), g.out_cnt.as<int32_t>(), n,
                                                    cfg.wave_row_max, bits, maxdeg, cfg.reorder,
-                                                   keys.as<uint32_t>(), g.perm.as<uint32_t>(), hubs.as<uint32_t>());
+                                                   keys.as<uint32_t>(), g.perm.as<uint32_t>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     EGX_TRY(radix_sort_u32(keys, keys_alt, &g.perm, &vals_alt, n, bits + 1, s));
-    uint32_t nh = 0;
-    EGX_HIP_TRY(hipMemcpyWithStream(&nh, hubs.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     keys.release();
     keys_alt.release();
     vals_alt.release();
@@ -1185,26 +1368,25 @@ int build_layout(Graph& g, const BinCfg& cfg) {
     EGX_TRY(exclusive_scan_u32(cnt.as<uint32_t>(), g.p_row.as<uint32_t>(), n, s));
     k_set_last<<<1, 64, 0, s>>>(g.p_row.as<int32_t>(), n, (int32_t)m);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     cnt.release();
 
     EGX_TRY(g.p_col.alloc(((size_t)std::max<int64_t>(m, 1) + kArcPad) * 4));
     EGX_HIP_TRY(hipMemsetAsync(g.p_col.as<int32_t>() + m, 0, kArcPad * 4, s), EGX_DEVICE_ERR);
-    if (g.weighted) {
+    if (g.has_values()) {
         EGX_TRY(g.p_val.alloc((size_t)std::max<int64_t>(m, 1) * 4));
         EGX_TRY(g.p_w.alloc((size_t)std::max<int64_t>(m, 1) * 8));
     }
     if (m > 0) {
-        k_layout_slots<<<nblocks(m, 256), 256, 0, s>>>(g.p_row.as<int32_t>(), g.perm.as<int32_t>(),
+        k_layout_slots<<<nblocks(m, kRunArcs), kRunThreads, 0, s>>>(g.p_row.as<int32_t>(), g.perm.as<int32_t>(),
                                                         g.rank.as<int32_t>(), g.in_row.as<int32_t>(),
                                                         g.in_col.as<int32_t>(), g.in_val.as<float>(),
-                                                        g.w_csc.as<double>(), n, m, g.weighted ? 1 : 0,
+                                                        g.w_csc.as<double>(), n, m, g.has_values() ? 1 : 0,
                                                         g.p_col.as<int32_t>(), g.p_val.as<float>(),
                                                         g.p_w.as<double>());
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     }
     g.reordered = true;
-    g.n_hub = (int32_t)nh;
+    g.n_hub = nh;
     g.it_row = g.p_row.as<int32_t>();
     g.it_col = g.p_col.as<int32_t>();
     g.it_val = g.p_val.as<float>();
@@ -1212,10 +1394,6 @@ int build_layout(Graph& g, const BinCfg& cfg) {
     g.it_outw = g.p_outw.as<double>();
     g.it_deg = g.p_deg.as<float>();
     EGX_HIP_TRY(hipEventRecord(g.ev1, s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipEventSynchronize(g.ev1), EGX_DEVICE_ERR);
-    float ms = 0.0f;
-    EGX_HIP_TRY(hipEventElapsedTime(&ms, g.ev0, g.ev1), EGX_DEVICE_ERR);
-    g.layout_seconds = (double)ms * 1e-3;
     g.layout_built = true;
     g.layout_hub = cfg.wave_row_max;
     g.layout_reorder = cfg.reorder;
@@ -1223,8 +1401,8 @@ int build_layout(Graph& g, const BinCfg& cfg) {
 }
 
 int refresh_alpha(Graph& g, double alpha) {
-    if (!g.weighted || alpha == g.alpha_vals) {
-        if (!g.weighted) g.alpha_vals = alpha;
+    if (!g.has_values() || alpha == g.alpha_vals) {
+        if (!g.has_values()) g.alpha_vals = alpha;
         return EGX_SUCC;
     }
     if (g.m > 0) {

@@ -154,6 +154,9 @@ struct Graph {
     // adjacency graph built with weights: the weighted kernels gather
     // fl32(alpha * w) (eigenvector centrality); false: unit weights
     bool adjacency_weights = false;
+    // the arc value arrays (in_val, w_csc, p_val, p_w, ...) exist: weighted
+    // graphs, and adjacency graphs whose kernels gather weights
+    bool has_values() const { return weighted && (!adjacency || adjacency_weights); }
     // propagation-blocked layout (bins.blocked): pb_src uint16 chunk-local
     // source per slot in (chunk, sub-bin, row, source) order; per kPbVec-slot
     // group of it, pb_mask uint8 (bit j: a stretch of one row starts at slot
@@ -232,7 +235,7 @@ struct Graph {
 // egx_build.hip.  With g.adjacency set, dW may be null (unit weights).
 int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const double* dW, int32_t n,
                           int64_t m, double alpha);
-int build_layout(Graph& g, const BinCfg& cfg);
+int build_layout(Graph& g, const BinCfg& cfg, int32_t known_hubs = -1);
 // Queue the device check of a host CSR's arcs on s: *flags (device, zeroed
 // here) gets kArcBadEndpoint / kArcBadWeight (not finite or negative; dW may
 // be null).
@@ -242,7 +245,8 @@ int check_arcs(const int32_t* dE, const double* dW, int32_t n, int64_t m, uint32
 // of (Vt, Et) lists the u with u->v.  Endpoints outside [0, n) leave Vt and Et unspecified.
 int transpose_csr(const int32_t* dV, const int32_t* dE, int32_t n, int64_t m, DevBuf& Vt, DevBuf& Et,
                   hipStream_t s);
-int rebuild_bins(Graph& g, const BinCfg& cfg);
+// known_hubs: the number of rows above the hub threshold, if the caller counted them (else < 0)
+int rebuild_bins(Graph& g, const BinCfg& cfg, int32_t known_hubs = -1);
 int refresh_alpha(Graph& g, double alpha);
 int download_csc(Graph& g, int32_t* in_row, int32_t* in_col, float* in_val, int32_t* dangling01);
 
