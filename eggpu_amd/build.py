@@ -21,6 +21,7 @@ ARCH = os.environ.get("EGX_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = [
     "egx_prim.hip",
+    "egx_xfer.hip",
     "egx_build.hip",
     "egx_gen.hip",
     "egx_pagerank.hip",

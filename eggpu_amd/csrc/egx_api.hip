@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "egx_graph.h"
+#include "egx_xfer.h"
 
 namespace egx {
 
@@ -188,11 +189,6 @@ int graph_from_host_csr(const int32_t* V, const int32_t* E, const double* W, int
     DevBuf dV, dE, dW;
     EGX_TRY(dV.alloc(((size_t)n + 1) * 4));
     EGX_TRY(dE.alloc((size_t)std::max(m, 1) * 4));
-    // pageable copies: a pinned staging arena measured 0.3 ms faster per
-    // build at R-MAT 14 but its first allocation (1 MB) took 7-8 ms
-    if (n > 0) EGX_HIP_TRY(hipMemcpyWithStream(dV.p, V, ((size_t)n + 1) * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
-    else EGX_HIP_TRY(hipMemsetAsync(dV.p, 0, 4, g.stream), EGX_DEVICE_ERR);
-    if (m > 0) EGX_HIP_TRY(hipMemcpyWithStream(dE.p, E, (size_t)m * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
     // weights that are all exactly 1 (the reference's unweighted_W, gen_CSR
     // graph.cpp:881) give the unweighted graph: the same pull CSC bit for bit
     // (in_val = fl32(alpha * (1/outdeg)) either way), iterated by the
@@ -200,10 +196,11 @@ int graph_from_host_csr(const int32_t* V, const int32_t* E, const double* W, int
     bool unit = W != nullptr;
     for (int32_t i = 0; unit && i < m; ++i) unit = W[i] == 1.0;
     const bool upload_w = W && (!unit || keep_csr);
-    if (upload_w) {
-        EGX_TRY(dW.alloc((size_t)std::max(m, 1) * 8));
-        if (m > 0) EGX_HIP_TRY(hipMemcpyWithStream(dW.p, W, (size_t)m * 8, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
-    }
+    if (upload_w) EGX_TRY(dW.alloc((size_t)std::max(m, 1) * 8));
+    if (n == 0) EGX_HIP_TRY(hipMemsetAsync(dV.p, 0, 4, g.stream), EGX_DEVICE_ERR);
+    EGX_TRY(upload({Upload{dV.p, V, n > 0 ? ((size_t)n + 1) * 4 : 0}, Upload{dE.p, E, (size_t)m * 4},
+                    Upload{dW.p, W, upload_w ? (size_t)m * 8 : 0}},
+                   g.stream));
     EGX_TRY(build_from_device_csr(g, dV.as<int32_t>(), dE.as<int32_t>(), (W && !unit) ? dW.as<double>() : nullptr,
                                   n, m, alpha));
     if (keep_csr) {
@@ -353,7 +350,6 @@ Graph::~Graph() {
     if (stream) (void)hipStreamSynchronize(stream);
     for (DevBuf* b : buffers()) b->release_idle();
     give_state_slot(host_state);
-    if (host_result) (void)hipHostFree(host_result);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     give_stream(device, stream);

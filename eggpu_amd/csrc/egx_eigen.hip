@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "egx_graph.h"
+#include "egx_xfer.h"
 
 extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const double* W, int32_t n, int32_t m,
                                    const double* x0, const egx_eig_opts* opts, double* out, int32_t* iterations,
@@ -164,12 +165,11 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
     DevBuf dV, dE, dW, dx, flags;
     EGX_TRY(dV.alloc(((size_t)n + 1) * 4));
     EGX_TRY(dE.alloc((size_t)m * 4));
-    EGX_HIP_TRY(hipMemcpyWithStream(dV.p, V, ((size_t)n + 1) * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpyWithStream(dE.p, E, (size_t)m * 4, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
-    if (W) {
-        EGX_TRY(dW.alloc((size_t)m * 8));
-        EGX_HIP_TRY(hipMemcpyWithStream(dW.p, W, (size_t)m * 8, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
-    }
+    if (W) EGX_TRY(dW.alloc((size_t)m * 8));
+    EGX_TRY(dx.alloc((size_t)n * 8));
+    EGX_TRY(upload({Upload{dV.p, V, ((size_t)n + 1) * 4}, Upload{dE.p, E, (size_t)m * 4},
+                    Upload{dW.p, W, W ? (size_t)m * 8 : 0}, Upload{dx.p, x.data(), (size_t)n * 8}},
+                   g.stream));
     uint32_t bad = 0;
     EGX_TRY(flags.alloc(4));
     EGX_TRY(check_arcs(dE.as<int32_t>(), W ? dW.as<double>() : nullptr, n, m, flags.as<uint32_t>(), g.stream));
@@ -180,9 +180,6 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
     dV.release();
     dE.release();
     dW.release();
-    EGX_TRY(dx.alloc((size_t)n * 8));
-    EGX_HIP_TRY(hipMemcpyWithStream(dx.p, x.data(), (size_t)n * 8, hipMemcpyHostToDevice, g.stream), EGX_DEVICE_ERR);
-
     SolveParams p;
     p.alpha = 1.0;
     p.max_iter = o.max_iter;

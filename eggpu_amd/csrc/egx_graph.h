@@ -222,10 +222,6 @@ struct Graph {
     DevBuf x[2], s[2], state, partials, red_part, out;
     int64_t partial_blocks = 0;
     void* host_state = nullptr;  // pinned PrState
-    // pinned staging of a packed PageRank result (kPackedHeader + 4 n bytes),
-    // made on the first download and kept
-    char* host_result = nullptr;
-
     ~Graph();
     static constexpr size_t kBuffers = 46;  // every DevBuf above
     std::array<DevBuf*, kBuffers> buffers();
@@ -354,7 +350,7 @@ constexpr size_t kPackedHeader = 16;  // the sum, padded so the floats start 16-
 int batch_result_enqueue(egx_batch* b, int32_t slot, void* host_out, hipEvent_t done);
 
 // out[v] = (double)x[v] * (1.0 / s) if s > 0, else 1.0 / n: the arithmetic
-// of the device's FP64 output (k_spmm_output), on a packed result.
+// of the device's FP64 output (k_pr_output), on a packed result.
 inline void unpack_result(const void* packed, int32_t n, double* out) {
     const double s = *static_cast<const double*>(packed);
     const float* x = reinterpret_cast<const float*>(static_cast<const char*>(packed) + kPackedHeader);

@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "egx_graph.h"
+#include "egx_xfer.h"
 
 namespace egx {
 namespace {
@@ -129,8 +130,7 @@ extern "C" int egx_katz_csr(const int32_t* V, const int32_t* E, int32_t n, int32
             EGX_TRY(cV.alloc(((size_t)n + 1) * 4));
             EGX_TRY(cE.alloc((size_t)m * 4));
             EGX_TRY(flags.alloc(4));
-            EGX_HIP_TRY(hipMemcpyWithStream(cV.p, V, ((size_t)n + 1) * 4, hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
-            EGX_HIP_TRY(hipMemcpyWithStream(cE.p, E, (size_t)m * 4, hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
+            EGX_TRY(upload({Upload{cV.p, V, ((size_t)n + 1) * 4}, Upload{cE.p, E, (size_t)m * 4}}, s));
             EGX_TRY(check_arcs(cE.as<int32_t>(), nullptr, n, m, flags.as<uint32_t>(), s));
             EGX_TRY(transpose_csr(cV.as<int32_t>(), cE.as<int32_t>(), n, m, dV, dE, s));
         }
@@ -170,7 +170,7 @@ extern "C" int egx_katz_csr(const int32_t* V, const int32_t* E, int32_t n, int32
             k_katz_scale<<<nblk(n, 1024), 256, 0, s>>>(part.as<double>(), n, res.as<double>());
             EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         }
-        EGX_HIP_TRY(hipMemcpyWithStream(out, res.p, (size_t)n * 8, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+        EGX_TRY(fetch({Fetch{res.p, out, n, false, 0.0}}, s));
         if (converged) *converged = stopped ? 1 : 0;
         return EGX_SUCC;
     }

@@ -45,6 +45,7 @@
 #include <vector>
 
 #include "egx_graph.h"
+#include "egx_xfer.h"
 
 namespace egx {
 
@@ -1197,19 +1198,28 @@ int prepare_graph(Graph& g, const SolveParams& p, hipStream_t s, IterArgs<T>& a)
     return EGX_SUCC;
 }
 
-// The packed form of the FP32 PageRank result: the iterate's sum (FP64) in
-// the header, then the FP32 iterate in caller order, half the bytes of the
-// FP64 result; unpack_result finishes it on the host with k_pr_output's
-// arithmetic, bit for bit.
+// The packed form of an FP32 PageRank result: the iterate in caller order,
+// half the bytes of the FP64 result; fetch() finishes it on the host with
+// k_pr_output's arithmetic, bit for bit.
 __global__ void k_pr_output_packed(const float* __restrict__ x0, const float* __restrict__ x1,
                                    const PrState* __restrict__ st, const int32_t* __restrict__ perm, int32_t n,
-                                   char* __restrict__ out) {
+                                   float* __restrict__ out) {
     const int32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r == 0) *reinterpret_cast<double*>(out) = st->sum;
     if (r >= n) return;
     const float* x = (st->iter & 1) ? x1 : x0;
     const int32_t v = perm ? perm[r] : r;
-    reinterpret_cast<float*>(out + kPackedHeader)[v] = x[r];
+    out[v] = x[r];
+}
+
+// The same for every graph of the table.
+__global__ void k_pr_output_packed_multi(const IterArgs<float>* __restrict__ table,
+                                         const uint32_t* __restrict__ nbase, int32_t count) {
+    const int32_t gi = graph_of_block(nbase, count, blockIdx.x);
+    const IterArgs<float>& a = table[gi];
+    const int32_t r = (int32_t)(blockIdx.x - nbase[gi]) * blockDim.x + threadIdx.x;
+    if (r >= a.n) return;
+    const float* x = (a.state->iter & 1) ? a.xb[1] : a.xb[0];
+    reinterpret_cast<float*>(a.out)[a.perm ? a.perm[r] : r] = x[r];
 }
 
 // Writes the result of graph g to a.out (and copies it to host_out):
@@ -1226,8 +1236,7 @@ int emit_result(const Graph& g, const IterArgs<T>& a, hipStream_t s, double* hos
     else
         k_pr_output<T><<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], a.state, perm, g.n, a.out);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    if (host_out)
-        EGX_HIP_TRY(hipMemcpyAsync(host_out, a.out, (size_t)g.n * 8, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+    if (host_out) return fetch({Fetch{a.out, host_out, g.n, false, 0.0}}, s);
     return EGX_SUCC;
 }
 
@@ -1350,20 +1359,13 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
     }
     if constexpr (std::is_same<T, float>::value) {
         // a PageRank result for the host only crosses PCIe packed (FP32
-        // iterate and its sum) and is finished here; a.out, the graph's own
-        // buffer of n >= 4 doubles, has room for the packed form
-        if (host_out && p.out_device == nullptr && p.bias == nullptr && p.eig_delta == 0 && g.n >= 4) {
-            const size_t bytes = kPackedHeader + (size_t)g.n * 4;
-            if (!g.host_result)
-                EGX_HIP_TRY(hipHostMalloc((void**)&g.host_result, bytes), EGX_FAILED_TO_ALLOCATE_HOST_MEM);
+        // iterate; its sum is in the state) and is finished here
+        if (host_out && p.out_device == nullptr && p.bias == nullptr && p.eig_delta == 0) {
             k_pr_output_packed<<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], a.state,
                                                              g.reordered ? g.perm.as<int32_t>() : nullptr, g.n,
-                                                             reinterpret_cast<char*>(a.out));
+                                                             reinterpret_cast<float*>(a.out));
             EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-            EGX_HIP_TRY(hipMemcpyAsync(g.host_result, a.out, bytes, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-            EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-            unpack_result(g.host_result, g.n, host_out);
-            return EGX_SUCC;
+            return fetch({Fetch{a.out, host_out, g.n, true, hs->sum}}, s);
         }
     }
     EGX_TRY(emit_result<T>(g, a, s, host_out, p.bias != nullptr, p.eig_delta != 0));
@@ -1639,16 +1641,29 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     EGX_HIP_TRY(hipMemcpyAsync(hs, d_states.p, sizeof(PrState) * (size_t)count, hipMemcpyDeviceToHost, s),
                 EGX_DEVICE_ERR);
-    // every normalised result in one launch; copies only where asked for
-    k_pr_output_multi<T><<<nbase[(size_t)count], 256, 0, s>>>(d_table.as<IterArgs<T>>(), d_nbase.as<uint32_t>(),
-                                                                count);
+    // every result in one launch (FP32 ones for the host packed), copied only where asked for
+    bool wanted = false;
+    for (int32_t i = 0; i < count; ++i) wanted = wanted || (host_out && host_out[i]);
+    constexpr bool kPacked = std::is_same<T, float>::value;
+    bool packed = false;
+    if constexpr (kPacked) {
+        packed = wanted;
+        if (packed)
+            k_pr_output_packed_multi<<<nbase[(size_t)count], 256, 0, s>>>(d_table.as<IterArgs<T>>(),
+                                                                          d_nbase.as<uint32_t>(), count);
+    }
+    if (!packed)
+        k_pr_output_multi<T><<<nbase[(size_t)count], 256, 0, s>>>(d_table.as<IterArgs<T>>(), d_nbase.as<uint32_t>(),
+                                                                    count);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    for (int32_t i = 0; i < count; ++i)
-        if (host_out && host_out[i])
-            EGX_HIP_TRY(hipMemcpyAsync(host_out[i], gs[(size_t)i]->out.p, (size_t)gs[(size_t)i]->n * 8,
-                                       hipMemcpyDeviceToHost, s),
-                        EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);  // the states are on the host
+    if (wanted) {
+        std::vector<Fetch> jobs;
+        for (int32_t i = 0; i < count; ++i)
+            if (host_out[i])
+                jobs.push_back(Fetch{gs[(size_t)i]->out.p, host_out[i], gs[(size_t)i]->n, packed, hs[i].sum});
+        EGX_TRY(fetch(jobs, s));
+    }
     if (st) {
         float ms = 0.0f;
         EGX_HIP_TRY(hipEventElapsedTime(&ms, ev0, ev1), EGX_DEVICE_ERR);

@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "egx_graph.h"
+#include "egx_xfer.h"
 
 struct egx_batch;
 
@@ -870,16 +871,31 @@ __global__ void k_spmm_repack(const float* __restrict__ src, int32_t cs, float* 
     dst[i] = (c < cs) ? src[v * cs + c] : 0.0f;
 }
 
-// out[perm[r]] = x[r][j] / sum_j, from the current X (read from ctl)
-__global__ void k_spmm_output(const float* __restrict__ x0, const float* __restrict__ x1,
-                              const BatchCtl* __restrict__ ctl, int32_t stride, const ColState* __restrict__ cols,
-                              const int32_t* perm, int32_t n, int32_t j, double* __restrict__ out) {
-    const int32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n) return;
+// Columns [j0, j0 + count) of the current X in caller order, packed: column
+// j0 + q at out + q * n.  X is row-major, so one column by itself reads whole
+// rows for 4 bytes each (64 columns of 300K nodes: 64 launches of 7.7 us);
+// a workgroup turns kTurn rows around in LDS instead, reading each row once
+// and writing kTurn consecutive values per column.
+constexpr int kTurn = 64;
+template <int C>
+__global__ __launch_bounds__(kRowThreads) void k_spmm_columns(const float* __restrict__ x0,
+                                                              const float* __restrict__ x1,
+                                                              const BatchCtl* __restrict__ ctl,
+                                                              const int32_t* __restrict__ rank, int32_t n, int32_t j0,
+                                                              int32_t count, float* __restrict__ out) {
+    __shared__ float tile[kTurn][C + 1];
     const float* x = ctl->cur ? x1 : x0;
-    const double s = cols[j].sum;
-    const int32_t v = perm ? perm[r] : r;
-    out[v] = (s > 0.0) ? (double)x[(size_t)r * stride + j] * (1.0 / s) : 1.0 / (double)n;
+    const int32_t v0 = (int32_t)blockIdx.x * kTurn;
+    const int32_t rows = min(kTurn, n - v0);
+    for (int i = threadIdx.x; i < rows * C; i += kRowThreads) {
+        const int32_t v = v0 + i / C;
+        const int32_t r = rank ? rank[v] : v;
+        tile[i / C][i % C] = x[(size_t)r * C + i % C];
+    }
+    __syncthreads();
+    const int l = lane_id();
+    if (l < rows)
+        for (int32_t q = wave_id(); q < count; q += kRowWaves) out[(size_t)q * n + v0 + l] = tile[l][j0 + q];
 }
 
 // The packed form of column j's result: its sum (FP64) in the header, then
@@ -1542,14 +1558,52 @@ int batch_result(Batch& b, int32_t j, double* host_out) {
         return EGX_UNSUPPORTED_GRAPH;
     }
     EGX_TRY(flush_init(b));
-    k_spmm_output<<<nblk(g.n, 256), 256, 0, s>>>(b.X[0].as<float>(), b.X[1].as<float>(), b.ctl.as<BatchCtl>(),
-                                                  b.width, b.cols.as<ColState>(),
-                                                  g.reordered ? g.perm.as<int32_t>() : nullptr, g.n, j,
-                                                  b.out.as<double>());
+    k_spmm_output_packed<<<nblk(g.n, 256), 256, 0, s>>>(b.X[0].as<float>(), b.X[1].as<float>(),
+                                                         b.ctl.as<BatchCtl>(), b.width, b.cols.as<ColState>(),
+                                                         g.reordered ? g.perm.as<int32_t>() : nullptr, g.n, j,
+                                                         b.out.as<char>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    if (host_out)
-        EGX_HIP_TRY(hipMemcpyAsync(host_out, b.out.p, (size_t)g.n * 8, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
+    double sum = 0.0;
+    EGX_HIP_TRY(hipMemcpyWithStream(&sum, b.out.p, sizeof(double), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+    if (!host_out) return EGX_SUCC;
+    return fetch({Fetch{b.out.as<char>() + kPackedHeader, host_out, g.n, true, sum}}, s);
+}
+
+// The results of columns [0, k) (after batch_poll) to host_out, k rows of n
+// doubles.
+constexpr int64_t kColumnsBytes = (int64_t)256 << 20;  // of packed columns on the device at a time
+int batch_results(Batch& b, int32_t k, double* host_out) {
+    Graph& g = *b.g;
+    hipStream_t s = b.stream;
+    if (k > b.width) {
+        set_last_error("batch slot holds no request");
+        return EGX_UNSUPPORTED_GRAPH;
+    }
+    EGX_TRY(flush_init(b));
+    const int64_t n = g.n;
+    const int32_t step = (int32_t)std::min<int64_t>(k, std::max<int64_t>(1, kColumnsBytes / (4 * n)));
+    DevBuf cols;
+    EGX_TRY(cols.alloc((size_t)step * n * 4, s));
+    const int32_t* rank = g.reordered ? g.rank.as<int32_t>() : nullptr;
+    const unsigned grid = nblk(n, kTurn);
+    for (int32_t j0 = 0; j0 < k; j0 += step) {
+        const int32_t count = std::min(step, k - j0);
+        const float *x0 = b.X[0].as<float>(), *x1 = b.X[1].as<float>();
+        const BatchCtl* ctl = b.ctl.as<BatchCtl>();
+        float* out = cols.as<float>();
+        switch (b.width) {
+            case 8: k_spmm_columns<8><<<grid, kRowThreads, 0, s>>>(x0, x1, ctl, rank, g.n, j0, count, out); break;
+            case 16: k_spmm_columns<16><<<grid, kRowThreads, 0, s>>>(x0, x1, ctl, rank, g.n, j0, count, out); break;
+            case 32: k_spmm_columns<32><<<grid, kRowThreads, 0, s>>>(x0, x1, ctl, rank, g.n, j0, count, out); break;
+            default: k_spmm_columns<64><<<grid, kRowThreads, 0, s>>>(x0, x1, ctl, rank, g.n, j0, count, out); break;
+        }
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        std::vector<Fetch> jobs;
+        for (int32_t q = 0; q < count; ++q)
+            jobs.push_back(Fetch{out + (size_t)q * n, host_out + (size_t)(j0 + q) * n, n, true,
+                                 b.host_cols[(size_t)(j0 + q)].sum});
+        EGX_TRY(fetch(jobs, s));
+    }
     return EGX_SUCC;
 }
 
@@ -1826,9 +1880,11 @@ int egx_graph_ppr(egx_graph* gh, int32_t k, const int32_t* seed_offsets, const i
     EGX_TRY(egx_batch_run(bh, launches, tol > 0.0 ? 0 : launches, kernel_seconds));
     std::vector<int32_t> it(egx::kCols);
     EGX_TRY(egx_batch_poll(bh, nullptr, nullptr, it.data(), nullptr));
-    for (int32_t j = 0; j < k; ++j) {
-        if (iterations) iterations[j] = it[(size_t)j];
-        if (PR) EGX_TRY(egx_batch_result(bh, j, PR + (size_t)j * gh->g.n));
+    if (iterations) std::copy(it.begin(), it.begin() + k, iterations);
+    if (PR) {
+        BatchDevice dg(bh->b->device);
+        if (!dg.ok) return EGX_DEVICE_ERR;
+        EGX_TRY(egx::batch_results(*bh->b, k, PR));
     }
     drop.ok = true;
     return EGX_SUCC;
