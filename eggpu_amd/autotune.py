@@ -2,12 +2,13 @@
 
 The knobs are those of egx_graph_set_bins:
 
-* thread_row_max -- a tile whose mean row length is at most this reduces its
-  rows one thread per row, otherwise one wavefront per row;
+* thread_row_max -- rows of up to 4 times this many arcs are reduced one lane
+  per row, longer ones one wavefront per row;
 * wave_row_max   -- rows with more in-arcs are hub rows (split into
   segments; they also lead the relabelled iteration layout);
 * hub_segment    -- arcs per hub segment (one workgroup each);
-* tile_items     -- rows + arcs per merge-path tile (LDS-staged);
+* tile_items     -- rows + arcs per merge-path tile (LDS-staged); the default
+  value stands for a size chosen by the graph's;
 * tile_sort      -- gather a tile's arcs in source order (1) or row order (0);
 * hot_sources    -- sources past this relabelled id are gathered with
   non-temporal loads, keeping the hot prefix resident (0: off);

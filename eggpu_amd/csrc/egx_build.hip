@@ -154,7 +154,7 @@ enum : int {
     kCtrMaxIn,     // largest in-degree
     kCtrLong,      // rows longer than kOutLong
     kCtrHubs,      // rows above the hub threshold
-    kCtrWaveRows,  // rows of tiles reduced a wavefront per row
+    kCtrWaveRows,  // rows reduced by a wavefront each
     kCtrWords
 };
 
@@ -505,16 +505,13 @@ __global__ __launch_bounds__(kRunThreads) void k_layout_slots(
     }
 }
 
-// Rows of tiles whose mean row length is above thread_row_max (egx_graph_info).
-__global__ __launch_bounds__(256) void k_tile_stats(const int32_t* __restrict__ row, const int32_t* __restrict__ tiles,
-                                                    int64_t n_tiles, int32_t thread_row_max,
-                                                    uint32_t* __restrict__ ctr) {
+// Non-hub rows with more than row_lane_max arcs (egx_graph_info).
+__global__ __launch_bounds__(256) void k_row_stats(const int32_t* __restrict__ row, int32_t n_hub, int32_t n,
+                                                   int32_t lane_max, uint32_t* __restrict__ ctr) {
     __shared__ uint32_t sh[4];
     uint32_t rows = 0;
-    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n_tiles; k += (int64_t)gridDim.x * 256) {
-        const int32_t r0 = tiles[k], r1 = tiles[k + 1];
-        if ((int64_t)(row[r1] - row[r0]) > (int64_t)thread_row_max * (r1 - r0)) rows += (uint32_t)(r1 - r0);
-    }
+    for (int64_t v = n_hub + (int64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (int64_t)gridDim.x * 256)
+        rows += row[v + 1] - row[v] > lane_max ? 1u : 0u;
     rows = block_sum_u32(rows, sh);
     if (threadIdx.x == 0 && rows) atomicAdd(&ctr[kCtrWaveRows], rows);
 }
@@ -1022,6 +1019,20 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     return EGX_SUCC;
 }
 
+// Items per tile: what the caller set, or at the default a size for the
+// graph.  Large tiles leave a small graph's device idle, small ones pay more
+// for their barriers than for their arcs.  Measured (us per SpMV launch at
+// tiles of 512 / 1024 / 2048 / 4096 / 5888 items, FP32): 244K items 10.4 /
+// 10.8 / 13.6 / 17.6 / 18.9; 1M items 14.1 / 11.0 / 12.2 / 17.0 / 20.0; 4.5M 45.6 / 32.9
+// / 28.5 / 35.7 / 37.1; 8M 82.9 / 55.7 / 42.5 / 38.2 / 43.5; 34M 345 / 243 / 184 / 160 / 172;
+// FP64 alike (34M: 206 / 192 / 220 at 2048 / 4096 / 5888).  A graph of a few thousand
+// items is cut into up to 64 tiles of at least 256 (7.5K items: 8.1 us at 256, 11.7 at 5888).
+int32_t tile_size(const BinCfg& cfg, int64_t items) {
+    if (cfg.tile_items != BinCfg{}.tile_items) return cfg.tile_items;
+    const int64_t fill = std::min<int64_t>(4096, std::max<int64_t>(1024, items / 2048));
+    return (int32_t)std::min(fill, std::max<int64_t>(256, items / 64));
+}
+
 int rebuild_bins(Graph& g, const BinCfg& cfg_in, int32_t known_hubs) {
     BinCfg cfg = cfg_in;
     if (cfg.thread_row_max < 0) cfg.thread_row_max = 0;
@@ -1080,19 +1091,19 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in, int32_t known_hubs) {
 
     // merge-path tiles over rows [n_hub, n)
     const int64_t items = (g.m - row[(size_t)g.n_hub]) + (int64_t)(n - g.n_hub);
-    g.n_tiles = (items + cfg.tile_items - 1) / cfg.tile_items;
+    const int32_t per_tile = tile_size(cfg, items);
+    g.n_tiles = (items + per_tile - 1) / per_tile;
+    g.tile_lds = per_tile + cfg.wave_row_max;
     DevBuf ctr;
     EGX_TRY(ctr.alloc(kCtrWords * sizeof(uint32_t)));
     EGX_HIP_TRY(hipMemsetAsync(ctr.p, 0, kCtrWords * sizeof(uint32_t), s), EGX_DEVICE_ERR);
     EGX_TRY(g.tiles.alloc(((size_t)g.n_tiles + 1) * 4));
-    k_tile_starts<<<nblocks(g.n_tiles + 1, 256), 256, 0, s>>>(g.it_row, g.n_hub, n, cfg.tile_items, g.n_tiles,
+    k_tile_starts<<<nblocks(g.n_tiles + 1, 256), 256, 0, s>>>(g.it_row, g.n_hub, n, per_tile, g.n_tiles,
                                                                g.tiles.as<int32_t>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    if (g.n_tiles > 0) {
-        k_tile_stats<<<std::min<unsigned>(nblocks(g.n_tiles, 256), kNodeBlocks), 256, 0, s>>>(
-            g.it_row, g.tiles.as<int32_t>(), g.n_tiles, cfg.thread_row_max, ctr.as<uint32_t>());
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    }
+    k_row_stats<<<std::min<unsigned>(nblocks(n, 256), kNodeBlocks), 256, 0, s>>>(g.it_row, g.n_hub, n,
+                                                                                 row_lane_max(cfg), ctr.as<uint32_t>());
+    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     // (also waits for the copies out of segs and hub_rows)
     uint32_t wave_rows = 0;
     EGX_HIP_TRY(hipMemcpyWithStream(&wave_rows, ctr.as<uint32_t>() + kCtrWaveRows, 4, hipMemcpyDeviceToHost, s),

@@ -34,6 +34,7 @@
 // double buffered, sized for FP64; partials (3 x grid, SoA), hub_part, out.
 #pragma once
 
+#include <algorithm>
 #include <array>
 #include <memory>
 #include <mutex>
@@ -83,7 +84,7 @@ constexpr int32_t kTileLds = 7936;
 constexpr int64_t kArcPad = 64;
 
 struct BinCfg {
-    int32_t thread_row_max = 12;  // tiles with mean row length <= this: thread per row, else wavefront per row
+    int32_t thread_row_max = 12;  // rows of up to kRowLaneFactor times this are reduced by one lane, longer ones by a wavefront
     int32_t wave_row_max = 2048;  // hub threshold: rows with more arcs go to the hub bin
     int32_t hub_segment = 8192;   // arcs per hub segment (one workgroup)
     int32_t tile_items = 5888;    // rows + arcs per tile (merge-path split)
@@ -93,6 +94,12 @@ struct BinCfg {
     int32_t blocked = 0;          // propagation-blocked iterations (unweighted, FP32)
     int32_t blocked_shared = 0;   // blocked items sized for shared multi-graph launches
 };
+
+// Rows of a tile with at most this many arcs are added by one lane.
+constexpr int32_t kRowLaneFactor = 4;
+inline int32_t row_lane_max(const BinCfg& cfg) {
+    return (int32_t)std::min<int64_t>((int64_t)std::max(cfg.thread_row_max, 0) * kRowLaneFactor, INT32_MAX);
+}
 
 // Propagation-blocked iteration (bins.blocked).  Sources are cut into chunks
 // of kPbChunk labels and destination rows into sub-bins of kPbRows rows.
@@ -209,6 +216,7 @@ struct Graph {
     int32_t n_hub = 0;            // rows [0, n_hub) of the iteration layout are hub rows
     DevBuf tiles;
     int64_t n_tiles = 0;
+    int32_t tile_lds = 0;         // LDS entries that a tile may need: its items and one row
     // tile arcs in source order (tile_sort): t_col source, t_pos slot of the
     // arc in its tile's row-order LDS staging, t_val weight (weighted); same
     // arc index space as it_col, entries [row[n_hub], m) used

@@ -17,9 +17,8 @@
 //   * tile (all other rows): the rows whose merge-path diagonal starts in
 //     the tile.  Their arcs are contiguous; the block first stages every
 //     gathered term into LDS (coalesced index loads, 8 independent gathers
-//     per thread), then reduces rows from LDS -- one thread per row when the
-//     tile's mean row length is at most thread_row_max, one wavefront per
-//     row with a wave64 shuffle reduction otherwise -- and finalises them.
+//     per thread), then reduces rows from LDS -- one lane per row up to
+//     row_lane_max arcs, one wavefront per longer row -- and finalises them.
 // Reduce (a few workgroups, then one wavefront) finalises hub rows from
 // their segment partials in segment order and folds the per-block (err, sum,
 // dang) slots in a fixed order: results are run-to-run deterministic and no
@@ -86,7 +85,7 @@ struct IterArgs {
     double* red_part;  // SoA: err[n_red], sum[n_red], dang[n_red]
     int64_t n_hrows;
     int32_t n;
-    int32_t thread_row_max;
+    int32_t row_lane_max;  // rows of a tile with more arcs are added by a wavefront
     uint32_t nblk_h;
     uint32_t grid;
     uint32_t n_red;    // reduce-part workgroups
@@ -170,6 +169,31 @@ __device__ __forceinline__ double jump_of(const IterArgs<T>& a) {
     return (1.0 - a.alpha) / n_d + a.alpha * a.state->dang / n_d;
 }
 
+// A DPP move of a double (two 32-bit moves): lanes without a source, and
+// the rows RowMask leaves out, read 0.
+template <int Ctrl, int RowMask>
+__device__ __forceinline__ double dpp_f64(double x) {
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, Ctrl, RowMask, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), Ctrl, RowMask, 0xf, false);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// Sum over the wavefront by DPP row shifts and row broadcasts (no LDS), in a
+// fixed order; the value of lane 63, broadcast.
+__device__ __forceinline__ double wave_total(double v) {
+    v += dpp_f64<0x111, 0xf>(v);  // row_shr:1
+    v += dpp_f64<0x112, 0xf>(v);  // row_shr:2
+    v += dpp_f64<0x114, 0xf>(v);  // row_shr:4
+    v += dpp_f64<0x118, 0xf>(v);  // row_shr:8
+    v += dpp_f64<0x142, 0xa>(v);  // row_bcast:15
+    v += dpp_f64<0x143, 0xc>(v);  // row_bcast:31
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, kWave - 1);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), kWave - 1);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
 // Gather the terms of a tile's arcs [a0, a0+na) into lds[] in row order.
 // S: the arcs are read in source order (neighbouring lanes then hit the same
 // cache lines) and each term is written to its row-order slot.
@@ -249,25 +273,33 @@ __device__ __forceinline__ void spmv_block(const IterArgs<T>& a, uint32_t b, T* 
     else stage_tile<T, W, false>(a, a0, na, lds);
     __syncthreads();
     double err = 0.0, sum = 0.0, dang = 0.0;
-    if ((int64_t)na > (int64_t)a.thread_row_max * nr) {
-        // wavefront per row
-        for (int32_t i = wave_id(); i < nr; i += kWavesPerBlock) {
-            const int32_t v = r0 + i;
-            const int32_t beg = a.row[v] - a0, end = a.row[v + 1] - a0;
-            double acc = 0.0;
-            for (int32_t j = beg + lane_id(); j < end; j += kWave) acc += (double)lds[j];
-            acc = wave_sum(acc);
-            if (lane_id() == 0) finalize_row<T, W>(a, v, acc, jump, err, sum, dang);
-        }
-    } else {
-        // thread per row
-        for (int32_t i = t; i < nr; i += kThreads) {
-            const int32_t v = r0 + i;
-            const int32_t beg = a.row[v] - a0, end = a.row[v + 1] - a0;
-            double acc = 0.0;
+    // A wavefront takes 64 rows at a time, one per lane.  Rows of up to
+    // row_lane_max arcs are added by their lane; the others by the whole
+    // wavefront, one after the other, each leaving its sum with its lane.
+    // Then the 64 rows are finalised together.  (One choice per tile by its
+    // mean row length left long rows to single lanes and short ones to whole
+    // wavefronts, which paid six shuffles and the loads of the update per row: 58 us per
+    // launch at 4.2M FP64 arcs.)
+    for (int32_t i0 = wave_id() * kWave; i0 < nr; i0 += kThreads) {
+        const int32_t i = i0 + lane_id();
+        const int32_t v = r0 + min(i, nr - 1);
+        const int32_t beg = a.row[v] - a0;
+        const int32_t end = i < nr ? a.row[v + 1] - a0 : beg;
+        double acc = 0.0;
+        const bool is_long = end - beg > a.row_lane_max;
+        if (!is_long)
             for (int32_t j = beg; j < end; ++j) acc += (double)lds[j];
-            finalize_row<T, W>(a, v, acc, jump, err, sum, dang);
+        uint64_t todo = __ballot(is_long);
+        while (todo) {
+            const int l = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const int32_t lb = __builtin_amdgcn_readlane(beg, l), le = __builtin_amdgcn_readlane(end, l);
+            double part = 0.0;
+            for (int32_t j = lb + lane_id(); j < le; j += kWave) part += (double)lds[j];
+            part = wave_total(part);
+            if (lane_id() == l) acc = part;
         }
+        if (i < nr) finalize_row<T, W>(a, v, acc, jump, err, sum, dang);
     }
     block_sum3(err, sum, dang, sh_red);
     if (t == 0) {
@@ -363,7 +395,8 @@ __device__ __forceinline__ void reduce_final_wave(const IterArgs<T>& a) {
 
 template <typename T, bool W>
 __global__ __launch_bounds__(kThreads) void k_pr_spmv(IterArgs<T> a) {
-    __shared__ T lds[kTileLds];
+    extern __shared__ __align__(16) unsigned char tile_lds[];
+    T* lds = reinterpret_cast<T*>(tile_lds);
     __shared__ double sh_red[3 * kWavesPerBlock];
     if (a.state->done) return;  // uniform: written by an earlier launch
     bind(a);
@@ -503,21 +536,11 @@ __device__ __forceinline__ void pb_emit_stage(const float (&v)[kPbVec], uint32_t
     }
 }
 
-// A DPP move of a double (two 32-bit moves): lanes without a source, and
-// the rows RowMask leaves out, read 0.
-template <int Ctrl, int RowMask>
-__device__ __forceinline__ double pb_dpp(double x) {
-    const uint64_t u = (uint64_t)__double_as_longlong(x);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, Ctrl, RowMask, 0xf, false);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), Ctrl, RowMask, 0xf, false);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
 // One step of the chain scan: the lanes whose bit of B is set add the a
 // that DPP control Ctrl brings them (0 where it brings none).
 template <int Ctrl, int RowMask>
 __device__ __forceinline__ void pb_chain_step(double& a, uint64_t B) {
-    const double an = pb_dpp<Ctrl, RowMask>(a);
+    const double an = dpp_f64<Ctrl, RowMask>(a);
     a = __builtin_amdgcn_inverse_ballot_w64(B) ? a + an : a;
 }
 
@@ -546,7 +569,7 @@ __device__ __forceinline__ double pb_window_carry(double a, bool b) {
     B &= 0x0000ffff0000ffffull | (((B >> 15) & 1u) ? 0x00000000ffff0000ull : 0ull) |
          (((B >> 47) & 1u) ? 0xffff000000000000ull : 0ull);
     pb_chain_step<0x143, 0xc>(a, B);  // row_bcast:31: rows 2 and 3 take lane 31
-    return pb_dpp<0x138, 0xf>(a);     // wave_shr:1
+    return dpp_f64<0x138, 0xf>(a);     // wave_shr:1
 }
 
 __device__ __forceinline__ void wave_lds_sync() {
@@ -906,7 +929,8 @@ template <typename T, bool W>
 __global__ __launch_bounds__(kThreads) void k_pr_spmv_multi(const IterArgs<T>* __restrict__ table,
                                                             const int32_t* __restrict__ blk_graph,
                                                             const uint32_t* __restrict__ blk_local) {
-    __shared__ T lds[kTileLds];
+    extern __shared__ __align__(16) unsigned char tile_lds[];
+    T* lds = reinterpret_cast<T*>(tile_lds);
     __shared__ double sh_red[3 * kWavesPerBlock];
     const int32_t gi = blk_graph[blockIdx.x];
     if (gi < 0) return;
@@ -1151,7 +1175,7 @@ int fill_args(Graph& g, const SolveParams& p, IterArgs<T>& a, bool* refreshed = 
     }
     a.n_hrows = g.n_hrows;
     a.n = n;
-    a.thread_row_max = g.bins.thread_row_max;
+    a.row_lane_max = row_lane_max(g.bins);
     a.cold_from = (g.bins.hot_sources > 0 && g.bins.hot_sources < n) ? g.bins.hot_sources : n;
     a.nblk_h = (uint32_t)g.n_hseg;
     a.grid = grid;
@@ -1282,7 +1306,7 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
                 return;
             }
         }
-        k_pr_spmv<T, W><<<grid, kThreads, 0, s>>>(a);
+        k_pr_spmv<T, W><<<grid, kThreads, (size_t)g.tile_lds * sizeof(T), s>>>(a);
     };
 
     // eigenvector mode finds iteration k's delta in launch k+1
@@ -1570,6 +1594,9 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
     } pg{pinned};
     PrState* hs = static_cast<PrState*>(pinned);
 
+    size_t tile_lds = 0;  // LDS of the largest tile among the pull members
+    for (int32_t i = 0; i < count; ++i)
+        if (!is_pb[(size_t)i]) tile_lds = std::max(tile_lds, (size_t)gs[(size_t)i]->tile_lds * sizeof(T));
     const int32_t chunk = p.check_every > 0 ? p.check_every : 8;
     // the SpMV of one iteration for every member: blocked members' scatter,
     // the others' pull work items, then the blocked members' sums
@@ -1580,7 +1607,7 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
                                                                       d_scg.as<int32_t>(), d_scl.as<uint32_t>());
         }
         if (total > 0)
-            k_pr_spmv_multi<T, W><<<(unsigned)total, kThreads, 0, s>>>(d_table.as<IterArgs<T>>(), d_blk.as<int32_t>(),
+            k_pr_spmv_multi<T, W><<<(unsigned)total, kThreads, tile_lds, s>>>(d_table.as<IterArgs<T>>(), d_blk.as<int32_t>(),
                                                                       d_base.as<uint32_t>());
         if constexpr (kBlockable) {
             if (n_sum > 0)

@@ -108,7 +108,7 @@ typedef struct {
     int32_t tile_sort;       /* 1: tile arcs gathered in source order */
     int32_t hot_sources;     /* gathers past this relabelled id are non-temporal (0: none) */
     int32_t blocked;         /* 1: iterations run propagation-blocked (egx_bin_opts.blocked) */
-    int64_t rows_thread;     /* rows reduced one thread per row */
+    int64_t rows_thread;     /* rows reduced one lane per row */
     int64_t rows_wave;       /* rows reduced one wavefront per row */
     int64_t rows_hub;        /* rows of the hub bin (segmented, one workgroup per segment) */
     int64_t hub_segments;
@@ -120,9 +120,9 @@ typedef struct {
 
 /* Degree bins of the SpMV.  Rows with in-degree above wave_row_max form the
  * hub bin (cut into hub_segment-arc segments, one workgroup each); the other
- * rows are split into tiles of tile_items rows+arcs whose gathered terms are
- * staged in LDS and reduced one thread per row when the tile's mean row
- * length is at most thread_row_max, else one wavefront per row.
+ * rows are split into tiles of tile_items rows+arcs (at the default value, of
+ * a size for the graph) whose gathered terms are staged in LDS and reduced
+ * one lane per row up to 4 * thread_row_max arcs, one wavefront per longer row.
  * tile_items + wave_row_max <= 7936. */
 typedef struct {
     int32_t thread_row_max;
