@@ -100,7 +100,7 @@ void give_stream(int dev, hipStream_t s) {
 // state): made 64 at a time in one page-aligned block, since each
 // hipHostMalloc costs tens of microseconds, and handed back to a free list
 // by freed graphs.  The blocks live until the process ends.
-constexpr size_t kStateSlotBytes = (sizeof(PrState) + 255) / 256 * 256;
+constexpr size_t kStateSlotBytes = (sizeof(HostState) + 255) / 256 * 256;
 constexpr size_t kStateSlotsPerBlock = 64;
 struct StateSlots {
     std::mutex mu;

@@ -534,6 +534,12 @@ __global__ void k_set_last(int32_t* __restrict__ arr, int64_t idx, int32_t value
     if (blockIdx.x == 0 && threadIdx.x == 0) arr[idx] = value;
 }
 
+// Rows of many partials first (in their order); returns how many those are.
+int64_t many_first(std::vector<HubRow>& rows) {
+    return std::stable_partition(rows.begin(), rows.end(), [](const HubRow& h) { return h.nseg >= kHubMany; }) -
+           rows.begin();
+}
+
 // The in-degree above which a row is a hub row.
 inline int32_t hub_threshold(const BinCfg& cfg) { return std::min(std::max(cfg.wave_row_max, 1), kTileLds - 256); }
 
@@ -807,7 +813,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     for (DevBuf* d : {&g.pb_src, &g.pb_dst, &g.pb_vals, &g.pb_vgrp, &g.pb_mask, &g.pb_scatter, &g.pb_sum,
                       &g.pb_hrows, &g.pb_hub_part, &g.pb_w, &g.pb_arc})
         d->release();
-    g.n_pb_scatter = g.n_pb_sum = g.n_pb_hrows = 0;
+    g.n_pb_scatter = g.n_pb_sum = g.n_pb_hrows = g.n_pb_hrows_many = 0;
     g.pb_scatter_size.clear();
     g.pb_sum_size.clear();
     if (!cfg.blocked || g.n <= 0 || g.m <= 0) return EGX_SUCC;
@@ -974,6 +980,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
         for (int32_t i = 0; i < nr; ++i) hrows.push_back(HubRow{r0 + i, (int32_t)(parts + (int64_t)i * np), np, 0});
         parts += (int64_t)nr * np;
     }
+    const int64_t many = many_first(hrows);
     // every range the kernels will touch, checked before any item upload
     // (the groups' value slots and rows were checked on the device)
     bool ok = bad_h == 0;
@@ -1009,6 +1016,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     g.n_pb_scatter = (int64_t)scat.size();
     g.n_pb_sum = (int64_t)sums.size();
     g.n_pb_hrows = (int64_t)hrows.size();
+    g.n_pb_hrows_many = many;
     g.pb_scatter_size.resize(scat.size());
     for (size_t i = 0; i < scat.size(); ++i) g.pb_scatter_size[i] = scat[i].g1 - scat[i].g0;
     g.pb_sum_size.resize(sums.size());
@@ -1049,7 +1057,7 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in, int32_t known_hubs) {
     g.bins = cfg;
     hipStream_t s = g.stream;
     const int32_t n = g.n;
-    g.n_hseg = g.n_hrows = g.n_tiles = 0;
+    g.n_hseg = g.n_hrows = g.n_hrows_split = g.n_hrows_many = g.n_tiles = 0;
     g.rows_thread = g.rows_wave = 0;
     if (n <= 0) return EGX_SUCC;
 
@@ -1064,7 +1072,8 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in, int32_t known_hubs) {
         const int32_t b = row[(size_t)v], e = row[(size_t)v + 1];
         const int32_t nseg = (int32_t)(((int64_t)(e - b) + cfg.hub_segment - 1) / cfg.hub_segment);
         const int32_t first = (int32_t)segs.size();
-        hub_rows.push_back(HubRow{v, first, nseg, 0});
+        // a row of one segment is finished by its workgroup
+        if (nseg > 1) hub_rows.push_back(HubRow{v, first, nseg, 0});
         for (int32_t k = 0; k < nseg; ++k) {
             HubSeg sg;
             sg.row = v;
@@ -1076,7 +1085,9 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in, int32_t known_hubs) {
             segs.push_back(sg);
         }
     }
-    g.n_hrows = (int64_t)hub_rows.size();
+    g.n_hrows = g.n_hub;
+    g.n_hrows_split = (int64_t)hub_rows.size();
+    g.n_hrows_many = many_first(hub_rows);
     g.n_hseg = (int64_t)segs.size();
     EGX_TRY(g.hsegs.alloc(std::max<size_t>(segs.size(), 1) * sizeof(HubSeg)));
     if (!segs.empty())

@@ -191,7 +191,7 @@ extern "C" int egx_eigenvector_csr(const int32_t* V, const int32_t* E, const dou
     p.eig_x0 = dx.as<double>();
     SolveStats st;
     EGX_TRY(solve_pagerank(g, p, out, &st));
-    const PrState* hs = static_cast<const PrState*>(g.host_state);
+    const PrState* hs = &static_cast<const HostState*>(g.host_state)->st;
     if (iterations) *iterations = hs->eig_iters;
     if (stop) *stop = hs->eig_stop;
     if (kernel_seconds) *kernel_seconds = st.kernel_seconds;

@@ -60,6 +60,10 @@ struct HubRow {
     int32_t pad;
 };
 
+// A hub row with this many partials is added by kHubLanes lanes.
+constexpr int32_t kHubLanes = 8;
+constexpr int32_t kHubMany = 7;
+
 struct PrState {
     double dang;      // dangling mass of the current iterate
     double err;       // L1(x' - x) of the last iteration
@@ -72,6 +76,15 @@ struct PrState {
     double scale_prev;
     int32_t eig_iters;  // iterations the reference loop counts at the stop
     int32_t eig_stop;   // 1 delta below tol, 2 max_iter, 3 norm below the floor
+    int32_t fresh;      // initial state: no iteration has been folded into it yet
+    int32_t pad;
+};
+
+// The pinned slot of a graph: a copy of the last state, and the progress of
+// the running solve, (done << 32) | launches begun, in one word that the device stores whole.
+struct HostState {
+    PrState st;
+    uint64_t progress;
 };
 
 // LDS entries (of the iterate type) a tile may stage: tile_items + hub
@@ -174,7 +187,7 @@ struct Graph {
     // (-1 for padding) for refreshing pb_w after an alpha change
     bool pb_ready = false;
     DevBuf pb_src, pb_dst, pb_vals, pb_vgrp, pb_mask, pb_scatter, pb_sum, pb_hrows, pb_hub_part, pb_w, pb_arc;
-    int64_t n_pb_scatter = 0, n_pb_sum = 0, n_pb_hrows = 0;
+    int64_t n_pb_scatter = 0, n_pb_sum = 0, n_pb_hrows = 0, n_pb_hrows_many = 0;
     // host copies of the items' sizes (groups per scatter item, value slots
     // per sum item), for ordering them in multi-graph launches
     std::vector<int32_t> pb_scatter_size, pb_sum_size;
@@ -224,12 +237,14 @@ struct Graph {
     bool tsorted = false;
     DevBuf hsegs, hrows, hub_part;
     int64_t n_hseg = 0, n_hrows = 0;
+    int64_t n_hrows_split = 0;    // hub rows of several segments: the entries of hrows
+    int64_t n_hrows_many = 0;     // of them with kHubMany segments or more, which come first
     int64_t rows_thread = 0, rows_wave = 0;
 
     // solve workspace (allocated on first use, sized for FP64)
     DevBuf x[2], s[2], state, partials, red_part, out;
     int64_t partial_blocks = 0;
-    void* host_state = nullptr;  // pinned PrState
+    void* host_state = nullptr;  // pinned HostState
     ~Graph();
     static constexpr size_t kBuffers = 46;  // every DevBuf above
     std::array<DevBuf*, kBuffers> buffers();
@@ -306,7 +321,7 @@ struct SolveParams {
 struct SolveBufs {
     void* x[2];
     void* s[2];
-    PrState* state;
+    PrState* state;  // two of them
     double* partials;
     double* red_part;
 };

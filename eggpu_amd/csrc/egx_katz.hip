@@ -159,7 +159,7 @@ extern "C" int egx_katz_csr(const int32_t* V, const int32_t* E, int32_t n, int32
         p.out_device = res.as<double>();
         SolveStats st;
         EGX_TRY(solve_pagerank(g, p, nullptr, &st));
-        const PrState* hs = static_cast<const PrState*>(g.host_state);
+        const PrState* hs = &static_cast<const HostState*>(g.host_state)->st;
         if (iterations) *iterations = hs->iter;
         if (kernel_seconds) *kernel_seconds = st.kernel_seconds;
         const bool stopped = hs->err < tol;  // else by max_iter

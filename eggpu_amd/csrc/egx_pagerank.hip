@@ -19,20 +19,20 @@
 //     gathered term into LDS (coalesced index loads, 8 independent gathers
 //     per thread), then reduces rows from LDS -- one lane per row up to
 //     row_lane_max arcs, one wavefront per longer row -- and finalises them.
-// Reduce (a few workgroups, then one wavefront) finalises hub rows from
-// their segment partials in segment order and folds the per-block (err, sum,
-// dang) slots in a fixed order: results are run-to-run deterministic and no
+// Reduce (a few workgroups) finalises the hub rows of several segments from
+// their partials and folds the per-block (err, sum, dang) slots; the next
+// iteration's first launch folds what is left, every workgroup for itself (begin_fold).
+// Every order is fixed: results are run-to-run deterministic and no
 // launch uses a global atomic (device-scope atomics on one address serialise
 // across the 8 XCDs).  Row sums, the teleport term, the dangling mass and the L1 residual
 // are FP64; iterates are stored as T (float or double).  Unweighted graphs
 // keep s = x/outdeg beside x, so each arc costs one 4-byte index and one
 // gather.
 //
-// The ping-pong buffer of an iteration is chosen on the device from the
-// graph's own iteration counter, so kernel arguments never change between
-// iterations: a run of iterations can be captured once in a hipGraph and
-// replayed, and many graphs -- each stopping on its own -- can share one
-// launch through a table of per-graph arguments (k_pr_spmv_multi /
+// A launch of one graph's solve knows its parity from its own number, which
+// a captured run of an even number of iterations repeats on every replay.
+// Many graphs -- each stopping on its own, their buffers chosen on the device
+// by their iteration counters -- can share one launch through a table of per-graph arguments (k_pr_spmv_multi /
 // k_pr_reduce_multi run the same block code as the one-graph kernels, so a
 // graph's result is bit-identical alone and in a batch).
 #include <algorithm>
@@ -54,9 +54,13 @@ namespace {
 // 5 with 256-thread blocks); the many small tiles of batched graphs gain most
 constexpr int kThreads = 512;
 constexpr int kWavesPerBlock = kThreads / kWave;
-constexpr int kReduceThreads = 256;  // per reduce-part workgroup
-constexpr int kRedItems = 512;       // hub rows + partial slots per reduce-part workgroup (target)
-constexpr int kMaxRed = 1024;        // reduce-part workgroups per graph, at most
+constexpr int kReduceThreads = 1024;  // per reduce workgroup
+constexpr int kRedSlots = 4096;      // or partial slots
+constexpr int kMaxRed = 256;         // reduce workgroups per graph, at most: each workgroup of the next launch adds their sums
+// Grids of up to kDirectFold workgroups without split hub rows need no
+// reduce launch: the next iteration folds their partials as they are, two
+// sets in turn (one is read while the other is written).
+constexpr uint32_t kDirectFold = 256;
 constexpr int kXcds = 8;             // MI355X: accelerator complex dies, one L2 each
 constexpr int64_t kAffineBytes = (int64_t)2 << 20;  // gathered vector kept on one XCD up to this size
 constexpr int kBatch = 8;  // gathers in flight per thread
@@ -80,10 +84,18 @@ struct IterArgs {
     const T* s_in;
     T* x_out;
     T* s_out;
-    PrState* state;
+    double cur_dang, cur_scale, cur_scale_prev;  // of the state the launch works from
+    int32_t cur_iter;
+    PrState* state;    // multi-graph: the state; one graph: two, by launch parity
     double* partials;  // SoA: err[grid], sum[grid], dang[grid]
     double* red_part;  // SoA: err[n_red], sum[n_red], dang[n_red]
+    uint32_t it;           // one graph: number of the iteration's launch
+    const double* fold;    // what begin_fold adds up: SoA of fold_n partial sums each
+    uint32_t fold_n;
+    HostState* host;       // pinned
+    int32_t hub_fix;       // hub_part holds 2^-62 fixed-point sums (blocked layouts)
     int64_t n_hrows;
+    int64_t n_hrows_many;  // of them with kHubMany partials or more, the first ones
     int32_t n;
     int32_t row_lane_max;  // rows of a tile with more arcs are added by a wavefront
     uint32_t nblk_h;
@@ -104,13 +116,27 @@ struct IterArgs {
 };
 
 template <typename T>
-__device__ __forceinline__ void bind(IterArgs<T>& a) {
+__device__ __forceinline__ void bind_parity(IterArgs<T>& a, bool odd) {
     // selects, not an index: a runtime index would move the argument block to scratch
-    const bool odd = (a.state->iter & 1) != 0;
     a.x_in = odd ? a.xb[1] : a.xb[0];
     a.x_out = odd ? a.xb[0] : a.xb[1];
     a.s_in = odd ? a.sb[1] : a.sb[0];
     a.s_out = odd ? a.sb[0] : a.sb[1];
+}
+
+template <typename T>
+__device__ __forceinline__ void use_state(IterArgs<T>& a, const PrState& st) {
+    a.cur_dang = st.dang;
+    a.cur_scale = st.scale;
+    a.cur_scale_prev = st.scale_prev;
+    a.cur_iter = st.iter;
+}
+
+// Multi-graph launches: everything from the graph's own state.
+template <typename T>
+__device__ __forceinline__ void bind(IterArgs<T>& a) {
+    bind_parity(a, (a.state->iter & 1) != 0);
+    use_state(a, *a.state);
 }
 
 // The gathered term of an arc from u: x[u] * in_val (weighted) or
@@ -133,9 +159,8 @@ __device__ __forceinline__ void finalize_row(const IterArgs<T>& a, int32_t v, do
         // the other buffer's old y (the iterate before x) gives the delta
         const double xc = jump * (double)a.x_in[v];
         const double yn = jump * acc + a.eig_shift * xc;
-        const PrState* st = a.state;
-        if (st->iter > 0) {
-            const double d = xc - st->scale_prev * (double)a.x_out[v];
+        if (a.cur_iter > 0) {
+            const double d = xc - a.cur_scale_prev * (double)a.x_out[v];
             err += (a.eig == 1) ? fabs(d) : d * d;
         }
         sum += yn * yn;
@@ -163,10 +188,10 @@ __device__ __forceinline__ void finalize_row(const IterArgs<T>& a, int32_t v, do
 // this returns (1-alpha) + alpha*dang, scaled by p[v] per row.
 template <typename T>
 __device__ __forceinline__ double jump_of(const IterArgs<T>& a) {
-    if (a.eig) return a.state->scale;
-    if (a.tele) return (1.0 - a.alpha) + a.alpha * a.state->dang;
+    if (a.eig) return a.cur_scale;
+    if (a.tele) return (1.0 - a.alpha) + a.alpha * a.cur_dang;
     const double n_d = (double)a.n;
-    return (1.0 - a.alpha) / n_d + a.alpha * a.state->dang / n_d;
+    return (1.0 - a.alpha) / n_d + a.alpha * a.cur_dang / n_d;
 }
 
 // A DPP move of a double (two 32-bit moves): lanes without a source, and
@@ -223,12 +248,101 @@ __device__ __forceinline__ void stage_tile(const IterArgs<T>& a, int32_t a0, int
     }
 }
 
+// The state after folding the sums of the launch before into `st`.
+template <typename T>
+__device__ __forceinline__ void advance_state(const IterArgs<T>& a, PrState& st, double e, double su, double dg) {
+    if (a.eig) {
+        // launch p found delta_p (x_p against x_{p-1}, p >= 1) and ||A x_p||;
+        // the reference's iteration p tests the delta, iteration p+1 the norm
+        const int32_t p = st.iter;
+        const double delta = (a.eig == 2) ? sqrt(e) : e;
+        const double nrm = sqrt(su);
+        st.err = delta;
+        st.sum = nrm;
+        int32_t stop = 0, counted = p;
+        if (p >= 1 && delta < a.tol_n) stop = 1;
+        else if (p >= a.max_iter) stop = 2;
+        else if (!(nrm >= a.eig_floor) || !(nrm > 0.0)) {
+            stop = 3;
+            counted = p + 1;
+        }
+        if (stop) {
+            // x_p (input buffer, scale) is the result; iter keeps its parity
+            st.eig_stop = stop;
+            st.eig_iters = counted;
+            st.done = 1;
+        } else {
+            st.scale_prev = st.scale;
+            st.scale = 1.0 / nrm;
+            st.iter = p + 1;
+        }
+    } else {
+        const int32_t it = st.iter + 1;
+        st.err = e;
+        st.sum = su;
+        st.dang = dg;
+        st.iter = it;
+        st.done = (e < a.tol_n || it >= a.max_iter) ? 1 : 0;
+    }
+}
+
+// First launch of iteration a.it, wavefront 0 of every workgroup: the state
+// this iteration works from, into *sh.  It is the one of the launch before
+// (slot of the other parity) plus that iteration's sums, which every
+// workgroup adds up for itself in the same fixed order -- a launch of its own
+// for that took 4.7 us per iteration.  Workgroup 0 leaves it in this parity's
+// slot for the iteration's other launches and reports the progress to the
+// host.  The fresh initial state, and a done one, go on as they are.  The
+// first sums are loaded (begin_load) before the workgroup's own work and
+// added (begin_fold) after it, so that their latency costs nothing.
+struct FoldSums {
+    double e, su, dg;
+};
+template <typename T>
+__device__ __forceinline__ FoldSums begin_load(const IterArgs<T>& a) {
+    const uint32_t r = (uint32_t)lane_id();
+    FoldSums f{0.0, 0.0, 0.0};
+    if (r < a.fold_n) {
+        f.e = a.fold[r];
+        f.su = a.fold[a.fold_n + r];
+        f.dg = a.fold[2 * (size_t)a.fold_n + r];
+    }
+    return f;
+}
+
+template <typename T>
+__device__ __forceinline__ void begin_fold(const IterArgs<T>& a, FoldSums f, PrState* sh) {
+    const int l = lane_id();
+    PrState st = a.state[(a.it + 1) & 1];
+    if (!st.done && !st.fresh) {
+        for (uint32_t r = l + kWave; r < a.fold_n; r += kWave) {
+            f.e += a.fold[r];
+            f.su += a.fold[a.fold_n + r];
+            f.dg += a.fold[2 * (size_t)a.fold_n + r];
+        }
+        advance_state(a, st, wave_total(f.e), wave_total(f.su), wave_total(f.dg));
+    }
+    st.fresh = 0;
+    if (l == 0) {
+        *sh = st;
+        if (blockIdx.x == 0) {
+            a.state[a.it & 1] = st;
+            __hip_atomic_store(&a.host->progress, ((uint64_t)(uint32_t)st.done << 32) | (uint64_t)(a.it + 1),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+}
+
 // One SpMV work item.  col / val are streamed once per iteration:
 // non-temporal loads keep them from evicting the gathered vector from L2.
-template <typename T, bool W>
-__device__ __forceinline__ void spmv_block(const IterArgs<T>& a, uint32_t b, T* lds, double* sh_red) {
-    const double jump = jump_of(a);
+// Fold: an iteration's first launch of one graph.  The gathers need only the
+// launch's parity; the state arrives in *sh with the barrier that ends them,
+// and a workgroup that then finds the solve done writes nothing.
+template <typename T, bool W, bool Fold>
+__device__ __forceinline__ void spmv_block(IterArgs<T>& a, uint32_t b, T* lds, double* sh_red, PrState* sh) {
     const int t = threadIdx.x;
+    FoldSums f{0.0, 0.0, 0.0};
+    if (Fold && wave_id() == 0) f = begin_load(a);
 
     if (b < a.nblk_h) {
         const HubSeg sg = a.hsegs[b];
@@ -251,14 +365,21 @@ __device__ __forceinline__ void spmv_block(const IterArgs<T>& a, uint32_t b, T* 
         }
         acc = wave_sum(acc);
         if (lane_id() == 0) sh_red[wave_id()] = acc;
+        if (Fold && wave_id() == 0) begin_fold(a, f, sh);
         __syncthreads();
+        if (Fold) {
+            if (sh->done) return;
+            use_state(a, *sh);
+        }
         if (t == 0) {
             double tot = 0.0;
             for (int w = 0; w < kWavesPerBlock; ++w) tot += sh_red[w];
-            a.hub_part[b] = tot;
-            a.partials[b] = 0.0;
-            a.partials[(size_t)a.grid + b] = 0.0;
-            a.partials[2 * (size_t)a.grid + b] = 0.0;
+            double err = 0.0, sum = 0.0, dang = 0.0;
+            if (sg.nseg == 1) finalize_row<T, W>(a, sg.row, tot, jump_of(a), err, sum, dang);
+            else a.hub_part[b] = tot;
+            a.partials[b] = err;
+            a.partials[(size_t)a.grid + b] = sum;
+            a.partials[2 * (size_t)a.grid + b] = dang;
         }
         return;
     }
@@ -271,7 +392,13 @@ __device__ __forceinline__ void spmv_block(const IterArgs<T>& a, uint32_t b, T* 
     const int32_t nr = r1 - r0;
     if (a.tpos) stage_tile<T, W, true>(a, a0, na, lds);
     else stage_tile<T, W, false>(a, a0, na, lds);
+    if (Fold && wave_id() == 0) begin_fold(a, f, sh);
     __syncthreads();
+    if (Fold) {
+        if (sh->done) return;
+        use_state(a, *sh);
+    }
+    const double jump = jump_of(a);
     double err = 0.0, sum = 0.0, dang = 0.0;
     // A wavefront takes 64 rows at a time, one per lane.  Rows of up to
     // row_lane_max arcs are added by their lane; the others by the whole
@@ -309,29 +436,70 @@ __device__ __forceinline__ void spmv_block(const IterArgs<T>& a, uint32_t b, T* 
     }
 }
 
-// Reduce, in two launches.  Part r (of n_red workgroups) finalises its share
-// of the hub rows from their segment partials (segment order) and folds its
-// share of the per-block partial slots; the final launch (one wavefront)
-// folds the n_red part sums in index order, updates the state and takes the
-// stop decision err < tol*n (pagerank.py:131) on the device.  Every sum has
-// a fixed order, so results are run-to-run deterministic.
+// Reduce.  Part r (of n_red workgroups) finalises its share of the hub rows
+// from their partials and folds its share of the per-block partial slots.
+// The first n_hrows_many rows have many partials (kHubMany): kHubLanes lanes
+// share one, adding strided and combining in a fixed tree; the others take a
+// lane each.  Measured (us per launch, one lane / kHubLanes for every row): R-MAT 20, up to 60
+// partials per row, 13.1 / 7.7; 3M nodes weighted, mostly 2 or 3, 7.1 / 16.4.
+// Partials of blocked layouts are fixed-point integers, whose sum has no order.
+constexpr double kPbUnfix = 1.0 / 4611686018427387904.0;  // 2^-62
+
+template <typename P>
+__device__ __forceinline__ P hub_row_sum(const P* __restrict__ part, const HubRow& hr, bool many, int sub) {
+    P acc = 0;
+    if (!many) {
+#pragma unroll 4
+        for (int32_t q = 0; q < hr.nseg; ++q) acc += part[hr.first + q];
+        return acc;
+    }
+    for (int32_t q = sub; q < hr.nseg; q += kHubLanes) acc += part[hr.first + q];
+#pragma unroll
+    for (int off = kHubLanes / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kHubLanes);
+    return acc;
+}
+
 template <typename T, bool W>
 __device__ __forceinline__ void reduce_part_block(const IterArgs<T>& a, uint32_t r, double* sh_red) {
     const double jump = jump_of(a);
     const int t = threadIdx.x;
-    const int64_t stride = (int64_t)a.n_red * kReduceThreads;
-    const int64_t first = (int64_t)r * kReduceThreads + t;
     double e = 0.0, su = 0.0, dg = 0.0;
-    for (int64_t h = first; h < a.n_hrows; h += stride) {
-        const HubRow hr = a.hrows[h];
-        double row = 0.0;
-        for (int32_t q = 0; q < hr.nseg; ++q) row += a.hub_part[hr.first + q];
-        finalize_row<T, W>(a, hr.row, row, jump, e, su, dg);
+    if (a.n_hrows == 0 && a.grid <= kDirectFold) {
+        // (many-graph launches) the order in which begin_fold adds the
+        // partials of a graph solved alone; n_red is 1
+        if (wave_id() != 0) return;
+        for (uint32_t i = t; i < a.grid; i += kWave) {
+            e += a.partials[i];
+            su += a.partials[a.grid + i];
+            dg += a.partials[2 * (size_t)a.grid + i];
+        }
+        e = wave_total(e);
+        su = wave_total(su);
+        dg = wave_total(dg);
+        if (t == 0) {
+            a.red_part[r] = e;
+            a.red_part[a.n_red + r] = su;
+            a.red_part[2 * (size_t)a.n_red + r] = dg;
+        }
+        return;
     }
+    const int64_t many_units = a.n_hrows_many * kHubLanes;
+    const int64_t units = many_units + (a.n_hrows - a.n_hrows_many);
+    for (int64_t u = (int64_t)r * kReduceThreads + t; u < units; u += (int64_t)a.n_red * kReduceThreads) {
+        const bool many = u < many_units;  // the same for the kHubLanes lanes of a row
+        const int sub = many ? (int)(u % kHubLanes) : 0;
+        const HubRow hr = a.hrows[many ? u / kHubLanes : u - many_units + a.n_hrows_many];
+        const double row =
+            a.hub_fix ? (double)hub_row_sum(reinterpret_cast<const unsigned long long*>(a.hub_part), hr, many, sub) *
+                            kPbUnfix
+                      : hub_row_sum(static_cast<const double*>(a.hub_part), hr, many, sub);
+        if (sub == 0) finalize_row<T, W>(a, hr.row, row, jump, e, su, dg);
+    }
+    const int64_t stride = (int64_t)a.n_red * kReduceThreads;
     const double* pe = a.partials;
     const double* ps = a.partials + a.grid;
     const double* pd = a.partials + 2 * (size_t)a.grid;
-    for (int64_t i = first; i < (int64_t)a.grid; i += stride) {
+    for (int64_t i = (int64_t)r * kReduceThreads + t; i < (int64_t)a.grid; i += stride) {
         e += pe[i];
         su += ps[i];
         dg += pd[i];
@@ -344,6 +512,7 @@ __device__ __forceinline__ void reduce_part_block(const IterArgs<T>& a, uint32_t
     }
 }
 
+// Multi-graph: one wavefront per graph folds the part sums into its state.
 template <typename T>
 __device__ __forceinline__ void reduce_final_wave(const IterArgs<T>& a) {
     const int l = lane_id();
@@ -353,68 +522,42 @@ __device__ __forceinline__ void reduce_final_wave(const IterArgs<T>& a) {
         su += a.red_part[a.n_red + r];
         dg += a.red_part[2 * (size_t)a.n_red + r];
     }
-    e = wave_sum(e);
-    su = wave_sum(su);
-    dg = wave_sum(dg);
-    if (l == 0 && a.eig) {
-        // launch p found delta_p (x_p against x_{p-1}, p >= 1) and ||A x_p||;
-        // the reference's iteration p tests the delta, iteration p+1 the norm
-        PrState* st = a.state;
-        const int32_t p = st->iter;
-        const double delta = (a.eig == 2) ? sqrt(e) : e;
-        const double nrm = sqrt(su);
-        st->err = delta;
-        st->sum = nrm;
-        int32_t stop = 0, counted = p;
-        if (p >= 1 && delta < a.tol_n) stop = 1;
-        else if (p >= a.max_iter) stop = 2;
-        else if (!(nrm >= a.eig_floor) || !(nrm > 0.0)) {
-            stop = 3;
-            counted = p + 1;
-        }
-        if (stop) {
-            // x_p (input buffer, scale) is the result; iter keeps its parity
-            st->eig_stop = stop;
-            st->eig_iters = counted;
-            st->done = 1;
-        } else {
-            st->scale_prev = st->scale;
-            st->scale = 1.0 / nrm;
-            st->iter = p + 1;
-        }
-    } else if (l == 0) {
-        PrState* st = a.state;
-        const int32_t it = st->iter + 1;
-        st->err = e;
-        st->sum = su;
-        st->dang = dg;
-        st->iter = it;
-        st->done = (e < a.tol_n || it >= a.max_iter) ? 1 : 0;
+    e = wave_total(e);
+    su = wave_total(su);
+    dg = wave_total(dg);
+    if (l == 0) {
+        PrState st = *a.state;
+        advance_state(a, st, e, su, dg);
+        *a.state = st;
     }
 }
 
 template <typename T, bool W>
-__global__ __launch_bounds__(kThreads) void k_pr_spmv(IterArgs<T> a) {
+__global__ __launch_bounds__(kThreads, 8) void k_pr_spmv(IterArgs<T> a) {
     extern __shared__ __align__(16) unsigned char tile_lds[];
     T* lds = reinterpret_cast<T*>(tile_lds);
     __shared__ double sh_red[3 * kWavesPerBlock];
-    if (a.state->done) return;  // uniform: written by an earlier launch
-    bind(a);
-    spmv_block<T, W>(a, blockIdx.x, lds, sh_red);
+    __shared__ PrState sh;
+    bind_parity(a, (a.it & 1) != 0);
+    spmv_block<T, W, true>(a, blockIdx.x, lds, sh_red, &sh);
 }
 
 template <typename T, bool W>
 __global__ __launch_bounds__(kReduceThreads) void k_pr_reduce(IterArgs<T> a) {
     __shared__ double sh_red[3 * (kReduceThreads / kWave)];
-    if (a.state->done) return;
-    bind(a);
+    const PrState* st = &a.state[a.it & 1];
+    if (st->done) return;
+    bind_parity(a, (a.it & 1) != 0);
+    use_state(a, *st);
     reduce_part_block<T, W>(a, blockIdx.x, sh_red);
 }
 
+// After the last iteration: its sums into the state, and the state to the host.
 template <typename T>
-__global__ __launch_bounds__(kWave) void k_pr_final(IterArgs<T> a) {
-    if (a.state->done) return;
-    reduce_final_wave<T>(a);
+__global__ __launch_bounds__(kWave) void k_pr_state(IterArgs<T> a) {
+    __shared__ PrState sh;
+    begin_fold(a, begin_load(a), &sh);
+    if (threadIdx.x == 0) a.host->st = sh;
 }
 
 // Propagation-blocked iteration (unweighted, FP32 iterates): the layout of
@@ -665,9 +808,9 @@ __device__ __forceinline__ void pb_scatter_batch(const PbScatterBatch<W>& cur, i
 // Scatter item `item` of one graph, in a workgroup of kPbThreads threads
 // with sc (kPbChunk + 4 floats) and stage (kPbThreads / kWave rows of
 // kPbStage floats) in LDS.
-template <typename T, bool W>
+template <typename T, bool W, bool Fold>
 __device__ __forceinline__ void pb_scatter_item(const IterArgs<T>& a, const PbArgs& pb, uint32_t item, float* sc,
-                                                float (*stage)[kPbStage]) {
+                                                float (*stage)[kPbStage], PrState* sh) {
     const PbScatter it = pb.scatter[item];
     const int l = lane_id();
     // every lane of a wavefront runs the loop the same number of times (the
@@ -693,7 +836,9 @@ __device__ __forceinline__ void pb_scatter_item(const IterArgs<T>& a, const PbAr
         for (int32_t i = threadIdx.x; i < cnt; i += kPbThreads) sc[i] = (float)sv[base + i];
     }
     if (threadIdx.x == 0) sc[kPbChunk] = 0.0f;
+    if (Fold && wave_id() == 0) begin_fold(a, begin_load(a), sh);
     __syncthreads();
+    if (Fold && sh->done) return;  // the state arrives with the barrier
     float* stg = stage[wave_id()];
     // software pipelined over two batches in turn: the next batch's loads
     // are issued before this batch's LDS reads and term stores, and neither
@@ -712,9 +857,9 @@ template <typename T, bool W>
 __global__ __launch_bounds__(kPbThreads) void k_pb_scatter(IterArgs<T> a, PbArgs pb) {
     __shared__ __align__(16) float sc[kPbChunk + 4];
     __shared__ float stage[kPbThreads / kWave][kPbStage];
-    if (a.state->done) return;
-    bind(a);
-    pb_scatter_item<T, W>(a, pb, blockIdx.x, sc, stage);
+    __shared__ PrState sh;
+    bind_parity(a, (a.it & 1) != 0);
+    pb_scatter_item<T, W, true>(a, pb, blockIdx.x, sc, stage, &sh);
 }
 
 // Many graphs, one launch: workgroup b runs scatter item item_local[b] of
@@ -730,7 +875,7 @@ __global__ __launch_bounds__(kPbThreads) void k_pb_scatter_multi(const IterArgs<
     IterArgs<T> a = table[gi];
     if (a.state->done) return;
     bind(a);
-    pb_scatter_item<T, W>(a, pbs[gi], item_local[blockIdx.x], sc, stage);
+    pb_scatter_item<T, W, false>(a, pbs[gi], item_local[blockIdx.x], sc, stage, nullptr);
 }
 
 // One sum item (one workgroup of kPbSumWaves wavefronts): its value slots
@@ -749,7 +894,6 @@ __global__ __launch_bounds__(kPbThreads) void k_pb_scatter_multi(const IterArgs<
 constexpr int kPbSumWaves = 4;
 constexpr int kPbSumGroups = 2;  // value groups per lane per batch (70 VGPRs: 7 wavefronts per SIMD)
 constexpr int kPbSumThreads = kPbSumWaves * kWave;
-constexpr double kPbUnfix = 1.0 / 4611686018427387904.0;  // 2^-62
 
 // t * 2^62 as an integer, truncated, for FP32 t in [0, 4): t = m * 2^(e - 150)
 // with m the significand (implicit bit included for normal numbers), so
@@ -889,7 +1033,8 @@ __device__ __forceinline__ void pb_sum_item(const IterArgs<T>& a, const PbArgs& 
         block_sum3(err, sum, dang, sh_red);
     } else {
         for (int32_t i = t; i < nr; i += kPbSumThreads)
-            a.hub_part[(size_t)it.part0 + (size_t)i * it.pieces + it.piece] = (double)acc[i] * kPbUnfix;
+            reinterpret_cast<unsigned long long*>(a.hub_part)[(size_t)it.part0 + (size_t)i * it.pieces + it.piece] =
+                acc[i];
     }
     if (t == 0) {
         a.partials[item] = err;
@@ -902,8 +1047,10 @@ template <typename T, bool W>
 __global__ __launch_bounds__(kPbSumThreads) void k_pb_sum(IterArgs<T> a, PbArgs pb) {
     __shared__ unsigned long long acc[kPbRows];
     __shared__ double sh_red[3 * kPbSumWaves];
-    if (a.state->done) return;
-    bind(a);
+    const PrState* st = &a.state[a.it & 1];
+    if (st->done) return;
+    bind_parity(a, (a.it & 1) != 0);
+    use_state(a, *st);
     pb_sum_item<T, W>(a, pb, blockIdx.x, acc, sh_red);
 }
 
@@ -926,7 +1073,7 @@ __global__ __launch_bounds__(kPbSumThreads) void k_pb_sum_multi(const IterArgs<T
 // Many graphs, one launch: block b works for graph blk_graph[b], as its
 // local block blk_local[b]; blk_graph[b] < 0 is padding.
 template <typename T, bool W>
-__global__ __launch_bounds__(kThreads) void k_pr_spmv_multi(const IterArgs<T>* __restrict__ table,
+__global__ __launch_bounds__(kThreads, 8) void k_pr_spmv_multi(const IterArgs<T>* __restrict__ table,
                                                             const int32_t* __restrict__ blk_graph,
                                                             const uint32_t* __restrict__ blk_local) {
     extern __shared__ __align__(16) unsigned char tile_lds[];
@@ -937,7 +1084,7 @@ __global__ __launch_bounds__(kThreads) void k_pr_spmv_multi(const IterArgs<T>* _
     IterArgs<T> a = table[gi];
     if (a.state->done) return;
     bind(a);
-    spmv_block<T, W>(a, blk_local[blockIdx.x], lds, sh_red);
+    spmv_block<T, W, false>(a, blk_local[blockIdx.x], lds, sh_red, nullptr);
 }
 
 template <typename T, bool W>
@@ -1019,13 +1166,23 @@ __global__ void k_fill_f64(double* __restrict__ out, int32_t n, double v) {
     if (i < n) out[i] = v;
 }
 
-// x0 = init (1/n for PageRank, 1 for Katz; as T), s0 = x0/deg.
+// x0 = init (1/n for PageRank, 1 for Katz; as T), s0 = x0/deg, and the
+// fresh state (in the slot that iteration 0 starts from).
 template <typename T>
-__global__ void k_pr_init(const float* __restrict__ deg, int32_t n, double init, T* __restrict__ x,
-                          T* __restrict__ s) {
+__global__ void k_pr_init(const float* __restrict__ deg, int32_t n, double init, int64_t n_dangling,
+                          T* __restrict__ x, T* __restrict__ s, PrState* __restrict__ state) {
     const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= n) return;
     const T x0 = (T)init;
+    if (v == 0) {
+        PrState st{};
+        st.dang = (double)n_dangling * (double)(T)(1.0 / (double)n);
+        st.sum = 1.0;
+        st.scale = 1.0;
+        st.scale_prev = 1.0;
+        st.fresh = 1;
+        state[1] = st;
+    }
+    if (v >= n) return;
     x[v] = x0;
     const float d = deg[v];
     s[v] = (d > 0.0f) ? (T)(x0 / (T)d) : (T)0;
@@ -1048,8 +1205,15 @@ __global__ void k_pr_output(const T* __restrict__ x0, const T* __restrict__ x1, 
 // (out-weight 1); state: no iterations, scale 1.
 template <typename T>
 __global__ void k_eig_init(const double* __restrict__ x0, const int32_t* __restrict__ perm, int32_t n,
-                           T* __restrict__ x, T* __restrict__ s) {
+                           T* __restrict__ x, T* __restrict__ s, PrState* __restrict__ state) {
     const int32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r == 0) {
+        PrState st{};
+        st.scale = 1.0;
+        st.scale_prev = 1.0;
+        st.fresh = 1;
+        state[1] = st;
+    }
     if (r >= n) return;
     const T v = (T)x0[perm ? perm[r] : r];
     x[r] = v;
@@ -1082,6 +1246,9 @@ __global__ void k_katz_output(const T* __restrict__ x0, const T* __restrict__ x1
 
 inline unsigned nblk(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
+// Partial slots that any grid of up to `grid` workgroups needs.
+int64_t partial_slots(int64_t grid) { return std::max(grid, 2 * std::min<int64_t>(grid, kDirectFold)); }
+
 int ensure_workspace(Graph& g, uint32_t grid) {
     const size_t nb = (size_t)std::max(g.n, 1) * 8;
     for (int i = 0; i < 2; ++i) {
@@ -1089,13 +1256,13 @@ int ensure_workspace(Graph& g, uint32_t grid) {
         if (g.s[i].bytes < nb) EGX_TRY(g.s[i].alloc(nb));
     }
     if (g.out.bytes < nb) EGX_TRY(g.out.alloc(nb));
-    if (g.state.bytes < sizeof(PrState)) EGX_TRY(g.state.alloc(sizeof(PrState)));
+    if (g.state.bytes < 2 * sizeof(PrState)) EGX_TRY(g.state.alloc(2 * sizeof(PrState)));
     if ((int64_t)grid > g.partial_blocks) {
-        EGX_TRY(g.partials.alloc((size_t)grid * 3 * 8));
+        EGX_TRY(g.partials.alloc((size_t)partial_slots(grid) * 3 * 8));
         g.partial_blocks = grid;
     }
     if (g.red_part.bytes < (size_t)kMaxRed * 3 * 8) EGX_TRY(g.red_part.alloc((size_t)kMaxRed * 3 * 8));
-    if (!g.host_state) EGX_HIP_TRY(hipHostMalloc(&g.host_state, sizeof(PrState)), EGX_FAILED_TO_ALLOCATE_HOST_MEM);
+    if (!g.host_state) EGX_HIP_TRY(hipHostMalloc(&g.host_state, sizeof(HostState)), EGX_FAILED_TO_ALLOCATE_HOST_MEM);
     return EGX_SUCC;
 }
 
@@ -1130,6 +1297,18 @@ struct CapturedRun {
 
 // Fills the launch arguments of graph g (refreshing its values for p.alpha
 // on the graph's own stream; *refreshed reports whether that queued work).
+// The reduce launch for `rows` hub rows, the first `many` of them shared by
+// kHubLanes lanes each: one round of its lanes if kMaxRed allows.
+template <typename T>
+void set_reduce(IterArgs<T>& a, int64_t rows, int64_t many) {
+    a.n_hrows = rows;
+    a.n_hrows_many = many;
+    const int64_t units = many * kHubLanes + (rows - many);
+    const int64_t want = std::max((units + kReduceThreads - 1) / kReduceThreads,
+                                  ((int64_t)a.grid + kRedSlots - 1) / kRedSlots);
+    a.n_red = (uint32_t)std::min<int64_t>(kMaxRed, std::max<int64_t>(1, want));
+}
+
 template <typename T>
 int fill_args(Graph& g, const SolveParams& p, IterArgs<T>& a, bool* refreshed = nullptr) {
     const uint32_t grid = (uint32_t)g.n_hseg + (uint32_t)g.n_tiles;
@@ -1173,13 +1352,13 @@ int fill_args(Graph& g, const SolveParams& p, IterArgs<T>& a, bool* refreshed = 
         a.partials = g.partials.as<double>();
         a.red_part = g.red_part.as<double>();
     }
-    a.n_hrows = g.n_hrows;
     a.n = n;
     a.row_lane_max = row_lane_max(g.bins);
     a.cold_from = (g.bins.hot_sources > 0 && g.bins.hot_sources < n) ? g.bins.hot_sources : n;
     a.nblk_h = (uint32_t)g.n_hseg;
     a.grid = grid;
-    a.n_red = (uint32_t)std::min<int64_t>(kMaxRed, std::max<int64_t>(1, (g.n_hrows + grid + kRedItems - 1) / kRedItems));
+    set_reduce(a, g.n_hrows_split, g.n_hrows_many);
+    a.host = static_cast<HostState*>(g.host_state);
     a.bias = p.bias;
     a.tele = p.tele;
     a.eig = p.eig_delta;
@@ -1200,25 +1379,13 @@ template <typename T>
 int prepare_graph(Graph& g, const SolveParams& p, hipStream_t s, IterArgs<T>& a) {
     EGX_TRY(fill_args<T>(g, p, a));
     const int32_t n = g.n;
-    if (p.eig_delta) {
+    if (p.eig_delta)
         k_eig_init<T><<<nblk(n, 256), 256, 0, s>>>(p.eig_x0, g.reordered ? g.perm.as<int32_t>() : nullptr, n,
-                                                   a.xb[0], a.sb[0]);
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        PrState* st0 = static_cast<PrState*>(g.host_state);
-        *st0 = PrState{};
-        st0->scale = 1.0;
-        st0->scale_prev = 1.0;
-        EGX_HIP_TRY(hipMemcpyAsync(a.state, st0, sizeof(PrState), hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
-        return EGX_SUCC;
-    }
-    k_pr_init<T><<<nblk(n, 256), 256, 0, s>>>(g.it_deg, n, p.bias ? 1.0 : 1.0 / (double)n, a.xb[0], a.sb[0]);
+                                                   a.xb[0], a.sb[0], a.state);
+    else
+        k_pr_init<T><<<nblk(n, 256), 256, 0, s>>>(g.it_deg, n, p.bias ? 1.0 : 1.0 / (double)n, g.n_dangling, a.xb[0],
+                                                  a.sb[0], a.state);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    // staged through the pinned state buffer: the copy may run after return
-    PrState* st0 = static_cast<PrState*>(g.host_state);
-    *st0 = PrState{};
-    st0->dang = (double)g.n_dangling * (double)(T)(1.0 / (double)n);
-    st0->sum = 1.0;
-    EGX_HIP_TRY(hipMemcpyAsync(a.state, st0, sizeof(PrState), hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
     return EGX_SUCC;
 }
 
@@ -1250,18 +1417,43 @@ __global__ void k_pr_output_packed_multi(const IterArgs<float>* __restrict__ tab
 // PageRank's normalised iterate, Katz's unnormalised previous iterate, or
 // the eigenvector iterate.
 template <typename T>
-int emit_result(const Graph& g, const IterArgs<T>& a, hipStream_t s, double* host_out, bool katz = false,
-                bool eig = false) {
+int emit_result(const Graph& g, const IterArgs<T>& a, const PrState* state, hipStream_t s, double* host_out,
+                bool katz = false, bool eig = false) {
     const int32_t* perm = g.reordered ? g.perm.as<int32_t>() : nullptr;
     if (eig)
-        k_eig_output<T><<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], a.state, perm, g.n, a.out);
+        k_eig_output<T><<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], state, perm, g.n, a.out);
     else if (katz)
-        k_katz_output<T><<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], a.state, perm, g.n, a.out);
+        k_katz_output<T><<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], state, perm, g.n, a.out);
     else
-        k_pr_output<T><<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], a.state, perm, g.n, a.out);
+        k_pr_output<T><<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], state, perm, g.n, a.out);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     if (host_out) return fetch({Fetch{a.out, host_out, g.n, false, 0.0}}, s);
     return EGX_SUCC;
+}
+
+constexpr int32_t kAhead = 4;
+
+// Waits until the device has begun iteration `begun` of the running solve
+// (or found it done).  The device stores its progress into pinned memory;
+// the stream is asked now and then, so that a failed launch ends the wait.
+int wait_progress(HostState* hs, int32_t begun, hipStream_t s, bool* done) {
+    for (int spins = 0;; ++spins) {
+        const uint64_t w = __atomic_load_n(&hs->progress, __ATOMIC_ACQUIRE);
+        *done = (w >> 32) != 0;
+        if (*done || begun <= 0 || (int64_t)(uint32_t)w >= (int64_t)begun) return EGX_SUCC;
+        if (spins % 1024 == 1023) {
+            const hipError_t q = hipStreamQuery(s);
+            if (q == hipSuccess) {  // all of it ran: the word is final
+                *done = (__atomic_load_n(&hs->progress, __ATOMIC_ACQUIRE) >> 32) != 0;
+                return EGX_SUCC;
+            }
+            (void)hipGetLastError();
+            if (q != hipErrorNotReady) {
+                set_last_error(std::string("solve: ") + hipGetErrorString(q));
+                return EGX_DEVICE_ERR;
+            }
+        }
+    }
 }
 
 template <typename T, bool W>
@@ -1282,11 +1474,10 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
         }
         a.hrows = g.pb_hrows.as<HubRow>();
         a.hub_part = g.pb_hub_part.as<double>();
-        a.n_hrows = g.n_pb_hrows;
         a.nblk_h = 0;
         a.grid = (uint32_t)g.n_pb_sum;
-        a.n_red = (uint32_t)std::min<int64_t>(
-            kMaxRed, std::max<int64_t>(1, (a.n_hrows + a.grid + kRedItems - 1) / kRedItems));
+        a.hub_fix = 1;
+        set_reduce(a, g.n_pb_hrows, g.n_pb_hrows_many);
         pb.src = g.pb_src.as<uint16_t>();
         pb.dst = g.pb_dst.as<uint16_t>();
         pb.vals = g.pb_vals.as<float>();
@@ -1297,6 +1488,19 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
         pb.w = W ? g.pb_w.as<float>() : nullptr;
     }
     const uint32_t grid = a.grid;
+    // what the next iteration folds: the reduce launch's sums, or without one the partials
+    const bool reduce = a.n_hrows > 0 || grid > kDirectFold;
+    double* const partials = a.partials;
+    a.fold_n = reduce ? a.n_red : grid;
+    auto set_iteration = [&](int32_t it) {
+        a.it = (uint32_t)it;
+        a.partials = partials;
+        a.fold = a.red_part;
+        if (!reduce) {
+            a.partials = partials + ((it & 1) ? 3 * (size_t)grid : 0);
+            a.fold = partials + ((it & 1) ? 0 : 3 * (size_t)grid);
+        }
+    };
     // the SpMV of one iteration: pull kernel, or scatter + sum
     auto launch_spmv = [&]() {
         if constexpr (kBlockable) {
@@ -1308,6 +1512,9 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
         }
         k_pr_spmv<T, W><<<grid, kThreads, (size_t)g.tile_lds * sizeof(T), s>>>(a);
     };
+    auto launch_reduce = [&]() {
+        if (reduce) k_pr_reduce<T, W><<<a.n_red, kReduceThreads, 0, s>>>(a);
+    };
 
     // eigenvector mode finds iteration k's delta in launch k+1
     const int32_t max_launch = p.max_iter + (p.eig_delta ? 1 : 0);
@@ -1315,54 +1522,85 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
     if (p.time_each_launch) EGX_TRY(timer.reserve((size_t)4 * max_launch));
     CapturedRun cap;
     cap.stream = s;
+    HostState* hs = static_cast<HostState*>(g.host_state);
+    // a solve that fails on the way leaves nothing queued that would write its progress into the next one's
+    struct Drain {
+        hipStream_t s;
+        bool ok = false;
+        ~Drain() {
+            if (!ok) (void)hipStreamSynchronize(s);
+        }
+    } drain{s};
+    __atomic_store_n(&hs->progress, (uint64_t)0, __ATOMIC_RELAXED);
     EGX_HIP_TRY(hipEventRecord(g.ev0, s), EGX_DEVICE_ERR);
     int32_t launched = 0;
-    int32_t chunk = p.check_every > 0 ? p.check_every : 4;
     const bool can_stop_early = p.tol > 0.0 || p.eig_delta != 0;
-    PrState* hs = static_cast<PrState*>(g.host_state);
+    // iterations queued past the last one whose start the device has
+    // reported: enough to keep it busy, few to run empty after the stop
+    const int32_t ahead = p.check_every > 0 ? p.check_every : kAhead;
+    // a replayed run repeats its iterations' parities: even lengths only
+    const bool replay = p.use_graph && !p.time_each_launch && can_stop_early && p.check_every > 0 &&
+                        p.check_every % 2 == 0;
     while (launched < max_launch) {
-        const int32_t todo = can_stop_early ? std::min(chunk, max_launch - launched) : (max_launch - launched);
-        if (p.use_graph && !p.time_each_launch && can_stop_early && todo == p.check_every) {
+        if (replay && max_launch - launched >= p.check_every) {
             // replay one captured chunk of `check_every` iterations
             if (!cap.exec) {
                 EGX_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), EGX_DEVICE_ERR);
-                for (int32_t q = 0; q < todo; ++q) {
+                for (int32_t q = 0; q < p.check_every; ++q) {
+                    set_iteration(q);
                     launch_spmv();
-                    k_pr_reduce<T, W><<<a.n_red, kReduceThreads, 0, s>>>(a);
-                    k_pr_final<T><<<1, kWave, 0, s>>>(a);
+                    launch_reduce();
                 }
                 EGX_HIP_TRY(hipStreamEndCapture(s, &cap.graph), EGX_DEVICE_ERR);
                 EGX_HIP_TRY(hipGraphInstantiate(&cap.exec, cap.graph, nullptr, nullptr, 0), EGX_DEVICE_ERR);
             }
             EGX_HIP_TRY(hipGraphLaunch(cap.exec, s), EGX_DEVICE_ERR);
-            launched += todo;
-        } else {
-            for (int32_t q = 0; q < todo; ++q, ++launched) {
-                if (p.time_each_launch) EGX_HIP_TRY(hipEventRecord(timer.ev[4 * launched], s), EGX_DEVICE_ERR);
-                launch_spmv();
-                EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-                if (p.time_each_launch) {
-                    EGX_HIP_TRY(hipEventRecord(timer.ev[4 * launched + 1], s), EGX_DEVICE_ERR);
-                    EGX_HIP_TRY(hipEventRecord(timer.ev[4 * launched + 2], s), EGX_DEVICE_ERR);
-                }
-                k_pr_reduce<T, W><<<a.n_red, kReduceThreads, 0, s>>>(a);
-                EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-                k_pr_final<T><<<1, kWave, 0, s>>>(a);
-                EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-                if (p.time_each_launch) EGX_HIP_TRY(hipEventRecord(timer.ev[4 * launched + 3], s), EGX_DEVICE_ERR);
-            }
+            launched += p.check_every;
+            EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
+            if (__atomic_load_n(&hs->progress, __ATOMIC_ACQUIRE) >> 32) break;
+            continue;
         }
-        if (launched >= max_launch) break;
-        EGX_HIP_TRY(hipMemcpyAsync(hs, a.state, sizeof(PrState), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-        EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-        if (hs->done) break;
-        if (p.check_every <= 0) chunk = std::min(chunk * 2, 64);
+        if (can_stop_early) {
+            bool done = false;
+            EGX_TRY(wait_progress(hs, launched - ahead, s, &done));
+            if (done) break;
+        }
+        if (p.time_each_launch) EGX_HIP_TRY(hipEventRecord(timer.ev[4 * launched], s), EGX_DEVICE_ERR);
+        set_iteration(launched);
+        launch_spmv();
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        if (p.time_each_launch) {
+            EGX_HIP_TRY(hipEventRecord(timer.ev[4 * launched + 1], s), EGX_DEVICE_ERR);
+            EGX_HIP_TRY(hipEventRecord(timer.ev[4 * launched + 2], s), EGX_DEVICE_ERR);
+        }
+        launch_reduce();
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        if (p.time_each_launch) EGX_HIP_TRY(hipEventRecord(timer.ev[4 * launched + 3], s), EGX_DEVICE_ERR);
+        ++launched;
     }
     EGX_HIP_TRY(hipEventRecord(g.ev1, s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpyAsync(hs, a.state, sizeof(PrState), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipEventSynchronize(g.ev1), EGX_DEVICE_ERR);
+    // the last iteration's sums into the state, and the state to the host
+    set_iteration(launched);
+    k_pr_state<T><<<1, kWave, 0, s>>>(a);
+    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    const PrState* last = a.state + (launched & 1);
+    // a PageRank result for the host only crosses PCIe packed (FP32 iterate;
+    // its sum is in the state) and is finished there
+    bool packed = false;
+    if constexpr (std::is_same<T, float>::value) {
+        packed = host_out && p.out_device == nullptr && p.bias == nullptr && p.eig_delta == 0;
+        if (packed) {
+            k_pr_output_packed<<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], last,
+                                                             g.reordered ? g.perm.as<int32_t>() : nullptr, g.n,
+                                                             reinterpret_cast<float*>(a.out));
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        }
+    }
+    if (!packed) EGX_TRY(emit_result<T>(g, a, last, s, host_out, p.bias != nullptr, p.eig_delta != 0));
+    if (packed) EGX_TRY(fetch({Fetch{a.out, host_out, g.n, true, 0.0, &hs->st.sum}}, s));
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    const int32_t iters = hs->iter;
+    drain.ok = true;
+    const int32_t iters = hs->st.iter;
     if (st) {
         float ms = 0.0f;
         EGX_HIP_TRY(hipEventElapsedTime(&ms, g.ev0, g.ev1), EGX_DEVICE_ERR);
@@ -1371,7 +1609,8 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
         st->spmv_grid = grid;
         if (p.time_each_launch) {
             // launches after the stop flag return at once; time the real ones
-            for (int32_t q = 0; q < iters; ++q) {
+            const int32_t timed = std::min(iters, launched);
+            for (int32_t q = 0; q < timed; ++q) {
                 float a_ms = 0.0f, b_ms = 0.0f;
                 EGX_HIP_TRY(hipEventElapsedTime(&a_ms, timer.ev[4 * q], timer.ev[4 * q + 1]), EGX_DEVICE_ERR);
                 EGX_HIP_TRY(hipEventElapsedTime(&b_ms, timer.ev[4 * q + 2], timer.ev[4 * q + 3]), EGX_DEVICE_ERR);
@@ -1381,19 +1620,6 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
             st->spmv_launches = iters;
         }
     }
-    if constexpr (std::is_same<T, float>::value) {
-        // a PageRank result for the host only crosses PCIe packed (FP32
-        // iterate; its sum is in the state) and is finished here
-        if (host_out && p.out_device == nullptr && p.bias == nullptr && p.eig_delta == 0) {
-            k_pr_output_packed<<<nblk(g.n, 256), 256, 0, s>>>(a.xb[0], a.xb[1], a.state,
-                                                             g.reordered ? g.perm.as<int32_t>() : nullptr, g.n,
-                                                             reinterpret_cast<float*>(a.out));
-            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-            return fetch({Fetch{a.out, host_out, g.n, true, hs->sum}}, s);
-        }
-    }
-    EGX_TRY(emit_result<T>(g, a, s, host_out, p.bias != nullptr, p.eig_delta != 0));
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     return EGX_SUCC;
 }
 
@@ -1451,11 +1677,10 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
             a.partials = g.partials.as<double>();
             a.hrows = g.pb_hrows.as<HubRow>();
             a.hub_part = g.pb_hub_part.as<double>();
-            a.n_hrows = g.n_pb_hrows;
             a.nblk_h = 0;
             a.grid = (uint32_t)g.n_pb_sum;
-            a.n_red = (uint32_t)std::min<int64_t>(
-                kMaxRed, std::max<int64_t>(1, (a.n_hrows + a.grid + kRedItems - 1) / kRedItems));
+            a.hub_fix = 1;
+            set_reduce(a, g.n_pb_hrows, g.n_pb_hrows_many);
             PbArgs& pb = pbt[(size_t)i];
             pb.src = g.pb_src.as<uint16_t>();
             pb.dst = g.pb_dst.as<uint16_t>();
@@ -1726,7 +1951,7 @@ int64_t solve_grid(const Graph& g) {
 int64_t solve_scratch_bytes(const Graph& g, int32_t precision) {
     const int64_t elem = precision == EGX_PRECISION_FP64 ? 8 : 4;
     const int64_t vec = align_up((int64_t)std::max(g.n, 1) * elem);
-    return 4 * vec + align_up((int64_t)sizeof(PrState)) + align_up(solve_grid(g) * 3 * 8) +
+    return 4 * vec + align_up(2 * (int64_t)sizeof(PrState)) + align_up(partial_slots(solve_grid(g)) * 3 * 8) +
            align_up((int64_t)kMaxRed * 3 * 8);
 }
 
@@ -1741,9 +1966,9 @@ void carve_solve_bufs(const Graph& g, int32_t precision, char* base, SolveBufs& 
         p += vec;
     }
     b.state = reinterpret_cast<PrState*>(p);
-    p += align_up((int64_t)sizeof(PrState));
+    p += align_up(2 * (int64_t)sizeof(PrState));
     b.partials = reinterpret_cast<double*>(p);
-    p += align_up(solve_grid(g) * 3 * 8);
+    p += align_up(partial_slots(solve_grid(g)) * 3 * 8);
     b.red_part = reinterpret_cast<double*>(p);
 }
 

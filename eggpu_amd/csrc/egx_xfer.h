@@ -26,6 +26,7 @@ struct Fetch {
     int64_t n;
     bool packed;
     double sum;
+    const double* sum_at = nullptr;  // instead of sum: pinned, written by work queued before the values'
 };
 
 // All of `jobs`, whose values are written by work queued on s; returns when

@@ -171,8 +171,9 @@ void finish_values(const Fetch& f, int64_t i0, int64_t n, const char* from) {
         return;
     }
     const float* x = reinterpret_cast<const float*>(from);
-    if (f.sum > 0.0) {
-        const double inv = 1.0 / f.sum;
+    const double sum = f.sum_at ? *f.sum_at : f.sum;
+    if (sum > 0.0) {
+        const double inv = 1.0 / sum;
         for (int64_t i = 0; i < n; ++i) out[i] = (double)x[i] * inv;
     } else {
         const double u = 1.0 / (double)f.n;
