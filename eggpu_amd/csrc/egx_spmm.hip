@@ -41,6 +41,10 @@ constexpr int kCols = 64;            // columns per batch (one per lane)
 constexpr int kRowThreads = 256;     // 4 wavefronts
 constexpr int kRowWaves = kRowThreads / kWave;
 constexpr int kSpmmHubSeg = 2048;    // arcs per hub segment (one workgroup)
+// hub rows + partial slots that one workgroup reduces (1,500 nodes: an
+// iteration 10.9 us at width 8 against 12.7 with two launches; with 400 items
+// and width 64 two launches are 3 us faster)
+constexpr int64_t kOneReduce = 128;
 constexpr int kMinWidth = 8;         // narrowest X row (columns)
 // merge-path weight of a row against one arc: finishing a row (class tree,
 // new value, three column sums, the store) costs several times an arc's
@@ -642,7 +646,8 @@ __device__ __forceinline__ void hub_block(const SpmmArgs& a, uint32_t b) {
         double tot = 0.0;
         for (int k = 0; k < kRowWaves; ++k) tot += sh[k][lane];
         if (lane < C) a.hub_part[(size_t)b * kCols + lane] = tot;
-        for (int q = 0; q < 3; ++q) a.partials[((size_t)b * 3 + q) * kCols + lane] = 0.0;
+        if (lane < C)
+            for (int q = 0; q < 3; ++q) a.partials[((size_t)b * 3 + q) * kCols + lane] = 0.0;
     }
 }
 
@@ -680,7 +685,7 @@ __device__ __forceinline__ void rows_block(const SpmmArgs& a, uint32_t b) {
         for (int q = 0; q < 3; ++q) {
             double t = 0.0;
             for (int k = 0; k < kRowWaves; ++k) t += sh[q][k][lane];
-            a.partials[(slot * 3 + q) * kCols + lane] = t;
+            if (owner) a.partials[(slot * 3 + q) * kCols + lane] = t;
         }
     }
 }
@@ -699,101 +704,85 @@ __global__ __launch_bounds__(kRowThreads) void k_spmm_iter(SpmmArgs a) {
     else rows_block<C>(a, blockIdx.x - a.nblk_h);
 }
 
-// Reduce, in two launches.  Part r (of n_red workgroups, 4 wavefronts,
-// lane = column) finalises its share of the hub rows from their segment
-// partials (segment order) and folds its share of the per-block partial
-// slots; the final launch (one wavefront) folds the part sums in index
-// order, updates the column states, takes each column's stop decision and
-// flips the buffer parity.  Every order is fixed by the layout alone, so
-// column sums do not depend on the launch width.
-template <int C>
-__global__ __launch_bounds__(kRowThreads) void k_spmm_reduce_part(SpmmArgs a) {
-    __shared__ double sh[3][kRowWaves][kCols];
-    if (!a.ctl->any_active) return;
-    const int cur = a.ctl->cur;
-    // selects, not an index: a runtime index would move the argument block to scratch
-    a.x_in = cur ? a.xbuf[1] : a.xbuf[0];
-    a.x_out = cur ? a.xbuf[0] : a.xbuf[1];
+// Sums of hub rows [h0, h1) and partial slots [b0, b1) by a workgroup of W
+// wavefronts: err, sum and dang of column lane % C, whole in wavefront 0.
+// Rows and slots go round 8 W chains, 8 of them a wavefront's: a lane group
+// of C columns holds 8 / G of them (G = 64 / C), so a narrow launch has as
+// many rows and slots in flight as a wide one has columns.  A chain adds its
+// hub rows (finalised here from their segment partials, in segment order)
+// and then its slots, in order; chains are combined in the 8-leaf tree and
+// wavefronts in order, so a column's sums do not depend on the width.
+// (One slot a wavefront at a time with 64 lanes at every width took 6.7 us
+// at width 8 and 9.2 at 64, for the up to 64 items of a workgroup.)
+template <int C, int W>
+__device__ __forceinline__ void fold_items(const SpmmArgs& a, int64_t h0, int64_t h1, const double* parts, uint64_t b0,
+                                           uint64_t b1, double& err, double& sum, double& dang) {
+    __shared__ double sh[3][W][kCols];
+    constexpr int G = kWave / C;
+    constexpr int R = 8 / G;
+    constexpr int kChains = 8 * W;
     const int lane = lane_id();
     const int w = wave_id();
-    const uint32_t r = blockIdx.x;
-    const ColState cs = a.cols[lane];
-    const double cj = (1.0 - cs.alpha) + cs.alpha * cs.dang;
-    const double inv_n = 1.0 / (double)a.n;
-    double err = 0.0, sum = 0.0, dang = 0.0;
-    const int64_t h0 = (a.n_hrows * r) / a.n_red, h1 = (a.n_hrows * (r + 1)) / a.n_red;
-    if (lane < C) {
-        for (int64_t h = h0 + w; h < h1; h += kRowWaves) {
-            const HubRow hr = a.hrows[h];
-            double acc = 0.0;
-            for (int32_t k = 0; k < hr.nseg; ++k) acc += a.hub_part[(size_t)(hr.first + k) * kCols + lane];
-            double e, su, dg;
-            finalize<C>(a, cs, cj, hr.row, acc, inv_n, row_inputs<C>(a, hr.row), e, su, dg);
-            err += e;
-            sum += su;
-            dang += dg;
+    const int c = lane % C;
+    const int q0 = w * 8 + (lane / C) * R;  // the lane's first chain
+    double acc[3][R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) acc[0][k] = acc[1][k] = acc[2][k] = 0.0;
+    if (h0 < h1) {
+        const ColState cs = a.cols[c];
+        const double cj = (1.0 - cs.alpha) + cs.alpha * cs.dang;
+        const double inv_n = 1.0 / (double)a.n;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            for (int64_t h = h0 + q0 + k; h < h1; h += kChains) {
+                const HubRow hr = a.hrows[h];
+                double tot = 0.0;
+                for (int32_t i = 0; i < hr.nseg; ++i) tot += a.hub_part[(size_t)(hr.first + i) * kCols + c];
+                double e, su, dg;
+                finalize<C>(a, cs, cj, hr.row, tot, inv_n, row_inputs<C>(a, hr.row), e, su, dg);
+                acc[0][k] += e;
+                acc[1][k] += su;
+                acc[2][k] += dg;
+            }
         }
     }
-    const uint64_t b0 = ((uint64_t)a.grid * r) / a.n_red, b1 = ((uint64_t)a.grid * (r + 1)) / a.n_red;
-    for (uint64_t b = b0 + w; b < b1; b += kRowWaves) {
-        err += a.partials[(b * 3 + 0) * kCols + lane];
-        sum += a.partials[(b * 3 + 1) * kCols + lane];
-        dang += a.partials[(b * 3 + 2) * kCols + lane];
+    for (uint64_t b = b0 + q0; b < b1; b += kChains) {
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const uint64_t at = min(b + k, b1 - 1);
+            const bool in = b + k < b1;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const double t = parts[(at * 3 + q) * kCols + c];
+                acc[q][k] += in ? t : 0.0;
+            }
+        }
     }
-    sh[0][w][lane] = err;
-    sh[1][w][lane] = sum;
-    sh[2][w][lane] = dang;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+#pragma unroll
+        for (int span = 1; span < R; span <<= 1) {
+#pragma unroll
+            for (int k = 0; k < R; k += 2 * span) acc[q][k] += acc[q][k + span];
+        }
+        const double t = across_groups<C>(acc[q][0]);
+        if (lane < C) sh[q][w][lane] = t;
+    }
     __syncthreads();
-    if (w == 0) {
-        for (int q = 0; q < 3; ++q) {
-            double t = 0.0;
-            for (int k = 0; k < kRowWaves; ++k) t += sh[q][k][lane];
-            a.red_part[((size_t)r * 3 + q) * kCols + lane] = t;
-        }
+    if (w != 0) return;
+    err = sum = dang = 0.0;
+    for (int k = 0; k < W; ++k) {
+        err += sh[0][k][c];
+        sum += sh[1][k][c];
+        dang += sh[2][k][c];
     }
 }
 
-// One workgroup (lane = column): wavefront w adds parts [r0, r1) in four
-// interleaved chains, so that its loads are in flight together (one chain
-// over up to 1,024 parts took 54 us at R-MAT 22), and the chains and
-// wavefronts are combined in a fixed order.
+// Column states and stop decisions of an iteration, by one wavefront (lane =
+// column) from the column's sums; flips the buffer parity.
 template <int C>
-__global__ __launch_bounds__(kRowThreads) void k_spmm_reduce_final(SpmmArgs a) {
-    __shared__ double sh[3][kRowWaves][kCols];
-    if (!a.ctl->any_active) return;
-    const int cur = a.ctl->cur;
+__device__ __forceinline__ void close_iteration(const SpmmArgs& a, int cur, double e, double s, double d) {
     const int lane = lane_id();
-    const int w = wave_id();
-    const uint32_t r0 = (uint32_t)(((uint64_t)a.n_red * w) / kRowWaves);
-    const uint32_t r1 = (uint32_t)(((uint64_t)a.n_red * (w + 1)) / kRowWaves);
-    double ce[4] = {0.0, 0.0, 0.0, 0.0}, cs4[4] = {0.0, 0.0, 0.0, 0.0}, cd[4] = {0.0, 0.0, 0.0, 0.0};
-    uint32_t r = r0;
-    for (; r + 4 <= r1; r += 4) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const size_t base = ((size_t)(r + k) * 3) * kCols + lane;
-            ce[k] += a.red_part[base];
-            cs4[k] += a.red_part[base + kCols];
-            cd[k] += a.red_part[base + 2 * kCols];
-        }
-    }
-    for (; r < r1; ++r) {
-        const size_t base = ((size_t)r * 3) * kCols + lane;
-        ce[0] += a.red_part[base];
-        cs4[0] += a.red_part[base + kCols];
-        cd[0] += a.red_part[base + 2 * kCols];
-    }
-    sh[0][w][lane] = (ce[0] + ce[1]) + (ce[2] + ce[3]);
-    sh[1][w][lane] = (cs4[0] + cs4[1]) + (cs4[2] + cs4[3]);
-    sh[2][w][lane] = (cd[0] + cd[1]) + (cd[2] + cd[3]);
-    __syncthreads();
-    if (w != 0) return;  // wavefront 0 finishes alone (the other waves read ctl before the barrier)
-    double e = 0.0, s = 0.0, d = 0.0;
-    for (int k = 0; k < kRowWaves; ++k) {
-        e += sh[0][k][lane];
-        s += sh[1][k][lane];
-        d += sh[2][k][lane];
-    }
     ColState* st = &a.cols[lane];
     int running = 0;
     if (lane < C && st->active && !st->done) {
@@ -810,6 +799,51 @@ __global__ __launch_bounds__(kRowThreads) void k_spmm_reduce_final(SpmmArgs a) {
         a.ctl->any_active = any ? 1 : 0;
         a.ctl->cur = cur ^ 1;
     }
+}
+
+// The reduce of an iteration: one workgroup where the layout has at most
+// kOneReduce hub rows and partial slots, else parts (part r of n_red: its
+// share of both) and a launch that folds the parts in order.  Which one it
+// is depends on the layout alone.
+template <int C>
+__global__ __launch_bounds__(kRowThreads) void k_spmm_reduce(SpmmArgs a) {
+    if (!a.ctl->any_active) return;
+    const int cur = a.ctl->cur;
+    // selects, not an index: a runtime index would move the argument block to scratch
+    a.x_in = cur ? a.xbuf[1] : a.xbuf[0];
+    a.x_out = cur ? a.xbuf[0] : a.xbuf[1];
+    double e, s, d;
+    fold_items<C, kRowWaves>(a, 0, a.n_hrows, a.partials, 0, a.grid, e, s, d);
+    // the other wavefronts read the column states and ctl before the fold's barrier
+    if (wave_id() == 0) close_iteration<C>(a, cur, e, s, d);
+}
+
+template <int C>
+__global__ __launch_bounds__(kRowThreads) void k_spmm_reduce_part(SpmmArgs a) {
+    if (!a.ctl->any_active) return;
+    const int cur = a.ctl->cur;
+    a.x_in = cur ? a.xbuf[1] : a.xbuf[0];
+    a.x_out = cur ? a.xbuf[0] : a.xbuf[1];
+    const uint32_t r = blockIdx.x;
+    const int64_t h0 = (a.n_hrows * r) / a.n_red, h1 = (a.n_hrows * (r + 1)) / a.n_red;
+    const uint64_t b0 = ((uint64_t)a.grid * r) / a.n_red, b1 = ((uint64_t)a.grid * (r + 1)) / a.n_red;
+    double e, s, d;
+    fold_items<C, kRowWaves>(a, h0, h1, a.partials, b0, b1, e, s, d);
+    const int lane = lane_id();
+    if (wave_id() == 0 && lane < C) {
+        a.red_part[((size_t)r * 3 + 0) * kCols + lane] = e;
+        a.red_part[((size_t)r * 3 + 1) * kCols + lane] = s;
+        a.red_part[((size_t)r * 3 + 2) * kCols + lane] = d;
+    }
+}
+
+template <int C>
+__global__ __launch_bounds__(kRowThreads) void k_spmm_reduce_final(SpmmArgs a) {
+    if (!a.ctl->any_active) return;
+    const int cur = a.ctl->cur;
+    double e, s, d;
+    fold_items<C, kRowWaves>(a, 0, 0, a.red_part, 0, a.n_red, e, s, d);
+    if (wave_id() == 0) close_iteration<C>(a, cur, e, s, d);
 }
 
 // Column j of the current X (row stride C) := 1/n (networkx starts
@@ -1129,13 +1163,21 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
                     EGX_DEVICE_ERR);
     EGX_TRY(b->hub_part.alloc(std::max<size_t>(segs.size(), 1) * kCols * 8));
 
-    // merge-path split of the other rows: about 8 wavefronts per CU-slot
     int32_t row_end_hub = 0, row_end = 0;
     EGX_HIP_TRY(hipMemcpyWithStream(&row_end_hub, g.it_row + g.n_hub, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     EGX_HIP_TRY(hipMemcpyWithStream(&row_end, g.it_row + n, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     // wavefront k holds the rows whose merge-path diagonal starts in its share
     const int64_t work = (int64_t)(row_end - row_end_hub) + kRowItems * (int64_t)(n - g.n_hub);
-    int64_t waves = std::min<int64_t>(16384, std::max<int64_t>(1, (work + 511) / 512));
+    // Arcs and row weights per wavefront: 512 where that makes 8,192
+    // wavefronts or more (with rows finished one after another, longer
+    // shares balance no better), and down to 64 so that smaller graphs have
+    // as many.  512 throughout, us per iteration at widths 8 and 64: 700
+    // nodes 33 and 35, 4,000 39 and 40, 20,000 42 and 57, 60,000 48 and 67;
+    // now 10 and 16, 15 and 38, 20 and 60, 35 and 67 (32 at least: 9 and 19
+    // at 700).  At 300,007 nodes (512) 106 and 158 became 100 and 155 with
+    // the reduce.
+    const int64_t share = std::min<int64_t>(512, std::max<int64_t>(64, (work + 8191) / 8192));
+    int64_t waves = std::min<int64_t>(16384, std::max<int64_t>(1, (work + share - 1) / share));
     const int64_t per_wave = std::max<int64_t>(1, (work + waves - 1) / waves);
     waves = std::max<int64_t>(1, (work + per_wave - 1) / per_wave);
     b->n_waves = (uint32_t)waves;
@@ -1145,8 +1187,13 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     b->grid = b->nblk_h + (uint32_t)((waves + kRowWaves - 1) / kRowWaves);
     EGX_TRY(b->partials.alloc((size_t)b->grid * 3 * kCols * 8));
-    // reduce parts: about 64 hub rows + partial slots each
-    b->n_red = (uint32_t)std::min<int64_t>(1024, std::max<int64_t>(1, (b->n_hrows + b->grid + 63) / 64));
+    // Reduce parts: 32 hub rows and partial slots each, 16 where those are so
+    // many that hub rows, each a serial chain, bound the launch (2,097,152
+    // nodes, width 64: 55 us with 64 a part; an iteration 1,175 us, 1,162
+    // with 32, 1,154 with 16; at 300,007 nodes 16 cost 1 us more than 32).
+    const int64_t items = b->n_hrows + b->grid;
+    const int64_t parts = (items + 31) / 32;
+    b->n_red = items <= kOneReduce ? 1u : (uint32_t)std::min<int64_t>(512, parts <= 256 ? parts : 2 * parts);
     EGX_TRY(b->red_part.alloc((size_t)b->n_red * 3 * kCols * 8));
     EGX_TRY(b->out.alloc(std::max((size_t)n * 8, kPackedHeader + (size_t)n * 4)));  // FP64 or packed result
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
@@ -1510,6 +1557,16 @@ int enqueue_iterations(Batch& b, const SpmmArgs& a, int32_t iters, hipStream_t s
                 default: k_spmm_iter<64><<<b.grid, kRowThreads, 0, s>>>(a); break;
             }
             EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        }
+        if (a.n_red == 1) {
+            switch (b.width) {
+                case 8: k_spmm_reduce<8><<<1, kRowThreads, 0, s>>>(a); break;
+                case 16: k_spmm_reduce<16><<<1, kRowThreads, 0, s>>>(a); break;
+                case 32: k_spmm_reduce<32><<<1, kRowThreads, 0, s>>>(a); break;
+                default: k_spmm_reduce<64><<<1, kRowThreads, 0, s>>>(a); break;
+            }
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+            continue;
         }
         switch (b.width) {
             case 8: k_spmm_reduce_part<8><<<a.n_red, kRowThreads, 0, s>>>(a); break;
