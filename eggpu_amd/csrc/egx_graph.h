@@ -362,15 +362,15 @@ namespace egx {
 // A new, empty handle bound to the current device, with its stream and events.
 int make_graph(std::unique_ptr<egx_graph>& out);
 
-// egx_batch_result without the wait, and with half the copy: queues the
-// packed result of `slot` on the batch's stream -- the column's FP64 sum s,
-// then its FP32 iterate in caller order (n floats) -- copies it to host_out
-// (pinned, at least kPackedHeader + 4 n bytes; may be null) and records
-// `done` (may be null) after the copy.  unpack_result turns it into the
-// doubles egx_batch_result returns, bit for bit.  host_out must stay valid
+// egx_batch_result of several columns without the wait, and with half the
+// bytes: queues one launch on the batch's stream that writes the packed
+// result of slots[i] -- the column's FP64 sum s, then its FP32 iterate in
+// caller order (n floats) -- to out[i] (pinned, at least kPackedHeader + 4 n
+// bytes), and records `done` after it.  unpack_result turns it into the
+// doubles egx_batch_result returns, bit for bit.  The buffers must stay valid
 // until `done` completes.
 constexpr size_t kPackedHeader = 16;  // the sum, padded so the floats start 16-byte aligned
-int batch_result_enqueue(egx_batch* b, int32_t slot, void* host_out, hipEvent_t done);
+int batch_results_enqueue(egx_batch* b, int32_t count, const int32_t* slots, char* const* out, hipEvent_t done);
 
 // out[v] = (double)x[v] * (1.0 / s) if s > 0, else 1.0 / n: the arithmetic
 // of the device's FP64 output (k_pr_output), on a packed result.

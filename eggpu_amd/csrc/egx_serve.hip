@@ -93,8 +93,8 @@ int64_t session_bytes(const egx_graph_info& inf) {
 // A finished column on its way to the callers' buffers.
 struct Delivery {
     std::shared_ptr<Request> r;
-    char* staged = nullptr;    // pinned packed copy of the result (null: nobody asked for it)
-    hipEvent_t ev = nullptr;   // recorded after the copy into `staged`
+    char* staged = nullptr;           // pinned packed result (null: nobody asked for it)
+    std::shared_ptr<hipEvent_t> ev;   // recorded after the launch that writes it; shared by a step's columns
 };
 
 }  // namespace
@@ -148,46 +148,57 @@ struct egx_server {
         for (char* p : staged_all) (void)hipHostFree(p);
     }
 
-    // A pinned buffer for one result of `graph` and an event, from the pools.
-    int take_staging(int32_t graph, char** buf, hipEvent_t* ev) {
+    // A pinned buffer for one result of `graph`, from the pool.
+    int take_staging(int32_t graph, char** buf) {
         *buf = nullptr;
-        *ev = nullptr;
         {
             std::lock_guard<std::mutex> lk(mu);
             auto& fl = staged_free[(size_t)graph];
             if (!fl.empty()) {
                 *buf = fl.back();
                 fl.pop_back();
-            }
-            if (!events_free.empty()) {
-                *ev = events_free.back();
-                events_free.pop_back();
+                return EGX_SUCC;
             }
         }
-        if (!*buf) {
-            void* p = nullptr;
-            const size_t bytes = egx::kPackedHeader + (size_t)info[(size_t)graph].n * sizeof(float);
-            if (hipHostMalloc(&p, bytes) != hipSuccess) return EGX_FAILED_TO_ALLOCATE_HOST_MEM;
-            *buf = static_cast<char*>(p);
-            std::lock_guard<std::mutex> lk(mu);
-            staged_all.push_back(*buf);
-        }
-        if (!*ev) {
-            if (hipEventCreateWithFlags(ev, hipEventDisableTiming) != hipSuccess) {
-                give_back(graph, *buf, nullptr);
-                *buf = nullptr;
-                return EGX_DEVICE_ERR;
-            }
-            std::lock_guard<std::mutex> lk(mu);
-            events_all.push_back(*ev);
-        }
+        void* p = nullptr;
+        const size_t bytes = egx::kPackedHeader + (size_t)info[(size_t)graph].n * sizeof(float);
+        if (hipHostMalloc(&p, bytes) != hipSuccess) return EGX_FAILED_TO_ALLOCATE_HOST_MEM;
+        *buf = static_cast<char*>(p);
+        std::lock_guard<std::mutex> lk(mu);
+        staged_all.push_back(*buf);
         return EGX_SUCC;
     }
 
-    void give_back(int32_t graph, char* buf, hipEvent_t ev) {
+    void give_back(int32_t graph, char* buf) {
+        if (!buf) return;
         std::lock_guard<std::mutex> lk(mu);
-        if (buf) staged_free[(size_t)graph].push_back(buf);
-        if (ev) events_free.push_back(ev);
+        staged_free[(size_t)graph].push_back(buf);
+    }
+
+    // An event from the pool; the last holder's release (never under mu)
+    // returns it.
+    int take_event(std::shared_ptr<hipEvent_t>* out) {
+        hipEvent_t ev = nullptr;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            if (!events_free.empty()) {
+                ev = events_free.back();
+                events_free.pop_back();
+            }
+        }
+        if (!ev) {
+            if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return EGX_DEVICE_ERR;
+            std::lock_guard<std::mutex> lk(mu);
+            events_all.push_back(ev);
+        }
+        *out = std::shared_ptr<hipEvent_t>(new hipEvent_t(ev), [this](hipEvent_t* e) {
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                events_free.push_back(*e);
+            }
+            delete e;
+        });
+        return EGX_SUCC;
     }
 
     // Delivery thread: wait for a staged (packed) result, finish its FP64
@@ -206,7 +217,7 @@ struct egx_server {
             }
             int st = EGX_SUCC;
             if (d.ev) {
-                const hipError_t e = hipEventSynchronize(d.ev);
+                const hipError_t e = hipEventSynchronize(*d.ev);
                 if (e != hipSuccess) {
                     egx::set_last_error(std::string("result copy event: ") + hipGetErrorString(e));
                     st = EGX_DEVICE_ERR;
@@ -229,7 +240,7 @@ struct egx_server {
                     }
                 }
             }
-            give_back(d.r->graph, d.staged, d.ev);
+            give_back(d.r->graph, d.staged);
             finish(d.r, st);
         }
     }
@@ -420,6 +431,8 @@ struct egx_server {
         int32_t width = 8;
         while (width < hi) width <<= 1;
         std::vector<std::pair<int32_t, Delivery>> finished;
+        std::vector<int32_t> wanted_slots;
+        std::vector<char*> wanted_out;
         for (int32_t j = 0; j < kSlots; ++j) {
             auto& r = s.slot[(size_t)j];
             if (!r || !done[j]) continue;
@@ -430,11 +443,12 @@ struct egx_server {
             Delivery d;
             d.r = r;
             int st = EGX_SUCC;
-            if (wanted) {
-                st = take_staging(s.graph, &d.staged, &d.ev);
-                if (st == EGX_SUCC) st = egx::batch_result_enqueue(s.b, j, d.staged, d.ev);
-            }
+            if (wanted) st = take_staging(s.graph, &d.staged);
             if (st == EGX_SUCC) {
+                if (d.staged) {
+                    wanted_slots.push_back(j);
+                    wanted_out.push_back(d.staged);
+                }
                 finished.emplace_back(j, std::move(d));
             } else {
                 drop_delivery(s, d, st);
@@ -442,6 +456,27 @@ struct egx_server {
             r = nullptr;
             s.busy -= 1;
             s.last_used = Clock::now();
+        }
+        if (!wanted_slots.empty()) {
+            // every result of this step in one launch and one event
+            std::shared_ptr<hipEvent_t> ev;
+            int st = take_event(&ev);
+            if (st == EGX_SUCC)
+                st = egx::batch_results_enqueue(s.b, (int32_t)wanted_slots.size(), wanted_slots.data(),
+                                                wanted_out.data(), *ev);
+            if (st != EGX_SUCC) {
+                // the launch may be queued: nothing writes the buffers once the stream has drained
+                (void)egx_batch_poll(s.b, nullptr, nullptr, nullptr, nullptr);
+                std::vector<std::pair<int32_t, Delivery>> rest;
+                for (auto& f : finished) {
+                    if (f.second.staged) drop_delivery(s, f.second, st);
+                    else rest.push_back(std::move(f));
+                }
+                finished.swap(rest);
+            } else {
+                for (auto& f : finished)
+                    if (f.second.staged) f.second.ev = ev;
+            }
         }
         if (finished.empty()) return;
         // one update releases every finished column (stream order: after
@@ -461,11 +496,12 @@ struct egx_server {
         cv_deliver.notify_all();
     }
 
-    // A result that will not be delivered: its copy lands first, its buffer
-    // goes back to the pool, and its request fails with `status`.
+    // A result that will not be delivered: it lands first, its buffer goes
+    // back to the pool, and its request fails with `status`.
     void drop_delivery(Session& s, Delivery& d, int status) {
-        if (d.ev) (void)hipEventSynchronize(d.ev);
-        give_back(s.graph, d.staged, d.ev);
+        if (d.ev) (void)hipEventSynchronize(*d.ev);
+        d.ev.reset();
+        give_back(s.graph, d.staged);
         finish(d.r, status);
     }
 

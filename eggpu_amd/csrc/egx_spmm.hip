@@ -75,6 +75,12 @@ struct BatchCtl {
     int32_t pad[2];
 };
 
+// The column states and the control word, in device-visible host memory.
+struct HostBatch {
+    ColState cols[kCols];
+    BatchCtl ctl;
+};
+
 struct SpmmArgs {
     const int32_t* row;
     const int32_t* col;
@@ -99,6 +105,7 @@ struct SpmmArgs {
     uint32_t grid;
     uint32_t n_waves;
     uint32_t n_red;            // reduce-part workgroups
+    HostBatch* publish;        // a step's last iteration: the states go here (else null)
     int32_t off32;             // width 64: X rows and arc slots addressable by 32-bit byte offsets
 };
 
@@ -778,6 +785,16 @@ __device__ __forceinline__ void fold_items(const SpmmArgs& a, int64_t h0, int64_
     }
 }
 
+// The states to the host (one wavefront, lane = column), so that a poll
+// after a step waits for the stream and reads memory: its two copies and
+// their wait took about 25 us a step.
+__device__ __forceinline__ void publish(const SpmmArgs& a) {
+    if (!a.publish) return;
+    const int lane = lane_id();
+    a.publish->cols[lane] = a.cols[lane];
+    if (lane == 0) a.publish->ctl = *a.ctl;
+}
+
 // Column states and stop decisions of an iteration, by one wavefront (lane =
 // column) from the column's sums; flips the buffer parity.
 template <int C>
@@ -799,6 +816,7 @@ __device__ __forceinline__ void close_iteration(const SpmmArgs& a, int cur, doub
         a.ctl->any_active = any ? 1 : 0;
         a.ctl->cur = cur ^ 1;
     }
+    publish(a);
 }
 
 // The reduce of an iteration: one workgroup where the layout has at most
@@ -807,7 +825,10 @@ __device__ __forceinline__ void close_iteration(const SpmmArgs& a, int cur, doub
 // is depends on the layout alone.
 template <int C>
 __global__ __launch_bounds__(kRowThreads) void k_spmm_reduce(SpmmArgs a) {
-    if (!a.ctl->any_active) return;
+    if (!a.ctl->any_active) {
+        if (wave_id() == 0) publish(a);
+        return;
+    }
     const int cur = a.ctl->cur;
     // selects, not an index: a runtime index would move the argument block to scratch
     a.x_in = cur ? a.xbuf[1] : a.xbuf[0];
@@ -839,7 +860,10 @@ __global__ __launch_bounds__(kRowThreads) void k_spmm_reduce_part(SpmmArgs a) {
 
 template <int C>
 __global__ __launch_bounds__(kRowThreads) void k_spmm_reduce_final(SpmmArgs a) {
-    if (!a.ctl->any_active) return;
+    if (!a.ctl->any_active) {
+        if (wave_id() == 0) publish(a);
+        return;
+    }
     const int cur = a.ctl->cur;
     double e, s, d;
     fold_items<C, kRowWaves>(a, 0, 0, a.red_part, 0, a.n_red, e, s, d);
@@ -946,6 +970,44 @@ __global__ void k_spmm_output_packed(const float* __restrict__ x0, const float* 
     reinterpret_cast<float*>(out + kPackedHeader)[v] = x[(size_t)r * stride + j];
 }
 
+// Packed results of several columns: columns j[0..count) to dst[0..count).
+struct ResultList {
+    int32_t count;
+    int32_t j[kCols];
+    char* dst[kCols];
+};
+
+// The packed results of every listed column (sum in the header, FP32 iterate
+// in caller order), a block per kTurn nodes as in k_spmm_columns, written
+// straight to the pinned buffers that the host reads: one launch for all
+// columns that finished in a step, where each took a launch of
+// k_spmm_output_packed and a copy.  Bound by the link (whole 256-byte runs).
+template <int C>
+__global__ __launch_bounds__(kRowThreads) void k_spmm_results(const float* __restrict__ x0,
+                                                              const float* __restrict__ x1,
+                                                              const BatchCtl* __restrict__ ctl,
+                                                              const ColState* __restrict__ cols,
+                                                              const int32_t* __restrict__ rank, int32_t n,
+                                                              ResultList list) {
+    __shared__ float tile[kTurn][C + 1];
+    const float* x = ctl->cur ? x1 : x0;
+    const int32_t v0 = (int32_t)blockIdx.x * kTurn;
+    const int32_t rows = min(kTurn, n - v0);
+    for (int i = threadIdx.x; i < rows * C; i += kRowThreads) {
+        const int32_t v = v0 + i / C;
+        const int32_t r = rank ? rank[v] : v;
+        tile[i / C][i % C] = x[(size_t)r * C + i % C];
+    }
+    __syncthreads();
+    const int l = lane_id();
+    for (int32_t q = wave_id(); q < list.count; q += kRowWaves) {
+        char* dst = list.dst[q];
+        const int32_t j = list.j[q];
+        if (l < rows) reinterpret_cast<float*>(dst + kPackedHeader)[v0 + l] = tile[l][j];
+        if (blockIdx.x == 0 && l == 0) *reinterpret_cast<double*>(dst) = cols[j].sum;
+    }
+}
+
 __global__ void k_set_tslot(int32_t* __restrict__ tslot, const int32_t* __restrict__ rows,
                             const int32_t* __restrict__ slots, int32_t count) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1016,7 +1078,8 @@ struct Batch {
     std::vector<std::vector<float>> host_ptab;
     std::vector<ColState> host_cols;          // active flags are host-owned; the rest as last polled
     std::vector<int32_t> rank_h;              // caller id -> iteration row (relabelled graphs)
-    void* pinned = nullptr;  // ColState[64] + BatchCtl
+    HostBatch* pinned = nullptr;
+    bool published = false;   // a step was the last to change the states: *pinned holds them once it is done
     // pinned staging for queued updates: copies from it run in stream order,
     // the arena is recycled after a stream sync
     char* arena = nullptr;
@@ -1120,7 +1183,7 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
     EGX_HIP_TRY(hipMemsetAsync(b->ctl.p, 0, sizeof(BatchCtl), s), EGX_DEVICE_ERR);
     b->host_cols.assign(kCols, ColState{});
     b->seeds.assign(kCols, {});
-    EGX_HIP_TRY(hipHostMalloc(&b->pinned, sizeof(ColState) * kCols + sizeof(BatchCtl)),
+    EGX_HIP_TRY(hipHostMalloc((void**)&b->pinned, sizeof(HostBatch)),
                 EGX_FAILED_TO_ALLOCATE_HOST_MEM);
     EGX_HIP_TRY(hipHostMalloc((void**)&b->arena, kArenaBytes), EGX_FAILED_TO_ALLOCATE_HOST_MEM);
     EGX_TRY(b->upd.alloc(sizeof(BatchUpdateBuf)));
@@ -1212,6 +1275,7 @@ int batch_queue_update(Batch& b, const BatchUpdateBuf& u) {
         EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);  // earlier copies out of the arena are done
         b.arena_used = 0;
     }
+    b.published = false;
     char* slot = b.arena + b.arena_used;
     b.arena_used += (bytes + 255) & ~(size_t)255;
     std::memcpy(slot, &u, bytes);
@@ -1319,8 +1383,9 @@ int batch_set_width(Batch& b, int32_t want) {
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         next = b.cur ^ 1;
     }
-    BatchCtl* hc = reinterpret_cast<BatchCtl*>(static_cast<char*>(b.pinned) + sizeof(ColState) * kCols);
+    BatchCtl* hc = &b.pinned->ctl;
     hc->cur = next;
+    b.published = false;
     EGX_HIP_TRY(hipMemcpyAsync(b.ctl.p, hc, sizeof(BatchCtl), hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     b.cur = next;
@@ -1446,7 +1511,7 @@ int batch_release(Batch& b, int32_t j) {
     return finish_update(b, u);
 }
 
-int enqueue_iterations(Batch& b, const SpmmArgs& a, int32_t iters, hipStream_t s);
+int enqueue_iterations(Batch& b, SpmmArgs a, int32_t iters, hipStream_t s);
 
 // Step graphs are captured on one stream per device, shared by every batch
 // there, never on a batch's own stream: other threads may be waiting on events
@@ -1537,18 +1602,21 @@ int batch_step(Batch& b, int32_t iters, bool record_time) {
         }
         if (record_time) EGX_HIP_TRY(hipEventRecord(b.ev0, s), EGX_DEVICE_ERR);
         EGX_HIP_TRY(hipGraphLaunch(sg.exec, s), EGX_DEVICE_ERR);
+        b.published = true;
         if (record_time) EGX_HIP_TRY(hipEventRecord(b.ev1, s), EGX_DEVICE_ERR);
         return EGX_SUCC;
     }
     if (record_time) EGX_HIP_TRY(hipEventRecord(b.ev0, s), EGX_DEVICE_ERR);
     EGX_TRY(enqueue_iterations(b, a, iters, s));
+    if (iters > 0) b.published = true;
     if (record_time) EGX_HIP_TRY(hipEventRecord(b.ev1, s), EGX_DEVICE_ERR);
     return EGX_SUCC;
 }
 
 // `iters` iterations (rows + reduce launches) at the batch's current width.
-int enqueue_iterations(Batch& b, const SpmmArgs& a, int32_t iters, hipStream_t s) {
+int enqueue_iterations(Batch& b, SpmmArgs a, int32_t iters, hipStream_t s) {
     for (int32_t i = 0; i < iters; ++i) {
+        if (i + 1 == iters) a.publish = b.pinned;
         if (b.grid > 0) {
             switch (b.width) {
                 case 8: k_spmm_iter<8><<<b.grid, kRowThreads, 0, s>>>(a); break;
@@ -1589,20 +1657,21 @@ int enqueue_iterations(Batch& b, const SpmmArgs& a, int32_t iters, hipStream_t s
 // Copy the column states to the host (synchronises the batch stream).
 int batch_poll(Batch& b) {
     hipStream_t s = b.stream;
-    char* p = static_cast<char*>(b.pinned);
-    EGX_HIP_TRY(hipMemcpyAsync(p, b.cols.p, sizeof(ColState) * kCols, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipMemcpyAsync(p + sizeof(ColState) * kCols, b.ctl.p, sizeof(BatchCtl), hipMemcpyDeviceToHost, s),
-                EGX_DEVICE_ERR);
+    if (!b.published) {
+        EGX_HIP_TRY(hipMemcpyAsync(b.pinned->cols, b.cols.p, sizeof(ColState) * kCols, hipMemcpyDeviceToHost, s),
+                    EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyAsync(&b.pinned->ctl, b.ctl.p, sizeof(BatchCtl), hipMemcpyDeviceToHost, s),
+                    EGX_DEVICE_ERR);
+    }
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    std::memcpy(b.host_cols.data(), p, sizeof(ColState) * kCols);
-    b.cur = reinterpret_cast<const BatchCtl*>(p + sizeof(ColState) * kCols)->cur;
+    std::memcpy(b.host_cols.data(), b.pinned->cols, sizeof(ColState) * kCols);
+    b.cur = b.pinned->ctl.cur;
     return EGX_SUCC;
 }
 
 int batch_any_active(Batch& b, int32_t* any) {
     EGX_TRY(batch_poll(b));
-    const BatchCtl* c = reinterpret_cast<const BatchCtl*>(static_cast<char*>(b.pinned) + sizeof(ColState) * kCols);
-    *any = c->any_active;
+    *any = b.pinned->ctl.any_active;
     return EGX_SUCC;
 }
 
@@ -1727,33 +1796,41 @@ int run_until_done(egx::Batch& b, int32_t max_launches, int32_t check_every, dou
 
 }  // namespace
 
-int egx::batch_result_enqueue(egx_batch* bh, int32_t j, void* host_out, hipEvent_t done) {
+int egx::batch_results_enqueue(egx_batch* bh, int32_t count, const int32_t* slots, char* const* out,
+                               hipEvent_t done) {
     using namespace egx;
-    if (!bh || !bh->b) return EGX_UNSUPPORTED_GRAPH;
+    if (!bh || !bh->b || count < 0 || count > kCols) return EGX_UNSUPPORTED_GRAPH;
     BatchDevice dg(bh->b->device);
     if (!dg.ok) return EGX_DEVICE_ERR;
     Batch& b = *bh->b;
     Graph& g = *b.g;
     hipStream_t s = b.stream;
-    if (j < 0 || j >= b.width) {
-        set_last_error("batch slot holds no request");
-        return EGX_UNSUPPORTED_GRAPH;
+    ResultList list{};
+    list.count = count;
+    for (int32_t i = 0; i < count; ++i) {
+        if (slots[i] < 0 || slots[i] >= b.width) {
+            set_last_error("batch slot holds no request");
+            return EGX_UNSUPPORTED_GRAPH;
+        }
+        list.j[i] = slots[i];
+        list.dst[i] = out[i];
     }
-    // b.out is reused by the next result on this stream only after this copy
     EGX_TRY(flush_init(b));
-    // b.out holds n doubles: room for the header and n floats (n >= 1)
-    const size_t bytes = kPackedHeader + (size_t)g.n * 4;
-    if (bytes > b.out.bytes) {
-        set_last_error("batch result buffer too small for the packed result");
-        return EGX_UNSUPPORTED_GRAPH;
+    if (count > 0) {
+        const unsigned grid = nblk(g.n, kTurn);
+        const float *x0 = b.X[0].as<float>(), *x1 = b.X[1].as<float>();
+        const BatchCtl* ctl = b.ctl.as<BatchCtl>();
+        const ColState* cols = b.cols.as<ColState>();
+        const int32_t* rank = g.reordered ? g.rank.as<int32_t>() : nullptr;
+        switch (b.width) {
+            case 8: k_spmm_results<8><<<grid, kRowThreads, 0, s>>>(x0, x1, ctl, cols, rank, g.n, list); break;
+            case 16: k_spmm_results<16><<<grid, kRowThreads, 0, s>>>(x0, x1, ctl, cols, rank, g.n, list); break;
+            case 32: k_spmm_results<32><<<grid, kRowThreads, 0, s>>>(x0, x1, ctl, cols, rank, g.n, list); break;
+            default: k_spmm_results<64><<<grid, kRowThreads, 0, s>>>(x0, x1, ctl, cols, rank, g.n, list); break;
+        }
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     }
-    k_spmm_output_packed<<<nblk(g.n, 256), 256, 0, s>>>(b.X[0].as<float>(), b.X[1].as<float>(),
-                                                         b.ctl.as<BatchCtl>(), b.width, b.cols.as<ColState>(),
-                                                         g.reordered ? g.perm.as<int32_t>() : nullptr, g.n, j,
-                                                         b.out.as<char>());
-    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    if (host_out) EGX_HIP_TRY(hipMemcpyAsync(host_out, b.out.p, bytes, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-    if (done) EGX_HIP_TRY(hipEventRecord(done, s), EGX_DEVICE_ERR);
+    EGX_HIP_TRY(hipEventRecord(done, s), EGX_DEVICE_ERR);
     return EGX_SUCC;
 }
 
