@@ -904,30 +904,69 @@ struct BatchUpdateBuf {
     int32_t t_idx[kMaxUpdateEntries];
     int32_t t_val[kMaxUpdateEntries];
     int32_t col_idx[kCols];
-    ColState cs[kCols];  // last: a copy stops after the n_cols in use
+    ColState cs[kCols];  // last: only the n_cols in use are staged
 };
 
-// Entries are applied in list order by one thread: a list may write one
-// address twice (a slot freed and re-used within one update, a column
-// released and assigned again), and the later entry must win.
-__global__ void k_batch_update(const BatchUpdateBuf* __restrict__ u, float* __restrict__ ptab,
-                               int32_t* __restrict__ tslot, ColState* __restrict__ cols, BatchCtl* __restrict__ ctl) {
-    if (threadIdx.x != 0) return;
-    for (int i = 0; i < u->h.n_ptab; ++i) ptab[u->p_idx[i]] = u->p_val[i];
-    for (int i = 0; i < u->h.n_tslot; ++i) tslot[u->t_idx[i]] = u->t_val[i];
-    for (int i = 0; i < u->h.n_cols; ++i) cols[u->col_idx[i]] = u->cs[i];
-    if (u->h.set_any) ctl->any_active = 1;
+// One workgroup reads the update where the host left it (one round trip over
+// the link; a copy to the device first cost a launch, and one thread that
+// walked the lists in memory up to 17 us).  A list may write one address
+// twice (a slot freed and re-used within one update, a column released and
+// assigned again) and the later entry must win: an entry with a later one of
+// the same index writes nothing.
+constexpr int kUpdateThreads = kMaxUpdateEntries;
+__global__ __launch_bounds__(kUpdateThreads) void k_batch_update(const BatchUpdateBuf* __restrict__ u, BatchUpdate h,
+                                                                 float* __restrict__ ptab, int32_t* __restrict__ tslot,
+                                                                 ColState* __restrict__ cols,
+                                                                 BatchCtl* __restrict__ ctl) {
+    constexpr int kWords = sizeof(ColState) / 4;
+    __shared__ int32_t p_idx[kMaxUpdateEntries], t_idx[kMaxUpdateEntries], col_idx[kCols];
+    __shared__ uint32_t cs[kCols * kWords];
+    const int t = threadIdx.x;
+    const uint32_t* words = reinterpret_cast<const uint32_t*>(u->cs);
+    float p_val = 0.0f;
+    int32_t t_val = 0;
+    if (t < h.n_ptab) {
+        p_idx[t] = u->p_idx[t];
+        p_val = u->p_val[t];
+    }
+    if (t < h.n_tslot) {
+        t_idx[t] = u->t_idx[t];
+        t_val = u->t_val[t];
+    }
+    if (t < h.n_cols) col_idx[t] = u->col_idx[t];
+    for (int i = t; i < h.n_cols * kWords; i += kUpdateThreads) cs[i] = words[i];
+    __syncthreads();
+    auto last = [](const int32_t* idx, int i, int n) {
+        for (int k = i + 1; k < n; ++k)
+            if (idx[k] == idx[i]) return false;
+        return true;
+    };
+    if (t < h.n_ptab && last(p_idx, t, h.n_ptab)) ptab[p_idx[t]] = p_val;
+    if (t < h.n_tslot && last(t_idx, t, h.n_tslot)) tslot[t_idx[t]] = t_val;
+    for (int i = t; i < h.n_cols * kWords; i += kUpdateThreads) {
+        const int k = i / kWords;
+        if (last(col_idx, k, h.n_cols))
+            reinterpret_cast<uint32_t*>(cols + col_idx[k])[i % kWords] = cs[i];
+    }
+    if (t == 0 && h.set_any) ctl->any_active = 1;
 }
 
-// dst (row stride cd) := src (row stride cs) for columns < min(cs, cd), 0 beyond.
-__global__ void k_spmm_repack(const float* __restrict__ src, int32_t cs, float* __restrict__ dst, int32_t cd,
-                              int32_t n) {
+// The current X (row stride cs) to d1 if it is x0, to d0 if it is x1 (row
+// stride cd): columns < min(cs, cd), 0 beyond.
+__global__ void k_spmm_repack(const float* x0, const float* x1, const BatchCtl* __restrict__ ctl, int32_t cs,
+                              float* d0, float* d1, int32_t cd, int32_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (int64_t)n * cd) return;
+    const int cur = ctl->cur;
+    const float* src = cur ? x1 : x0;
+    float* dst = cur ? d0 : d1;
     const int64_t v = i / cd;
-    const int32_t c = (int32_t)(i - v * cd);
-    dst[i] = (c < cs) ? src[v * cs + c] : 0.0f;
+    const int32_t j = (int32_t)(i - v * cd);
+    dst[i] = j < cs ? src[v * cs + j] : 0.0f;
 }
+
+// After a repack: its destination is current.
+__global__ void k_spmm_repacked(BatchCtl* ctl, int32_t into_first) { ctl->cur = into_first ? 0 : ctl->cur ^ 1; }
 
 // Columns [j0, j0 + count) of the current X in caller order, packed: column
 // j0 + q at out + q * n.  X is row-major, so one column by itself reads whole
@@ -1062,7 +1101,6 @@ struct Batch {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     DevBuf X[2], nval, tslot, ptab, cols, ctl, partials, red_part, hub_part, hsegs, hrows, wave_rows, out;
     uint32_t n_red = 1;
-    int cur = 0;
     int32_t width = 0;     // columns per X row (8, 16, 32 or 64): covers every assigned slot
     int32_t cap_cols = 0;  // columns the X buffers hold
     int32_t n = 0;
@@ -1080,11 +1118,10 @@ struct Batch {
     std::vector<int32_t> rank_h;              // caller id -> iteration row (relabelled graphs)
     HostBatch* pinned = nullptr;
     bool published = false;   // a step was the last to change the states: *pinned holds them once it is done
-    // pinned staging for queued updates: copies from it run in stream order,
-    // the arena is recycled after a stream sync
+    // pinned updates that their launches read in stream order; the arena is
+    // recycled after a stream sync
     char* arena = nullptr;
     size_t arena_used = 0;
-    DevBuf upd;               // device copy of the update being applied
     double last_kernel_seconds = 0.0;
     // captured runs of `iters` iterations, one per width (8, 16, 32, 64),
     // replayed by later steps of the same shape: a session narrows and
@@ -1117,7 +1154,7 @@ struct Batch {
         if (device >= 0) (void)hipSetDevice(device);
         if (stream) (void)hipStreamSynchronize(stream);
         for (DevBuf* d : {&X[0], &X[1], &nval, &tslot, &ptab, &cols, &ctl, &partials, &red_part, &hub_part, &hsegs,
-                          &hrows, &wave_rows, &out, &upd})
+                          &hrows, &wave_rows, &out})
             d->release_idle();
         pool_stream_idle(stream);
         drop_step_graphs();
@@ -1186,7 +1223,6 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
     EGX_HIP_TRY(hipHostMalloc((void**)&b->pinned, sizeof(HostBatch)),
                 EGX_FAILED_TO_ALLOCATE_HOST_MEM);
     EGX_HIP_TRY(hipHostMalloc((void**)&b->arena, kArenaBytes), EGX_FAILED_TO_ALLOCATE_HOST_MEM);
-    EGX_TRY(b->upd.alloc(sizeof(BatchUpdateBuf)));
     if (const char* e = std::getenv("EGGPU_AMD_BATCH_GRAPHS")) b->use_graph = std::strcmp(e, "0") != 0;
     if (g.reordered) {
         b->rank_h.resize((size_t)n);
@@ -1264,24 +1300,21 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
     return EGX_SUCC;
 }
 
-int batch_poll(Batch& b);
-
 // Queue one update (applied in stream order, no host wait unless the
 // staging arena wraps).
 int batch_queue_update(Batch& b, const BatchUpdateBuf& u) {
     hipStream_t s = b.stream;
     const size_t bytes = offsetof(BatchUpdateBuf, cs) + (size_t)u.h.n_cols * sizeof(ColState);
     if (b.arena_used + bytes > kArenaBytes) {
-        EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);  // earlier copies out of the arena are done
+        EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);  // earlier updates out of the arena are done
         b.arena_used = 0;
     }
     b.published = false;
     char* slot = b.arena + b.arena_used;
     b.arena_used += (bytes + 255) & ~(size_t)255;
     std::memcpy(slot, &u, bytes);
-    EGX_HIP_TRY(hipMemcpyAsync(b.upd.p, slot, bytes, hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
-    k_batch_update<<<1, kWave, 0, s>>>(b.upd.as<BatchUpdateBuf>(), b.ptab.as<float>(), b.tslot.as<int32_t>(),
-                                     b.cols.as<ColState>(), b.ctl.as<BatchCtl>());
+    k_batch_update<<<1, kUpdateThreads, 0, s>>>(reinterpret_cast<const BatchUpdateBuf*>(slot), u.h, b.ptab.as<float>(),
+                                                b.tslot.as<int32_t>(), b.cols.as<ColState>(), b.ctl.as<BatchCtl>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     return EGX_SUCC;
 }
@@ -1312,7 +1345,6 @@ int stage_col(Batch& b, BatchUpdateBuf& u, int32_t j, const ColState& cs) {
 }
 
 // Record ptab[t][j] = v in the host mirror and in update u.
-
 int stage_ptab(Batch& b, BatchUpdateBuf& u, int32_t t, int32_t j, float v) {
     if (u.h.n_ptab >= kMaxUpdateEntries) EGX_TRY(flush_update(b, u));
     b.host_ptab[(size_t)t][(size_t)j] = v;
@@ -1343,9 +1375,6 @@ int32_t width_for(int32_t need) {
     return w;
 }
 
-// Re-lay X for `want` columns per row: the current iterate is repacked into
-// the other buffer (or into new, larger buffers) and becomes current.  The
-// stream is idle afterwards.
 // Write x0 into the columns assigned since the last flush (one launch).
 int flush_init(Batch& b) {
     if (!b.init_pending) return EGX_SUCC;
@@ -1357,38 +1386,39 @@ int flush_init(Batch& b) {
     return EGX_SUCC;
 }
 
+// Re-lay X for `want` columns per row: the current iterate is repacked into
+// the other buffer (or into new, larger buffers) and becomes current.  Which
+// buffer that is stays on the device: asking for it and writing it back were
+// two waits, 60 us of the host's time per change.  The host waits only when
+// the buffers grow.
 int batch_set_width(Batch& b, int32_t want) {
     if (want == b.width) return EGX_SUCC;
     EGX_TRY(flush_init(b));
-    EGX_TRY(batch_poll(b));
     hipStream_t s = b.stream;
     const int64_t total = (int64_t)b.n * want;
-    int next;
-    if (want > b.cap_cols) {
+    const float *x0 = b.X[0].as<float>(), *x1 = b.X[1].as<float>();
+    BatchCtl* ctl = b.ctl.as<BatchCtl>();
+    const bool grow = want > b.cap_cols;
+    DevBuf nx[2];
+    if (grow) {
         StreamScope scope(s);
-        DevBuf nx[2];
         EGX_TRY(nx[0].alloc((size_t)total * 4));
         EGX_TRY(nx[1].alloc((size_t)total * 4));
-        k_spmm_repack<<<nblk(total, 256), 256, 0, s>>>(b.X[b.cur].as<float>(), b.width, nx[0].as<float>(), want, b.n);
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    }
+    float* d0 = grow ? nx[0].as<float>() : b.X[0].as<float>();
+    float* d1 = grow ? nx[0].as<float>() : b.X[1].as<float>();
+    k_spmm_repack<<<nblk(total, 256), 256, 0, s>>>(x0, x1, ctl, b.width, d0, d1, want, b.n);
+    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    k_spmm_repacked<<<1, 1, 0, s>>>(ctl, grow ? 1 : 0);
+    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    b.published = false;
+    if (grow) {
         EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
         b.drop_step_graphs();  // they address the old X buffers (and the stream is idle)
         b.X[0] = std::move(nx[0]);
         b.X[1] = std::move(nx[1]);
         b.cap_cols = want;
-        next = 0;
-    } else {
-        k_spmm_repack<<<nblk(total, 256), 256, 0, s>>>(b.X[b.cur].as<float>(), b.width, b.X[b.cur ^ 1].as<float>(),
-                                                        want, b.n);
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        next = b.cur ^ 1;
     }
-    BatchCtl* hc = &b.pinned->ctl;
-    hc->cur = next;
-    b.published = false;
-    EGX_HIP_TRY(hipMemcpyAsync(b.ctl.p, hc, sizeof(BatchCtl), hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
-    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
-    b.cur = next;
     b.width = want;
     return EGX_SUCC;
 }
@@ -1480,7 +1510,7 @@ int assign_into(Batch& b, BatchUpdateBuf& u, int32_t j, const int32_t* seeds, in
 
 // Assign column j: seeds (original node ids) or none (global PageRank).
 // Queued in stream order behind any iterations already enqueued: the host
-// waits only when the X layout has to widen.
+// waits only when the X buffers have to grow.
 int batch_assign(Batch& b, int32_t j, const int32_t* seeds, int32_t nseeds, double alpha, int32_t max_iter,
                  double tol) {
     EGX_TRY(check_assign(b, j, seeds, nseeds));
@@ -1665,7 +1695,6 @@ int batch_poll(Batch& b) {
     }
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     std::memcpy(b.host_cols.data(), b.pinned->cols, sizeof(ColState) * kCols);
-    b.cur = b.pinned->ctl.cur;
     return EGX_SUCC;
 }
 
