@@ -767,24 +767,40 @@ __global__ void k_pb_groups(const uint32_t* __restrict__ soff, const uint32_t* _
 }
 
 // Work-item sizes of the blocked iteration, in slots (multiples of kPbVec).
-// A scatter block holds a whole CU's LDS, so a graph needs about
-// kPbScatterItems items to keep every CU busy.  A sum item is one
-// wavefront; sub-bins larger than total / kPbSumItems value slots are cut
-// into pieces, so that mid-size graphs (few sub-bins, long ones) fill the
-// CUs and the heavy sub-bins of skewed graphs do not trail.  Items never
-// shrink below the minimums: a scatter item stages its chunk's 128 KB of
-// sources, and a sub-bin cut into pieces hands its row sums to the reduce
-// launch.  Measured on R-MAT 18, 20, 22 and 24 (ms per iteration, fixed
-// 256K-slot scatter and 128K-slot sum items -> these sizes): 0.125 -> 0.047,
-// 0.163 -> 0.083, 0.243 -> 0.184, 0.609 -> 0.611.
+// A scatter block holds a whole CU's LDS and stages its chunk's 128 KB of
+// sources, so an item is at least 32K slots, and kPbCus items run at a time.
+// Where such items of at most 64K slots fit one such round, the smallest that
+// do are taken.  Larger graphs take total / items, down to 64K slots, which
+// is one batch of 8 groups a lane (weighted: 32K, batches hold 2 groups).
+// us per iteration with items of 32K -> 64K slots: 1,048,576 nodes and 16
+// arcs each 50 -> 47, 2,097,152 89 -> 86, 4,194,304 151 -> 145; weighted, one
+// round: 700,001 nodes 50 -> 41; weighted above that, 32K and 64K: 3,000,017
+// nodes 124 and 127, R-MAT 24 with 64K to 256K 633 to 664.
+constexpr int64_t kPbCus = 256;
 constexpr int64_t kPbScatterItems = 1024;
-// weighted graphs: their scatter keeps 2 groups per lane per batch, and
-// shorter items balance better (R-MAT 24: 0.65-0.67 ms per pair at 2048-4096
-// items against 0.70 at 1024; unweighted within noise)
 constexpr int64_t kPbScatterItemsW = 4096;
 constexpr int64_t kPbScatterMin = 32768;
-constexpr int64_t kPbSumItems = 512;
-constexpr int64_t kPbSumMin = 16384;
+constexpr int64_t kPbScatterMax1 = 65536;  // one round; unweighted graphs of several take no less
+// A sum item is a workgroup; sub-bins larger than total / items value slots
+// are cut into pieces, so that mid-size graphs (few sub-bins, long ones) fill
+// the CUs and the heavy sub-bins of skewed graphs do not trail; each piece
+// hands its row sums to the reduce launch.  From kPbSumBins sub-bins on fewer
+// pieces are the better choice: us per iteration with total / 512 of 16K or
+// more against total / 256 of 32K or more: 1,048,576 nodes 46.6 and 48.0,
+// 2,097,152 85.0 and 77.7, 4,194,304 142.6 and 134.4, weighted 3,000,017 124
+// and 119, R-MAT 24 494 and 494.
+constexpr int64_t kPbSumBins = 1024;
+constexpr int64_t kPbSumItems = 512, kPbSumMin = 16384;
+constexpr int64_t kPbSumItemsMany = 256, kPbSumMinMany = 32768;
+// Graphs laid out for shared launches: one size for all, as the set fills the
+// device.  us per iteration of sets of 16 to 100 graphs, items of 256K and
+// 128K slots -> 96K and 32K: 48 graphs of 1,000 to 300,000 nodes 128 -> 101,
+// 24 of them 107 -> 63, 96 of them 185 -> 175, 16 of 20,000 to 1,000,000
+// 181 -> 156, 100 of 1,000 to 20,000 69 -> 50 (scatter items of 64K to 192K
+// differ by how they fill the last round: 108, 70, 186, 166, 46 and 99, 78,
+// 160, 167, 61).
+constexpr int64_t kPbScatterShared = 98304;
+constexpr int64_t kPbSumShared = 32768;
 
 int64_t pb_item_slots(int64_t total, int64_t items, int64_t lo, int64_t hi) {
     const int64_t want = (total / items) / kPbVec * kPbVec;
@@ -936,19 +952,39 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     EGX_HIP_TRY(hipMemcpyWithStream(&bad_h, bad.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
 
-    // scatter work: contiguous group ranges of at most scat_slots slots per chunk
-    // (a graph laid out for shared launches takes the largest items: the set fills the device)
-    const int64_t scat_items = g.weighted ? kPbScatterItemsW : kPbScatterItems;
-    // whole windows: an item starts on its chunk's window grid
-    const int32_t scat_groups = std::max<int32_t>(
-        kPbWindow, (int32_t)(pb_item_slots(slots, cfg.blocked_shared ? 1 : scat_items, kPbScatterMin, kPbScatterItem) /
-                             kPbVec / kPbWindow * kPbWindow));
+    // scatter work: contiguous group ranges of at most scat_groups groups per
+    // chunk, whole windows: an item starts on its chunk's window grid
+    auto chunk_groups = [&](int64_t c, int32_t& c0, int32_t& c1) {
+        c0 = (int32_t)(soff_h[(size_t)(c * B)] / kPbVec);
+        c1 = (int32_t)(soff_h[(size_t)((c + 1) * B)] / kPbVec);
+    };
+    auto scatter_slots = [&]() -> int64_t {
+        if (cfg.blocked_shared) return kPbScatterShared;
+        constexpr int64_t kStep = 4 * kPbWindow * kPbVec;
+        const int64_t first = std::max<int64_t>(kPbScatterMin, (slots / kPbCus) / kStep * kStep);
+        for (int64_t z = first; z <= kPbScatterMax1; z += kStep) {
+            int64_t items = 0;
+            for (int64_t c = 0; c < S; ++c) {
+                int32_t c0, c1;
+                chunk_groups(c, c0, c1);
+                items += (c1 - c0 + z / kPbVec - 1) / (z / kPbVec);
+            }
+            if (items <= kPbCus) return z;
+        }
+        return g.weighted ? pb_item_slots(slots, kPbScatterItemsW, kPbScatterMin, kPbScatterItem)
+                          : pb_item_slots(slots, kPbScatterItems, kPbScatterMax1, kPbScatterItem);
+    };
+    const int32_t scat_groups =
+        std::max<int32_t>(kPbWindow, (int32_t)(scatter_slots() / kPbVec / kPbWindow * kPbWindow));
+    const bool many_bins = B >= kPbSumBins;
     const int32_t sum_slots =
-        (int32_t)pb_item_slots(nvals, cfg.blocked_shared ? 1 : kPbSumItems, kPbSumMin, kPbItem);
+        (int32_t)(cfg.blocked_shared ? kPbSumShared
+                                     : pb_item_slots(nvals, many_bins ? kPbSumItemsMany : kPbSumItems,
+                                                     many_bins ? kPbSumMinMany : kPbSumMin, kPbItem));
     std::vector<PbScatter> scat;
     for (int64_t c = 0; c < S; ++c) {
-        const int32_t c0 = (int32_t)(soff_h[(size_t)(c * B)] / kPbVec);
-        const int32_t c1 = (int32_t)(soff_h[(size_t)((c + 1) * B)] / kPbVec);
+        int32_t c0, c1;
+        chunk_groups(c, c0, c1);
         for (int32_t q0 = c0; q0 < c1; q0 += scat_groups)
             scat.push_back(PbScatter{(int32_t)c, q0, (int32_t)std::min<int64_t>(c1, (int64_t)q0 + scat_groups), 0});
     }

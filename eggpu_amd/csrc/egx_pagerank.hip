@@ -768,6 +768,7 @@ __device__ __forceinline__ void pb_scatter_batch(const PbScatterBatch<W>& cur, i
                                                  const float* sc, float* stg, float* vals, int l) {
 #pragma unroll
     for (int q = 0; q < PbScatterBatch<W>::kG; ++q) {
+        if (g0 + q * kPbThreads >= g1) break;  // (wavefront-uniform) the item ends before
         const bool ok = g0 + q * kPbThreads + l < g1;
         const int32_t vgq = cur.vg[q];
         const uint32_t mkq = ok ? cur.mk[q] : 0u;
