@@ -1777,6 +1777,27 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
     std::vector<int32_t> rblk((size_t)rtotal);
     for (int32_t i = 0; i < count; ++i)
         std::fill(rblk.begin() + rbase[(size_t)i], rblk.begin() + rbase[(size_t)i] + table[(size_t)i].n_red, i);
+    // The results that the host asks for lie one after another, so that they
+    // cross the link in whole chunks (48 of them, 14 MB, took 48 copies and
+    // 0.95 ms).  Without the memory for that each goes to its graph's own.
+    bool wanted = false;
+    for (int32_t i = 0; i < count; ++i) wanted = wanted || (host_out && host_out[i]);
+    const bool packed = wanted && std::is_same<T, float>::value;  // FP32 results are finished by the host
+    DevBuf results;
+    if (wanted) {
+        const size_t elem = packed ? 4 : 8;
+        size_t values = 0;
+        for (int32_t i = 0; i < count; ++i)
+            if (host_out[i]) values += (size_t)gs[(size_t)i]->n;
+        if (results.alloc(std::max<size_t>(values, 1) * elem, s) == EGX_SUCC) {
+            size_t at = 0;
+            for (int32_t i = 0; i < count; ++i) {
+                if (!host_out[i]) continue;
+                table[(size_t)i].out = reinterpret_cast<double*>(results.as<char>() + at);
+                at += (size_t)gs[(size_t)i]->n * elem;
+            }
+        }
+    }
     DevBuf d_table, d_blk, d_base, d_rblk, d_rbase, d_nbase, d_states, d_pbt, d_scg, d_scl, d_sumg, d_suml;
     const uint32_t n_sc = (uint32_t)sc_graph.size(), n_sum = (uint32_t)sum_graph.size();
     if (n_sc > 0) {
@@ -1823,7 +1844,9 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
     size_t tile_lds = 0;  // LDS of the largest tile among the pull members
     for (int32_t i = 0; i < count; ++i)
         if (!is_pb[(size_t)i]) tile_lds = std::max(tile_lds, (size_t)gs[(size_t)i]->tile_lds * sizeof(T));
-    const int32_t chunk = p.check_every > 0 ? p.check_every : 8;
+    // at tol 0 every member runs to max_iter: nothing to look at in between
+    const bool can_stop_early = p.tol > 0.0 || p.use_graph;
+    const int32_t chunk = !can_stop_early ? p.max_iter : p.check_every > 0 ? p.check_every : 8;
     // the SpMV of one iteration for every member: blocked members' scatter,
     // the others' pull work items, then the blocked members' sums
     auto launch_spmv = [&]() {
@@ -1895,12 +1918,7 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
     EGX_HIP_TRY(hipMemcpyAsync(hs, d_states.p, sizeof(PrState) * (size_t)count, hipMemcpyDeviceToHost, s),
                 EGX_DEVICE_ERR);
     // every result in one launch (FP32 ones for the host packed), copied only where asked for
-    bool wanted = false;
-    for (int32_t i = 0; i < count; ++i) wanted = wanted || (host_out && host_out[i]);
-    constexpr bool kPacked = std::is_same<T, float>::value;
-    bool packed = false;
-    if constexpr (kPacked) {
-        packed = wanted;
+    if constexpr (std::is_same<T, float>::value) {
         if (packed)
             k_pr_output_packed_multi<<<nbase[(size_t)count], 256, 0, s>>>(d_table.as<IterArgs<T>>(),
                                                                           d_nbase.as<uint32_t>(), count);
@@ -1914,7 +1932,7 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
         std::vector<Fetch> jobs;
         for (int32_t i = 0; i < count; ++i)
             if (host_out[i])
-                jobs.push_back(Fetch{gs[(size_t)i]->out.p, host_out[i], gs[(size_t)i]->n, packed, hs[i].sum});
+                jobs.push_back(Fetch{table[(size_t)i].out, host_out[i], gs[(size_t)i]->n, packed, hs[i].sum});
         EGX_TRY(fetch(jobs, s));
     }
     if (st) {

@@ -188,18 +188,25 @@ size_t part_bytes(size_t total) {
     return std::min(kChunkBytes, std::max(kInlineBytes, even));
 }
 
+// Values [i0, i0 + n) of a job, `at` bytes into the part that carries them.
+struct Piece {
+    const Fetch* f;
+    int64_t i0, n;
+    size_t at;
+};
+
 struct Part {
-    const Fetch* f;    // the job (fetch)
-    int64_t i0, n;     // its values (fetch)
-    const char* host;  // source (upload)
+    const char* host;      // source (upload)
     char* dev;
     size_t bytes;
+    size_t first, pieces;  // of the run's pieces (fetch): one job's values, or those of jobs that follow each other
 };
 
 // The transfer's parts, taken in order by several threads; part k uses
 // chunk k % chunks, after part k - chunks is through with it.
 struct Run {
     std::vector<Part> parts;
+    std::vector<Piece> pieces;
     std::vector<Chunk> chunks;
     std::unique_ptr<std::atomic<int>[]> stage;  // per part: 1 queued (fetch), 2 through
     std::atomic<int64_t> next{0};
@@ -221,6 +228,10 @@ struct Run {
         }
         return true;
     }
+    void finish(const Part& p, const char* from) const {
+        for (size_t q = p.first; q < p.first + p.pieces; ++q)
+            finish_values(*pieces[q].f, pieces[q].i0, pieces[q].n, from + pieces[q].at);
+    }
     void queue_fetch(int64_t k) {
         const Part& p = parts[(size_t)k];
         const Chunk& c = chunks[(size_t)k % chunks.size()];
@@ -236,7 +247,7 @@ struct Run {
             const Part& p = parts[(size_t)k];
             const Chunk& c = chunks[(size_t)k % chunks.size()];
             if (!ok(hipEventSynchronize(c.ev))) return;
-            finish_values(*p.f, p.i0, p.n, c.p);
+            finish(p, c.p);
             stage[(size_t)k].store(2, std::memory_order_release);
             if (k + ring < total) queue_fetch(k + ring);
         }
@@ -288,8 +299,8 @@ int upload_chunked(const std::vector<Upload>& jobs, size_t total_bytes, hipStrea
     const size_t step = part_bytes(total_bytes);
     for (const Upload& u : jobs)
         for (size_t at = 0; at < u.bytes; at += step)
-            r.parts.push_back(Part{nullptr, 0, 0, static_cast<const char*>(u.host) + at,
-                                   static_cast<char*>(u.dev) + at, std::min(step, u.bytes - at)});
+            r.parts.push_back(Part{static_cast<const char*>(u.host) + at, static_cast<char*>(u.dev) + at,
+                                   std::min(step, u.bytes - at), 0, 0});
     const std::function<void()> work = [&] { r.upload_parts(); };
     if (begin_run(r, r.parts.size(), s) != 0) {  // no pinned memory
         for (const Upload& u : jobs)
@@ -302,13 +313,21 @@ int upload_chunked(const std::vector<Upload>& jobs, size_t total_bytes, hipStrea
 
 int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_t s) {
     Run r;
+    const size_t step = part_bytes(total_bytes);
     for (const Fetch& f : jobs) {
         const size_t elem = f.packed ? 4 : 8;
-        const int64_t step = (int64_t)(part_bytes(total_bytes) / elem);
-        for (int64_t i = 0; i < f.n; i += step) {
-            const int64_t k = std::min(step, f.n - i);
-            r.parts.push_back(Part{&f, i, k, nullptr, static_cast<char*>(const_cast<void*>(f.dev)) + (size_t)i * elem,
-                                   (size_t)k * elem});
+        char* dev = static_cast<char*>(const_cast<void*>(f.dev));
+        for (int64_t i = 0; i < f.n;) {
+            char* at = dev + (size_t)i * elem;
+            if (r.parts.empty() || r.pieces.back().f->packed != f.packed ||
+                r.parts.back().dev + r.parts.back().bytes != at || r.parts.back().bytes + elem > step)
+                r.parts.push_back(Part{nullptr, at, 0, r.pieces.size(), 0});
+            Part& p = r.parts.back();
+            const int64_t k = std::min((int64_t)((step - p.bytes) / elem), f.n - i);
+            r.pieces.push_back(Piece{&f, i, k, p.bytes});
+            p.bytes += (size_t)k * elem;
+            p.pieces += 1;
+            i += k;
         }
     }
     if (r.parts.empty()) return EGX_SUCC;
@@ -318,7 +337,7 @@ int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_
         std::vector<char> buf(kChunkBytes);
         for (const Part& p : r.parts) {
             EGX_HIP_TRY(hipMemcpyWithStream(buf.data(), p.dev, p.bytes, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-            finish_values(*p.f, p.i0, p.n, buf.data());
+            r.finish(p, buf.data());
         }
         return EGX_SUCC;
     }
