@@ -182,45 +182,87 @@ __device__ __forceinline__ double arc_weight(const int32_t* __restrict__ E, cons
 
 // Out-weight and valid out-arc count of every row.  The sum is the one of
 // adding the row's weights one after the other in CSR order (pagerank.cu:308-315),
-// bit for bit.  kOutLanes lanes share a row: they load that many arcs
-// together and each adds them in order (shuffles inside the group), so the
-// only serial part is the chain of additions; one thread walking a row by
-// itself paid a memory latency per arc (95 ns: 7.6 ms for the longest row of
-// an 11M-arc R-MAT graph, 4.3 ms at 8M arcs, whatever the other rows did).
-// Rows longer than kOutLong go to k_row_out_long.
-constexpr int kOutLanes = 8;
+// bit for bit.  A workgroup takes the rows that begin in its kOutTile arcs:
+// their arcs come in whole lines into LDS, where each row has a thread that
+// adds them (8 lanes per row that loaded their own arcs and passed them on
+// by shuffles: 190 us for 9.3M arcs; one thread walking a row in memory paid a
+// latency per arc, 95 ns).  Rows longer than kOutLong, listed beforehand,
+// are the first workgroups' of the same launch: one of them each (they ran
+// 114 us by themselves).  9.3M weighted arcs: 304 us -> 113, the longest row's
+// chain of additions, and 18 for the list.
+constexpr int kOutThreads = 256;
 constexpr int32_t kOutLong = 256;
+constexpr int32_t kOutTile = 4096;
+constexpr int kLongStage = 1024;
+constexpr int kLongBlocks = 1024;
+struct OutTile {
+    double w[kOutTile + kOutLong];
+    int32_t rows[2];
+    uint32_t bad;
+};
+struct OutLong {
+    double stage[2][kLongStage];
+    double s[4];
+    int32_t c[4], low[4];
+};
+
+// First row whose offset is at least q (V[n] >= q), by one wavefront.
+__device__ __forceinline__ int32_t wave_first_row(const int32_t* __restrict__ V, int32_t n, int64_t q) {
+    int32_t lo = 0, hi = n;  // V[hi] >= q
+    while (lo < hi) {
+        const int64_t step = ((int64_t)hi - lo + kWave - 1) / kWave;
+        const int64_t at = (int64_t)lo + (lane_id() + 1) * step - 1;
+        const bool below = at < hi && (int64_t)V[at] < q;
+        const int k = __popcll(__ballot(below));  // offsets ascend: a prefix of the lanes
+        const int64_t nlo = (int64_t)lo + k * step, nhi = nlo + step - 1;
+        lo = (int32_t)min(nlo, (int64_t)hi);
+        hi = (int32_t)min(nhi, (int64_t)hi);
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+}
+
 template <bool HasW>
-__global__ __launch_bounds__(256) void k_row_out(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
-                                                 const double* __restrict__ W, int32_t n,
-                                                 double* __restrict__ out_w, int32_t* __restrict__ outcnt,
-                                                 int32_t* __restrict__ long_rows, uint32_t* __restrict__ n_long) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)n * kOutLanes) return;  // whole groups: 64 is a multiple of kOutLanes
-    const int32_t u = (int32_t)(t / kOutLanes);
-    const int sub = (int)(t % kOutLanes);
-    const int32_t beg = V[u], end = V[u + 1];
-    if (end - beg > kOutLong) {
-        if (sub == 0) long_rows[atomicAdd(n_long, 1u)] = u;
-        return;
+__device__ __forceinline__ void row_out_tile(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
+                                             const double* __restrict__ W, int32_t n, int64_t tile, bool last,
+                                             double* __restrict__ out_w, int32_t* __restrict__ outcnt, OutTile& sh) {
+    const int t = threadIdx.x;
+    const int64_t q0 = tile * kOutTile;
+    if (t == 0) sh.bad = 0;
+    if (wave_id() < 2) {
+        const int32_t r = (wave_id() == 1 && last) ? n : wave_first_row(V, n, q0 + wave_id() * kOutTile);
+        if (lane_id() == 0) sh.rows[wave_id()] = r;
     }
-    double s = 0.0;
-    int32_t c = 0;
-    double w = (int64_t)beg + sub < end ? arc_weight<HasW>(E, W, (int64_t)beg + sub, n, c) : 0.0;
-    for (int64_t p = beg; p < end; p += kOutLanes) {
-        const int64_t nx = p + kOutLanes + sub;  // the next arcs are loaded before these are added
-        const double wn = nx < end ? arc_weight<HasW>(E, W, nx, n, c) : 0.0;
-        if (HasW) {
-#pragma unroll
-            for (int j = 0; j < kOutLanes; ++j) s += __shfl(w, j, kOutLanes);
+    __syncthreads();
+    const int32_t r0 = sh.rows[0], r1 = sh.rows[1];
+    if (r0 >= r1) return;  // (uniform)
+    // the arcs of these rows, but no further than the longest row that ends here could reach
+    const int64_t a0 = V[r0], a1 = min((int64_t)V[r1], q0 + kOutTile + kOutLong);
+    for (int64_t p = a0 + t; p < a1; p += kOutThreads) {
+        int32_t ok = 0;
+        const double w = arc_weight<HasW>(E, W, p, n, ok);
+        sh.w[p - q0] = w;
+        if (!ok) sh.bad = 1;
+    }
+    __syncthreads();
+    const bool bad = sh.bad != 0;
+    for (int32_t r = r0 + t; r < r1; r += kOutThreads) {
+        const int32_t beg = V[r], len = V[r + 1] - beg;
+        if (len > kOutLong) continue;
+        int32_t c = len;
+        if (bad) {
+            c = 0;
+            for (int32_t k = 0; k < len; ++k) {
+                const int32_t v = E[beg + k];
+                c += (v >= 0 && v < n) ? 1 : 0;
+            }
         }
-        w = wn;
-    }
-#pragma unroll
-    for (int off = kOutLanes / 2; off > 0; off >>= 1) c += __shfl_xor(c, off, kOutLanes);
-    if (sub == 0) {
-        out_w[u] = HasW ? s : (double)c;
-        outcnt[u] = c;
+        double s = 0.0;
+        if (HasW) {
+            const double* w = sh.w + (beg - q0);
+            for (int32_t k = 0; k < len; ++k) s += w[k];
+        }
+        out_w[r] = HasW ? s : (double)c;
+        outcnt[r] = c;
     }
 }
 
@@ -240,20 +282,13 @@ __device__ __forceinline__ int32_t lowest_bit(double w) {
 // the parallel sum is the sequential one.  That holds for unit weights and
 // for weights that came from 32-bit floats.  Other rows are staged through
 // LDS and added in CSR order by one wavefront.
-constexpr int kLongStage = 1024;
-constexpr int kLongBlocks = 1024;
 template <bool HasW>
-__global__ __launch_bounds__(256) void k_row_out_long(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
-                                                      const double* __restrict__ W, int32_t n,
-                                                      double* __restrict__ out_w, int32_t* __restrict__ outcnt,
-                                                      const int32_t* __restrict__ long_rows,
-                                                      const uint32_t* __restrict__ n_long) {
-    __shared__ double stage[2][kLongStage];
-    __shared__ double sh_s[4];
-    __shared__ int32_t sh_c[4], sh_low[4];
+__device__ __forceinline__ void row_out_long(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
+                                             const double* __restrict__ W, int32_t n, uint32_t first, uint32_t step,
+                                             double* __restrict__ out_w, int32_t* __restrict__ outcnt,
+                                             const int32_t* __restrict__ long_rows, uint32_t rows, OutLong& sh) {
     const int t = threadIdx.x;
-    const uint32_t rows = *n_long;
-    for (uint32_t i = blockIdx.x; i < rows; i += gridDim.x) {
+    for (uint32_t i = first; i < rows; i += step) {
         const int32_t u = long_rows[i];
         const int32_t beg = V[u], end = V[u + 1];
         double s = 0.0;
@@ -270,31 +305,31 @@ __global__ __launch_bounds__(256) void k_row_out_long(const int32_t* __restrict_
             low = min(low, __shfl_xor(low, off, kWave));
         }
         if (lane_id() == 0) {
-            sh_s[wave_id()] = s;
-            sh_c[wave_id()] = c;
-            sh_low[wave_id()] = low;
+            sh.s[wave_id()] = s;
+            sh.c[wave_id()] = c;
+            sh.low[wave_id()] = low;
         }
         __syncthreads();
-        s = (sh_s[0] + sh_s[1]) + (sh_s[2] + sh_s[3]);
-        c = sh_c[0] + sh_c[1] + sh_c[2] + sh_c[3];
-        low = min(min(sh_low[0], sh_low[1]), min(sh_low[2], sh_low[3]));
+        s = (sh.s[0] + sh.s[1]) + (sh.s[2] + sh.s[3]);
+        c = sh.c[0] + sh.c[1] + sh.c[2] + sh.c[3];
+        low = min(min(sh.low[0], sh.low[1]), min(sh.low[2], sh.low[3]));
         const bool exact = !HasW || low == 4096 || s < ldexp(1.0, low + 53);  // uniform over the workgroup
         if (!exact) {
             int32_t dummy = 0;
             double run = 0.0;
             for (int32_t q = t; q < kLongStage; q += 256)
-                stage[0][q] = (int64_t)beg + q < end ? arc_weight<HasW>(E, W, (int64_t)beg + q, n, dummy) : 0.0;
+                sh.stage[0][q] = (int64_t)beg + q < end ? arc_weight<HasW>(E, W, (int64_t)beg + q, n, dummy) : 0.0;
             __syncthreads();
             int cur = 0;
             for (int64_t p = beg; p < end; p += kLongStage, cur ^= 1) {
                 if (wave_id() == 0) {  // every lane reads the same entries
-                    const double* st = stage[cur];
+                    const double* st = sh.stage[cur];
 #pragma unroll 16
                     for (int q = 0; q < kLongStage; ++q) run += st[q];
                 } else {
                     const int64_t nb = p + kLongStage;
                     for (int32_t q = t - kWave; q < kLongStage; q += 256 - kWave)
-                        stage[cur ^ 1][q] = nb + q < end ? arc_weight<HasW>(E, W, nb + q, n, dummy) : 0.0;
+                        sh.stage[cur ^ 1][q] = nb + q < end ? arc_weight<HasW>(E, W, nb + q, n, dummy) : 0.0;
                 }
                 __syncthreads();
             }
@@ -304,8 +339,40 @@ __global__ __launch_bounds__(256) void k_row_out_long(const int32_t* __restrict_
             out_w[u] = s;
             outcnt[u] = c;
         }
-        __syncthreads();  // sh_* are reused by the next row
+        __syncthreads();  // sh is reused by the next row
     }
+}
+
+// Workgroups [0, long_blocks) take the listed rows, the others a tile each.
+template <bool HasW>
+__global__ __launch_bounds__(kOutThreads) void k_row_out(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
+                                                         const double* __restrict__ W, int32_t n, uint32_t tiles,
+                                                         double* __restrict__ out_w, int32_t* __restrict__ outcnt,
+                                                         const int32_t* __restrict__ long_rows,
+                                                         const uint32_t* __restrict__ n_long, uint32_t long_blocks) {
+    __shared__ union {
+        OutTile tile;
+        OutLong row;
+    } sh;
+    if (blockIdx.x < long_blocks) {
+        row_out_long<HasW>(V, E, W, n, blockIdx.x, long_blocks, out_w, outcnt, long_rows, *n_long, sh.row);
+    } else {
+        const uint32_t tile = blockIdx.x - long_blocks;
+        row_out_tile<HasW>(V, E, W, n, tile, tile + 1 == tiles, out_w, outcnt, sh.tile);
+    }
+}
+
+// The rows longer than kOutLong.
+__global__ void k_long_rows(const int32_t* __restrict__ V, int32_t n, int32_t* __restrict__ long_rows,
+                            uint32_t* __restrict__ n_long) {
+    const int32_t u = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool is_long = u < n && V[u + 1] - V[u] > kOutLong;
+    const uint64_t mask = __ballot(is_long);
+    if (mask == 0) return;
+    uint32_t at = 0;
+    if (lane_id() == 0) at = atomicAdd(n_long, (uint32_t)__popcll(mask));
+    at = __builtin_amdgcn_readfirstlane(at);
+    if (is_long) long_rows[at + __popcll(mask & ((1ull << lane_id()) - 1ull))] = u;
 }
 
 // Sum / maximum over a 256-thread workgroup, valid in thread 0.
@@ -1242,15 +1309,14 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
         int32_t* lr = long_rows.as<int32_t>();
         uint32_t* nl = ctr + kCtrLong;
         const unsigned lb = (unsigned)std::min<int64_t>(max_long, kLongBlocks);
-        const unsigned sb = nblocks((int64_t)n * kOutLanes, 256);
-        if (dW) k_row_out<true><<<sb, 256, 0, s>>>(dV, dE, dW, n, out_w, outcnt_p, lr, nl);
-        else k_row_out<false><<<sb, 256, 0, s>>>(dV, dE, nullptr, n, out_w, outcnt_p, lr, nl);
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         if (lb > 0) {
-            if (dW) k_row_out_long<true><<<lb, 256, 0, s>>>(dV, dE, dW, n, out_w, outcnt_p, lr, nl);
-            else k_row_out_long<false><<<lb, 256, 0, s>>>(dV, dE, nullptr, n, out_w, outcnt_p, lr, nl);
+            k_long_rows<<<nblocks(n, 256), 256, 0, s>>>(dV, n, lr, nl);
             EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         }
+        const unsigned tiles = nblocks(std::max<int64_t>(m, 1), kOutTile);
+        if (dW) k_row_out<true><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, dW, n, tiles, out_w, outcnt_p, lr, nl, lb);
+        else k_row_out<false><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, nullptr, n, tiles, out_w, outcnt_p, lr, nl, lb);
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         return EGX_SUCC;
     };
     auto unit_out = [&]() -> int {

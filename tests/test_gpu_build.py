@@ -7,8 +7,8 @@ from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# out-degrees around the lanes per row (8), the long-row limit (1024) and the long rows' staging chunk (1024)
-OUT_LENGTHS = [0, 1, 7, 8, 9, 15, 16, 17, 1023, 1024, 1025, 2047, 2048, 2049, 5000]
+# out-degrees around the long-row limit (256) and the long rows' staging chunk (1024)
+OUT_LENGTHS = [0, 1, 7, 8, 9, 15, 16, 17, 255, 256, 257, 1023, 1024, 1025, 2047, 2048, 2049, 5000]
 
 
 def _weights(rng, kind, m):
@@ -45,6 +45,39 @@ def test_out_weight_sums_bit_exact(gpu_ready, kind, invalid):
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     assert np.array_equal(got[2].view(np.uint32), want[2].view(np.uint32))
     assert np.array_equal(got[3], want[3])
+
+
+# rows against the 4096-arc tiles: a row of the limit that starts at a tile's last arc, empty rows on an edge and at the
+# end, whole tiles without a row's start, an arc count of whole tiles
+OUT_TILES = {
+    "over_the_edge": [255] * 16 + [15, 256, 256, 1, 0, 0, 3],
+    "empty_on_the_edge": [256] * 16 + [0] * 700 + [256] * 16 + [0] * 300,
+    "tile_without_a_start": [4095, 9000, 2, 257, 256, 0],
+    "long_first": [300, 0, 5],
+    "one_arc": [0, 1, 0],
+}
+
+
+@pytest.mark.parametrize("name", sorted(OUT_TILES))
+@pytest.mark.parametrize("invalid", [False, True])
+def test_out_weight_tiles_bit_exact(gpu_ready, name, invalid):
+    print(f"out weight tiles {name} invalid={invalid}", flush=True)
+    rng = np.random.default_rng(8)
+    lengths = np.array(OUT_TILES[name])
+    n = len(lengths)
+    V = np.zeros(n + 1, np.int32)
+    V[1:] = np.cumsum(lengths)
+    m = int(V[-1])
+    E = rng.integers(0, n, m).astype(np.int32)
+    if invalid:
+        E[rng.choice(m, (m + 6) // 7, replace=False)] = -1
+    for W in (_weights(rng, "double", m), np.ones(m)):
+        with native.DeviceGraph.from_csr(V, E, W, alpha=0.85) as g:
+            got = g.download_csc()
+        want = O.build_inbound(V, E, W, 0.85)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        assert np.array_equal(got[2].view(np.uint32), want[2].view(np.uint32))
+        assert np.array_equal(got[3], want[3])
 
 
 @pytest.mark.parametrize("n,m", [(1, 3), (2, 2), (255, 1000), (257, 4096), (65537, 200001)])
