@@ -154,18 +154,8 @@ enum : int {
     kCtrMaxIn,     // largest in-degree
     kCtrLong,      // rows longer than kOutLong
     kCtrHubs,      // rows above the hub threshold
-    kCtrWaveRows,  // rows reduced by a wavefront each
-    kCtrWords
+    kCtrWords = 16  // 64 bytes: a clear is one launch
 };
-
-__global__ void k_outcnt_from_V(const int32_t* __restrict__ V, int32_t n, double* __restrict__ out_w,
-                                int32_t* __restrict__ outcnt) {
-    const int32_t u = blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= n) return;
-    const int32_t c = V[u + 1] - V[u];
-    outcnt[u] = c;
-    out_w[u] = (double)c;
-}
 
 // The weight of arc p as the build counts it (pagerank.cu:308-315): 0 when
 // its endpoint is outside [0, n) or the weight is not finite or negative.
@@ -398,17 +388,27 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t* sh) {
 // (one per 256 nodes took 67 us at 700K nodes).
 constexpr int kNodeBlocks = 512;
 
-// deg (0 == dangling), dangling count, max out-degree.
-__global__ __launch_bounds__(256) void k_node_arrays(const double* __restrict__ out_w,
-                                                     const int32_t* __restrict__ outcnt, int32_t n, int weighted,
-                                                     float* __restrict__ deg, uint32_t* __restrict__ ctr) {
+// deg (0 == dangling), dangling count, max out-degree.  Count: the out-arcs
+// are the offsets' differences, written here with the out-weights (1 each
+// with unit_out, else the counts).
+template <bool Count>
+__global__ __launch_bounds__(256) void k_node_arrays(const int32_t* __restrict__ V, double* __restrict__ out_w,
+                                                     int32_t* __restrict__ outcnt, int32_t n, int unit_out,
+                                                     int weighted, float* __restrict__ deg,
+                                                     uint32_t* __restrict__ ctr) {
     __shared__ uint32_t sh[4];
     uint32_t nd = 0, most = 0;
     for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < n; u += (int64_t)gridDim.x * 256) {
-        const bool dang = !(out_w[u] > 0.0);  // pagerank.cu:323-326: outW <= 0
-        deg[u] = weighted ? (dang ? 0.0f : 1.0f) : (dang ? 0.0f : (float)outcnt[u]);
+        const int32_t c = Count ? V[u + 1] - V[u] : outcnt[u];
+        const double w = Count ? (unit_out ? 1.0 : (double)c) : out_w[u];
+        if (Count) {
+            outcnt[u] = c;
+            out_w[u] = w;
+        }
+        const bool dang = !(w > 0.0);  // pagerank.cu:323-326: outW <= 0
+        deg[u] = weighted ? (dang ? 0.0f : 1.0f) : (dang ? 0.0f : (float)c);
         nd += dang ? 1u : 0u;
-        most = max(most, (uint32_t)outcnt[u]);
+        most = max(most, (uint32_t)c);
     }
     nd = block_sum_u32(nd, sh);
     most = block_max_u32(most, sh);
@@ -469,8 +469,9 @@ __global__ __launch_bounds__(256) void k_in_degrees(const int32_t* __restrict__ 
 // equal keys.  perm[r] = original id of row r, rank = its inverse.
 __global__ void k_layout_keys(const int32_t* __restrict__ in_row, const int32_t* __restrict__ out_cnt, int32_t n,
                               int32_t hub, int32_t bits, uint32_t maxdeg, int reorder, uint32_t* __restrict__ keys,
-                              uint32_t* __restrict__ vals) {
+                              uint32_t* __restrict__ vals, int32_t* __restrict__ pad) {
     const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v < kArcPad) pad[v] = 0;  // the zeroed slots past in_col's arcs
     if (v >= n) return;
     const bool is_hub = (in_row[v + 1] - in_row[v]) > hub;
     const uint32_t sec = reorder ? (maxdeg - (uint32_t)out_cnt[v]) : 0u;
@@ -481,8 +482,9 @@ __global__ void k_layout_keys(const int32_t* __restrict__ in_row, const int32_t*
 // tiles[k] = first row v in [n_hub, n] whose merge-path diagonal
 // (it_row[v] - it_row[n_hub]) + (v - n_hub) reaches k * tile_items.
 __global__ void k_tile_starts(const int32_t* __restrict__ row, int32_t n_hub, int32_t n, int32_t tile_items,
-                              int64_t n_tiles, int32_t* __restrict__ tiles) {
+                              int64_t n_tiles, int32_t* __restrict__ tiles, uint32_t* __restrict__ wave_rows) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k == 0) *wave_rows = 0;
     if (k > n_tiles) return;
     if (k == n_tiles) {
         tiles[k] = n;
@@ -539,8 +541,10 @@ __global__ void k_tile_vals(const int32_t* __restrict__ row, const int32_t* __re
 __global__ void k_layout_nodes(const uint32_t* __restrict__ perm, const int32_t* __restrict__ in_row,
                                const float* __restrict__ deg, const double* __restrict__ out_w, int32_t n,
                                int32_t* __restrict__ rank, uint32_t* __restrict__ cnt, float* __restrict__ p_deg,
-                               double* __restrict__ p_outw) {
+                               double* __restrict__ p_outw, int32_t* __restrict__ pad) {
     const int32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < kArcPad) pad[r] = 0;  // the zeroed slots past p_col's arcs
+    if (r == 0) cnt[n] = 0;
     if (r >= n) return;
     const int32_t v = (int32_t)perm[r];
     rank[v] = r;
@@ -574,13 +578,13 @@ __global__ __launch_bounds__(kRunThreads) void k_layout_slots(
 
 // Non-hub rows with more than row_lane_max arcs (egx_graph_info).
 __global__ __launch_bounds__(256) void k_row_stats(const int32_t* __restrict__ row, int32_t n_hub, int32_t n,
-                                                   int32_t lane_max, uint32_t* __restrict__ ctr) {
+                                                   int32_t lane_max, uint32_t* __restrict__ wave_rows) {
     __shared__ uint32_t sh[4];
     uint32_t rows = 0;
     for (int64_t v = n_hub + (int64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (int64_t)gridDim.x * 256)
         rows += row[v + 1] - row[v] > lane_max ? 1u : 0u;
     rows = block_sum_u32(rows, sh);
-    if (threadIdx.x == 0 && rows) atomicAdd(&ctr[kCtrWaveRows], rows);
+    if (threadIdx.x == 0 && rows) atomicAdd(wave_rows, rows);
 }
 
 __global__ void k_check_arcs(const int32_t* __restrict__ E, const double* __restrict__ W, int32_t n, int64_t m,
@@ -595,10 +599,6 @@ __global__ void k_check_arcs(const int32_t* __restrict__ E, const double* __rest
         }
     }
     if (f) atomicOr(flags, f);
-}
-
-__global__ void k_set_last(int32_t* __restrict__ arr, int64_t idx, int32_t value) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) arr[idx] = value;
 }
 
 // Rows of many partials first (in their order); returns how many those are.
@@ -1208,30 +1208,30 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in, int32_t known_hubs) {
     const int32_t per_tile = tile_size(cfg, items);
     g.n_tiles = (items + per_tile - 1) / per_tile;
     g.tile_lds = per_tile + cfg.wave_row_max;
-    DevBuf ctr;
-    EGX_TRY(ctr.alloc(kCtrWords * sizeof(uint32_t)));
-    EGX_HIP_TRY(hipMemsetAsync(ctr.p, 0, kCtrWords * sizeof(uint32_t), s), EGX_DEVICE_ERR);
+    DevBuf wave_rows;
+    EGX_TRY(wave_rows.alloc(sizeof(uint32_t)));
     EGX_TRY(g.tiles.alloc(((size_t)g.n_tiles + 1) * 4));
     k_tile_starts<<<nblocks(g.n_tiles + 1, 256), 256, 0, s>>>(g.it_row, g.n_hub, n, per_tile, g.n_tiles,
-                                                               g.tiles.as<int32_t>());
+                                                               g.tiles.as<int32_t>(), wave_rows.as<uint32_t>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    k_row_stats<<<std::min<unsigned>(nblocks(n, 256), kNodeBlocks), 256, 0, s>>>(g.it_row, g.n_hub, n,
-                                                                                 row_lane_max(cfg), ctr.as<uint32_t>());
+    k_row_stats<<<std::min<unsigned>(nblocks(n, 256), kNodeBlocks), 256, 0, s>>>(
+        g.it_row, g.n_hub, n, row_lane_max(cfg), wave_rows.as<uint32_t>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    // (also waits for the copies out of segs and hub_rows)
-    uint32_t wave_rows = 0;
-    EGX_HIP_TRY(hipMemcpyWithStream(&wave_rows, ctr.as<uint32_t>() + kCtrWaveRows, 4, hipMemcpyDeviceToHost, s),
-                EGX_DEVICE_ERR);
-    g.rows_wave = wave_rows;
+    int rc = build_tile_sort(g, cfg);
+    if (rc == EGX_SUCC) {
+        rc = build_blocked(g, cfg, layout_changed);
+        if (rc != EGX_SUCC) g.bins.blocked = 0;  // the pull layout stays usable
+    }
+    // the one wait (also for the copies out of segs and hub_rows), after all that can be queued without it
+    uint32_t rows_wave = 0;
+    EGX_HIP_TRY(hipMemcpyWithStream(&rows_wave, wave_rows.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+    g.rows_wave = rows_wave;
     g.rows_thread = (int64_t)(n - g.n_hub) - g.rows_wave;
     if (layout_changed) {
         float ms = 0.0f;
         EGX_HIP_TRY(hipEventElapsedTime(&ms, g.ev0, g.ev1), EGX_DEVICE_ERR);
         g.layout_seconds = (double)ms * 1e-3;
     }
-    EGX_TRY(build_tile_sort(g, cfg));
-    const int rc = build_blocked(g, cfg, layout_changed);
-    if (rc != EGX_SUCC) g.bins.blocked = 0;  // the pull layout stays usable
     return rc;
 }
 
@@ -1301,7 +1301,10 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
     EGX_TRY(vals_alt.alloc((mm + kArcPad) * 4));
     if (values) EGX_TRY(rec.alloc(mm * sizeof(ArcRec)));
 
-    // out-weights and counts by the arcs themselves (weights, or endpoints to skip), or by the offsets
+    // Out-weights, counts and what follows from them: by the arcs themselves
+    // (weights that count, or endpoints to skip), or by the offsets.
+    const bool sum_weights = dW && !g.adjacency;  // out-weights of adjacency graphs are 1
+    const unsigned node_blocks = std::min<unsigned>(nblocks(n, 256), kNodeBlocks);
     auto out_by_arcs = [&]() -> int {
         // at most m / kOutLong rows are longer than kOutLong
         const int64_t max_long = m / kOutLong;
@@ -1314,32 +1317,29 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
             EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         }
         const unsigned tiles = nblocks(std::max<int64_t>(m, 1), kOutTile);
-        if (dW) k_row_out<true><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, dW, n, tiles, out_w, outcnt_p, lr, nl, lb);
-        else k_row_out<false><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, nullptr, n, tiles, out_w, outcnt_p, lr, nl, lb);
+        if (sum_weights)
+            k_row_out<true><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, dW, n, tiles, out_w, outcnt_p, lr, nl, lb);
+        else
+            k_row_out<false><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, nullptr, n, tiles, out_w, outcnt_p, lr, nl,
+                                                                lb);
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        return EGX_SUCC;
-    };
-    auto unit_out = [&]() -> int {
-        if (!g.adjacency) return EGX_SUCC;
-        k_unit_out_w<<<nblocks(n, 256), 256, 0, s>>>(out_w, n);
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        return EGX_SUCC;
-    };
-    const unsigned node_blocks = std::min<unsigned>(nblocks(n, 256), kNodeBlocks);
-    auto node_arrays = [&]() -> int {
-        k_node_arrays<<<node_blocks, 256, 0, s>>>(out_w, outcnt_p, n, g.weighted ? 1 : 0, g.deg.as<float>(), ctr);
+        if (g.adjacency) {
+            k_unit_out_w<<<nblocks(n, 256), 256, 0, s>>>(out_w, n);
+            EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        }
+        k_node_arrays<false><<<node_blocks, 256, 0, s>>>(dV, out_w, outcnt_p, n, 0, g.weighted ? 1 : 0,
+                                                         g.deg.as<float>(), ctr);
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         return EGX_SUCC;
     };
     if (n > 0) {
-        if (dW) {
+        if (sum_weights) {
             EGX_TRY(out_by_arcs());
         } else {
-            k_outcnt_from_V<<<nblocks(n, 256), 256, 0, s>>>(dV, n, out_w, outcnt_p);
+            k_node_arrays<true><<<node_blocks, 256, 0, s>>>(dV, out_w, outcnt_p, n, g.adjacency ? 1 : 0,
+                                                            g.weighted ? 1 : 0, g.deg.as<float>(), ctr);
             EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         }
-        EGX_TRY(unit_out());
-        EGX_TRY(node_arrays());
     }
     if (m > 0) {
         const unsigned rb = nblocks(m, kRunArcs);
@@ -1360,12 +1360,10 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
     }
     uint32_t hctr[kCtrWords];
     EGX_HIP_TRY(hipMemcpyWithStream(hctr, ctr, sizeof(hctr), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
-    if (hctr[kCtrInvalid] > 0 && !dW && n > 0) {
+    if (hctr[kCtrInvalid] > 0 && !sum_weights && n > 0) {
         // skipped endpoints: the offsets counted them
         EGX_HIP_TRY(hipMemsetAsync(ctr, 0, kCtrWords * sizeof(uint32_t), s), EGX_DEVICE_ERR);
         EGX_TRY(out_by_arcs());
-        EGX_TRY(unit_out());
-        EGX_TRY(node_arrays());
         uint32_t again[kCtrWords];
         EGX_HIP_TRY(hipMemcpyWithStream(again, ctr, sizeof(again), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
         hctr[kCtrDangling] = again[kCtrDangling];
@@ -1398,7 +1396,7 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
         g.in_val.release();
         g.w_csc.release();
     }
-    EGX_HIP_TRY(hipMemsetAsync(g.in_col.as<int32_t>() + m_valid, 0, kArcPad * 4, s), EGX_DEVICE_ERR);
+    if (n <= 0) EGX_HIP_TRY(hipMemsetAsync(g.in_col.p, 0, kArcPad * 4, s), EGX_DEVICE_ERR);  // else the layout's
     g.layout_built = false;
     EGX_TRY(rebuild_bins(g, g.bins, (int32_t)hctr[kCtrHubs]));
     // large PageRank graphs iterate propagation-blocked; one the layout
@@ -1473,7 +1471,8 @@ int build_layout(Graph& g, const BinCfg& cfg, int32_t known_hubs) {
     EGX_TRY(vals_alt.alloc((size_t)n * 4));
     k_layout_keys<<<nblocks(n, 256), 256, 0, s>>>(g.in_row.as<int32_t>(), g.out_cnt.as<int32_t>(), n,
                                                    cfg.wave_row_max, bits, maxdeg, cfg.reorder,
-                                                   keys.as<uint32_t>(), g.perm.as<uint32_t>());
+                                                   keys.as<uint32_t>(), g.perm.as<uint32_t>(),
+                                                   g.in_col.as<int32_t>() + m);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     EGX_TRY(radix_sort_u32(keys, keys_alt, &g.perm, &vals_alt, n, bits + 1, s));
     keys.release();
@@ -1481,21 +1480,18 @@ int build_layout(Graph& g, const BinCfg& cfg, int32_t known_hubs) {
     vals_alt.release();
 
     EGX_TRY(g.rank.alloc((size_t)n * 4));
-    EGX_TRY(cnt.alloc((size_t)n * 4));
+    EGX_TRY(cnt.alloc(((size_t)n + 1) * 4));
+    EGX_TRY(g.p_col.alloc(((size_t)std::max<int64_t>(m, 1) + kArcPad) * 4));
     EGX_TRY(g.p_deg.alloc((size_t)n * 4));
     EGX_TRY(g.p_outw.alloc((size_t)n * 8));
     EGX_TRY(g.p_row.alloc(((size_t)n + 1) * 4));
     k_layout_nodes<<<nblocks(n, 256), 256, 0, s>>>(g.perm.as<uint32_t>(), g.in_row.as<int32_t>(), g.deg.as<float>(),
                                                     g.out_w.as<double>(), n, g.rank.as<int32_t>(),
-                                                    cnt.as<uint32_t>(), g.p_deg.as<float>(), g.p_outw.as<double>());
+                                                    cnt.as<uint32_t>(), g.p_deg.as<float>(), g.p_outw.as<double>(),
+                                                    g.p_col.as<int32_t>() + m);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    EGX_TRY(exclusive_scan_u32(cnt.as<uint32_t>(), g.p_row.as<uint32_t>(), n, s));
-    k_set_last<<<1, 64, 0, s>>>(g.p_row.as<int32_t>(), n, (int32_t)m);
-    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    EGX_TRY(exclusive_scan_u32(cnt.as<uint32_t>(), g.p_row.as<uint32_t>(), (int64_t)n + 1, s));
     cnt.release();
-
-    EGX_TRY(g.p_col.alloc(((size_t)std::max<int64_t>(m, 1) + kArcPad) * 4));
-    EGX_HIP_TRY(hipMemsetAsync(g.p_col.as<int32_t>() + m, 0, kArcPad * 4, s), EGX_DEVICE_ERR);
     if (g.has_values()) {
         EGX_TRY(g.p_val.alloc((size_t)std::max<int64_t>(m, 1) * 4));
         EGX_TRY(g.p_w.alloc((size_t)std::max<int64_t>(m, 1) * 8));

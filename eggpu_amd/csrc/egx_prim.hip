@@ -249,11 +249,29 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_reduce(const T* __restric
     if (threadIdx.x == 0) partial[blockIdx.x] = total;
 }
 
+// Scan of one tile.  What comes before it is offsets[tile], or, with each > 0,
+// the sum of before[0, tile * each): the tiles' sums (each 1), or the input
+// itself (each kScanTile; not in place).
 template <typename T>
 __global__ __launch_bounds__(kScanThreads) void k_scan_tile(const T* in, T* out, int64_t n,
-                                                            const T* __restrict__ offsets) {
+                                                            const T* __restrict__ offsets, const T* before,
+                                                            int32_t each) {
     __shared__ T sh[kScanTile];
     __shared__ T sh_w[kScanThreads / kWave];
+    T start = 0;
+    if (each > 0) {
+        const int64_t k = (int64_t)blockIdx.x * each;
+        T sum = 0;
+#pragma unroll 8
+        for (int64_t i = threadIdx.x; i < k; i += kScanThreads) sum += before[i];
+        __shared__ T total;
+        const T got = block_reduce_sum(sum, sh_w);
+        if (threadIdx.x == 0) total = got;
+        __syncthreads();
+        start = total;
+    } else if (offsets) {
+        start = offsets[blockIdx.x];
+    }
     const int64_t base = (int64_t)blockIdx.x * kScanTile;
 #pragma unroll
     for (int i = 0; i < kScanItems; ++i) {
@@ -269,7 +287,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tile(const T* in, T* out,
         tsum += local[i];
     }
     T run = block_exclusive_scan(tsum, sh_w);
-    if (offsets) run += offsets[blockIdx.x];
+    run += start;
 #pragma unroll
     for (int i = 0; i < kScanItems; ++i) {
         sh[threadIdx.x * kScanItems + i] = run;
@@ -283,12 +301,17 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tile(const T* in, T* out,
     }
 }
 
+// Up to kScanDirect tiles out of place, each adds up all before it (one
+// launch: 16,384 elements took three, 10 us and the gaps between them); up to kScanSelf
+// tiles, each adds up the tiles' sums; above, those are scanned first.
+constexpr int64_t kScanDirect = 16;
+constexpr int64_t kScanSelf = 1024;
 template <typename T>
 int scan_impl(const T* in, T* out, int64_t n, hipStream_t s) {
     if (n <= 0) return EGX_SUCC;
     const int64_t nb = (n + kScanTile - 1) / kScanTile;
-    if (nb == 1) {
-        k_scan_tile<T><<<1, kScanThreads, 0, s>>>(in, out, n, nullptr);
+    if (nb == 1 || (nb <= kScanDirect && in != out)) {
+        k_scan_tile<T><<<(unsigned)nb, kScanThreads, 0, s>>>(in, out, n, nullptr, in, nb == 1 ? 0 : kScanTile);
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         return EGX_SUCC;
     }
@@ -296,8 +319,9 @@ int scan_impl(const T* in, T* out, int64_t n, hipStream_t s) {
     EGX_TRY(part.alloc((size_t)nb * sizeof(T), s));  // released in s's order: no wait
     k_scan_reduce<T><<<(unsigned)nb, kScanThreads, 0, s>>>(in, n, part.as<T>());
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    EGX_TRY(scan_impl<T>(part.as<T>(), part.as<T>(), nb, s));
-    k_scan_tile<T><<<(unsigned)nb, kScanThreads, 0, s>>>(in, out, n, part.as<T>());
+    if (nb > kScanSelf) EGX_TRY(scan_impl<T>(part.as<T>(), part.as<T>(), nb, s));
+    k_scan_tile<T><<<(unsigned)nb, kScanThreads, 0, s>>>(in, out, n, part.as<T>(), part.as<T>(),
+                                                         nb > kScanSelf ? 0 : 1);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     return EGX_SUCC;
 }

@@ -133,3 +133,23 @@ def test_sorted_build_bit_exact(gpu_ready, n, m):
         got = g.download_csc()
     want = O.build_inbound(V, E, None, 0.85)
     assert all(np.array_equal(a, b) for a, b in zip(got, want[:4]))
+
+
+# rows against the scans of their arc counts: one tile (2,048), the last size of one launch (16 tiles) and of two (1,024)
+@pytest.mark.parametrize("n", [2046, 2047, 2048, 32766, 32767, 32768, 2097150, 2097152])
+def test_row_offsets_at_scan_sizes(gpu_ready, n):
+    print(f"scan sizes n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    m = 3 * n
+    src = np.sort(rng.integers(0, n, m))
+    E = (rng.integers(0, n, m) ** 2 // n).astype(np.int32)  # low heads more often
+    V = np.zeros(n + 1, np.int32)
+    V[1:] = np.cumsum(np.bincount(src, minlength=n))
+    with native.DeviceGraph.from_csr(V, E) as g:
+        got, it, _ = g.pagerank(max_iter=3, tol=0.0, precision=native.PRECISION_FP64)
+    out = np.bincount(src, minlength=n)
+    x = np.full(n, 1.0 / n)
+    for _ in range(3):
+        s = np.divide(x, out, out=np.zeros(n), where=out > 0)
+        x = 0.85 * np.bincount(E, weights=s[src], minlength=n) + (0.15 + 0.85 * x[out == 0].sum()) / n
+    assert it == 3 and np.max(np.abs(got - x / x.sum()) / x) <= 1e-10  # sums of up to m terms of 2^-53 each
