@@ -94,15 +94,6 @@ __device__ __forceinline__ const int32_t* run_rows(const int32_t* __restrict__ V
 }
 static_assert(kRunItems == 8, "a thread spreads two int4 of marks");
 
-__global__ __launch_bounds__(kRunThreads) void k_expand_src(const int32_t* __restrict__ V, int32_t n, int64_t m,
-                                                            int32_t* __restrict__ src) {
-    __shared__ RunRows sh;
-    const int64_t q0 = (int64_t)blockIdx.x * kRunArcs;
-    const int32_t cnt = (int32_t)min((int64_t)kRunArcs, m - q0);
-    const int32_t* rows = run_rows(V, n, q0, cnt, sh);
-    for (int32_t i = threadIdx.x; i < cnt; i += kRunThreads) src[q0 + i] = rows[i];
-}
-
 // What a weighted arc carries to its place in the pull CSC: gathered as one
 // 16-byte record instead of its weight, source and the source's out-weight
 // one by one (k_fill_csc over 9.3M arcs: 310 us).
@@ -1244,25 +1235,6 @@ int check_arcs(const int32_t* dE, const double* dW, int32_t n, int64_t m, uint32
     return EGX_SUCC;
 }
 
-int transpose_csr(const int32_t* dV, const int32_t* dE, int32_t n, int64_t m, DevBuf& Vt, DevBuf& Et,
-                  hipStream_t s) {
-    // a stable sort of (head, source) pairs in arc order
-    const size_t mm = (size_t)std::max<int64_t>(m, 1);
-    DevBuf keys, keys_alt, vals_alt;
-    EGX_TRY(keys.alloc(mm * 4, s));
-    EGX_TRY(keys_alt.alloc(mm * 4, s));
-    EGX_TRY(vals_alt.alloc(mm * 4, s));
-    EGX_TRY(Et.alloc(mm * 4, s));
-    EGX_TRY(Vt.alloc(((size_t)n + 1) * 4, s));
-    if (m > 0) {
-        EGX_HIP_TRY(hipMemcpyAsync(keys.p, dE, (size_t)m * 4, hipMemcpyDeviceToDevice, s), EGX_DEVICE_ERR);
-        k_expand_src<<<nblocks(m, kRunArcs), kRunThreads, 0, s>>>(dV, n, m, Et.as<int32_t>());
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    }
-    EGX_TRY(radix_sort_u32(keys, keys_alt, &Et, &vals_alt, m, bits_for((uint64_t)std::max(n - 1, 0)), s));
-    return lower_bound_iota_u32(keys.as<uint32_t>(), m, Vt.as<int32_t>(), (int64_t)n + 1, s);
-}
-
 // out_w[u] = 1: adjacency values keep alpha * w undivided.
 __global__ void k_unit_out_w(double* __restrict__ out_w, int32_t n) {
     const int32_t u = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1411,6 +1383,61 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
             EGX_TRY(build_blocked(g, cfg, true));  // releases what the attempt allocated
         }
     }
+    EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
+    pool_stream_idle(s);
+    g.build_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
+    return EGX_SUCC;
+}
+
+int build_from_device_rows(Graph& g, DevBuf&& V, DevBuf&& E, int32_t n, int64_t m, double alpha, bool* bad_endpoint) {
+    hipStream_t s = g.stream;
+    g.n = n;
+    g.m = m;
+    g.weighted = true;
+    g.adjacency_weights = false;
+    g.alpha_vals = alpha;
+    g.alpha_orig = alpha;
+    const auto t_start = std::chrono::steady_clock::now();
+    g.in_row = std::move(V);
+    g.in_col = std::move(E);
+    g.in_val.release();
+    g.w_csc.release();
+    DevBuf ctr_buf, keys, keys_alt, offsets;
+    EGX_TRY(ctr_buf.alloc(kCtrWords * sizeof(uint32_t)));
+    uint32_t* ctr = ctr_buf.as<uint32_t>();
+    EGX_HIP_TRY(hipMemsetAsync(ctr, 0, kCtrWords * sizeof(uint32_t), s), EGX_DEVICE_ERR);
+    EGX_TRY(g.out_w.alloc((size_t)n * 8));
+    EGX_TRY(g.deg.alloc((size_t)n * 4));
+    EGX_TRY(g.out_cnt.alloc((size_t)n * 4));
+    EGX_TRY(keys.alloc((size_t)m * 4));
+    EGX_TRY(keys_alt.alloc((size_t)m * 4));
+    EGX_TRY(offsets.alloc(((size_t)n + 1) * 4));
+    k_check_arcs<<<(unsigned)std::min<int64_t>((m + 255) / 256, 4096), 256, 0, s>>>(g.in_col.as<int32_t>(), nullptr, n,
+                                                                                  m, ctr + kCtrInvalid);
+    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    // how often each node is a source: by a sort of the sources alone (one
+    // counter per node would take a device-wide atomic per arc)
+    EGX_HIP_TRY(hipMemcpyAsync(keys.p, g.in_col.p, (size_t)m * 4, hipMemcpyDeviceToDevice, s), EGX_DEVICE_ERR);
+    EGX_TRY(radix_sort_u32(keys, keys_alt, nullptr, nullptr, m, bits_for((uint64_t)(n - 1)), s));
+    EGX_TRY(lower_bound_iota_u32(keys.as<uint32_t>(), m, offsets.as<int32_t>(), (int64_t)n + 1, s));
+    const unsigned node_blocks = std::min<unsigned>(nblocks(n, 256), kNodeBlocks);
+    k_node_arrays<true><<<node_blocks, 256, 0, s>>>(offsets.as<int32_t>(), g.out_w.as<double>(),
+                                                    g.out_cnt.as<int32_t>(), n, 1, 1, g.deg.as<float>(), ctr);
+    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    k_in_degrees<<<node_blocks, 256, 0, s>>>(g.in_row.as<int32_t>(), n, hub_threshold(g.bins), ctr);
+    EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    uint32_t hctr[kCtrWords];
+    EGX_HIP_TRY(hipMemcpyWithStream(hctr, ctr, sizeof(hctr), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+    *bad_endpoint = hctr[kCtrInvalid] != 0;
+    if (*bad_endpoint) return EGX_SUCC;  // the caller's to report; nothing else was built
+    g.n_dangling = hctr[kCtrDangling];
+    g.max_out_degree = (int32_t)hctr[kCtrMaxOut];
+    g.max_in_degree = (int32_t)hctr[kCtrMaxIn];
+    keys.release();
+    keys_alt.release();
+    offsets.release();
+    g.layout_built = false;
+    EGX_TRY(rebuild_bins(g, g.bins, (int32_t)hctr[kCtrHubs]));
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     pool_stream_idle(s);
     g.build_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();

@@ -254,16 +254,17 @@ struct Graph {
 // egx_build.hip.  With g.adjacency set, dW may be null (unit weights).
 int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const double* dW, int32_t n,
                           int64_t m, double alpha);
+// The adjacency graph (g.adjacency set, unit weights) whose row v gathers from
+// E[V[v]], ..., E[V[v + 1] - 1], in that order; V and E (m + kArcPad slots) become the
+// graph's, n and m are positive.  *bad_endpoint: an entry of E is outside
+// [0, n), and nothing was built.
+int build_from_device_rows(Graph& g, DevBuf&& V, DevBuf&& E, int32_t n, int64_t m, double alpha, bool* bad_endpoint);
 int build_layout(Graph& g, const BinCfg& cfg, int32_t known_hubs = -1);
 // Queue the device check of a host CSR's arcs on s: *flags (device, zeroed
 // here) gets kArcBadEndpoint / kArcBadWeight (not finite or negative; dW may
 // be null).
 constexpr uint32_t kArcBadEndpoint = 1u, kArcBadWeight = 2u;
 int check_arcs(const int32_t* dE, const double* dW, int32_t n, int64_t m, uint32_t* flags, hipStream_t s);
-// Queue the transposed arcs of (dV, dE) on s, stable in source order: row v
-// of (Vt, Et) lists the u with u->v.  Endpoints outside [0, n) leave Vt and Et unspecified.
-int transpose_csr(const int32_t* dV, const int32_t* dE, int32_t n, int64_t m, DevBuf& Vt, DevBuf& Et,
-                  hipStream_t s);
 // known_hubs: the number of rows above the hub threshold, if the caller counted them (else < 0)
 int rebuild_bins(Graph& g, const BinCfg& cfg, int32_t known_hubs = -1);
 int refresh_alpha(Graph& g, double alpha);
