@@ -2,6 +2,7 @@
 #pragma once
 
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "egx_common.h"
@@ -32,5 +33,40 @@ struct Fetch {
 // All of `jobs`, whose values are written by work queued on s; returns when
 // the callers' arrays hold them.
 int fetch(const std::vector<Fetch>& jobs, hipStream_t s);
+
+// A small result that its last kernel writes to pinned memory itself, which
+// saves the launch that carries it there: begin() gives the memory (false:
+// too large, or none to be had), the kernel ends in raise_flag(), finish()
+// waits for it and hands the values (f.dev is not read) to the caller.
+class DirectFetch {
+  public:
+    DirectFetch();
+    ~DirectFetch();
+    DirectFetch(const DirectFetch&) = delete;
+    DirectFetch& operator=(const DirectFetch&) = delete;
+    bool begin(size_t bytes, hipStream_t s);
+    int finish(const Fetch& f);
+    char* to = nullptr;
+    uint32_t* count = nullptr;
+    uint32_t* flag = nullptr;
+
+  private:
+    struct State;
+    std::unique_ptr<State> st_;
+};
+
+// The end of a kernel that writes to the host: all threads of every
+// workgroup take part.  The last workgroup knows that the others' writes are
+// out (each thread fences before its workgroup counts), raises the flag, and
+// leaves the count at 0 for the next use.
+__device__ __forceinline__ void raise_flag(uint32_t* count, uint32_t* flag) {
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    if (atomicAdd(count, 1u) + 1u == gridDim.x) {
+        atomicExch(count, 0u);
+        __hip_atomic_store(flag, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
 
 }  // namespace egx

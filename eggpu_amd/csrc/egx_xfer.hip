@@ -54,9 +54,7 @@ struct Chunk {
 // Bound by the link.  A copy call and an event for each part left 10 us between
 // parts of 512 KB, which the link carries in 9.7; queued kernels follow each
 // other at once, and the host reads the flag (a solve of 1,048,576 nodes,
-// 20 iterations: 1.22 ms -> 1.16; 64 columns of 300,007 6.5 -> 6.3).  The last workgroup to finish
-// knows that the others' writes are out (each fences before it counts), and
-// leaves the count at 0 for the chunk's next use.
+// 20 iterations: 1.22 ms -> 1.16; 64 columns of 300,007 6.5 -> 6.3).
 constexpr int kFetchThreads = 256;
 constexpr int kFetchBlocks = 64;
 __global__ __launch_bounds__(kFetchThreads) void k_fetch_part(const char* __restrict__ from, char* __restrict__ to,
@@ -74,13 +72,7 @@ __global__ __launch_bounds__(kFetchThreads) void k_fetch_part(const char* __rest
     }
     for (int64_t i = words + t; i < bytes / 4; i += stride)
         reinterpret_cast<uint32_t*>(to)[i] = reinterpret_cast<const uint32_t*>(from)[i];
-    __threadfence_system();
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    if (atomicAdd(count, 1u) + 1u == gridDim.x) {
-        atomicExch(count, 0u);
-        __hip_atomic_store(flag, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    raise_flag(count, flag);
 }
 
 __global__ void k_fetch_reset(uint32_t* count) { *count = 0; }
@@ -427,6 +419,41 @@ int upload(const std::vector<Upload>& jobs, hipStream_t s) {
         set_last_error("host transfer: out of host memory");
         return EGX_FAILED_TO_ALLOCATE_HOST_MEM;
     }
+}
+
+struct DirectFetch::State {
+    Run r;
+};
+
+DirectFetch::DirectFetch() = default;
+
+DirectFetch::~DirectFetch() {
+    if (st_) (void)finish_run(st_->r);  // the kernel may still write
+}
+
+bool DirectFetch::begin(size_t bytes, hipStream_t s) {
+    if (bytes > kInlineBytes) return false;
+    try {
+        std::unique_ptr<State> st(new State());
+        if (begin_run(st->r, 1, s) != 0) return false;
+        st_ = std::move(st);
+    } catch (const std::bad_alloc&) {
+        return false;
+    }
+    const Chunk& c = st_->r.chunks[0];
+    __atomic_store_n(c.flag(), 0u, __ATOMIC_RELEASE);
+    to = c.p;
+    count = c.count;
+    flag = c.flag();
+    return true;
+}
+
+int DirectFetch::finish(const Fetch& f) {
+    Run& r = st_->r;
+    if (r.landed(r.chunks[0])) finish_values(f, 0, f.n, r.chunks[0].p);
+    const int rc = finish_run(r);
+    st_.reset();
+    return rc;
 }
 
 int fetch(const std::vector<Fetch>& jobs, hipStream_t s) {
