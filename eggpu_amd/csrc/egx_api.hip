@@ -33,7 +33,7 @@ struct DeviceGuard {
     }
 };
 
-// Streams of freed graphs and finished multi-graph solves, kept per device
+// Streams of freed graphs, closed batches and finished multi-graph solves, kept per device
 // for the next ones: creating a HIP stream costs more than the rest of a
 // small graph's set-up.  At most kIdleStreams idle streams per device are
 // kept; the pool lives until the process ends.
@@ -46,9 +46,12 @@ struct DeviceGuard {
 // (its solves capture hipGraphs on it).
 constexpr size_t kIdleStreams = 16;
 constexpr int kWarmStreams = 4;
+//
+// Batches have theirs apart: graphs' streams capture, and a thread that still
+// waits for an event of a closed batch must not meet a capture on its stream.
 struct StreamPool {
     std::mutex mu;
-    std::vector<std::pair<int, hipStream_t>> idle;
+    std::vector<std::pair<int, hipStream_t>> idle[2];  // by StreamUse
     std::vector<int> warmed;  // devices whose first streams were made together
 };
 StreamPool& stream_pool() {
@@ -56,22 +59,25 @@ StreamPool& stream_pool() {
     return *p;
 }
 
+}  // namespace
+
 // A stream on the current device `dev`: an idle one, else a new one.
-hipError_t take_stream(int dev, hipStream_t* s) {
+hipError_t take_stream(int dev, hipStream_t* s, StreamUse use) {
     StreamPool& p = stream_pool();
     std::lock_guard<std::mutex> lk(p.mu);
-    if (std::find(p.warmed.begin(), p.warmed.end(), dev) == p.warmed.end()) {
+    auto& idle = p.idle[(int)use];
+    if (use == StreamUse::kGraph && std::find(p.warmed.begin(), p.warmed.end(), dev) == p.warmed.end()) {
         p.warmed.push_back(dev);
         for (int i = 1; i < kWarmStreams; ++i) {
             hipStream_t w = nullptr;
             if (hipStreamCreate(&w) != hipSuccess) break;  // the request below reports a failure
-            p.idle.emplace_back(dev, w);
+            idle.emplace_back(dev, w);
         }
     }
-    for (size_t i = p.idle.size(); i-- > 0;) {
-        if (p.idle[i].first == dev) {
-            *s = p.idle[i].second;
-            p.idle.erase(p.idle.begin() + (std::ptrdiff_t)i);
+    for (size_t i = idle.size(); i-- > 0;) {
+        if (idle[i].first == dev) {
+            *s = idle[i].second;
+            idle.erase(idle.begin() + (std::ptrdiff_t)i);
             return hipSuccess;
         }
     }
@@ -79,22 +85,25 @@ hipError_t take_stream(int dev, hipStream_t* s) {
 }
 
 // Return stream s of device dev (current) once its work is done.
-void give_stream(int dev, hipStream_t s) {
+void give_stream(int dev, hipStream_t s, StreamUse use) {
     if (!s) return;
     (void)hipStreamSynchronize(s);
     pool_stream_idle(s);
     StreamPool& p = stream_pool();
     {
         std::lock_guard<std::mutex> lk(p.mu);
+        auto& idle = p.idle[(int)use];
         size_t on_dev = 0;
-        for (const auto& e : p.idle) on_dev += e.first == dev ? 1 : 0;
+        for (const auto& e : idle) on_dev += e.first == dev ? 1 : 0;
         if (on_dev < kIdleStreams) {
-            p.idle.emplace_back(dev, s);
+            idle.emplace_back(dev, s);
             return;
         }
     }
     (void)hipStreamDestroy(s);
 }
+
+namespace {
 
 // Pinned state slots (one per graph, the staging of its solves' stop
 // state): made 64 at a time in one page-aligned block, since each

@@ -251,6 +251,12 @@ struct Graph {
     size_t device_bytes() const;
 };
 
+// Streams from the process's pool (egx_api.hip): take one for device dev
+// (current); give it back once its work is done (this waits for it).
+enum class StreamUse { kGraph = 0, kBatch = 1 };
+hipError_t take_stream(int dev, hipStream_t* s, StreamUse use = StreamUse::kGraph);
+void give_stream(int dev, hipStream_t s, StreamUse use = StreamUse::kGraph);
+
 // egx_build.hip.  With g.adjacency set, dW may be null (unit weights).
 int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const double* dW, int32_t n,
                           int64_t m, double alpha);

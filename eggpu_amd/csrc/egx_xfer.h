@@ -28,11 +28,15 @@ struct Fetch {
     bool packed;
     double sum;
     const double* sum_at = nullptr;  // instead of sum: pinned, written by work queued before the values'
+    int32_t* words = nullptr;        // (download) packed 4-byte words, copied here as they are
 };
 
 // All of `jobs`, whose values are written by work queued on s; returns when
 // the callers' arrays hold them.
 int fetch(const std::vector<Fetch>& jobs, hipStream_t s);
+
+// 4-byte words at dev, written by work queued on s, to host as they are.
+int download(const void* dev, int32_t* host, int64_t n, hipStream_t s);
 
 // A small result that its last kernel writes to pinned memory itself, which
 // saves the launch that carries it there: begin() gives the memory (false:

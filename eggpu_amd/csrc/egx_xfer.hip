@@ -205,6 +205,10 @@ void run_together(const std::function<void()>& fn, int more) {
 
 // values [i0, i0 + n) of a job, from a chunk
 void finish_values(const Fetch& f, int64_t i0, int64_t n, const char* from) {
+    if (f.words) {
+        std::memcpy(f.words + i0, from, (size_t)n * 4);
+        return;
+    }
     double* out = f.host + i0;
     if (!f.packed) {
         std::memcpy(out, from, (size_t)n * 8);
@@ -465,6 +469,10 @@ int fetch(const std::vector<Fetch>& jobs, hipStream_t s) {
         set_last_error("host transfer: out of host memory");
         return EGX_FAILED_TO_ALLOCATE_HOST_MEM;
     }
+}
+
+int download(const void* dev, int32_t* host, int64_t n, hipStream_t s) {
+    return fetch({Fetch{dev, nullptr, n, true, 0.0, nullptr, host}}, s);
 }
 
 }  // namespace egx
