@@ -144,7 +144,11 @@ enum : int {
     kCtrMaxOut,    // largest out-degree
     kCtrMaxIn,     // largest in-degree
     kCtrLong,      // rows longer than kOutLong
-    kCtrHubs,      // rows above the hub threshold
+    kCtrHubs,      // rows above the hub threshold,
+    kCtrHubArcs,   // their arcs,
+    kCtrHubSegs,   // their segments,
+    kCtrHubSplit,  // those of more than one segment
+    kCtrHubMany,   // and of kHubMany or more
     kCtrWords = 16  // 64 bytes: a clear is one launch
 };
 
@@ -439,20 +443,105 @@ __global__ void k_unit_vals(const int32_t* __restrict__ in_col, const double* __
 
 // Largest in-degree, and the rows above the hub threshold.
 __global__ __launch_bounds__(256) void k_in_degrees(const int32_t* __restrict__ in_row, int32_t n, int32_t hub,
-                                                    uint32_t* __restrict__ ctr) {
+                                                    int32_t seg, uint32_t* __restrict__ ctr) {
     __shared__ uint32_t sh[4];
-    uint32_t most = 0, hubs = 0;
+    uint32_t most = 0, hubs = 0, arcs = 0, segs = 0, split = 0, many = 0;
     for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (int64_t)gridDim.x * 256) {
         const int32_t d = in_row[v + 1] - in_row[v];
         most = max(most, (uint32_t)d);
-        hubs += d > hub ? 1u : 0u;
+        if (d > hub) {
+            const uint32_t k = ((uint32_t)d + (uint32_t)seg - 1u) / (uint32_t)seg;
+            hubs += 1u;
+            arcs += (uint32_t)d;
+            segs += k;
+            split += k > 1u ? 1u : 0u;
+            many += k >= (uint32_t)kHubMany ? 1u : 0u;
+        }
     }
     most = block_max_u32(most, sh);
     hubs = block_sum_u32(hubs, sh);
+    if (threadIdx.x == 0 && most) atomicMax(&ctr[kCtrMaxIn], most);
+    __shared__ uint32_t any;
+    if (threadIdx.x == 0) any = hubs;
+    __syncthreads();
+    if (any == 0) return;
+    arcs = block_sum_u32(arcs, sh);
+    segs = block_sum_u32(segs, sh);
+    split = block_sum_u32(split, sh);
+    many = block_sum_u32(many, sh);
     if (threadIdx.x == 0) {
-        if (most) atomicMax(&ctr[kCtrMaxIn], most);
-        if (hubs) atomicAdd(&ctr[kCtrHubs], hubs);
+        atomicAdd(&ctr[kCtrHubs], hubs);
+        atomicAdd(&ctr[kCtrHubArcs], arcs);
+        atomicAdd(&ctr[kCtrHubSegs], segs);
+        if (split) atomicAdd(&ctr[kCtrHubSplit], split);
+        if (many) atomicAdd(&ctr[kCtrHubMany], many);
     }
+}
+
+// First segment of every hub row (rows [0, n_hub); one past them at n_hub),
+// and the rows of several segments: those of kHubMany or more first, each
+// part in row order.  One workgroup; with the counts known from the degrees
+// the host waits for none of it (it read the offsets back and copied both
+// lists up: a build and solve of 16,384 nodes 381 us, 374 so).
+constexpr int kHubThreads = 1024;
+__global__ __launch_bounds__(kHubThreads) void k_hub_rows(const int32_t* __restrict__ row, int32_t n_hub, int32_t seg,
+                                                          int32_t n_many, int32_t* __restrict__ first,
+                                                          HubRow* __restrict__ rows) {
+    __shared__ int32_t sums[3][kHubThreads / kWave];
+    int32_t base[3] = {0, 0, n_many};  // segments, rows of many, other rows of several
+    const int l = lane_id();
+    const uint64_t below = (1ull << l) - 1ull;
+    for (int32_t v0 = 0; v0 < n_hub; v0 += kHubThreads) {
+        const int32_t v = v0 + (int32_t)threadIdx.x;
+        const int32_t len = v < n_hub ? row[v + 1] - row[v] : 0;
+        const int32_t k = (int32_t)(((int64_t)len + seg - 1) / seg);
+        const bool is_many = k >= kHubMany, is_split = k > 1 && !is_many;
+        int32_t inc = k;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int32_t o = __shfl_up(inc, off, kWave);
+            if (l >= off) inc += o;
+        }
+        const uint64_t bm = __ballot(is_many), bs = __ballot(is_split);
+        if (l == kWave - 1) {
+            sums[0][wave_id()] = inc;
+            sums[1][wave_id()] = __popcll(bm);
+            sums[2][wave_id()] = __popcll(bs);
+        }
+        __syncthreads();
+        int32_t at[3] = {base[0] + inc - k, base[1] + (int32_t)__popcll(bm & below),
+                         base[2] + (int32_t)__popcll(bs & below)};
+        for (int q = 0; q < 3; ++q)
+            for (int w = 0; w < kHubThreads / kWave; ++w) {
+                base[q] += sums[q][w];
+                if (w < wave_id()) at[q] += sums[q][w];
+            }
+        if (v < n_hub) first[v] = at[0];
+        if (is_many) rows[at[1]] = HubRow{v, at[0], k, 0};
+        if (is_split) rows[at[2]] = HubRow{v, at[0], k, 0};
+        __syncthreads();  // sums is reused
+    }
+    if (threadIdx.x == 0) first[n_hub] = base[0];
+}
+
+__global__ void k_hub_segs(const int32_t* __restrict__ row, const int32_t* __restrict__ first, int32_t n_hub,
+                           int32_t seg, int32_t n_segs, HubSeg* __restrict__ out) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_segs) return;
+    int32_t lo = 0, hi = n_hub;  // first[lo] <= i < first[hi]
+    while (hi - lo > 1) {
+        const int32_t mid = lo + ((hi - lo) >> 1);
+        if (first[mid] <= i) lo = mid;
+        else hi = mid;
+    }
+    HubSeg sg;
+    sg.row = lo;
+    sg.beg = row[lo] + (i - first[lo]) * seg;
+    sg.end = (int32_t)min((int64_t)sg.beg + seg, (int64_t)row[lo + 1]);
+    sg.slot = lo;
+    sg.nseg = first[lo + 1] - first[lo];
+    sg.first = first[lo];
+    out[i] = sg;
 }
 
 // Relabelling key: hub rows (in-degree > hub) first, then descending
@@ -600,6 +689,9 @@ int64_t many_first(std::vector<HubRow>& rows) {
 
 // The in-degree above which a row is a hub row.
 inline int32_t hub_threshold(const BinCfg& cfg) { return std::min(std::max(cfg.wave_row_max, 1), kTileLds - 256); }
+
+// Arcs per hub segment.
+inline int32_t hub_segment(const BinCfg& cfg) { return std::max(cfg.hub_segment, 256); }
 
 inline unsigned nblocks(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
@@ -1135,67 +1227,60 @@ int32_t tile_size(const BinCfg& cfg, int64_t items) {
     return (int32_t)std::min(fill, std::max<int64_t>(256, items / 64));
 }
 
-int rebuild_bins(Graph& g, const BinCfg& cfg_in, int32_t known_hubs) {
+int rebuild_bins(Graph& g, const BinCfg& cfg_in, const uint32_t* counters) {
     BinCfg cfg = cfg_in;
     if (cfg.thread_row_max < 0) cfg.thread_row_max = 0;
     cfg.wave_row_max = hub_threshold(cfg);
     if (cfg.tile_items < 256) cfg.tile_items = 256;
     if (cfg.tile_items > kTileLds - cfg.wave_row_max) cfg.tile_items = kTileLds - cfg.wave_row_max;
-    if (cfg.hub_segment < 256) cfg.hub_segment = 256;
+    cfg.hub_segment = hub_segment(cfg);
     if (cfg.reorder != 0) cfg.reorder = 1;
     if (cfg.tile_sort != 0) cfg.tile_sort = 1;
     if (cfg.blocked != 0) cfg.blocked = 1;
     const bool layout_changed =
         !g.layout_built || g.layout_hub != cfg.wave_row_max || g.layout_reorder != cfg.reorder;
-    if (layout_changed) EGX_TRY(build_layout(g, cfg, known_hubs));
-    g.bins = cfg;
     hipStream_t s = g.stream;
     const int32_t n = g.n;
+    uint32_t hctr[kCtrWords] = {};
+    if (counters) {
+        std::copy(counters, counters + kCtrWords, hctr);
+    } else if (n > 0) {
+        DevBuf ctr;
+        EGX_TRY(ctr.alloc(sizeof(hctr)));
+        EGX_HIP_TRY(hipMemsetAsync(ctr.p, 0, sizeof(hctr), s), EGX_DEVICE_ERR);
+        k_in_degrees<<<std::min<unsigned>(nblocks(n, 256), kNodeBlocks), 256, 0, s>>>(
+            g.in_row.as<int32_t>(), n, cfg.wave_row_max, cfg.hub_segment, ctr.as<uint32_t>());
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        EGX_HIP_TRY(hipMemcpyWithStream(hctr, ctr.p, sizeof(hctr), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
+    }
+    if (layout_changed) EGX_TRY(build_layout(g, cfg, (int32_t)hctr[kCtrHubs]));
+    g.bins = cfg;
     g.n_hseg = g.n_hrows = g.n_hrows_split = g.n_hrows_many = g.n_tiles = 0;
     g.rows_thread = g.rows_wave = 0;
     if (n <= 0) return EGX_SUCC;
 
-    // hub rows [0, n_hub): fixed-size segments
-    std::vector<int32_t> row((size_t)g.n_hub + 1, 0);
-    if (g.n_hub > 0)
-        EGX_HIP_TRY(hipMemcpyWithStream(row.data(), g.it_row, row.size() * 4, hipMemcpyDeviceToHost, s),
-                    EGX_DEVICE_ERR);
-    std::vector<HubSeg> segs;
-    std::vector<HubRow> hub_rows;
-    for (int32_t v = 0; v < g.n_hub; ++v) {
-        const int32_t b = row[(size_t)v], e = row[(size_t)v + 1];
-        const int32_t nseg = (int32_t)(((int64_t)(e - b) + cfg.hub_segment - 1) / cfg.hub_segment);
-        const int32_t first = (int32_t)segs.size();
-        // a row of one segment is finished by its workgroup
-        if (nseg > 1) hub_rows.push_back(HubRow{v, first, nseg, 0});
-        for (int32_t k = 0; k < nseg; ++k) {
-            HubSeg sg;
-            sg.row = v;
-            sg.beg = b + k * cfg.hub_segment;
-            sg.end = (int32_t)std::min<int64_t>((int64_t)sg.beg + cfg.hub_segment, e);
-            sg.slot = v;
-            sg.nseg = nseg;
-            sg.first = first;
-            segs.push_back(sg);
-        }
-    }
+    // hub rows [0, n_hub): fixed-size segments; a row of one segment is
+    // finished by its workgroup
     g.n_hrows = g.n_hub;
-    g.n_hrows_split = (int64_t)hub_rows.size();
-    g.n_hrows_many = many_first(hub_rows);
-    g.n_hseg = (int64_t)segs.size();
-    EGX_TRY(g.hsegs.alloc(std::max<size_t>(segs.size(), 1) * sizeof(HubSeg)));
-    if (!segs.empty())
-        EGX_HIP_TRY(hipMemcpyAsync(g.hsegs.p, segs.data(), segs.size() * sizeof(HubSeg), hipMemcpyHostToDevice, s),
-                    EGX_DEVICE_ERR);
-    EGX_TRY(g.hrows.alloc(std::max<size_t>(hub_rows.size(), 1) * sizeof(HubRow)));
-    if (!hub_rows.empty())
-        EGX_HIP_TRY(hipMemcpyAsync(g.hrows.p, hub_rows.data(), hub_rows.size() * sizeof(HubRow),
-                                   hipMemcpyHostToDevice, s),
-                    EGX_DEVICE_ERR);
-    EGX_TRY(g.hub_part.alloc(std::max<size_t>(segs.size(), 1) * 8));
+    g.n_hrows_split = hctr[kCtrHubSplit];
+    g.n_hrows_many = hctr[kCtrHubMany];
+    g.n_hseg = hctr[kCtrHubSegs];
+    EGX_TRY(g.hsegs.alloc(std::max<size_t>((size_t)g.n_hseg, 1) * sizeof(HubSeg)));
+    EGX_TRY(g.hrows.alloc(std::max<size_t>((size_t)g.n_hrows_split, 1) * sizeof(HubRow)));
+    EGX_TRY(g.hub_part.alloc(std::max<size_t>((size_t)g.n_hseg, 1) * 8));
+    DevBuf first_seg;
+    if (g.n_hub > 0) {
+        EGX_TRY(first_seg.alloc(((size_t)g.n_hub + 1) * 4));
+        k_hub_rows<<<1, kHubThreads, 0, s>>>(g.it_row, g.n_hub, cfg.hub_segment, (int32_t)g.n_hrows_many,
+                                             first_seg.as<int32_t>(), g.hrows.as<HubRow>());
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+        k_hub_segs<<<nblocks(g.n_hseg, 256), 256, 0, s>>>(g.it_row, first_seg.as<int32_t>(), g.n_hub, cfg.hub_segment,
+                                                          (int32_t)g.n_hseg, g.hsegs.as<HubSeg>());
+        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
+    }
 
     // merge-path tiles over rows [n_hub, n)
-    const int64_t items = (g.m - row[(size_t)g.n_hub]) + (int64_t)(n - g.n_hub);
+    const int64_t items = (g.m - (int64_t)hctr[kCtrHubArcs]) + (int64_t)(n - g.n_hub);
     const int32_t per_tile = tile_size(cfg, items);
     g.n_tiles = (items + per_tile - 1) / per_tile;
     g.tile_lds = per_tile + cfg.wave_row_max;
@@ -1213,7 +1298,7 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in, int32_t known_hubs) {
         rc = build_blocked(g, cfg, layout_changed);
         if (rc != EGX_SUCC) g.bins.blocked = 0;  // the pull layout stays usable
     }
-    // the one wait (also for the copies out of segs and hub_rows), after all that can be queued without it
+    // the one wait, after all that can be queued without it
     uint32_t rows_wave = 0;
     EGX_HIP_TRY(hipMemcpyWithStream(&rows_wave, wave_rows.p, 4, hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
     g.rows_wave = rows_wave;
@@ -1327,7 +1412,8 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
     EGX_TRY(radix_sort_u32(keys, keys_alt, &vals, &vals_alt, m, bits_for((uint64_t)n), s));
     EGX_TRY(lower_bound_iota_u32(keys.as<uint32_t>(), m, g.in_row.as<int32_t>(), (int64_t)n + 1, s));
     if (n > 0) {
-        k_in_degrees<<<node_blocks, 256, 0, s>>>(g.in_row.as<int32_t>(), n, hub_threshold(g.bins), ctr);
+        k_in_degrees<<<node_blocks, 256, 0, s>>>(g.in_row.as<int32_t>(), n, hub_threshold(g.bins),
+                                             hub_segment(g.bins), ctr);
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     }
     uint32_t hctr[kCtrWords];
@@ -1370,7 +1456,7 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
     }
     if (n <= 0) EGX_HIP_TRY(hipMemsetAsync(g.in_col.p, 0, kArcPad * 4, s), EGX_DEVICE_ERR);  // else the layout's
     g.layout_built = false;
-    EGX_TRY(rebuild_bins(g, g.bins, (int32_t)hctr[kCtrHubs]));
+    EGX_TRY(rebuild_bins(g, g.bins, hctr));
     // large PageRank graphs iterate propagation-blocked; one the layout
     // cannot hold keeps the pull layout alone
     if (!g.adjacency && m >= kPbDefaultArcs && !g.bins.blocked) {
@@ -1424,7 +1510,8 @@ int build_from_device_rows(Graph& g, DevBuf&& V, DevBuf&& E, int32_t n, int64_t 
     k_node_arrays<true><<<node_blocks, 256, 0, s>>>(offsets.as<int32_t>(), g.out_w.as<double>(),
                                                     g.out_cnt.as<int32_t>(), n, 1, 1, g.deg.as<float>(), ctr);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-    k_in_degrees<<<node_blocks, 256, 0, s>>>(g.in_row.as<int32_t>(), n, hub_threshold(g.bins), ctr);
+    k_in_degrees<<<node_blocks, 256, 0, s>>>(g.in_row.as<int32_t>(), n, hub_threshold(g.bins),
+                                             hub_segment(g.bins), ctr);
     EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     uint32_t hctr[kCtrWords];
     EGX_HIP_TRY(hipMemcpyWithStream(hctr, ctr, sizeof(hctr), hipMemcpyDeviceToHost, s), EGX_DEVICE_ERR);
@@ -1437,14 +1524,14 @@ int build_from_device_rows(Graph& g, DevBuf&& V, DevBuf&& E, int32_t n, int64_t 
     keys_alt.release();
     offsets.release();
     g.layout_built = false;
-    EGX_TRY(rebuild_bins(g, g.bins, (int32_t)hctr[kCtrHubs]));
+    EGX_TRY(rebuild_bins(g, g.bins, hctr));
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     pool_stream_idle(s);
     g.build_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
     return EGX_SUCC;
 }
 
-int build_layout(Graph& g, const BinCfg& cfg, int32_t known_hubs) {
+int build_layout(Graph& g, const BinCfg& cfg, int32_t hubs) {
     hipStream_t s = g.stream;
     const int32_t n = g.n;
     const int64_t m = g.m;
@@ -1479,19 +1566,6 @@ int build_layout(Graph& g, const BinCfg& cfg, int32_t known_hubs) {
     const uint32_t maxdeg = (uint32_t)g.max_out_degree;
     const int bits = cfg.reorder ? bits_for(maxdeg) : 0;
     DevBuf keys, keys_alt, vals_alt, cnt;
-    int32_t nh = known_hubs;
-    if (nh < 0) {
-        DevBuf ctr;
-        uint32_t hubs = 0;
-        EGX_TRY(ctr.alloc(kCtrWords * sizeof(uint32_t)));
-        EGX_HIP_TRY(hipMemsetAsync(ctr.p, 0, kCtrWords * sizeof(uint32_t), s), EGX_DEVICE_ERR);
-        k_in_degrees<<<std::min<unsigned>(nblocks(n, 256), kNodeBlocks), 256, 0, s>>>(
-            g.in_row.as<int32_t>(), n, cfg.wave_row_max, ctr.as<uint32_t>());
-        EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
-        EGX_HIP_TRY(hipMemcpyWithStream(&hubs, ctr.as<uint32_t>() + kCtrHubs, 4, hipMemcpyDeviceToHost, s),
-                    EGX_DEVICE_ERR);
-        nh = (int32_t)hubs;
-    }
     EGX_TRY(keys.alloc((size_t)n * 4));
     EGX_TRY(keys_alt.alloc((size_t)n * 4));
     EGX_TRY(g.perm.alloc((size_t)n * 4));
@@ -1533,7 +1607,7 @@ int build_layout(Graph& g, const BinCfg& cfg, int32_t known_hubs) {
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
     }
     g.reordered = true;
-    g.n_hub = nh;
+    g.n_hub = hubs;
     g.it_row = g.p_row.as<int32_t>();
     g.it_col = g.p_col.as<int32_t>();
     g.it_val = g.p_val.as<float>();

@@ -265,14 +265,14 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
 // graph's, n and m are positive.  *bad_endpoint: an entry of E is outside
 // [0, n), and nothing was built.
 int build_from_device_rows(Graph& g, DevBuf&& V, DevBuf&& E, int32_t n, int64_t m, double alpha, bool* bad_endpoint);
-int build_layout(Graph& g, const BinCfg& cfg, int32_t known_hubs = -1);
+int build_layout(Graph& g, const BinCfg& cfg, int32_t hubs);  // hubs: rows above the hub threshold
 // Queue the device check of a host CSR's arcs on s: *flags (device, zeroed
 // here) gets kArcBadEndpoint / kArcBadWeight (not finite or negative; dW may
 // be null).
 constexpr uint32_t kArcBadEndpoint = 1u, kArcBadWeight = 2u;
 int check_arcs(const int32_t* dE, const double* dW, int32_t n, int64_t m, uint32_t* flags, hipStream_t s);
-// known_hubs: the number of rows above the hub threshold, if the caller counted them (else < 0)
-int rebuild_bins(Graph& g, const BinCfg& cfg, int32_t known_hubs = -1);
+// counters: the build's, if the caller has them for cfg's hub threshold and segments (else counted here)
+int rebuild_bins(Graph& g, const BinCfg& cfg, const uint32_t* counters = nullptr);
 int refresh_alpha(Graph& g, double alpha);
 int download_csc(Graph& g, int32_t* in_row, int32_t* in_col, float* in_val, int32_t* dangling01);
 

@@ -153,3 +153,30 @@ def test_row_offsets_at_scan_sizes(gpu_ready, n):
         s = np.divide(x, out, out=np.zeros(n), where=out > 0)
         x = 0.85 * np.bincount(E, weights=s[src], minlength=n) + (0.15 + 0.85 * x[out == 0].sum()) / n
     assert it == 3 and np.max(np.abs(got - x / x.sum()) / x) <= 1e-10  # sums of up to m terms of 2^-53 each
+
+
+# hub rows against the 1,024 threads that list them; rows of one segment, of several, and of 7 and more
+@pytest.mark.parametrize("hubs", [0, 1, 1023, 1024, 1025, 2100])
+def test_hub_row_lists(gpu_ready, hubs):
+    print(f"hub rows {hubs}", flush=True)
+    n = 2200
+    rng = np.random.default_rng(hubs)
+    indeg = rng.integers(0, 65, n)
+    indeg[rng.choice(n, hubs, replace=False)] = rng.choice([65, 255, 256, 257, 512, 513, 1536, 1537, 1800], hubs)
+    dst = np.repeat(np.arange(n), indeg)
+    src = rng.integers(0, n, len(dst))
+    order = np.lexsort((dst, src))
+    src, dst = src[order], dst[order].astype(np.int32)
+    V = np.zeros(n + 1, np.int32)
+    V[1:] = np.cumsum(np.bincount(src, minlength=n))
+    out = np.bincount(src, minlength=n)
+    x = np.full(n, 1.0 / n)
+    for _ in range(3):
+        s = np.divide(x, out, out=np.zeros(n), where=out > 0)
+        x = 0.85 * np.bincount(dst, weights=s[src], minlength=n) + (0.15 + 0.85 * x[out == 0].sum()) / n
+    with native.DeviceGraph.from_csr(V, dst) as g:
+        for seg in (256, 512, 8192):
+            g.set_bins(wave_row_max=64, hub_segment=seg)
+            assert g.info()["rows_hub"] == hubs
+            got, it, _ = g.pagerank(max_iter=3, tol=0.0, precision=native.PRECISION_FP64)
+            assert it == 3 and np.max(np.abs(got - x / x.sum()) / x) <= 1e-11  # sums of at most 1,800 terms of 2^-53 each
