@@ -90,6 +90,8 @@ struct IterArgs {
     double* partials;  // SoA: err[grid], sum[grid], dang[grid]
     double* red_part;  // SoA: err[n_red], sum[n_red], dang[n_red]
     uint32_t it;           // one graph: number of the iteration's launch
+    uint32_t may_stop;     // before the last iteration
+    uint32_t prefolded;    // the state in this launch's slot is there already
     const double* fold;    // what begin_fold adds up: SoA of fold_n partial sums each
     uint32_t fold_n;
     HostState* host;       // pinned
@@ -333,19 +335,48 @@ __device__ __forceinline__ void begin_fold(const IterArgs<T>& a, FoldSums f, PrS
     }
 }
 
+// Launches queued past the stop end at once: the state of the launch before
+// (stop_slot), whose last sums are not yet folded, is a stopped one already,
+// and the first workgroup hands it on.  (Without this look they gathered all
+// their arcs before they learnt of it: 5 of 34 us each in a Katz solve of 6
+// iterations of 49 us.)  Only the first launch past the stop gathers in vain.  Graphs
+// of kPrefoldArcs or more that may stop early therefore fold the sums in a
+// launch of their own (k_pr_state, 5 us) before each iteration: R-MAT 24
+// stopping after one iteration 834 us, 796 so.
+constexpr int64_t kPrefoldArcs = (int64_t)1 << 26, kPrefoldArcsPull = (int64_t)1 << 24;
+template <typename T>
+__device__ __forceinline__ int32_t stop_slot(const IterArgs<T>& a) {
+    return (int32_t)((a.it + (a.prefolded ? 0u : 1u)) & 1u);
+}
+template <typename T>
+__device__ __forceinline__ void past_stop(const IterArgs<T>& a, PrState* sh) {
+    if (!a.prefolded && blockIdx.x == 0 && wave_id() == 0) begin_fold(a, FoldSums{0.0, 0.0, 0.0}, sh);
+}
+
+// begin_fold of an iteration's own launches.
+template <typename T>
+__device__ __forceinline__ void iteration_state(const IterArgs<T>& a, FoldSums f, PrState* sh) {
+    if (!a.prefolded) begin_fold(a, f, sh);
+    else if (lane_id() == 0) *sh = a.state[a.it & 1];
+}
+
 // One SpMV work item.  col / val are streamed once per iteration:
 // non-temporal loads keep them from evicting the gathered vector from L2.
 // Fold: an iteration's first launch of one graph.  The gathers need only the
 // launch's parity; the state arrives in *sh with the barrier that ends them,
-// and a workgroup that then finds the solve done writes nothing.
-template <typename T, bool W, bool Fold>
+// and a workgroup that then finds the solve done writes nothing.  Stop: looks for
+// a stop before the gathers (the code for it alone slows FP64 tiles by 3%).
+template <typename T, bool W, bool Fold, bool Stop>
 __device__ __forceinline__ void spmv_block(IterArgs<T>& a, uint32_t b, T* lds, double* sh_red, PrState* sh) {
     const int t = threadIdx.x;
     FoldSums f{0.0, 0.0, 0.0};
     if (Fold && wave_id() == 0) f = begin_load(a);
+    // looked at once the item's bounds are here
+    const int32_t stopped = Stop ? a.state[stop_slot(a)].done : 0;
 
     if (b < a.nblk_h) {
         const HubSeg sg = a.hsegs[b];
+        if (Stop && stopped) return past_stop(a, sh);
         double acc = 0.0;
         for (int32_t base = sg.beg; base < sg.end; base += kThreads * kBatch) {
             int32_t u[kBatch];
@@ -365,7 +396,7 @@ __device__ __forceinline__ void spmv_block(IterArgs<T>& a, uint32_t b, T* lds, d
         }
         acc = wave_sum(acc);
         if (lane_id() == 0) sh_red[wave_id()] = acc;
-        if (Fold && wave_id() == 0) begin_fold(a, f, sh);
+        if (Fold && wave_id() == 0) iteration_state(a, f, sh);
         __syncthreads();
         if (Fold) {
             if (sh->done) return;
@@ -390,9 +421,10 @@ __device__ __forceinline__ void spmv_block(IterArgs<T>& a, uint32_t b, T* lds, d
     const int32_t a0 = a.row[r0];
     const int32_t na = a.row[r1] - a0;
     const int32_t nr = r1 - r0;
+    if (Stop && stopped) return past_stop(a, sh);
     if (a.tpos) stage_tile<T, W, true>(a, a0, na, lds);
     else stage_tile<T, W, false>(a, a0, na, lds);
-    if (Fold && wave_id() == 0) begin_fold(a, f, sh);
+    if (Fold && wave_id() == 0) iteration_state(a, f, sh);
     __syncthreads();
     if (Fold) {
         if (sh->done) return;
@@ -532,14 +564,14 @@ __device__ __forceinline__ void reduce_final_wave(const IterArgs<T>& a) {
     }
 }
 
-template <typename T, bool W>
+template <typename T, bool W, bool Stop>
 __global__ __launch_bounds__(kThreads, 8) void k_pr_spmv(IterArgs<T> a) {
     extern __shared__ __align__(16) unsigned char tile_lds[];
     T* lds = reinterpret_cast<T*>(tile_lds);
     __shared__ double sh_red[3 * kWavesPerBlock];
     __shared__ PrState sh;
     bind_parity(a, (a.it & 1) != 0);
-    spmv_block<T, W, true>(a, blockIdx.x, lds, sh_red, &sh);
+    spmv_block<T, W, true, Stop>(a, blockIdx.x, lds, sh_red, &sh);
 }
 
 template <typename T, bool W>
@@ -813,6 +845,7 @@ template <typename T, bool W, bool Fold>
 __device__ __forceinline__ void pb_scatter_item(const IterArgs<T>& a, const PbArgs& pb, uint32_t item, float* sc,
                                                 float (*stage)[kPbStage], PrState* sh) {
     const PbScatter it = pb.scatter[item];
+    if (Fold && a.may_stop && a.state[stop_slot(a)].done) return past_stop(a, sh);
     const int l = lane_id();
     // every lane of a wavefront runs the loop the same number of times (the
     // bound depends on the wavefront's first thread only), so the shuffles
@@ -837,7 +870,7 @@ __device__ __forceinline__ void pb_scatter_item(const IterArgs<T>& a, const PbAr
         for (int32_t i = threadIdx.x; i < cnt; i += kPbThreads) sc[i] = (float)sv[base + i];
     }
     if (threadIdx.x == 0) sc[kPbChunk] = 0.0f;
-    if (Fold && wave_id() == 0) begin_fold(a, begin_load(a), sh);
+    if (Fold && wave_id() == 0) iteration_state(a, begin_load(a), sh);
     __syncthreads();
     if (Fold && sh->done) return;  // the state arrives with the barrier
     float* stg = stage[wave_id()];
@@ -1085,7 +1118,7 @@ __global__ __launch_bounds__(kThreads, 8) void k_pr_spmv_multi(const IterArgs<T>
     IterArgs<T> a = table[gi];
     if (a.state->done) return;
     bind(a);
-    spmv_block<T, W, false>(a, blk_local[blockIdx.x], lds, sh_red, nullptr);
+    spmv_block<T, W, false, false>(a, blk_local[blockIdx.x], lds, sh_red, nullptr);
 }
 
 template <typename T, bool W>
@@ -1508,8 +1541,12 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
             a.fold = partials + ((it & 1) ? 0 : 3 * (size_t)grid);
         }
     };
+    const bool can_stop_early = p.tol > 0.0 || p.eig_delta != 0;
+    a.may_stop = can_stop_early ? 1 : 0;
+    a.prefolded = can_stop_early && g.m >= (blocked ? kPrefoldArcs : kPrefoldArcsPull) ? 1 : 0;
     // the SpMV of one iteration: pull kernel, or scatter + sum
     auto launch_spmv = [&]() {
+        if (a.prefolded) k_pr_state<T><<<1, kWave, 0, s>>>(a);
         if constexpr (kBlockable) {
             if (blocked) {
                 k_pb_scatter<T, W><<<(uint32_t)g.n_pb_scatter, kPbThreads, 0, s>>>(a, pb);
@@ -1517,7 +1554,8 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
                 return;
             }
         }
-        k_pr_spmv<T, W><<<grid, kThreads, (size_t)g.tile_lds * sizeof(T), s>>>(a);
+        if (a.may_stop) k_pr_spmv<T, W, true><<<grid, kThreads, (size_t)g.tile_lds * sizeof(T), s>>>(a);
+        else k_pr_spmv<T, W, false><<<grid, kThreads, (size_t)g.tile_lds * sizeof(T), s>>>(a);
     };
     auto launch_reduce = [&]() {
         if (reduce) k_pr_reduce<T, W><<<a.n_red, kReduceThreads, 0, s>>>(a);
@@ -1541,7 +1579,6 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
     __atomic_store_n(&hs->progress, (uint64_t)0, __ATOMIC_RELAXED);
     EGX_HIP_TRY(hipEventRecord(g.ev0, s), EGX_DEVICE_ERR);
     int32_t launched = 0;
-    const bool can_stop_early = p.tol > 0.0 || p.eig_delta != 0;
     // iterations queued past the last one whose start the device has
     // reported: enough to keep it busy, few to run empty after the stop
     const int32_t ahead = p.check_every > 0 ? p.check_every : kAhead;
