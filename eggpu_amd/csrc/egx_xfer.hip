@@ -4,12 +4,12 @@
 // 16.7M doubles took 9 ms of a 19.5 ms solve, one thread touching 134 MB of new
 // pages (16.8 GB/s) after a 67 MB copy, and 112 MB of CSR arrays went up at
 // 27 GB/s.  Both directions now run in chunks of kChunkBytes through a ring
-// of pinned chunks: the copy engine moves one chunk while up to
+// of pinned chunks: queued kernels move one chunk over the link while up to
 // kThreads threads fill or empty others (PCIe carries 57 GB/s from pinned
 // memory).  Chunks and threads are kept for the process and shared by all
 // callers: a caller takes what is free (it always makes progress alone) and
 // gives it back before it returns.  Transfers down of at most kInlineBytes use one
-// chunk and no threads, those up of at most kUploadPlain the runtime's copy.
+// chunk and no threads, those up of at most kUploadSmall too.
 #include <sched.h>
 
 #include <algorithm>
@@ -34,20 +34,20 @@ namespace {
 // 2.76 / 6.74, 8 MiB 2.69 / 6.68; 4 threads 2.71 / 7.27, 16 threads 2.82 / 6.68.
 constexpr size_t kChunkBytes = (size_t)4 << 20;
 constexpr size_t kInlineBytes = (size_t)256 << 10;
-// Uploads up to here are the runtime's own copies: one array after the other at
-// 30 GB/s, but no threads to wake (16,384 nodes and 1 MB of arcs built and
-// solved: 494 us in chunks, 480 so).
-constexpr size_t kUploadPlain = (size_t)2 << 20;
+// Uploads up to here go through one chunk, by the calling thread: no threads
+// to wake.
+constexpr size_t kUploadSmall = (size_t)2 << 20;
 constexpr int kMaxChunks = 24;    // pinned chunks the process keeps, at most
 constexpr int kCallChunks = 12;   // of them for one transfer
 constexpr int kThreads = 8;       // the calling thread among them
 
 struct Chunk {
-    char* p = nullptr;           // kChunkBytes, and the flag behind them
+    char* p = nullptr;           // `bytes`, and the flag behind them
+    size_t bytes = 0;            // kChunkBytes, or kInlineBytes (making and pinning 4 MiB takes 6 ms, 256 KiB 0.2)
     uint32_t* count = nullptr;   // device: workgroups that have written their share
     hipEvent_t ev = nullptr;     // the chunk's last upload
     int dev = -1;                // of count and ev
-    uint32_t* flag() const { return reinterpret_cast<uint32_t*>(p + kChunkBytes); }
+    uint32_t* flag() const { return reinterpret_cast<uint32_t*>(p + bytes); }
 };
 
 // Device memory to a pinned chunk, and 1 to *flag once all of it is there.
@@ -57,12 +57,11 @@ struct Chunk {
 // 20 iterations: 1.22 ms -> 1.16; 64 columns of 300,007 6.5 -> 6.3).
 constexpr int kFetchThreads = 256;
 constexpr int kFetchBlocks = 64;
-__global__ __launch_bounds__(kFetchThreads) void k_fetch_part(const char* __restrict__ from, char* __restrict__ to,
-                                                              int64_t bytes, uint32_t* count, uint32_t* flag) {
+__device__ __forceinline__ void copy_words(const char* __restrict__ from, char* __restrict__ to, int64_t bytes) {
     const int64_t t = (int64_t)blockIdx.x * kFetchThreads + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * kFetchThreads;
     int64_t words = 0;  // 4-byte words already taken by 16-byte copies
-    if (reinterpret_cast<uintptr_t>(from) % 16 == 0) {  // (uniform) results of a set may begin at any float
+    if ((reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(to)) % 16 == 0) {  // (uniform) results of a set may begin at any float
         const uint4* f = reinterpret_cast<const uint4*>(from);
         uint4* o = reinterpret_cast<uint4*>(to);
         const int64_t n = bytes / 16;
@@ -72,7 +71,26 @@ __global__ __launch_bounds__(kFetchThreads) void k_fetch_part(const char* __rest
     }
     for (int64_t i = words + t; i < bytes / 4; i += stride)
         reinterpret_cast<uint32_t*>(to)[i] = reinterpret_cast<const uint32_t*>(from)[i];
+}
+
+__global__ __launch_bounds__(kFetchThreads) void k_fetch_part(const char* __restrict__ from, char* __restrict__ to,
+                                                              int64_t bytes, uint32_t* count, uint32_t* flag) {
+    copy_words(from, to, bytes);
     raise_flag(count, flag);
+}
+
+// The other way, from a pinned chunk.  The copy engine reaches the same rate,
+// but the first copy it makes for a process takes 6 ms to set up: the first
+// graph built from host arrays took 6.9 ms, and 1.1 so (16,384 nodes); later
+// builds 377 -> 361 us there, 4.98 -> 4.80 ms with 112 MB of weighted arcs.
+__global__ __launch_bounds__(kFetchThreads) void k_upload_part(const char* __restrict__ from, char* __restrict__ to,
+                                                               int64_t bytes) {
+    copy_words(from, to, bytes);
+}
+
+unsigned copy_blocks(size_t bytes) {
+    const int64_t blocks = ((int64_t)bytes + kFetchThreads * 16 - 1) / (kFetchThreads * 16);
+    return (unsigned)std::min<int64_t>(kFetchBlocks, std::max<int64_t>(blocks, 1));
 }
 
 __global__ void k_fetch_reset(uint32_t* count) { *count = 0; }
@@ -80,30 +98,33 @@ __global__ void k_fetch_reset(uint32_t* count) { *count = 0; }
 struct ChunkPool {
     std::mutex mu;
     std::vector<Chunk> idle;
-    int made = 0;
+    int made[2] = {0, 0};  // small, large
 };
 ChunkPool& chunk_pool() {
     static ChunkPool* p = new ChunkPool();  // kept until the process ends
     return *p;
 }
 
-// Up to `want` chunks usable on device dev (for work on s), at least one unless nothing is
+// Up to `want` chunks that hold `bytes`, usable on device dev (for work on s), at least one unless nothing is
 // free and no more may be made (then none).
-std::vector<Chunk> take_chunks(int want, int dev, hipStream_t s) {
+std::vector<Chunk> take_chunks(int want, size_t bytes, int dev, hipStream_t s) {
     ChunkPool& pool = chunk_pool();
+    bytes = bytes <= kInlineBytes ? kInlineBytes : kChunkBytes;
+    int& made = pool.made[bytes == kChunkBytes ? 1 : 0];
     std::vector<Chunk> got;
     got.reserve((size_t)want);
     std::lock_guard<std::mutex> lk(pool.mu);
-    pool.idle.reserve((size_t)kMaxChunks);  // so that giving back never allocates
+    pool.idle.reserve((size_t)kMaxChunks * 2);  // so that giving back never allocates
     for (size_t i = pool.idle.size(); i-- > 0 && (int)got.size() < want;) {
-        if (pool.idle[i].dev != dev) continue;
+        if (pool.idle[i].dev != dev || pool.idle[i].bytes != bytes) continue;
         got.push_back(pool.idle[i]);
         pool.idle.erase(pool.idle.begin() + (std::ptrdiff_t)i);
     }
-    while ((int)got.size() < want && pool.made < kMaxChunks) {
+    while ((int)got.size() < want && made < kMaxChunks) {
         Chunk c;
         c.dev = dev;
-        if (hipHostMalloc(reinterpret_cast<void**>(&c.p), kChunkBytes + 64) != hipSuccess) {
+        c.bytes = bytes;
+        if (hipHostMalloc(reinterpret_cast<void**>(&c.p), bytes + 64) != hipSuccess) {
             (void)hipGetLastError();
             break;
         }
@@ -119,7 +140,7 @@ std::vector<Chunk> take_chunks(int want, int dev, hipStream_t s) {
             (void)hipHostFree(c.p);
             break;
         }
-        pool.made += 1;
+        made += 1;
         got.push_back(c);
     }
     return got;
@@ -280,9 +301,7 @@ struct Run {
         const Part& p = parts[(size_t)k];
         const Chunk& c = chunks[(size_t)k % chunks.size()];
         __atomic_store_n(c.flag(), 0u, __ATOMIC_RELEASE);
-        const int64_t blocks = ((int64_t)p.bytes + kFetchThreads * 16 - 1) / (kFetchThreads * 16);
-        k_fetch_part<<<(unsigned)std::min<int64_t>(kFetchBlocks, blocks), kFetchThreads, 0, s>>>(
-            p.dev, c.p, (int64_t)p.bytes, c.count, c.flag());
+        k_fetch_part<<<copy_blocks(p.bytes), kFetchThreads, 0, s>>>(p.dev, c.p, (int64_t)p.bytes, c.count, c.flag());
         if (ok(hipGetLastError())) stage[(size_t)k].store(1, std::memory_order_release);
     }
     // Waits until the part in chunk c has landed; false when its stream failed.
@@ -322,9 +341,8 @@ struct Run {
             // the ring's previous part has been queued from this chunk, and its copy has ended
             if (k >= ring && (!reached(k - ring, 2) || !ok(hipEventSynchronize(c.ev)))) return;
             std::memcpy(c.p, p.host, p.bytes);
-            if (!ok(hipMemcpyAsync(p.dev, c.p, p.bytes, hipMemcpyHostToDevice, s)) ||
-                !ok(hipEventRecord(c.ev, s)))
-                return;
+            k_upload_part<<<copy_blocks(p.bytes), kFetchThreads, 0, s>>>(c.p, p.dev, (int64_t)p.bytes);
+            if (!ok(hipGetLastError()) || !ok(hipEventRecord(c.ev, s))) return;
             stage[(size_t)k].store(2, std::memory_order_release);
         }
     }
@@ -342,15 +360,44 @@ int finish_run(Run& r) {
     return EGX_SUCC;
 }
 
-// Chunks for `parts` parts; -1 when there are none to be had.
-int begin_run(Run& r, size_t parts, hipStream_t s) {
+size_t largest(const std::vector<Part>& parts) {
+    size_t most = 0;
+    for (const Part& p : parts) most = std::max(most, p.bytes);
+    return most;
+}
+
+// Chunks for `parts` parts of at most `bytes`; -1 when there are none to be had.
+int begin_run(Run& r, size_t parts, size_t bytes, hipStream_t s) {
     r.s = s;
     if (hipGetDevice(&r.dev) != hipSuccess) return -1;
-    r.chunks = take_chunks((int)std::min<size_t>(parts, kCallChunks), r.dev, s);
+    r.chunks = take_chunks((int)std::min<size_t>(parts, kCallChunks), bytes, r.dev, s);
     if (r.chunks.empty()) return -1;
     r.stage.reset(new std::atomic<int>[std::max<size_t>(parts, 1)]);
     for (size_t i = 0; i < parts; ++i) r.stage[i].store(0);
     return 0;
+}
+
+int upload_plain(const std::vector<Upload>& jobs, hipStream_t s) {
+    for (const Upload& u : jobs)
+        if (u.bytes)
+            EGX_HIP_TRY(hipMemcpyWithStream(u.dev, u.host, u.bytes, hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
+    return EGX_SUCC;
+}
+
+// All in one chunk, by the calling thread.
+int upload_small(const std::vector<Upload>& jobs, size_t total_bytes, hipStream_t s) {
+    Run r;
+    if (begin_run(r, 1, total_bytes + 16 * jobs.size(), s) != 0) return upload_plain(jobs, s);
+    size_t at = 0;
+    for (const Upload& u : jobs) {
+        if (u.bytes == 0) continue;
+        char* from = r.chunks[0].p + at;
+        std::memcpy(from, u.host, u.bytes);
+        k_upload_part<<<copy_blocks(u.bytes), kFetchThreads, 0, s>>>(from, static_cast<char*>(u.dev), (int64_t)u.bytes);
+        if (!r.ok(hipGetLastError())) break;
+        at += (u.bytes + 15) / 16 * 16;
+    }
+    return finish_run(r);
 }
 
 int upload_chunked(const std::vector<Upload>& jobs, size_t total_bytes, hipStream_t s) {
@@ -361,11 +408,7 @@ int upload_chunked(const std::vector<Upload>& jobs, size_t total_bytes, hipStrea
             r.parts.push_back(Part{static_cast<const char*>(u.host) + at, static_cast<char*>(u.dev) + at,
                                    std::min(step, u.bytes - at), 0, 0});
     const std::function<void()> work = [&] { r.upload_parts(); };
-    if (begin_run(r, r.parts.size(), s) != 0) {  // no pinned memory
-        for (const Upload& u : jobs)
-            EGX_HIP_TRY(hipMemcpyWithStream(u.dev, u.host, u.bytes, hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
-        return EGX_SUCC;
-    }
+    if (begin_run(r, r.parts.size(), largest(r.parts), s) != 0) return upload_plain(jobs, s);  // no pinned memory
     run_together(work, (int)std::min<size_t>(r.parts.size(), kThreads) - 1);
     return finish_run(r);
 }
@@ -391,7 +434,7 @@ int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_
     }
     if (r.parts.empty()) return EGX_SUCC;
     const std::function<void()> work = [&] { r.fetch_parts(); };
-    if (begin_run(r, r.parts.size(), s) != 0) {
+    if (begin_run(r, r.parts.size(), largest(r.parts), s) != 0) {
         // no pinned memory: through a pageable buffer
         std::vector<char> buf(kChunkBytes);
         for (const Part& p : r.parts) {
@@ -411,13 +454,9 @@ int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_
 int upload(const std::vector<Upload>& jobs, hipStream_t s) {
     size_t total = 0;
     for (const Upload& u : jobs) total += u.bytes;
-    if (total <= kUploadPlain) {
-        for (const Upload& u : jobs)
-            if (u.bytes)
-                EGX_HIP_TRY(hipMemcpyWithStream(u.dev, u.host, u.bytes, hipMemcpyHostToDevice, s), EGX_DEVICE_ERR);
-        return EGX_SUCC;
-    }
+    if (total == 0) return EGX_SUCC;
     try {
+        if (total <= kUploadSmall) return upload_small(jobs, total, s);
         return upload_chunked(jobs, total, s);
     } catch (const std::bad_alloc&) {
         set_last_error("host transfer: out of host memory");
@@ -439,7 +478,7 @@ bool DirectFetch::begin(size_t bytes, hipStream_t s) {
     if (bytes > kInlineBytes) return false;
     try {
         std::unique_ptr<State> st(new State());
-        if (begin_run(st->r, 1, s) != 0) return false;
+        if (begin_run(st->r, 1, bytes, s) != 0) return false;
         st_ = std::move(st);
     } catch (const std::bad_alloc&) {
         return false;
