@@ -942,15 +942,14 @@ constexpr int64_t kPbScatterMax1 = 65536;  // one round; unweighted graphs of se
 constexpr int64_t kPbSumBins = 1024;
 constexpr int64_t kPbSumItems = 512, kPbSumMin = 16384;
 constexpr int64_t kPbSumItemsMany = 256, kPbSumMinMany = 32768;
-// Graphs laid out for shared launches: one size for all, as the set fills the
-// device.  us per iteration of sets of 16 to 100 graphs, items of 256K and
-// 128K slots -> 96K and 32K: 48 graphs of 1,000 to 300,000 nodes 128 -> 101,
-// 24 of them 107 -> 63, 96 of them 185 -> 175, 16 of 20,000 to 1,000,000
-// 181 -> 156, 100 of 1,000 to 20,000 69 -> 50 (scatter items of 64K to 192K
-// differ by how they fill the last round: 108, 70, 186, 166, 46 and 99, 78,
-// 160, 167, 61).
+// Graphs laid out for shared launches: one size for all.  Scatter items of a
+// chunk are joined by the launch when the set is large (kJoinSlots); sum
+// items are not, so theirs is the one that costs large sets nothing.  us per
+// iteration at 256K and 128K slots, 192K and 64K, 96K and 32K: 48 graphs of
+// 1,000 to 300,000 nodes 130, 106, 104; 96 of them 189, 159, 179; 200 337,
+// 342, 391; 512 of 1,000 to 1,000,000 2,399, 2,424, 2,791.
 constexpr int64_t kPbScatterShared = 98304;
-constexpr int64_t kPbSumShared = 32768;
+constexpr int64_t kPbSumShared = 65536;
 
 int64_t pb_item_slots(int64_t total, int64_t items, int64_t lo, int64_t hi) {
     const int64_t want = (total / items) / kPbVec * kPbVec;
@@ -981,6 +980,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
         d->release();
     g.n_pb_scatter = g.n_pb_sum = g.n_pb_hrows = g.n_pb_hrows_many = 0;
     g.pb_scatter_size.clear();
+    g.pb_scatter_chunk.clear();
     g.pb_sum_size.clear();
     if (!cfg.blocked || g.n <= 0 || g.m <= 0) return EGX_SUCC;
     // test hook: a real device allocation failure at the start of the layout
@@ -1204,7 +1204,11 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     g.n_pb_hrows = (int64_t)hrows.size();
     g.n_pb_hrows_many = many;
     g.pb_scatter_size.resize(scat.size());
-    for (size_t i = 0; i < scat.size(); ++i) g.pb_scatter_size[i] = scat[i].g1 - scat[i].g0;
+    g.pb_scatter_chunk.resize(scat.size());
+    for (size_t i = 0; i < scat.size(); ++i) {
+        g.pb_scatter_size[i] = scat[i].g1 - scat[i].g0;
+        g.pb_scatter_chunk[i] = scat[i].chunk;
+    }
     g.pb_sum_size.resize(sums.size());
     for (size_t i = 0; i < sums.size(); ++i) g.pb_sum_size[i] = sums[i].e1 - sums[i].e0;
     g.pb_shared = cfg.blocked_shared;

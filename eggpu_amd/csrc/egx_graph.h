@@ -190,7 +190,7 @@ struct Graph {
     int64_t n_pb_scatter = 0, n_pb_sum = 0, n_pb_hrows = 0, n_pb_hrows_many = 0;
     // host copies of the items' sizes (groups per scatter item, value slots
     // per sum item), for ordering them in multi-graph launches
-    std::vector<int32_t> pb_scatter_size, pb_sum_size;
+    std::vector<int32_t> pb_scatter_size, pb_sum_size, pb_scatter_chunk;
     int32_t pb_shared = -1;  // item sizing the blocked layout was built with (BinCfg::blocked_shared)
     // the blocked layout merges stretches across groups (weighted solves);
     // only the kernels built for that merge read it

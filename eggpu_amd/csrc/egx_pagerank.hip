@@ -838,13 +838,15 @@ __device__ __forceinline__ void pb_scatter_batch(const PbScatterBatch<W>& cur, i
     }
 }
 
-// Scatter item `item` of one graph, in a workgroup of kPbThreads threads
+// Scatter items [item, item + count) of one graph, all of one chunk and one
+// after the other, in a workgroup of kPbThreads threads
 // with sc (kPbChunk + 4 floats) and stage (kPbThreads / kWave rows of
 // kPbStage floats) in LDS.
 template <typename T, bool W, bool Fold>
-__device__ __forceinline__ void pb_scatter_item(const IterArgs<T>& a, const PbArgs& pb, uint32_t item, float* sc,
-                                                float (*stage)[kPbStage], PrState* sh) {
-    const PbScatter it = pb.scatter[item];
+__device__ __forceinline__ void pb_scatter_item(const IterArgs<T>& a, const PbArgs& pb, uint32_t item, uint32_t count,
+                                                float* sc, float (*stage)[kPbStage], PrState* sh) {
+    PbScatter it = pb.scatter[item];
+    if (!Fold) it.g1 = pb.scatter[item + count - 1].g1;
     if (Fold && a.may_stop && a.state[stop_slot(a)].done) return past_stop(a, sh);
     const int l = lane_id();
     // every lane of a wavefront runs the loop the same number of times (the
@@ -893,11 +895,21 @@ __global__ __launch_bounds__(kPbThreads) void k_pb_scatter(IterArgs<T> a, PbArgs
     __shared__ float stage[kPbThreads / kWave][kPbStage];
     __shared__ PrState sh;
     bind_parity(a, (a.it & 1) != 0);
-    pb_scatter_item<T, W, true>(a, pb, blockIdx.x, sc, stage, &sh);
+    pb_scatter_item<T, W, true>(a, pb, blockIdx.x, 1, sc, stage, &sh);
 }
 
-// Many graphs, one launch: workgroup b runs scatter item item_local[b] of
-// graph item_graph[b].
+// Many graphs, one launch: workgroup b runs item_local[b] / kJoinOne scatter
+// items from item_local[b] % kJoinOne on of graph item_graph[b].
+constexpr uint32_t kJoinOne = 1u << 28;
+// Slots per scatter workgroup and round that items are joined towards, up to
+// kJoinMost of them: sets with less than 1.5 rounds of kJoinSlots leave them
+// as they are (fewer CUs would run), larger ones stage each chunk less often:
+// us per iteration with 96K, 192K and 256K slots a workgroup: 48 graphs of
+// 1,000 to 300,000 nodes 104, 106 and 117, 96 of them 169 (128K), 159 and 175,
+// 200 of them 366 (128K), 342 and 337.
+constexpr int64_t kJoinSlots = 168 * 1024;
+constexpr int64_t kJoinMost = 3;
+constexpr int64_t kScatterCus = 256;  // a scatter workgroup takes a CU
 template <typename T, bool W>
 __global__ __launch_bounds__(kPbThreads) void k_pb_scatter_multi(const IterArgs<T>* __restrict__ table,
                                                                  const PbArgs* __restrict__ pbs,
@@ -909,7 +921,8 @@ __global__ __launch_bounds__(kPbThreads) void k_pb_scatter_multi(const IterArgs<
     IterArgs<T> a = table[gi];
     if (a.state->done) return;
     bind(a);
-    pb_scatter_item<T, W, false>(a, pbs[gi], item_local[blockIdx.x], sc, stage, nullptr);
+    const uint32_t item = item_local[blockIdx.x];
+    pb_scatter_item<T, W, false>(a, pbs[gi], item & (kJoinOne - 1), item / kJoinOne, sc, stage, nullptr);
 }
 
 // One sum item (one workgroup of kPbSumWaves wavefronts): its value slots
@@ -1715,6 +1728,7 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
         uint32_t local;
     };
     std::vector<PbItem> sc_items, sum_items;
+    int64_t scatter_groups = 0;
     if constexpr (kBlockable) {
         for (int32_t i = 0; i < count; ++i) {
             Graph& g = *gs[(size_t)i];
@@ -1739,9 +1753,25 @@ int solve_multi_typed(std::vector<Graph*>& gs, const SolveParams& p, double* con
             pb.scatter = g.pb_scatter.as<PbScatter>();
             pb.sums = g.pb_sum.as<PbSum>();
             pb.w = W ? g.pb_w.as<float>() : nullptr;
-            for (int64_t k = 0; k < g.n_pb_scatter; ++k)
-                sc_items.push_back({g.pb_scatter_size[(size_t)k], i, (uint32_t)k});
+            for (int64_t k = 0; k < g.n_pb_scatter; ++k) scatter_groups += g.pb_scatter_size[(size_t)k];
             for (int64_t k = 0; k < g.n_pb_sum; ++k) sum_items.push_back({g.pb_sum_size[(size_t)k], i, (uint32_t)k});
+        }
+        const int64_t join =
+            std::min(kJoinMost, std::max<int64_t>(1, (scatter_groups * kPbVec / kScatterCus + kJoinSlots / 2) / kJoinSlots));
+        for (int32_t i = 0; i < count; ++i) {
+            if (!is_pb[(size_t)i]) continue;
+            const Graph& g = *gs[(size_t)i];
+            const int64_t most = g.n_pb_scatter < (int64_t)kJoinOne && g.pb_shared == 1 ? join : 1;
+            for (int64_t k = 0; k < g.n_pb_scatter;) {
+                int64_t q = 1;
+                int32_t size = g.pb_scatter_size[(size_t)k];
+                for (; q < most && k + q < g.n_pb_scatter &&
+                       g.pb_scatter_chunk[(size_t)(k + q)] == g.pb_scatter_chunk[(size_t)k];
+                     ++q)
+                    size += g.pb_scatter_size[(size_t)(k + q)];
+                sc_items.push_back({size, i, (uint32_t)k | (uint32_t)q * kJoinOne});
+                k += q;
+            }
         }
         // largest items first, so the small ones fill in behind them rather
         // than a large one running alone at the end of the launch

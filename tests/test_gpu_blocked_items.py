@@ -25,3 +25,22 @@ def test_item_sizes_do_not_change_the_iterate(gpu_ready, n, factor, weighted):
             assert np.abs(got - want).sum() <= 4 * 2.0 ** -24 / (1 - 0.85)
             (many,), _, _ = native.multi_pagerank([g], max_iter=10, tol=0.0)
             assert np.array_equal(many, got)
+
+
+# scatter items as they are, joined in twos, and in threes (75 and 130 million slots over 256 compute units)
+@pytest.mark.parametrize("count,factor", [(1, 4), (3, 26), (5, 28)])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_joined_items_in_shared_launches(gpu_ready, count, factor, weighted):
+    print(f"joined items count={count} factor={factor} weighted={weighted}", flush=True)
+    n = 1000003
+    graphs = [native.DeviceGraph.rmat_n(n, factor * n, seed=5 + k, weighted=weighted, wseed=4) for k in range(count)]
+    try:
+        for g in graphs:
+            g.set_bins(blocked=1, blocked_shared=1)
+        ranks, its, _ = native.multi_pagerank(graphs, max_iter=4, tol=0.0)
+        for g, r, it in zip(graphs, ranks, its):
+            want, w_it, _ = g.pagerank(max_iter=4, tol=0.0)
+            assert it == w_it and np.array_equal(r, want)
+    finally:
+        for g in graphs:
+            g.close()
