@@ -396,7 +396,7 @@ class DeviceGraph:
         tile_sort, blocked and blocked_shared < 0 keep theirs; hot_sources 0
         keeps it, < 0 turns non-temporal cold gathers off).  blocked_shared=1
         sizes the blocked layout's work items for graphs solved together in
-        multi_pagerank (the largest items); 0 for a graph solved alone."""
+        multi_pagerank; 0 for a graph solved alone."""
         o = BinOpts(int(thread_row_max), int(wave_row_max), int(hub_segment), int(tile_items), int(reorder),
                     int(tile_sort), int(hot_sources), int(blocked), int(blocked_shared))
         _check(lib().egx_graph_set_bins(self.handle, ctypes.byref(o)))

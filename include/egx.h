@@ -138,8 +138,8 @@ typedef struct {
                                through LDS, then summed per bin in LDS, with no
                                random gathers; 0: pull SpMV; < 0: keep setting */
     int32_t blocked_shared; /* 1: size the blocked layout's scatter and sum items for
-                               graphs solved together (egx_multi_pagerank): the
-                               largest items, since the set fills the device; 0: size
+                               graphs solved together (egx_multi_pagerank), which
+                               joins them when the set fills the device; 0: size
                                them so that the graph alone fills it (the default);
                                < 0: keep setting */
 } egx_bin_opts;
