@@ -34,6 +34,12 @@ namespace {
 constexpr int kRunThreads = 512;
 constexpr int kRunItems = 8;
 constexpr int kRunArcs = kRunThreads * kRunItems;  // arcs per workgroup
+// A run that spans more rows than this (most of them without arcs) has each
+// arc search between the first and the last instead: marking walks every row.
+// 1M arcs, us of k_arc_keys and k_layout_slots with marks | searches at 16K
+// rows a run 17 and 41 | 38 and 59, at 32K 27 and 58 | 43 and 71, at 64K 62 and 93 |
+// 60 and 91, at 128K 141 and 172 | 86 and 130, at 256K 283 and 304 | 110 and 155.
+constexpr int32_t kRunStretch = 65536;
 struct RunRows {
     int4 mark[kRunArcs / 4];
     int32_t wave_max[kRunThreads / kWave];
@@ -69,6 +75,19 @@ __device__ __forceinline__ const int32_t* run_rows(const int32_t* __restrict__ V
     for (int i = t; i < kRunArcs / 4; i += kRunThreads) sh.mark[i] = int4{0, 0, 0, 0};
     __syncthreads();
     const int32_t first = sh.ends[0], last = sh.ends[1];
+    if (last - first > kRunStretch) {  // (uniform)
+        for (int32_t i = t; i < cnt; i += kRunThreads) {
+            int32_t lo = first, hi = last + 1;  // V[lo] <= q0 + i, and it is below V[hi] or hi is past the last
+            while (hi - lo > 1) {
+                const int32_t mid = lo + (hi - lo) / 2;
+                if (V[mid] <= q0 + i) lo = mid;
+                else hi = mid;
+            }
+            mark[i] = lo;
+        }
+        __syncthreads();
+        return mark;
+    }
     // a row's first arc gets the row; of the rows that share it (all but the last have no arcs) the last wins
     for (int32_t r = first + 1 + t; r <= last; r += kRunThreads) atomicMax(&mark[V[r] - q0], r);
     if (t == 0) atomicMax(&mark[0], first);
@@ -167,7 +186,10 @@ __device__ __forceinline__ double arc_weight(const int32_t* __restrict__ E, cons
 
 // Out-weight and valid out-arc count of every row.  The sum is the one of
 // adding the row's weights one after the other in CSR order (pagerank.cu:308-315),
-// bit for bit.  A workgroup takes the rows that begin in its kOutTile arcs:
+// bit for bit.  A workgroup takes the rows whose merge-path diagonal (the arcs
+// and the rows before them) begins in its kOutTile, so that rows without arcs
+// are shared out too (by arcs alone, one workgroup took all that follow each
+// other: a build of 16 weighted arcs and 16M nodes 37 ms, now 0.8):
 // their arcs come in whole lines into LDS, where each row has a thread that
 // adds them (8 lanes per row that loaded their own arcs and passed them on
 // by shuffles: 190 us for 9.3M arcs; one thread walking a row in memory paid a
@@ -191,14 +213,14 @@ struct OutLong {
     int32_t c[4], low[4];
 };
 
-// First row whose offset is at least q (V[n] >= q), by one wavefront.
+// First row whose diagonal V[r] + r is at least q, n if none is, by one wavefront.
 __device__ __forceinline__ int32_t wave_first_row(const int32_t* __restrict__ V, int32_t n, int64_t q) {
-    int32_t lo = 0, hi = n;  // V[hi] >= q
+    int32_t lo = 0, hi = n;
     while (lo < hi) {
         const int64_t step = ((int64_t)hi - lo + kWave - 1) / kWave;
         const int64_t at = (int64_t)lo + (lane_id() + 1) * step - 1;
-        const bool below = at < hi && (int64_t)V[at] < q;
-        const int k = __popcll(__ballot(below));  // offsets ascend: a prefix of the lanes
+        const bool below = at < hi && V[at] + at < q;
+        const int k = __popcll(__ballot(below));  // diagonals ascend: a prefix of the lanes
         const int64_t nlo = (int64_t)lo + k * step, nhi = nlo + step - 1;
         lo = (int32_t)min(nlo, (int64_t)hi);
         hi = (int32_t)min(nhi, (int64_t)hi);
@@ -208,24 +230,24 @@ __device__ __forceinline__ int32_t wave_first_row(const int32_t* __restrict__ V,
 
 template <bool HasW>
 __device__ __forceinline__ void row_out_tile(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
-                                             const double* __restrict__ W, int32_t n, int64_t tile, bool last,
+                                             const double* __restrict__ W, int32_t n, int64_t tile,
                                              double* __restrict__ out_w, int32_t* __restrict__ outcnt, OutTile& sh) {
     const int t = threadIdx.x;
-    const int64_t q0 = tile * kOutTile;
     if (t == 0) sh.bad = 0;
     if (wave_id() < 2) {
-        const int32_t r = (wave_id() == 1 && last) ? n : wave_first_row(V, n, q0 + wave_id() * kOutTile);
+        const int32_t r = wave_first_row(V, n, (tile + wave_id()) * kOutTile);
         if (lane_id() == 0) sh.rows[wave_id()] = r;
     }
     __syncthreads();
     const int32_t r0 = sh.rows[0], r1 = sh.rows[1];
     if (r0 >= r1) return;  // (uniform)
-    // the arcs of these rows, but no further than the longest row that ends here could reach
-    const int64_t a0 = V[r0], a1 = min((int64_t)V[r1], q0 + kOutTile + kOutLong);
+    // the arcs of these rows, but no further than a short row that begins here
+    // could reach: every row begins less than kOutTile arcs after the first
+    const int64_t a0 = V[r0], a1 = min((int64_t)V[r1], a0 + kOutTile + kOutLong);
     for (int64_t p = a0 + t; p < a1; p += kOutThreads) {
         int32_t ok = 0;
         const double w = arc_weight<HasW>(E, W, p, n, ok);
-        sh.w[p - q0] = w;
+        sh.w[p - a0] = w;
         if (!ok) sh.bad = 1;
     }
     __syncthreads();
@@ -243,7 +265,7 @@ __device__ __forceinline__ void row_out_tile(const int32_t* __restrict__ V, cons
         }
         double s = 0.0;
         if (HasW) {
-            const double* w = sh.w + (beg - q0);
+            const double* w = sh.w + (beg - a0);
             for (int32_t k = 0; k < len; ++k) s += w[k];
         }
         out_w[r] = HasW ? s : (double)c;
@@ -331,7 +353,7 @@ __device__ __forceinline__ void row_out_long(const int32_t* __restrict__ V, cons
 // Workgroups [0, long_blocks) take the listed rows, the others a tile each.
 template <bool HasW>
 __global__ __launch_bounds__(kOutThreads) void k_row_out(const int32_t* __restrict__ V, const int32_t* __restrict__ E,
-                                                         const double* __restrict__ W, int32_t n, uint32_t tiles,
+                                                         const double* __restrict__ W, int32_t n,
                                                          double* __restrict__ out_w, int32_t* __restrict__ outcnt,
                                                          const int32_t* __restrict__ long_rows,
                                                          const uint32_t* __restrict__ n_long, uint32_t long_blocks) {
@@ -342,8 +364,7 @@ __global__ __launch_bounds__(kOutThreads) void k_row_out(const int32_t* __restri
     if (blockIdx.x < long_blocks) {
         row_out_long<HasW>(V, E, W, n, blockIdx.x, long_blocks, out_w, outcnt, long_rows, *n_long, sh.row);
     } else {
-        const uint32_t tile = blockIdx.x - long_blocks;
-        row_out_tile<HasW>(V, E, W, n, tile, tile + 1 == tiles, out_w, outcnt, sh.tile);
+        row_out_tile<HasW>(V, E, W, n, blockIdx.x - long_blocks, out_w, outcnt, sh.tile);
     }
 }
 
@@ -1377,12 +1398,11 @@ int build_from_device_csr(Graph& g, const int32_t* dV, const int32_t* dE, const 
             k_long_rows<<<nblocks(n, 256), 256, 0, s>>>(dV, n, lr, nl);
             EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         }
-        const unsigned tiles = nblocks(std::max<int64_t>(m, 1), kOutTile);
+        const unsigned tiles = nblocks(m + n, kOutTile);
         if (sum_weights)
-            k_row_out<true><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, dW, n, tiles, out_w, outcnt_p, lr, nl, lb);
+            k_row_out<true><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, dW, n, out_w, outcnt_p, lr, nl, lb);
         else
-            k_row_out<false><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, nullptr, n, tiles, out_w, outcnt_p, lr, nl,
-                                                                lb);
+            k_row_out<false><<<lb + tiles, kOutThreads, 0, s>>>(dV, dE, nullptr, n, out_w, outcnt_p, lr, nl, lb);
         EGX_CHECK_LAUNCH(EGX_DEVICE_ERR);
         if (g.adjacency) {
             k_unit_out_w<<<nblocks(n, 256), 256, 0, s>>>(out_w, n);
