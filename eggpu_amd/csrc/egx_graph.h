@@ -333,11 +333,15 @@ struct SolveBufs {
     double* red_part;
 };
 // Bytes a solve of graph g in this precision needs for its SolveBufs when
-// they are carved from one region with carve_solve_bufs (256-byte aligned).
+// they are carved from one region with carve_solve_bufs (256-byte aligned):
+// the per-workgroup partial sums, and all else.
+int64_t solve_partial_bytes(const Graph& g);
 int64_t solve_scratch_bytes(const Graph& g, int32_t precision);
 // Carves the SolveBufs of graph g out of base (at least
-// solve_scratch_bytes(g, precision) bytes, 256-byte aligned).
-void carve_solve_bufs(const Graph& g, int32_t precision, char* base, SolveBufs& b);
+// solve_scratch_bytes(g, precision) bytes, 256-byte aligned) and of partials
+// (solve_partial_bytes(g), 8-byte aligned), or out of base alone, which then
+// holds both, when partials is null.
+void carve_solve_bufs(const Graph& g, int32_t precision, char* base, double* partials, SolveBufs& b);
 struct SolveStats {
     double kernel_seconds = 0.0;  // first to last iteration launch
     double spmv_seconds = 0.0;    // sum of k_pr_spmv launch durations

@@ -6,7 +6,9 @@
 // The per-solve workspace that egx_graph_pagerank allocates on a graph's
 // first solve (two iterate and two contribution buffers, the device state,
 // per-block and reduce partial sums) comes from `scratch`, a static device
-// array; the normalised result goes to the caller's device buffer.  The
+// array; the normalised result goes to the caller's device buffer, which
+// holds the partial sums until then where the array has no room for them
+// (they grow with the tiles: graphs of 4.17M nodes and 16 arcs each).  The
 // graph's own layout buffers (built with the graph) are used as in
 // egx_graph_pagerank, and its pinned state slot exists from creation on.
 #include <mutex>
@@ -17,7 +19,7 @@ namespace egx {
 namespace {
 
 // 64 MiB per device: FP32 solves of graphs up to about 4M nodes, FP64 up to
-// about 2M (solve_scratch_bytes gives the exact need).  Every GPU the
+// about 2M (solve_scratch_bytes and solve_partial_bytes give the exact need).  Every GPU the
 // library runs on holds its own copy until the process ends.
 constexpr int64_t kNoAllocScratchBytes = (int64_t)64 << 20;
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
@@ -83,7 +85,10 @@ extern "C" int egx_graph_pagerank_noalloc(egx_graph* gh, const egx_solve_opts* o
         egx::set_last_error("egx_graph_pagerank_noalloc: PR_device is NULL");
         return EGX_UNSUPPORTED_GRAPH;
     }
-    const int64_t need = egx::solve_scratch_bytes(g, opts->precision);
+    const int64_t partial = egx::solve_partial_bytes(g);
+    int64_t need = egx::solve_scratch_bytes(g, opts->precision) + partial;
+    const bool lent = need > egx::kNoAllocScratchBytes && partial <= (int64_t)g.n * 8;
+    if (lent) need -= partial;
     if (need > egx::kNoAllocScratchBytes) {
         egx::set_last_error("egx_graph_pagerank_noalloc: this graph needs " + std::to_string(need) +
                             " bytes of per-solve scratch; the allocation-free entry point holds " +
@@ -99,7 +104,7 @@ extern "C" int egx_graph_pagerank_noalloc(egx_graph* gh, const egx_solve_opts* o
     char* base = nullptr;
     EGX_TRY(egx::scratch_of_current_device(g.device, &base));
     egx::SolveBufs bufs{};
-    egx::carve_solve_bufs(g, opts->precision, base, bufs);
+    egx::carve_solve_bufs(g, opts->precision, base, lent ? PR_device : nullptr, bufs);
     egx::SolveParams p;
     p.alpha = opts->alpha;
     p.max_iter = opts->max_iter;

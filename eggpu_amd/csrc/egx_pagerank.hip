@@ -2045,14 +2045,15 @@ int64_t solve_grid(const Graph& g) {
 
 }  // namespace
 
+int64_t solve_partial_bytes(const Graph& g) { return align_up(partial_slots(solve_grid(g)) * 3 * 8); }
+
 int64_t solve_scratch_bytes(const Graph& g, int32_t precision) {
     const int64_t elem = precision == EGX_PRECISION_FP64 ? 8 : 4;
     const int64_t vec = align_up((int64_t)std::max(g.n, 1) * elem);
-    return 4 * vec + align_up(2 * (int64_t)sizeof(PrState)) + align_up(partial_slots(solve_grid(g)) * 3 * 8) +
-           align_up((int64_t)kMaxRed * 3 * 8);
+    return 4 * vec + align_up(2 * (int64_t)sizeof(PrState)) + align_up((int64_t)kMaxRed * 3 * 8);
 }
 
-void carve_solve_bufs(const Graph& g, int32_t precision, char* base, SolveBufs& b) {
+void carve_solve_bufs(const Graph& g, int32_t precision, char* base, double* partials, SolveBufs& b) {
     const int64_t elem = precision == EGX_PRECISION_FP64 ? 8 : 4;
     const int64_t vec = align_up((int64_t)std::max(g.n, 1) * elem);
     char* p = base;
@@ -2064,9 +2065,9 @@ void carve_solve_bufs(const Graph& g, int32_t precision, char* base, SolveBufs& 
     }
     b.state = reinterpret_cast<PrState*>(p);
     p += align_up(2 * (int64_t)sizeof(PrState));
-    b.partials = reinterpret_cast<double*>(p);
-    p += align_up(partial_slots(solve_grid(g)) * 3 * 8);
     b.red_part = reinterpret_cast<double*>(p);
+    p += align_up((int64_t)kMaxRed * 3 * 8);
+    b.partials = partials ? partials : reinterpret_cast<double*>(p);
 }
 
 

@@ -231,7 +231,8 @@ int egx_graph_pagerank(egx_graph *g, const egx_solve_opts *opts, double *PR, int
  * egx_last_error.  opts as egx_graph_pagerank (check_every as there; no
  * per-launch timing, no graph replay).  PR_device: caller-owned device memory
  * on the graph's device, n doubles, written with the normalised ranks in
- * caller node order (the values egx_graph_pagerank returns, bit for bit).
+ * caller node order (the values egx_graph_pagerank returns, bit for bit); it
+ * may hold partial sums meanwhile.
  * iterations may be NULL.  Every call on one GPU shares that GPU's array:
  * calls that overlap on one GPU race, as do overlapping calls on one graph
  * through any entry point. */
