@@ -30,7 +30,7 @@
 // gather.
 //
 // A launch of one graph's solve knows its parity from its own number, which
-// a captured run of an even number of iterations repeats on every replay.
+// a captured run repeats on every replay.
 // Many graphs -- each stopping on its own, their buffers chosen on the device
 // by their iteration counters -- can share one launch through a table of per-graph arguments (k_pr_spmv_multi /
 // k_pr_reduce_multi run the same block code as the one-graph kernels, so a
@@ -1578,8 +1578,8 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
     const int32_t max_launch = p.max_iter + (p.eig_delta ? 1 : 0);
     LaunchTimer timer;
     if (p.time_each_launch) EGX_TRY(timer.reserve((size_t)4 * max_launch));
-    CapturedRun cap;
-    cap.stream = s;
+    CapturedRun caps[2];  // by the parity of their first iteration
+    caps[0].stream = caps[1].stream = s;
     HostState* hs = static_cast<HostState*>(g.host_state);
     // a solve that fails on the way leaves nothing queued that would write its progress into the next one's
     struct Drain {
@@ -1595,16 +1595,17 @@ int solve_typed(Graph& g, const SolveParams& p, double* host_out, SolveStats* st
     // iterations queued past the last one whose start the device has
     // reported: enough to keep it busy, few to run empty after the stop
     const int32_t ahead = p.check_every > 0 ? p.check_every : kAhead;
-    // a replayed run repeats its iterations' parities: even lengths only
-    const bool replay = p.use_graph && !p.time_each_launch && can_stop_early && p.check_every > 0 &&
-                        p.check_every % 2 == 0;
+    const bool replay = p.use_graph && !p.time_each_launch && can_stop_early && p.check_every > 0;
     while (launched < max_launch) {
         if (replay && max_launch - launched >= p.check_every) {
-            // replay one captured chunk of `check_every` iterations
+            // replay one captured chunk of `check_every` iterations; it
+            // repeats its iterations' parities, so odd lengths take two in turn
+            const int32_t odd = launched & 1;
+            CapturedRun& cap = caps[odd];
             if (!cap.exec) {
                 EGX_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), EGX_DEVICE_ERR);
                 for (int32_t q = 0; q < p.check_every; ++q) {
-                    set_iteration(q);
+                    set_iteration(odd + q);
                     launch_spmv();
                     launch_reduce();
                 }
