@@ -1129,6 +1129,7 @@ struct Batch {
     // far more than a replay.  The kernel arguments depend only on the width
     // and the X buffers (the buffer parity lives on the device).
     bool use_graph = true;
+    int32_t fail_after = -1;  // test hook: steps of more iterations fail once these are queued
     struct StepGraph {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
@@ -1222,6 +1223,7 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
     EGX_HIP_TRY(hipHostMalloc((void**)&b->pinned, kHostBatch + kArenaBytes), EGX_FAILED_TO_ALLOCATE_HOST_MEM);
     b->arena = reinterpret_cast<char*>(b->pinned) + kHostBatch;
     if (const char* e = std::getenv("EGGPU_AMD_BATCH_GRAPHS")) b->use_graph = std::strcmp(e, "0") != 0;
+    if (const char* e = std::getenv("EGGPU_AMD_TEST_FAIL_STEP")) b->fail_after = std::atoi(e);
     if (g.reordered) {
         b->rank_h.resize((size_t)n);
         EGX_TRY(download(g.rank.p, b->rank_h.data(), n, s));  // (a pageable copy: 0.5 ms of 240,000 ranks)
@@ -1629,14 +1631,18 @@ int batch_step(Batch& b, int32_t iters, bool record_time) {
             sg.x1 = b.X[1].p;
         }
         if (record_time) EGX_HIP_TRY(hipEventRecord(b.ev0, s), EGX_DEVICE_ERR);
+        b.published = false;  // until all of the step is queued
         EGX_HIP_TRY(hipGraphLaunch(sg.exec, s), EGX_DEVICE_ERR);
         b.published = true;
         if (record_time) EGX_HIP_TRY(hipEventRecord(b.ev1, s), EGX_DEVICE_ERR);
         return EGX_SUCC;
     }
     if (record_time) EGX_HIP_TRY(hipEventRecord(b.ev0, s), EGX_DEVICE_ERR);
-    EGX_TRY(enqueue_iterations(b, a, iters, s));
-    if (iters > 0) b.published = true;
+    if (iters > 0) {
+        b.published = false;  // until all of the step is queued: its first launches change the states
+        EGX_TRY(enqueue_iterations(b, a, iters, s));
+        b.published = true;
+    }
     if (record_time) EGX_HIP_TRY(hipEventRecord(b.ev1, s), EGX_DEVICE_ERR);
     return EGX_SUCC;
 }
@@ -1644,6 +1650,10 @@ int batch_step(Batch& b, int32_t iters, bool record_time) {
 // `iters` iterations (rows + reduce launches) at the batch's current width.
 int enqueue_iterations(Batch& b, SpmmArgs a, int32_t iters, hipStream_t s) {
     for (int32_t i = 0; i < iters; ++i) {
+        if (i == b.fail_after) {
+            set_last_error("batch step: failed as EGGPU_AMD_TEST_FAIL_STEP asks");
+            return EGX_DEVICE_ERR;
+        }
         if (i + 1 == iters) a.publish = b.pinned;
         if (b.grid > 0) {
             switch (b.width) {
