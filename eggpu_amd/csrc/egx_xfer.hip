@@ -39,6 +39,11 @@ constexpr size_t kInlineBytes = (size_t)256 << 10;
 constexpr size_t kUploadSmall = (size_t)2 << 20;
 constexpr int kMaxChunks = 24;    // pinned chunks the process keeps, at most
 constexpr int kCallChunks = 12;   // of them for one transfer
+constexpr int kAheadChunks = 2;   // of them for one that still waits for its values
+// A transfer down of several parts begins with one of this size: it tells the
+// waiting thread that the values are there, to queue the other parts and to wake the helpers
+// while the second part crosses.
+constexpr size_t kFirstBytes = (size_t)64 << 10;
 constexpr int kThreads = 8;       // the calling thread among them
 
 struct Chunk {
@@ -366,11 +371,11 @@ size_t largest(const std::vector<Part>& parts) {
     return most;
 }
 
-// Chunks for `parts` parts of at most `bytes`; -1 when there are none to be had.
-int begin_run(Run& r, size_t parts, size_t bytes, hipStream_t s) {
+// Chunks for `parts` parts of at most `bytes`, at most `most` of them; -1 when there are none to be had.
+int begin_run(Run& r, size_t parts, size_t bytes, hipStream_t s, int most = kCallChunks) {
     r.s = s;
     if (hipGetDevice(&r.dev) != hipSuccess) return -1;
-    r.chunks = take_chunks((int)std::min<size_t>(parts, kCallChunks), bytes, r.dev, s);
+    r.chunks = take_chunks((int)std::min<size_t>(parts, (size_t)most), bytes, r.dev, s);
     if (r.chunks.empty()) return -1;
     r.stage.reset(new std::atomic<int>[std::max<size_t>(parts, 1)]);
     for (size_t i = 0; i < parts; ++i) r.stage[i].store(0);
@@ -416,16 +421,19 @@ int upload_chunked(const std::vector<Upload>& jobs, size_t total_bytes, hipStrea
 int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_t s) {
     Run r;
     const size_t step = part_bytes(total_bytes);
+    size_t room = step;  // of the part being filled
     for (const Fetch& f : jobs) {
         const size_t elem = f.packed ? 4 : 8;
         char* dev = static_cast<char*>(const_cast<void*>(f.dev));
         for (int64_t i = 0; i < f.n;) {
             char* at = dev + (size_t)i * elem;
             if (r.parts.empty() || r.pieces.back().f->packed != f.packed ||
-                r.parts.back().dev + r.parts.back().bytes != at || r.parts.back().bytes + elem > step)
+                r.parts.back().dev + r.parts.back().bytes != at || r.parts.back().bytes + elem > room) {
+                room = r.parts.empty() && total_bytes > kInlineBytes ? kFirstBytes : step;
                 r.parts.push_back(Part{nullptr, at, 0, r.pieces.size(), 0});
+            }
             Part& p = r.parts.back();
-            const int64_t k = std::min((int64_t)((step - p.bytes) / elem), f.n - i);
+            const int64_t k = std::min((int64_t)((room - p.bytes) / elem), f.n - i);
             r.pieces.push_back(Piece{&f, i, k, p.bytes});
             p.bytes += (size_t)k * elem;
             p.pieces += 1;
@@ -433,8 +441,19 @@ int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_
         }
     }
     if (r.parts.empty()) return EGX_SUCC;
-    const std::function<void()> work = [&] { r.fetch_parts(); };
-    if (begin_run(r, r.parts.size(), largest(r.parts), s) != 0) {
+    size_t queued = 0;  // of the ring's first round
+    const std::thread::id caller = std::this_thread::get_id();
+    const std::function<void()> work = [&] {
+        if (std::this_thread::get_id() == caller)  // while the helpers wake
+            for (; queued < r.chunks.size(); ++queued) r.queue_fetch((int64_t)queued);
+        r.fetch_parts();
+    };
+    // The values may be behind a whole solve: until the first part lands the
+    // call holds kAheadChunks chunks, and one thread waits.  (With all of them
+    // and the helpers from the start, a solve of 4.2M nodes and 300 iterations
+    // kept 8.0 cores spinning, and half of the process's chunks from others.)
+    const size_t part = largest(r.parts);
+    if (begin_run(r, r.parts.size(), part, s, kAheadChunks) != 0) {
         // no pinned memory: through a pageable buffer
         std::vector<char> buf(kChunkBytes);
         for (const Part& p : r.parts) {
@@ -443,9 +462,15 @@ int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_
         }
         return EGX_SUCC;
     }
-    for (size_t k = 0; k < std::min(r.parts.size(), r.chunks.size()); ++k) r.queue_fetch((int64_t)k);
-    if (total_bytes <= kInlineBytes) work();
-    else run_together(work, (int)std::min<size_t>(r.parts.size(), kThreads) - 1);
+    for (; queued < r.chunks.size(); ++queued) r.queue_fetch((int64_t)queued);
+    if (r.parts.size() == 1) {
+        work();
+    } else if (r.landed(r.chunks[0])) {
+        const size_t all = std::min<size_t>(r.parts.size(), kCallChunks);
+        if (all > queued)
+            for (const Chunk& c : take_chunks((int)(all - queued), part, r.dev, s)) r.chunks.push_back(c);
+        run_together(work, (int)std::min<size_t>(r.parts.size(), kThreads) - 1);
+    }
     return finish_run(r);
 }
 
