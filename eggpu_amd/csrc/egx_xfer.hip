@@ -273,8 +273,18 @@ struct Part {
 };
 
 // The transfer's parts, taken in order by several threads; part k uses
-// chunk k % chunks, after part k - chunks is through with it.
+// chunk k % chunks, after part k - chunks is through with it.  Chunks that it
+// still holds when it ends (finish_run has given them back, unless something
+// failed on the way) go back once its stream is through with them.
 struct Run {
+    Run() = default;
+    Run(const Run&) = delete;
+    Run& operator=(const Run&) = delete;
+    ~Run() {
+        if (chunks.empty()) return;
+        (void)hipStreamSynchronize(s);
+        give_chunks(chunks);
+    }
     std::vector<Part> parts;
     std::vector<Piece> pieces;
     std::vector<Chunk> chunks;
@@ -357,6 +367,7 @@ int finish_run(Run& r) {
     // no copy may still use a chunk when another caller gets it
     const hipError_t e = hipStreamSynchronize(r.s);
     give_chunks(r.chunks);
+    r.chunks.clear();
     const hipError_t first = (hipError_t)r.err.load();
     if (first != hipSuccess || e != hipSuccess) {
         set_last_error(std::string("host transfer: ") + hipGetErrorString(first != hipSuccess ? first : e));
@@ -371,15 +382,20 @@ size_t largest(const std::vector<Part>& parts) {
     return most;
 }
 
+// Up to `want` chunks that hold `bytes` for the run, kCallChunks with those it has.
+void add_chunks(Run& r, size_t want, size_t bytes) {
+    for (const Chunk& c : take_chunks((int)want, bytes, r.dev, r.s)) r.chunks.push_back(c);  // begin_run has reserved them
+}
+
 // Chunks for `parts` parts of at most `bytes`, at most `most` of them; -1 when there are none to be had.
 int begin_run(Run& r, size_t parts, size_t bytes, hipStream_t s, int most = kCallChunks) {
     r.s = s;
     if (hipGetDevice(&r.dev) != hipSuccess) return -1;
-    r.chunks = take_chunks((int)std::min<size_t>(parts, (size_t)most), bytes, r.dev, s);
-    if (r.chunks.empty()) return -1;
     r.stage.reset(new std::atomic<int>[std::max<size_t>(parts, 1)]);
     for (size_t i = 0; i < parts; ++i) r.stage[i].store(0);
-    return 0;
+    r.chunks.reserve(kCallChunks);
+    add_chunks(r, std::min<size_t>(parts, (size_t)most), bytes);
+    return r.chunks.empty() ? -1 : 0;
 }
 
 int upload_plain(const std::vector<Upload>& jobs, hipStream_t s) {
@@ -467,8 +483,7 @@ int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_
         work();
     } else if (r.landed(r.chunks[0])) {
         const size_t all = std::min<size_t>(r.parts.size(), kCallChunks);
-        if (all > queued)
-            for (const Chunk& c : take_chunks((int)(all - queued), part, r.dev, s)) r.chunks.push_back(c);
+        if (all > queued) add_chunks(r, all - queued, part);
         run_together(work, (int)std::min<size_t>(r.parts.size(), kThreads) - 1);
     }
     return finish_run(r);
