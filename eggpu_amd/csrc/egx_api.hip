@@ -785,6 +785,8 @@ void egx_pagerank_cache_reset(void) {
     egx::g_hits = egx::g_misses = egx::g_builds = egx::g_refreshes = egx::g_evictions = 0;
 }
 
+void egx_device_trim(void) { egx::pool_trim(); }
+
 int egx_pagerank_cache_stats(egx_cache_stats* out) {
     if (!out) return EGX_UNSUPPORTED_GRAPH;
     out->hits = egx::g_hits.load();

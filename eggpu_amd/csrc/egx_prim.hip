@@ -25,8 +25,8 @@ namespace {
 // behind it; once the stream is known to be idle the tag is dropped and any
 // stream may have it.  The allocator itself never waits.  At most kPoolBytes
 // (and kPoolBlocks blocks) stay idle per process (the oldest blocks are freed first, a larger block
-// at once); a failed hipMalloc gives all of them back and tries again, and so
-// does egx_pagerank_cache_reset.
+// at once); a failed hipMalloc gives all of them back and tries again, and
+// egx_device_trim and egx_pagerank_cache_reset give them back.
 constexpr size_t kPoolBytes = (size_t)4 << 30;
 constexpr size_t kPoolBlocks = 4096;
 

@@ -133,7 +133,13 @@ std::vector<Chunk> take_chunks(int want, size_t bytes, int dev, hipStream_t s) {
             (void)hipGetLastError();
             break;
         }
-        if (hipMalloc(reinterpret_cast<void**>(&c.count), 64) != hipSuccess) {
+        hipError_t e = hipMalloc(reinterpret_cast<void**>(&c.count), 64);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            pool_trim();  // idle blocks may be what is missing
+            e = hipMalloc(reinterpret_cast<void**>(&c.count), 64);
+        }
+        if (e != hipSuccess) {
             (void)hipGetLastError();
             (void)hipHostFree(c.p);
             break;

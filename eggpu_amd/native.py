@@ -189,6 +189,7 @@ SIGNATURES = {
     "egx_pagerank": (ctypes.c_int, [_i32p, _i32p, _f64p, ctypes.c_int32, ctypes.c_int32, ctypes.c_double,
                                     ctypes.c_int32, ctypes.c_double, ctypes.c_uint64, _f64p, _i32p, _f64p]),
     "egx_pagerank_cache_reset": (None, []),
+    "egx_device_trim": (None, []),
     "egx_pagerank_cache_stats": (ctypes.c_int, [ctypes.POINTER(CacheStats)]),
     "egx_graph_from_csr": (ctypes.c_int, [_i32p, _i32p, _f64p, ctypes.c_int32, ctypes.c_int32, ctypes.c_double,
                                           ctypes.c_int32, ctypes.POINTER(_vp)]),
@@ -733,6 +734,12 @@ def cache_stats():
 
 def cache_reset():
     lib().egx_pagerank_cache_reset()
+
+
+def device_trim():
+    """Give device memory that closed graphs and batches left with the process
+    (at most 4 GiB, kept for the next ones) back to the devices."""
+    lib().egx_device_trim()
 
 
 def cpp_gpu_pagerank_dense(graph, alpha=0.85, max_iterator=200, threshold=1e-6, weight=None):

@@ -87,6 +87,13 @@ typedef struct {
 void egx_pagerank_cache_reset(void);
 int egx_pagerank_cache_stats(egx_cache_stats *out);
 
+/* Device memory that freed graphs, closed batches and finished calls leave is
+ * kept for the next ones: at most 4 GiB per process, which other allocators
+ * of the process do not see as free.  egx_device_trim gives the idle part
+ * back to the devices; egx_pagerank_cache_reset does so too, and a failed
+ * allocation of this library does before it reports the failure. */
+void egx_device_trim(void);
+
 /* ------------------------------------------------------------------------ */
 /* Device-resident graphs.  No counterpart in the reference, which keeps one  */
 /* thread-local workspace (pagerank.cu:44-132); these give the serving pool,  */
@@ -277,6 +284,7 @@ int egx_graph_ppr_single(egx_graph *g, const int32_t *seeds, int32_t nseeds, con
 int egx_multi_pagerank(egx_graph *const *graphs, int32_t count, const egx_solve_opts *opts,
                        double *const *PR, int32_t *iterations, egx_solve_stats *stats, int32_t flags);
 
+/* The graph's device memory may stay with the process (egx_device_trim). */
 void egx_graph_free(egx_graph *g);
 
 /* ------------------------------------------------------------------------ */
