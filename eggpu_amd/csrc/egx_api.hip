@@ -477,7 +477,7 @@ int egx_graph_info_get(const egx_graph* gh, egx_graph_info* out) {
     out->thread_row_max = g.bins.thread_row_max;
     out->wave_row_max = g.bins.wave_row_max;
     out->hub_segment = g.bins.hub_segment;
-    out->tile_items = g.bins.tile_items;
+    out->tile_items = g.tile_items;
     out->hub_rows_first = g.n_hub;
     out->tile_sort = g.tsorted ? 1 : 0;
     out->hot_sources = g.bins.hot_sources;
@@ -510,7 +510,7 @@ int egx_graph_set_bins(egx_graph* gh, const egx_bin_opts* opts) {
         egx::set_last_error("cannot re-bin a graph while batch sessions are open on it");
         return EGX_UNSUPPORTED_GRAPH;
     }
-    if (opts->tile_items > 0) cfg.tile_items = opts->tile_items;
+    if (opts->tile_items > 0 || opts->tile_items == EGX_TILE_ITEMS_AUTO) cfg.tile_items = opts->tile_items;
     if (opts->reorder >= 0) cfg.reorder = opts->reorder ? 1 : 0;
     if (opts->tile_sort >= 0) cfg.tile_sort = opts->tile_sort ? 1 : 0;
     if (opts->hot_sources != 0) cfg.hot_sources = opts->hot_sources > 0 ? opts->hot_sources : 0;

@@ -1238,7 +1238,7 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
     return EGX_SUCC;
 }
 
-// Items per tile: what the caller set, or at the default a size for the
+// Items per tile: what the caller set, or (EGX_TILE_ITEMS_AUTO) a size for the
 // graph.  Large tiles leave a small graph's device idle, small ones pay more
 // for their barriers than for their arcs.  Measured (us per SpMV launch at
 // tiles of 512 / 1024 / 2048 / 4096 / 5888 items, FP32): 244K items 10.4 /
@@ -1247,8 +1247,9 @@ int build_blocked(Graph& g, const BinCfg& cfg, bool layout_changed) {
 // FP64 alike (34M: 206 / 192 / 220 at 2048 / 4096 / 5888).  A graph of a few thousand
 // items is cut into up to 64 tiles of at least 256 (7.5K items: 8.1 us at 256, 11.7 at 5888).
 int32_t tile_size(const BinCfg& cfg, int64_t items) {
-    if (cfg.tile_items != BinCfg{}.tile_items) return cfg.tile_items;
-    const int64_t fill = std::min<int64_t>(4096, std::max<int64_t>(1024, items / 2048));
+    if (cfg.tile_items != EGX_TILE_ITEMS_AUTO) return cfg.tile_items;
+    const int64_t most = std::min(4096, kTileLds - cfg.wave_row_max);
+    const int64_t fill = std::min(most, std::max<int64_t>(1024, items / 2048));
     return (int32_t)std::min(fill, std::max<int64_t>(256, items / 64));
 }
 
@@ -1256,8 +1257,8 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in, const uint32_t* counters) {
     BinCfg cfg = cfg_in;
     if (cfg.thread_row_max < 0) cfg.thread_row_max = 0;
     cfg.wave_row_max = hub_threshold(cfg);
-    if (cfg.tile_items < 256) cfg.tile_items = 256;
-    if (cfg.tile_items > kTileLds - cfg.wave_row_max) cfg.tile_items = kTileLds - cfg.wave_row_max;
+    if (cfg.tile_items != EGX_TILE_ITEMS_AUTO)
+        cfg.tile_items = std::min(std::max(cfg.tile_items, 256), kTileLds - cfg.wave_row_max);
     cfg.hub_segment = hub_segment(cfg);
     if (cfg.reorder != 0) cfg.reorder = 1;
     if (cfg.tile_sort != 0) cfg.tile_sort = 1;
@@ -1307,6 +1308,7 @@ int rebuild_bins(Graph& g, const BinCfg& cfg_in, const uint32_t* counters) {
     // merge-path tiles over rows [n_hub, n)
     const int64_t items = (g.m - (int64_t)hctr[kCtrHubArcs]) + (int64_t)(n - g.n_hub);
     const int32_t per_tile = tile_size(cfg, items);
+    g.tile_items = per_tile;
     g.n_tiles = (items + per_tile - 1) / per_tile;
     g.tile_lds = per_tile + cfg.wave_row_max;
     DevBuf wave_rows;

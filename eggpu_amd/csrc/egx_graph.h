@@ -100,7 +100,7 @@ struct BinCfg {
     int32_t thread_row_max = 12;  // rows of up to kRowLaneFactor times this are reduced by one lane, longer ones by a wavefront
     int32_t wave_row_max = 2048;  // hub threshold: rows with more arcs go to the hub bin
     int32_t hub_segment = 8192;   // arcs per hub segment (one workgroup)
-    int32_t tile_items = 5888;    // rows + arcs per tile (merge-path split)
+    int32_t tile_items = EGX_TILE_ITEMS_AUTO;  // rows + arcs per tile (merge-path split), or a size for the graph
     int32_t reorder = 1;          // relabel by out-degree (hub rows always first)
     int32_t tile_sort = 0;        // gather each tile's arcs in source order (LDS scatter back to row order)
     int32_t hot_sources = 0;      // > 0: sources past this label are gathered non-temporally
@@ -229,6 +229,7 @@ struct Graph {
     int32_t n_hub = 0;            // rows [0, n_hub) of the iteration layout are hub rows
     DevBuf tiles;
     int64_t n_tiles = 0;
+    int32_t tile_items = 0;       // rows + arcs per tile
     int32_t tile_lds = 0;         // LDS entries that a tile may need: its items and one row
     // tile arcs in source order (tile_sort): t_col source, t_pos slot of the
     // arc in its tile's row-order LDS staging, t_val weight (weighted); same

@@ -30,6 +30,7 @@ EGX_NEGATIVE_CYCLE = 6
 
 PRECISION_FP32 = 0
 PRECISION_FP64 = 1
+TILE_ITEMS_AUTO = -(2**31)  # EGX_TILE_ITEMS_AUTO
 SOLVE_TIME_LAUNCHES = 1
 SOLVE_HIP_GRAPH = 2
 SOLVE_XCD_PLACEMENT = 4
@@ -397,7 +398,8 @@ class DeviceGraph:
         tile_sort, blocked and blocked_shared < 0 keep theirs; hot_sources 0
         keeps it, < 0 turns non-temporal cold gathers off).  blocked_shared=1
         sizes the blocked layout's work items for graphs solved together in
-        multi_pagerank; 0 for a graph solved alone."""
+        multi_pagerank; 0 for a graph solved alone.  tile_items
+        TILE_ITEMS_AUTO: a size for the graph, as a new graph has."""
         o = BinOpts(int(thread_row_max), int(wave_row_max), int(hub_segment), int(tile_items), int(reorder),
                     int(tile_sort), int(hot_sources), int(blocked), int(blocked_shared))
         _check(lib().egx_graph_set_bins(self.handle, ctypes.byref(o)))

@@ -106,7 +106,7 @@ typedef struct {
     int32_t weighted;        /* 1 when explicit weights were given */
     int32_t max_in_degree;
     int32_t max_out_degree;
-    int32_t thread_row_max;  /* bin settings in use (egx_bin_opts) */
+    int32_t thread_row_max;  /* bin settings in use (egx_bin_opts), tile_items the size that runs */
     int32_t wave_row_max;
     int32_t hub_segment;
     int32_t tile_items;
@@ -127,10 +127,11 @@ typedef struct {
 
 /* Degree bins of the SpMV.  Rows with in-degree above wave_row_max form the
  * hub bin (cut into hub_segment-arc segments, one workgroup each); the other
- * rows are split into tiles of tile_items rows+arcs (at the default value, of
- * a size for the graph) whose gathered terms are staged in LDS and reduced
- * one lane per row up to 4 * thread_row_max arcs, one wavefront per longer row.
- * tile_items + wave_row_max <= 7936. */
+ * rows are split into tiles of tile_items rows+arcs (EGX_TILE_ITEMS_AUTO, where
+ * a graph starts: of a size for the graph) whose gathered terms are staged in
+ * LDS and reduced one lane per row up to 4 * thread_row_max arcs, one wavefront
+ * per longer row.  tile_items + wave_row_max <= 7936. */
+#define EGX_TILE_ITEMS_AUTO INT32_MIN
 typedef struct {
     int32_t thread_row_max;
     int32_t wave_row_max;
@@ -210,7 +211,8 @@ int egx_graph_er(int32_t n, int64_t nedges, uint64_t seed, int32_t weighted, dou
 
 int egx_graph_info_get(const egx_graph *g, egx_graph_info *out);
 
-/* Re-bin rows for the SpMV kernels (autotuner hook). Fields <= 0 keep the current value. */
+/* Re-bin rows for the SpMV kernels (autotuner hook). Fields <= 0 keep the current value
+ * (tile_items EGX_TILE_ITEMS_AUTO: back to a size for the graph). */
 int egx_graph_set_bins(egx_graph *g, const egx_bin_opts *opts);
 
 /* Pull CSR (the reference's in_row/in_col/in_val/dangling01, pagerank.cu:286-347)
