@@ -84,9 +84,9 @@ struct Session {
 };
 
 int64_t session_bytes(const egx_graph_info& inf) {
-    // two X buffers at the widest layout, teleport slots, output, partials
+    // two X buffers at the widest layout, teleport slots, packed output, partials
     const int64_t n = inf.n;
-    return 2 * n * kSlots * 4 + n * 4 + n * 8 + (int64_t)1024 * kSlots * 4 +
+    return 2 * n * kSlots * 4 + n * 4 + n * 4 + (int64_t)1024 * kSlots * 4 +
            (int64_t)(inf.tiles + inf.hub_segments + 8192) * 3 * kSlots * 8 + ((int64_t)1 << 20);
 }
 

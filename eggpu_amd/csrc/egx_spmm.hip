@@ -1294,7 +1294,7 @@ int batch_open(Graph& g, std::unique_ptr<Batch>& out) {
     const int64_t parts = (items + 31) / 32;
     b->n_red = items <= kOneReduce ? 1u : (uint32_t)std::min<int64_t>(512, parts <= 256 ? parts : 2 * parts);
     EGX_TRY(b->red_part.alloc((size_t)b->n_red * 3 * kCols * 8));
-    EGX_TRY(b->out.alloc(std::max((size_t)n * 8, kPackedHeader + (size_t)n * 4)));  // FP64 or packed result
+    EGX_TRY(b->out.alloc(kPackedHeader + (size_t)n * 4));  // a packed result
     EGX_HIP_TRY(hipStreamSynchronize(s), EGX_DEVICE_ERR);
     out = std::move(b);
     return EGX_SUCC;
