@@ -1047,12 +1047,6 @@ __global__ __launch_bounds__(kRowThreads) void k_spmm_results(const float* __res
     }
 }
 
-__global__ void k_set_tslot(int32_t* __restrict__ tslot, const int32_t* __restrict__ rows,
-                            const int32_t* __restrict__ slots, int32_t count) {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) tslot[rows[i]] = slots[i];
-}
-
 __global__ void k_fill_i32(int32_t* __restrict__ a, int64_t n, int32_t v) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = v;
