@@ -342,8 +342,18 @@ __device__ __forceinline__ void begin_fold(const IterArgs<T>& a, FoldSums f, PrS
 // their arcs before they learnt of it: 5 of 34 us each in a Katz solve of 6
 // iterations of 49 us.)  Only the first launch past the stop gathers in vain.  Graphs
 // of kPrefoldArcs or more that may stop early therefore fold the sums in a
-// launch of their own (k_pr_state, 5 us) before each iteration: R-MAT 24
-// stopping after one iteration 834 us, 796 so.
+// launch of their own (k_pr_state, 3 to 5 us) before each iteration.  That
+// saves one pass and costs a launch per iteration, so it pays up to some ten
+// iterations, where solves of large graphs stop (at a tolerance of 1e-6 after
+// the first: the residual is compared with 1e-6 of the node count).  us of a
+// solve with | without it, stopping after 1, 5 to 7, 9 to 11, 20 and 56 to 60:
+// blocked, R-MAT 24 (263M arcs) 784 | 827, 2764 | 2788, 4730 | 4746, 10090 |
+// 10030, 29710 | 29540; R-MAT 23 (82M) 365 | 391, 1387 | 1391, 2375 | 2364,
+// 4106 | 4028, 12100 | 11860; below the line, R-MAT 22 (65M) 256 | 289, 990 |
+// 998, 1545 | 1541, 2898 | 2841, 8576 | 8381; R-MAT 20 (16M) 113 | 120, 419 |
+// 403, 613 | 582, 1016 | 965, 2801 | 2658.  Pull, R-MAT 21 in FP64 (32M) 338 |
+// 497, 1628 | 1767, 2492 | 2617, 4340 | 4292, 12970 | 12810; below the line,
+// R-MAT 20 in FP32 (16M) 178 | 228, 712 | 742, 1050 | 1078, 1792 | 1748, 4987 | 4916.
 constexpr int64_t kPrefoldArcs = (int64_t)1 << 26, kPrefoldArcsPull = (int64_t)1 << 24;
 template <typename T>
 __device__ __forceinline__ int32_t stop_slot(const IterArgs<T>& a) {

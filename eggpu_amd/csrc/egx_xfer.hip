@@ -8,7 +8,8 @@
 // kThreads threads fill or empty others (PCIe carries 57 GB/s from pinned
 // memory).  Chunks and threads are kept for the process and shared by all
 // callers: a caller takes what is free (it always makes progress alone) and
-// gives it back before it returns.  Transfers down of at most kInlineBytes use one
+// gives it back before it returns; while its values are still behind other work
+// it holds two chunks and waits by itself.  Transfers down of at most kInlineBytes use one
 // chunk and no threads, those up of at most kUploadSmall too.
 #include <sched.h>
 
@@ -48,7 +49,7 @@ constexpr int kThreads = 8;       // the calling thread among them
 
 struct Chunk {
     char* p = nullptr;           // `bytes`, and the flag behind them
-    size_t bytes = 0;            // kChunkBytes, or kInlineBytes (making and pinning 4 MiB takes 6 ms, 256 KiB 0.2)
+    size_t bytes = 0;            // kChunkBytes, or kInlineBytes for those that need no more (making either takes 0.05 ms)
     uint32_t* count = nullptr;   // device: workgroups that have written their share
     hipEvent_t ev = nullptr;     // the chunk's last upload
     int dev = -1;                // of count and ev
