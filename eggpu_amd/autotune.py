@@ -7,8 +7,8 @@ The knobs are those of egx_graph_set_bins:
 * wave_row_max   -- rows with more in-arcs are hub rows (split into
   segments; they also lead the relabelled iteration layout);
 * hub_segment    -- arcs per hub segment (one workgroup each);
-* tile_items     -- rows + arcs per merge-path tile (LDS-staged), or
-  native.TILE_ITEMS_AUTO for the library's choice by the graph's size;
+* tile_items     -- rows + arcs per merge-path tile (LDS-staged); the descent
+  starts from the library's choice by the graph's size;
 * tile_sort      -- gather a tile's arcs in source order (1) or row order (0);
 * hot_sources    -- sources past this relabelled id are gathered with
   non-temporal loads, keeping the hot prefix resident (0: off);
@@ -40,7 +40,7 @@ SPACE = {
     "thread_row_max": [4, 8, 12, 16, 24, 48],
     "wave_row_max": [512, 1024, 2048, 4096],
     "hub_segment": [2048, 4096, 8192, 16384, 32768],
-    "tile_items": [1536, 2944, 4416, 5888, 7424, native.TILE_ITEMS_AUTO],
+    "tile_items": [1536, 2944, 4416, 5888, 7424],
     "tile_sort": [0, 1],
     "hot_sources": [0, 1 << 18, 1 << 19, 1 << 20, 1 << 21],
 }
@@ -81,12 +81,16 @@ def measure(g, cfg, iters=5, precision=native.PRECISION_FP32, repeats=2):
 
 
 def tune(g, precision=native.PRECISION_FP32, iters=5, passes=2, space=None, start=None, log=None):
-    """Coordinate descent from ``start`` (default: DEFAULT).
+    """Coordinate descent from ``start`` (default: DEFAULT, with tiles of the
+    size that the library chooses for the graph).
     Returns (best cfg, seconds per iteration, trials).  Leaves ``g`` binned
     with the best setting."""
     space = space or SPACE
     cur = dict(DEFAULT, **(start or {}))
     cur["blocked"] = 0
+    if "tile_items" not in (start or {}):
+        set_bins(g, dict(cur, tile_items=native.TILE_ITEMS_AUTO))
+        cur["tile_items"] = g.info().get("tile_items", cur["tile_items"])
     trials = []
     seen = {}
 

@@ -33,3 +33,14 @@ def test_tiles_have_the_size_asked_for(gpu_ready, n):
         assert tiles() == min(own, 936)  # what the hub threshold leaves of a tile's LDS
         g.set_bins(wave_row_max=2048)
         assert tiles() == own
+
+
+def test_the_tuner_starts_from_the_graph_s_own_size(gpu_ready):
+    print("tile items, tuner", flush=True)
+    from eggpu_amd import autotune
+
+    with native.DeviceGraph.er(60000, 480000, seed=2) as g:
+        own = g.info()["tile_items"]
+        g.set_bins(tile_items=5888)
+        cfg, _, _ = autotune.tune(g, space={"tile_sort": [0, 1]}, passes=1, iters=2)
+        assert cfg["tile_items"] == own == g.info()["tile_items"]
