@@ -31,9 +31,17 @@ struct Fetch {
     int32_t* words = nullptr;        // (download) packed 4-byte words, copied here as they are
 };
 
+// Whether the values of a fetch, which are behind longer work, are about to
+// land: soon(of), asked again and again while one thread waits.  Without it
+// they are taken to land now.
+struct Due {
+    bool (*soon)(const void* of) = nullptr;
+    const void* of = nullptr;
+};
+
 // All of `jobs`, whose values are written by work queued on s; returns when
 // the callers' arrays hold them.
-int fetch(const std::vector<Fetch>& jobs, hipStream_t s);
+int fetch(const std::vector<Fetch>& jobs, hipStream_t s, const Due& due = Due{});
 
 // 4-byte words at dev, written by work queued on s, to host as they are.
 int download(const void* dev, int32_t* host, int64_t n, hipStream_t s);

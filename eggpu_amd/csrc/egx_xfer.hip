@@ -8,8 +8,8 @@
 // kThreads threads fill or empty others (PCIe carries 57 GB/s from pinned
 // memory).  Chunks and threads are kept for the process and shared by all
 // callers: a caller takes what is free (it always makes progress alone) and
-// gives it back before it returns; while its values are still behind other work
-// it holds two chunks and waits by itself.  Transfers down of at most kInlineBytes use one
+// gives it back before it returns; until its values are due it holds two chunks
+// and waits by itself.  Transfers down of at most kInlineBytes use one
 // chunk and no threads, those up of at most kUploadSmall too.
 #include <sched.h>
 
@@ -40,11 +40,7 @@ constexpr size_t kInlineBytes = (size_t)256 << 10;
 constexpr size_t kUploadSmall = (size_t)2 << 20;
 constexpr int kMaxChunks = 24;    // pinned chunks the process keeps, at most
 constexpr int kCallChunks = 12;   // of them for one transfer
-constexpr int kAheadChunks = 2;   // of them for one that still waits for its values
-// A transfer down of several parts begins with one of this size: it tells the
-// waiting thread that the values are there, to queue the other parts and to wake the helpers
-// while the second part crosses.
-constexpr size_t kFirstBytes = (size_t)64 << 10;
+constexpr int kAheadChunks = 2;   // of them for one whose values are not due yet
 constexpr int kThreads = 8;       // the calling thread among them
 
 struct Chunk {
@@ -326,10 +322,10 @@ struct Run {
         k_fetch_part<<<copy_blocks(p.bytes), kFetchThreads, 0, s>>>(p.dev, c.p, (int64_t)p.bytes, c.count, c.flag());
         if (ok(hipGetLastError())) stage[(size_t)k].store(1, std::memory_order_release);
     }
-    // Waits until the part in chunk c has landed; false when its stream failed.
-    bool landed(const Chunk& c) {
+    // Waits until the part in chunk c has landed, or is about to; false when its stream failed.
+    bool landed(const Chunk& c, const Due& due = Due{}) {
         for (uint32_t spins = 1;; ++spins) {
-            if (__atomic_load_n(c.flag(), __ATOMIC_ACQUIRE) != 0u) return true;
+            if (__atomic_load_n(c.flag(), __ATOMIC_ACQUIRE) != 0u || (due.soon && due.soon(due.of))) return true;
             if (spins % 4096 == 0) {
                 const hipError_t e = hipStreamQuery(s);
                 if (e == hipErrorNotReady) (void)hipGetLastError();  // not an error: clear it
@@ -441,22 +437,19 @@ int upload_chunked(const std::vector<Upload>& jobs, size_t total_bytes, hipStrea
     return finish_run(r);
 }
 
-int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_t s) {
+int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_t s, const Due& due) {
     Run r;
     const size_t step = part_bytes(total_bytes);
-    size_t room = step;  // of the part being filled
     for (const Fetch& f : jobs) {
         const size_t elem = f.packed ? 4 : 8;
         char* dev = static_cast<char*>(const_cast<void*>(f.dev));
         for (int64_t i = 0; i < f.n;) {
             char* at = dev + (size_t)i * elem;
             if (r.parts.empty() || r.pieces.back().f->packed != f.packed ||
-                r.parts.back().dev + r.parts.back().bytes != at || r.parts.back().bytes + elem > room) {
-                room = r.parts.empty() && total_bytes > kInlineBytes ? kFirstBytes : step;
+                r.parts.back().dev + r.parts.back().bytes != at || r.parts.back().bytes + elem > step)
                 r.parts.push_back(Part{nullptr, at, 0, r.pieces.size(), 0});
-            }
             Part& p = r.parts.back();
-            const int64_t k = std::min((int64_t)((room - p.bytes) / elem), f.n - i);
+            const int64_t k = std::min((int64_t)((step - p.bytes) / elem), f.n - i);
             r.pieces.push_back(Piece{&f, i, k, p.bytes});
             p.bytes += (size_t)k * elem;
             p.pieces += 1;
@@ -464,19 +457,13 @@ int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_
         }
     }
     if (r.parts.empty()) return EGX_SUCC;
-    size_t queued = 0;  // of the ring's first round
-    const std::thread::id caller = std::this_thread::get_id();
-    const std::function<void()> work = [&] {
-        if (std::this_thread::get_id() == caller)  // while the helpers wake
-            for (; queued < r.chunks.size(); ++queued) r.queue_fetch((int64_t)queued);
-        r.fetch_parts();
-    };
-    // The values may be behind a whole solve: until the first part lands the
-    // call holds kAheadChunks chunks, and one thread waits.  (With all of them
-    // and the helpers from the start, a solve of 4.2M nodes and 300 iterations
-    // kept 8.0 cores spinning, and half of the process's chunks from others.)
+    const std::function<void()> work = [&] { r.fetch_parts(); };
+    // Values behind a whole solve: until they are due the call holds
+    // kAheadChunks chunks, and one thread waits.  (With all of them and the
+    // helpers from the start, a solve of 4.2M nodes and 300 iterations kept 8.0
+    // cores spinning, and half of the process's chunks from others.)
     const size_t part = largest(r.parts);
-    if (begin_run(r, r.parts.size(), part, s, kAheadChunks) != 0) {
+    if (begin_run(r, r.parts.size(), part, s, due.soon ? kAheadChunks : kCallChunks) != 0) {
         // no pinned memory: through a pageable buffer
         std::vector<char> buf(kChunkBytes);
         for (const Part& p : r.parts) {
@@ -485,14 +472,19 @@ int fetch_chunked(const std::vector<Fetch>& jobs, size_t total_bytes, hipStream_
         }
         return EGX_SUCC;
     }
+    size_t queued = 0;
     for (; queued < r.chunks.size(); ++queued) r.queue_fetch((int64_t)queued);
     if (r.parts.size() == 1) {
         work();
-    } else if (r.landed(r.chunks[0])) {
+        return finish_run(r);
+    }
+    if (due.soon) {
+        if (!r.landed(r.chunks[0], due)) return finish_run(r);
         const size_t all = std::min<size_t>(r.parts.size(), kCallChunks);
         if (all > queued) add_chunks(r, all - queued, part);
-        run_together(work, (int)std::min<size_t>(r.parts.size(), kThreads) - 1);
+        for (; queued < r.chunks.size(); ++queued) r.queue_fetch((int64_t)queued);
     }
+    run_together(work, (int)std::min<size_t>(r.parts.size(), kThreads) - 1);
     return finish_run(r);
 }
 
@@ -546,11 +538,11 @@ int DirectFetch::finish(const Fetch& f) {
     return rc;
 }
 
-int fetch(const std::vector<Fetch>& jobs, hipStream_t s) {
+int fetch(const std::vector<Fetch>& jobs, hipStream_t s, const Due& due) {
     size_t total = 0;
     for (const Fetch& f : jobs) total += (size_t)f.n * (f.packed ? 4 : 8);
     try {
-        return fetch_chunked(jobs, total, s);
+        return fetch_chunked(jobs, total, s, due);
     } catch (const std::bad_alloc&) {
         set_last_error("host transfer: out of host memory");
         return EGX_FAILED_TO_ALLOCATE_HOST_MEM;
